@@ -1,16 +1,20 @@
-"""Builds libsglamd.so (the torch-free C-ABI library) for gfx950 with hipcc, in-tree.
+"""Builds, in-tree, libsglamd.so (the torch-free C-ABI library) for gfx950 with hipcc, and _C.so (the operators and
+whole-call functions on top of it, host.cpp) with the host compiler against torch's headers.
 
 Usage: python sglang_amd/csrc/build.py [-j N]   (run by path: importing the package needs the built library)
 """
+import importlib.util
 import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB_PATH = os.path.join(PKG, "libsglamd.so")
+HOST_PATH = os.path.join(PKG, "_C.so")
 SOURCES = ["gemm_mode_block_fp8.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
            "moe.hip", "quant.hip", "gemm.hip", "generic.hip", "ceilings.hip"]
 # packed fp32 ALU forms are switched off on purpose (the -Xclang -target-feature pair below)
@@ -66,6 +70,20 @@ def _require_complete_report(src: str, table) -> None:
         raise RuntimeError(f"{src}: no VGPR or scratch figure in the compiler's remarks for: " + ", ".join(unread))
 
 
+def _host_flags():
+    """Compile and link flags of host.cpp.  The library is found by its soname, so a copy that the process has loaded
+    from elsewhere (SGLAMD_LIBRARY) serves both; otherwise it is the one beside _C.so."""
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    include = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+               os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    compile_flags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+                     "-DTORCH_EXTENSION_NAME=_C", "-DTORCH_API_INCLUDE_EXTENSION_H", *("-isystem" + d for d in include)]
+    link_flags = ["-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+                  "-L" + PKG, "-l:libsglamd.so", "-Wl,-rpath,$ORIGIN"]
+    return compile_flags, link_flags
+
+
 def build(jobs: int = 4, verbose: bool = True) -> str:
     hipcc = _hipcc()
     objdir = os.path.join(HERE, "build")
@@ -92,16 +110,27 @@ def build(jobs: int = 4, verbose: bool = True) -> str:
                                + ", ".join(f"{row[0]} ({row[4]} B/lane)" for row in spilling))
         return obj
 
+    gxx = os.environ.get("CXX", "g++")
+    host_compile, host_link = _host_flags()
+    host_obj = os.path.join(objdir, "host.o")
+
+    def run(what, cmd):
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"{what} failed:\n{r.stdout}\n{r.stderr}")
+
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        host = ex.submit(run, "g++ for host.cpp", [gxx, *host_compile, "-c", os.path.join(HERE, "host.cpp"), "-o", host_obj])
         objs = list(ex.map(compile_one, srcs))
+        host.result()
     tmp = LIB_PATH + ".tmp"
-    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    run("link", [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname,libsglamd.so", "-o", tmp, *objs])
     os.replace(tmp, LIB_PATH)
+    tmp = HOST_PATH + ".tmp"
+    run("link of _C.so", [gxx, "-shared", "-o", tmp, host_obj, *host_link])
+    os.replace(tmp, HOST_PATH)
     if verbose:
-        print(f"built {LIB_PATH} from {srcs}", file=sys.stderr)
+        print(f"built {LIB_PATH} from {srcs} and {HOST_PATH}", file=sys.stderr)
     return LIB_PATH
 
 

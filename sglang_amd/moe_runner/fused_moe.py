@@ -332,6 +332,15 @@ _inplace_op = _register_custom_op(inplace_fused_experts, ["hidden_states"])
 _outplace_op = _register_custom_op(outplace_fused_experts, [])
 
 
+def _needs_operator(hidden_states: torch.Tensor) -> bool:
+    """Whether somebody has to see the layer as one operator node: a compiler or another tracing mode, a tensor
+    subclass, autograd.  Otherwise the function behind the operator is called as it is (the Python side of a custom
+    operator costs about 20 us a call, as much as a quarter of a one-token layer)."""
+    return (torch.compiler.is_compiling() or type(hidden_states) is not torch.Tensor
+            or torch._C._len_torch_dispatch_stack() > 0
+            or (hidden_states.requires_grad and torch.is_grad_enabled()))
+
+
 def fused_experts(
     hidden_states: torch.Tensor,
     w1: torch.Tensor,
@@ -360,18 +369,20 @@ def fused_experts(
     filter_expert = c.num_experts is None or c.num_experts != c.num_local_experts
     if c.inplace:
         assert not c.no_combine, "no combine + inplace makes no sense"
-        _inplace_op(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
-                    c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
-                    per_channel_quant, w1_scale, w2_scale, w1_zp, w2_zp, a1_scale, a2_scale, block_shape,
-                    c.routed_scaling_factor, c.gemm1_alpha, c.gemm1_clamp_limit, filter_expert,
-                    swiglu_limit=c.swiglu_limit)
+        layer = _inplace_op if _needs_operator(hidden_states) else inplace_fused_experts
+        layer(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
+              c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
+              per_channel_quant, w1_scale, w2_scale, w1_zp, w2_zp, a1_scale, a2_scale, block_shape,
+              c.routed_scaling_factor, c.gemm1_alpha, c.gemm1_clamp_limit, filter_expert,
+              swiglu_limit=c.swiglu_limit)
         return hidden_states
-    return _outplace_op(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
-                        c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
-                        per_channel_quant, w1_scale, w2_scale, w1_zp, w2_zp, a1_scale, a2_scale, block_shape,
-                        no_combine=c.no_combine, routed_scaling_factor=c.routed_scaling_factor,
-                        gemm1_alpha=c.gemm1_alpha, gemm1_limit=c.gemm1_clamp_limit, filter_expert=filter_expert,
-                        swiglu_limit=c.swiglu_limit)
+    layer = _outplace_op if _needs_operator(hidden_states) else outplace_fused_experts
+    return layer(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
+                 c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
+                 per_channel_quant, w1_scale, w2_scale, w1_zp, w2_zp, a1_scale, a2_scale, block_shape,
+                 no_combine=c.no_combine, routed_scaling_factor=c.routed_scaling_factor,
+                 gemm1_alpha=c.gemm1_alpha, gemm1_limit=c.gemm1_clamp_limit, filter_expert=filter_expert,
+                 swiglu_limit=c.swiglu_limit)
 
 
 def fused_moe(

@@ -9,6 +9,7 @@ from ..gemm import (
     sgl_per_token_group_quant_8bit,
     sgl_per_token_quant_fp8,
 )
+from ..ops import _C, block_scaled_mm_any_, static_quant_fp8_, tensor_absmax_scale_, ue8m0_unpack_, w8a8_block_fp8_matmul_
 
 fp8_dtype = torch.float8_e4m3fn
 fp8_max = 448.0
@@ -71,6 +72,11 @@ def sglang_per_token_group_quant_fp8(
     half its width.  `enable_v2=None` picks the second arithmetic for the group sizes it supports."""
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
+    if masked_m is None and enable_v2 is not False:
+        quantised = _C.group_quant_2d(x, group_size, eps, column_major_scales, scale_tma_aligned, scale_ue8m0,
+                                      fuse_silu_and_mul, False)
+        if quantised is not None:
+            return quantised
     width = x.shape[-1] // 2 if fuse_silu_and_mul else x.shape[-1]
     q_shape = x.shape[:-1] + (width,)
     x_q = x.new_empty(q_shape, dtype=fp8_dtype)
@@ -98,6 +104,10 @@ def sglang_per_token_group_quant_int8(x: torch.Tensor, group_size: int, eps: flo
     """int8 sibling (python/sglang/srt/layers/quantization/int8_kernel.py:184-225): row-major fp32 scales."""
     assert x.shape[-1] % group_size == 0
     assert x.is_contiguous()
+    if dtype == torch.int8 and enable_v2 is not False:
+        quantised = _C.group_quant_2d(x, group_size, eps, False, False, False, False, True)
+        if quantised is not None:
+            return quantised
     x_q = torch.empty_like(x, dtype=dtype)
     x_s = torch.empty(x.shape[:-1] + (x.shape[-1] // group_size,), device=x.device, dtype=torch.float32)
     if x.numel() > 0:
@@ -130,6 +140,10 @@ def sglang_per_token_group_quant_8bit(
 def sglang_per_token_quant_fp8(x: torch.Tensor, dtype: torch.dtype = fp8_dtype):
     """fp8_kernel.py:656-672: one scale per row, shape [rows, 1]."""
     assert x.is_contiguous(), "`x` is not contiguous"
+    if dtype == fp8_dtype:
+        quantised = _C.per_token_quant(x, False)
+        if quantised is not None:
+            return quantised
     x_q = x.new_empty(x.shape, dtype=dtype)
     x_s = x.new_empty((x.shape[0], 1), dtype=torch.float32)
     sgl_per_token_quant_fp8(x, x_q, x_s)
@@ -139,8 +153,6 @@ def sglang_per_token_quant_fp8(x: torch.Tensor, dtype: torch.dtype = fp8_dtype):
 def static_quant_fp8(x: torch.Tensor, x_s: torch.Tensor, repeat_scale: bool = False):
     """fp8_kernel.py:724-777: quantise with a given per-tensor scale, q = e4m3(clamp(x * (1 / x_s))); with
     `repeat_scale` the scale comes back broadcast to one per row, [rows, 1], as the row-scaled GEMM takes it."""
-    from ..ops import static_quant_fp8_
-
     assert x.is_contiguous(), "`x` is not contiguous"
     assert x_s.numel() == 1, "only supports per-tensor scale"
     x_q = torch.empty_like(x, dtype=fp8_dtype)
@@ -156,8 +168,6 @@ def scaled_fp8_quant(input: torch.Tensor, scale: Optional[torch.Tensor] = None,
     """fp8_kernel.py:1693-1777: FP8 quantisation of a 2D tensor with a given per-tensor scale (static), or with a
     scale computed here: one per token ([rows, 1]) or one for the tensor ([1], max|x| / 448).  The output has
     max(num_token_padding, rows) rows; rows past the input are left unwritten, as in the reference."""
-    from ..ops import static_quant_fp8_, tensor_absmax_scale_
-
     assert input.ndim == 2, f"Expected 2D input tensor, got {input.ndim}D"
     rows, hidden = input.shape
     out_rows = max(num_token_padding, rows) if num_token_padding else rows
@@ -226,14 +236,14 @@ def w8a8_block_fp8_matmul(A, B, As, Bs, block_size: List[int], output_dtype: tor
     (what the quantiser writes with scale_ue8m0=True; for the weights the same words on every row of a block)
     are expanded to the fp32 powers of two they stand for by one small launch each; when both operands came with
     such scales the GEMM is told so (the large-tile kernel then applies them inside the MFMA)."""
-    from ..ops import ue8m0_unpack_, w8a8_block_fp8_matmul_
-
+    if block_size[0] == 128 and block_size[1] == 128 and A.dtype == fp8_dtype:
+        out = _C.block_matmul(A, B, As, Bs, output_dtype, None)
+        if out is not None:
+            return out
     M, N, K, C = prepare_block_fp8_matmul_inputs(A, B, As, Bs, block_size, output_dtype)
     assert output_dtype in (torch.float16, torch.bfloat16)
     if list(block_size) != [128, 128]:
         # other scale-block shapes (the reference's kernel is generic in them): the generic kernel, float scales
-        from ..ops import block_scaled_mm_any_
-
         if not all(b in (64, 128) for b in block_size) or As.dtype != torch.float32 or Bs.dtype != torch.float32:
             raise NotImplementedError("scale blocks of 64 or 128 in each direction with float scales are implemented")
         As2 = As.reshape(M, As.shape[-1])

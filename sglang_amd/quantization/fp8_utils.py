@@ -5,6 +5,7 @@ from typing import Callable, List, Optional
 import torch
 
 from ..gemm import fp8_blockwise_scaled_mm, fp8_scaled_mm
+from ..ops import _C, tensor_absmax_scale_
 from .fp8_kernel import (
     per_token_group_quant_fp8,
     sglang_per_token_group_quant_fp8,
@@ -23,7 +24,16 @@ def _finish(out_2d: torch.Tensor, input: torch.Tensor, bias, dtype: torch.dtype)
     """Add the bias in place and restore the activation's leading dimensions."""
     if bias is not None:
         out_2d += bias
-    return out_2d.to(dtype).view(*input.shape[:-1], out_2d.shape[-1])
+    out_2d = out_2d.to(dtype)
+    return out_2d if input.dim() == 2 else out_2d.view(*input.shape[:-1], out_2d.shape[-1])
+
+
+def _plain_block_linear(x, weight, block_size, weight_scale, bias):
+    """The layer in one native call where its configuration is the plain one (128x128 scale blocks, whole groups of
+    128 columns); None otherwise."""
+    if block_size[0] != 128 or block_size[1] != 128:
+        return None
+    return _C.block_linear(x, weight, weight_scale, bias)
 
 
 def _dynamic_block_quant_only(input_scale, block_size) -> None:
@@ -39,6 +49,10 @@ def triton_w8a8_block_fp8_linear(input, weight, block_size: List[int], weight_sc
     """Row-major-scale variant (fp8_utils.py:814-834); accepts N, K that are not multiples of 128."""
     _dynamic_block_quant_only(input_scale, block_size)
     x = _rows(input)
+    if weight_scale.dtype == torch.float32:
+        out = _plain_block_linear(x, weight, block_size, weight_scale, bias)
+        if out is not None:
+            return _finish(out, input, None, x.dtype)
     x_q, x_scale = per_token_group_quant_fp8(x, block_size[1], column_major_scales=False)
     out = w8a8_block_fp8_matmul(x_q, weight, x_scale, weight_scale, block_size, output_dtype=x.dtype)
     return _finish(out, input, bias, x.dtype)
@@ -51,10 +65,13 @@ def cutlass_w8a8_block_fp8_linear_with_fallback(input, weight, block_size: List[
     _dynamic_block_quant_only(input_scale, block_size)
     if weight_scale.dtype == torch.int32:
         return deepgemm_w8a8_block_fp8_linear_with_fallback(input, weight, block_size, weight_scale, None, bias)
+    x = _rows(input)
+    out = _plain_block_linear(x, weight, block_size, weight_scale, bias)
+    if out is not None:
+        return _finish(out, input, None, x.dtype)
     n, k = weight.shape
     if n % 128 or k % 128 or list(block_size) != [128, 128]:
         return triton_w8a8_block_fp8_linear(input, weight, block_size, weight_scale, input_scale, bias)
-    x = _rows(input)
     x_q, x_scale = per_token_group_quant_fp8(x, block_size[1], column_major_scales=True)
     out = fp8_blockwise_scaled_mm(x_q, weight.T, x_scale, weight_scale.T, out_dtype=x.dtype)
     return _finish(out, input, bias, x.dtype)
@@ -70,6 +87,9 @@ def deepgemm_w8a8_block_fp8_linear_with_fallback(input, weight, block_size: List
     if weight_scale.dtype != torch.int32:
         return cutlass_w8a8_block_fp8_linear_with_fallback(input, weight, block_size, weight_scale, None, bias)
     x = _rows(input)
+    out = _plain_block_linear(x, weight, block_size, weight_scale, bias)
+    if out is not None:
+        return _finish(out, input, None, x.dtype)
     x_q, x_scale = sglang_per_token_group_quant_fp8(x, block_size[1], column_major_scales=True,
                                                     scale_tma_aligned=True, scale_ue8m0=True)
     out = w8a8_block_fp8_matmul(x_q, weight, x_scale, weight_scale, block_size, output_dtype=x.dtype)
@@ -88,8 +108,11 @@ def aiter_w8a8_block_fp8_linear(input, weight, block_size: List[int], weight_sca
     x_q = _rows(input)
     if input_scale.numel() != x_q.shape[0] * (-(-x_q.shape[1] // 128)):
         raise NotImplementedError("the input scale must hold one value per row and 128 columns")
-    out = w8a8_block_fp8_matmul(x_q, weight, input_scale.view(x_q.shape[0], -1), weight_scale, block_size,
-                                output_dtype=torch.bfloat16)
+    input_scale = input_scale.view(x_q.shape[0], -1)
+    out = _C.block_matmul(x_q, weight, input_scale, weight_scale, torch.bfloat16, bias)
+    if out is not None:
+        return _finish(out, input, None, torch.bfloat16)
+    out = w8a8_block_fp8_matmul(x_q, weight, input_scale, weight_scale, block_size, output_dtype=torch.bfloat16)
     return _finish(out, input, bias, torch.bfloat16)
 
 
@@ -126,12 +149,13 @@ def apply_fp8_linear(input, weight, weight_scale, input_scale=None, input_scale_
         x_q, x_scale = static_quant_fp8(x, input_scale, repeat_scale=True)
     elif per_tensor_dynamic:
         # max|x| / 448 computed on the device, then broadcast to the rows like a static scale
-        from ..ops import tensor_absmax_scale_
-
         scale = torch.empty(1, device=x.device, dtype=torch.float32)
         tensor_absmax_scale_(x if x.is_contiguous() else x.contiguous(), scale)
         x_q, x_scale = static_quant_fp8(x, scale, repeat_scale=True)
     else:
+        out = _C.row_linear(x, weight, weight_scale, bias)
+        if out is not None:
+            return _finish(out, input, None, input.dtype)
         x_q, x_scale = sglang_per_token_quant_fp8(x)
     w_scale = weight_scale.reshape(-1).to(torch.float32)
     if w_scale.numel() == 1:
