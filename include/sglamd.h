@@ -399,6 +399,18 @@ int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t M, int64_t
                                float routed_scaling_factor, int block_m, void* workspace, int64_t workspace_bytes,
                                void* stream);
 
+/* The same layer for every weight format the path has (triton_utils/fused_moe.py:401-785 with use_fp8_w8a8 /
+ * use_int8_w8a8): block scales as above, or row scales -- activations quantised per token, w13_scale [E, 2I] and
+ * w2_scale [E, H] one float per output channel, optional biases b13 [E, 2I] and b2 [E, H] in `dtype` (null without).
+ * Row-scaled layers take H and I up to 32768 and matrices below 2 GiB.  block_m: 0, 16, 32, 64, 128 or 192. */
+enum { SGLAMD_MOE_BLOCK_FP8 = 0, SGLAMD_MOE_ROW_FP8 = 1, SGLAMD_MOE_ROW_INT8 = 2, SGLAMD_MOE_BLOCK_INT8 = 3 };
+int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk, int block_m);
+int sglamd_fused_moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E, int topk,
+                           const void* w13, const float* w13_scale, const void* b13, const void* w2,
+                           const float* w2_scale, const void* b2, const float* topk_weights, const void* topk_ids,
+                           int ids_dtype, void* out, float routed_scaling_factor, int block_m, void* workspace,
+                           int64_t workspace_bytes, void* stream);
+
 /* sglamd_fused_moe_block_fp8 for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and results
  * as sglamd_fused_moe_block_fp8, without the workspace: the intermediates live in a 16 MiB device array that is

@@ -16,7 +16,7 @@ PKG = os.path.dirname(HERE)
 LIB_PATH = os.path.join(PKG, "libsglamd.so")
 HOST_PATH = os.path.join(PKG, "_C.so")
 SOURCES = ["gemm_mode_block_fp8.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
-           "moe.hip", "quant.hip", "gemm.hip", "generic.hip", "ceilings.hip"]
+           "moe.hip", "moe_rows.hip", "quant.hip", "gemm.hip", "generic.hip", "ceilings.hip"]
 # packed fp32 ALU forms are switched off on purpose (the -Xclang -target-feature pair below)
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -31,7 +31,7 @@ HIPCC_FLAGS = [
 # and the compiler spills accumulators into scratch memory, which still computes the right result, two to ten
 # times slower.  A build in which a kernel of these files uses scratch memory therefore fails.
 NO_SCRATCH = {"gemm_mode_block_fp8.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
-              "moe.hip"}
+              "moe.hip", "moe_rows.hip"}
 
 
 def _hipcc() -> str:

@@ -497,6 +497,8 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   // row modes: the weight-row scales (and bias) of this lane's 32 columns, fetched once for all row tiles
   float sbn[2][4][4], bia[2][4][4];
   if constexpr (!gemm_is_block(MODE)) {
+    const float* sb_row = g.sb + (MOE ? (int64_t)max(expert, 0) * g.sb_se : 0);
+    const OS* bias = g.bias ? (const OS*)g.bias + (MOE ? (int64_t)max(expert, 0) * g.sb_sk : 0) : nullptr;
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -504,8 +506,8 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           const int nn = min(n0 + wn * 64 + j * 32 + 8 * rq + 4 * fk + r, (int)g.N - 1);
-          sbn[j][rq][r] = g.sb[nn];
-          bia[j][rq][r] = g.bias ? OT::to_f32(((const OS*)g.bias)[nn]) : 0.f;
+          sbn[j][rq][r] = sb_row[MOE ? (int64_t)nn * g.sb_sn : nn];
+          bia[j][rq][r] = bias ? OT::to_f32(bias[nn]) : 0.f;
         }
   }
 #pragma unroll
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       m = min(m, (int)g.M - 1);
     }
     float sam = 1.f;
-    if (!gemm_is_block(MODE)) sam = g.sa[m];
+    if (!gemm_is_block(MODE)) sam = g.sa[MOE ? (int64_t)(m / g.top_k) * g.sa_sm : m];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
 #pragma unroll
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
         const int cl = wn * 64 + j * 32 + 8 * rq + 4 * fk;
         float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = (float)acc[i][j][rq * 4 + r] * wgt;
+        for (int r = 0; r < 4; r++) v[r] = (float)acc[i][j][rq * 4 + r];
         if constexpr (!gemm_is_block(MODE)) {
 #pragma unroll
           for (int r = 0; r < 4; r++) {
@@ -538,6 +540,10 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
             else v[r] = v[r] * (sbn[j][rq][r] * sam);
             if (g.bias) v[r] += bia[j][rq][r];
           }
+        }
+        if (MOE) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] *= wgt;
         }
         const v2i w = {(int)OT::pack2(v[0], v[1]), (int)OT::pack2(v[2], v[3])};
         *(v2i*)(smem + rl * CROW + cl * 2) = w;

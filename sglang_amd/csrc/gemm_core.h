@@ -36,6 +36,8 @@ struct GemmArgs {
   int64_t sa_sm, sa_sk;
   const float* sb;          // block: sb[e*sb_se + nb*sb_sn + kb*sb_sk]; rowwise: sb[n]
   int64_t sb_sn, sb_sk, sb_se;
+  // rowwise MoE: sa[(slot / top_k) * sa_sm] (0: per tensor), sb[e*sb_se + n*sb_sn] (sb_sn 0: per expert), and the
+  // bias rows of the experts lie sb_sk elements apart
   const void* bias;         // rowwise, optional, [N] in the output dtype
   void* C;
   int64_t ldc;

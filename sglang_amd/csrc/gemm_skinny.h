@@ -629,19 +629,27 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       if (!row_ok || n >= o_n_end) continue;
       float v[4];
       float sam = 1.f;
-      if (!gemm_is_block(MODE)) sam = g.sa[out_row];
+      const float* sb_row = g.sb;
+      const OS* bias = (const OS*)g.bias;
+      if constexpr (!gemm_is_block(MODE)) {
+        sam = g.sa[MOE ? (out_row / g.top_k) * g.sa_sm : out_row];
+        if (MOE) {
+          sb_row += (int64_t)max(o_expert, 0) * g.sb_se;
+          if (bias) bias += (int64_t)max(o_expert, 0) * g.sb_sk;
+        }
+      }
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         if constexpr (gemm_is_block(MODE)) {
           v[r] = a[r];
         } else {
-          const float sbn = (n + r) < g.N ? g.sb[n + r] : 0.f;
+          const float sbn = (n + r) < g.N ? sb_row[MOE ? (int64_t)(n + r) * g.sb_sn : n + r] : 0.f;
           if constexpr (MODE == GEMM_ROW_FP8) {
             v[r] = a[r] * sbn * sam;
           } else {
             v[r] = (float)a[r] * (sbn * sam);
           }
-          if (g.bias) v[r] += OT::to_f32(((const OS*)g.bias)[(n + r) < g.N ? n + r : 0]);
+          if (bias) v[r] += OT::to_f32(bias[(n + r) < g.N ? n + r : 0]);
         }
         if (MOE) {
           if (o_expert < 0) v[r] = 0.f;

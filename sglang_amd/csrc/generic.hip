@@ -4,7 +4,7 @@
 // Also the sigmoid router (topk_sigmoid), the twin of topk_softmax in moe.hip.
 #include <math.h>
 
-#include "gemm_core.h"
+#include "moe_dispatch.h"
 
 namespace sglamd {
 
@@ -295,6 +295,11 @@ extern "C" int sglamd_fused_moe_gemm_any(const void* a, int64_t lda, const float
   hipStream_t st = (hipStream_t)stream;
   const GemmArgsX gx = {g, GemmExt{block_n, block_k, as_stride_m, ws_stride_n, bias_stride_e}};
   if (row) {
+    if (moe_rows_ok(g)) {
+      GemmArgs r = g;
+      r.sb_sk = bias_stride_e;  // row modes: where GemmArgs keeps it
+      return moe_rows_gemm(q_dtype == SGLAMD_I8 ? GEMM_ROW_INT8 : GEMM_ROW_FP8, r, out_dtype, block_m, st);
+    }
     if (q_dtype == SGLAMD_I8) return generic_out<GEMM_ROW_INT8, true>(gx, block_m, out_dtype, st);
     return generic_out<GEMM_ROW_FP8, true>(gx, block_m, out_dtype, st);
   }

@@ -973,6 +973,58 @@ void fused_moe_block_fp8_(const Tensor& hidden, const Tensor& w1, const Tensor& 
                                    ws.numel() * ws.element_size(), stream_of(hidden)));
 }
 
+// The whole MoE layer (fused_moe.py:401-785) for gated SiLU experts in one of the four weight formats: 128x128 block
+// scales (block = true) or one scale per output channel, e4m3fn or int8.  block_m: 0 for the library's choice.
+optional<Tensor> moe_layer(const Tensor& hidden, const Tensor& w1, const Tensor& w2, const optional<Tensor>& w1_scale,
+                           const optional<Tensor>& w2_scale, const optional<Tensor>& b1, const optional<Tensor>& b2,
+                           const Tensor& topk_weights, const Tensor& topk_ids, bool block, bool int8, bool inplace,
+                           double routed_scaling_factor, int64_t block_m) {
+  const ScalarType t = hidden.scalar_type(), wt = int8 ? at::kChar : kFp8;
+  if (hidden.dim() != 2 || !hidden.is_cuda() || !is_half(t) || !hidden.is_contiguous() || hidden.size(0) == 0) return {};
+  const int64_t m = hidden.size(0), h = hidden.size(1);
+  if (w1.dim() != 3 || w2.dim() != 3 || w1.scalar_type() != wt || w2.scalar_type() != wt || !w1.is_contiguous() ||
+      !w2.is_contiguous() || w1.device() != hidden.device() || w2.device() != hidden.device())
+    return {};
+  const int64_t e = w1.size(0), n2 = w1.size(1), i = n2 / 2;
+  if (w1.size(2) != h || w2.size(0) != e || w2.size(1) != h || w2.size(2) != i || h % 128 || n2 % 256 || e + 1 > 2048 ||
+      h == 0 || n2 == 0)
+    return {};
+  auto plain_scale = [&](const optional<Tensor>& s, int64_t n, int64_t k) {
+    if (!s || s->scalar_type() != at::kFloat || !s->is_contiguous() || s->device() != hidden.device()) return false;
+    if (!block) return s->numel() == e * n;
+    return s->dim() == 3 && s->size(0) == e && s->size(1) == n / 128 && s->size(2) == k / 128;
+  };
+  if (!plain_scale(w1_scale, n2, h) || !plain_scale(w2_scale, h, i)) return {};
+  if (block && (b1 || b2)) return {};
+  // row-scaled layers: whole rows in registers, matrices behind 32-bit buffer offsets
+  if (!block && (h > 32768 || i > 32768 || n2 * h >= 0x7ffffff0ll || m * h >= 0x7ffffff0ll || m * topk_ids.size(-1) * i >= 0x7ffffff0ll))
+    return {};
+  auto plain_expert_bias = [&](const optional<Tensor>& b, int64_t n) {
+    return !b || (b->dim() == 2 && b->size(0) == e && b->size(1) == n && b->is_contiguous() && b->scalar_type() == t &&
+                  b->device() == hidden.device());
+  };
+  if (!plain_expert_bias(b1, n2) || !plain_expert_bias(b2, h)) return {};
+  if (topk_ids.dim() != 2 || topk_ids.sizes() != topk_weights.sizes() || topk_ids.size(0) != m || topk_ids.size(1) == 0 ||
+      topk_ids.device() != hidden.device() || topk_weights.device() != hidden.device() ||
+      (topk_ids.scalar_type() != at::kInt && topk_ids.scalar_type() != at::kLong))
+    return {};
+  const int64_t topk = topk_ids.size(1);
+  if (m * topk >= (1ll << 30)) return {};
+  const c10::DeviceGuard guard(hidden.device());
+  const Tensor tw = topk_weights.to(at::kFloat).contiguous(), ids = topk_ids.contiguous();
+  Tensor out = inplace ? hidden : empty({m, h}, t, hidden);
+  const int mode = block ? (int8 ? SGLAMD_MOE_BLOCK_INT8 : SGLAMD_MOE_BLOCK_FP8)
+                         : (int8 ? SGLAMD_MOE_ROW_INT8 : SGLAMD_MOE_ROW_FP8);
+  const int64_t need = sglamd_fused_moe_layer_workspace(mode, m, h, i, (int)e, (int)topk, (int)block_m);
+  const Tensor ws = empty({need}, at::kByte, hidden);
+  check(sglamd_fused_moe_layer(mode, hidden.data_ptr(), tag(t), m, h, i, (int)e, (int)topk, w1.data_ptr(),
+                               w1_scale->data_ptr<float>(), b1 ? b1->data_ptr() : nullptr, w2.data_ptr(),
+                               w2_scale->data_ptr<float>(), b2 ? b2->data_ptr() : nullptr, tw.data_ptr<float>(),
+                               ids.data_ptr(), tag(ids.scalar_type()), out.data_ptr(), (float)routed_scaling_factor,
+                               (int)block_m, ws.data_ptr(), need, stream_of(hidden)));
+  return out;
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(sgl_kernel, m) {
@@ -1072,6 +1124,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_moe_block_fp8_", &fused_moe_block_fp8_, Unlocked(), py::arg("hidden_states"), py::arg("w1"), py::arg("w2"),
         py::arg("w1_scale"), py::arg("w2_scale"), py::arg("topk_weights"), py::arg("topk_ids"), py::arg("out"),
         py::arg("routed_scaling_factor"), py::arg("block_m") = 0, py::arg("workspace") = py::none());
+  m.def("moe_layer", &moe_layer, Unlocked());
   m.def("fused_moe_block_fp8_workspace_bytes",
         [](int64_t m_, int64_t h, int64_t i, int64_t e, int64_t topk, int64_t block_m) {
           return sglamd_fused_moe_block_fp8_workspace(m_, h, i, (int)e, (int)topk, (int)block_m);

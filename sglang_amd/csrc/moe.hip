@@ -2,9 +2,7 @@
 // block-padded expert spans), the sorted-block grouped block-FP8 GEMM (same MFMA core as
 // the dense GEMM, rows gathered through the sorted token list), silu_and_mul and the
 // top-k sum reduce.
-#include "gemm_big.h"
-#include "gemm_big_moe_persist.h"
-#include "gemm_skinny.h"
+#include "moe_dispatch.h"
 #include "quant_core.h"
 
 namespace sglamd {
@@ -249,6 +247,20 @@ __global__ __launch_bounds__(1024) void moe_prologue_kernel(const IdT* __restric
   } else {
     group_quant_body<T, 128>(qa, (int64_t)((int)blockIdx.x - parts) * 1024 + threadIdx.x);
   }
+}
+
+// The same for the row-scaled layers: one row of hidden states per workgroup behind the sorting ones.
+template <typename IdT, typename T, bool INT8, int NV>
+__global__ __launch_bounds__(1024) void moe_row_prologue_kernel(const IdT* __restrict__ topk_ids, int32_t* sorted_ids,
+                                                                int32_t* expert_ids, int32_t* post_pad_out,
+                                                                int32_t* cumsum_out, int nb, int block_size, int numel,
+                                                                int max_padded, int parts, RowQuantArgs qa) {
+  __shared__ float red[16];
+  if ((int)blockIdx.x < parts)
+    moe_align_body<IdT>(topk_ids, sorted_ids, expert_ids, post_pad_out, cumsum_out, nb, block_size, numel, 1, max_padded,
+                        (int)blockIdx.x, parts);
+  else
+    row_quant_body<T, INT8, false, NV>(qa, (int)blockIdx.x - parts, red);
 }
 
 // prepare_moe_input: the stable sort above with block size 1, emitting permutations and problem sizes.
@@ -517,78 +529,10 @@ __global__ __launch_bounds__(256) void moe_sum_reduce_kernel(const u16* __restri
   }
 }
 
-// tuning knob: SGLAMD_MOE_PERSIST=0 runs the tall sorted blocks one tile per workgroup instead of the persistent walk
-static inline bool moe_persist_enabled() {
-  static const int v = getenv("SGLAMD_MOE_PERSIST") ? atoi(getenv("SGLAMD_MOE_PERSIST")) : 1;
-  return v != 0;
-}
-
-// tuning knob: SGLAMD_MOE_PERSIST128=0 keeps the 128-slot sorted blocks with one tile per workgroup
-static inline bool moe_persist128_enabled() {
-  static const int v = getenv("SGLAMD_MOE_PERSIST128") ? atoi(getenv("SGLAMD_MOE_PERSIST128")) : 1;
-  return v != 0 && moe_persist_enabled();
-}
-
 // tuning knob: SGLAMD_MOE_ACTQ=0 keeps SiLU * up and its quantisation a launch of their own behind the first GEMM
 static bool moe_actq_enabled() {
   static const int v = getenv("SGLAMD_MOE_ACTQ") ? atoi(getenv("SGLAMD_MOE_ACTQ")) : 1;
   return v != 0;
-}
-
-// The persistent walk hands out tiles by position, not by arrival.  A sorted block that is an expert's second one
-// finds the weights its first block has just streamed in L2 and finishes in half the time, and a fixed walk cannot
-// balance that the way the dispatch order of a one-tile-per-workgroup launch does; until the tiles went to XCDs in
-// contiguous ranges the walk therefore lost 5 % where half of the experts own one block and half two (6144 tokens
-// on the DeepSeek-V3 layer) and was only used where every expert owns the same number.  With an expert's blocks
-// meeting in one L2 it is level or ahead at every token count measured (3072 ... 12288: 0 ... -5.5 %), so it runs
-// wherever there are more tiles than CUs.
-template <int MODE, typename OT>
-static int dispatch_moe_gemm(const GemmArgs& g, int block_m, hipStream_t st) {
-  // number of sorted blocks that will actually run is data dependent; every valid slot could own one
-  const int64_t expect = g.num_valid < g.max_blocks_m ? g.num_valid : g.max_blocks_m;
-  const bool streaming_ok = gemm8_skinny_ok(g, g.num_valid / g.top_k);
-  switch (block_m) {
-    case 16:
-      if (streaming_ok) return gemm8_skinny_launch<1, MODE, OT, true>(g, st, expect);
-      return gemm8_launch<16, 128, 1, 2, MODE, OT, true>(g, st);  // operands of 2 GiB and more
-    case 32:
-      if (streaming_ok) return gemm8_skinny_launch<2, MODE, OT, true>(g, st, expect);
-      return gemm8_launch<32, 128, 1, 2, MODE, OT, true>(g, st);
-    case 64:
-      // the tile kernel with one 32-row tile per wave when its preconditions hold: the streaming kernel spends
-      // four MFMA row groups per weight fragment and falls far behind it at this height
-      if ((g.K % 128) == 0 && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll &&
-          (int64_t)g.N * g.ldb < 0x7fffffffll)
-        // (the persistent walk with its two stages is 12 % behind this kernel's three at this height)
-        return gemm8_big_moe_launch<MODE, OT, 1>(g, st);
-      if (streaming_ok) return gemm8_skinny_launch<4, MODE, OT, true>(g, st, expect);
-      return gemm8_launch<64, 128, 2, 2, MODE, OT, true>(g, st);
-    case 128:
-      // 32x32x64-MFMA tile kernel when its preconditions hold (K % 128 == 0, operands below 2 GiB per matrix)
-      if ((g.K % 128) == 0 && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll &&
-          (int64_t)g.N * g.ldb < 0x7fffffffll)
-      {
-        // more tiles than CUs: the persistent walk, as for the 192-slot blocks
-        if (moe_persist128_enabled() && gemm8_moe_persist_ok(g) &&
-            (int64_t)((g.N + 255) / 256) * g.max_blocks_m > device_cus())
-          return gemm8_moe_persist_launch<MODE, OT, 2>(g, st);
-        return gemm8_big_moe_launch<MODE, OT>(g, st);
-      }
-      return gemm8_launch<128, 128, 2, 2, MODE, OT, true>(g, st);
-    case 192:
-      // one block per expert when an expert gets 129..192 rows: its weights are streamed once
-      SGLAMD_REQUIRE((g.K % 128) == 0 && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll &&
-                         (int64_t)g.N * g.ldb < 0x7fffffffll,
-                     SGLAMD_EINVAL, "fused_moe_gemm: block_m 192 needs K %% 128 == 0 and operands below 2 GiB");
-      // more tiles than CUs: one workgroup per CU walks them and requests a tile's first blocks under the
-      // epilogue of the tile before
-      if (moe_persist_enabled() && gemm8_moe_persist_ok(g) &&
-          (int64_t)((g.N + 255) / 256) * g.max_blocks_m > device_cus())
-        return gemm8_moe_persist_launch<MODE, OT, 3>(g, st);
-      return gemm8_big_moe_launch<MODE, OT, 3>(g, st);
-    default:
-      return fail(SGLAMD_EINVAL, "fused_moe_gemm: block_m must be 16, 32, 64, 128 or 192 (got %d)", block_m);
-  }
 }
 
 }  // namespace sglamd
@@ -958,6 +902,10 @@ extern "C" int sglamd_fp8_blockwise_scaled_grouped_mm(void* output, int out_dtyp
 // Five launches on one stream (four for up to four tokens, three for one); all intermediates live in the
 // caller's workspace.
 // ---------------------------------------------------------------------------------------
+static_assert(GEMM_BLOCK_FP8 == (int)SGLAMD_MOE_BLOCK_FP8 && GEMM_ROW_FP8 == (int)SGLAMD_MOE_ROW_FP8 &&
+                  GEMM_ROW_INT8 == (int)SGLAMD_MOE_ROW_INT8 && GEMM_BLOCK_INT8 == (int)SGLAMD_MOE_BLOCK_INT8,
+              "the ABI's layer modes are the GEMM modes");
+
 namespace {
 struct MoeWs {
   int64_t sorted, expert, post, cumsum, xq, xs, c1, aq, as, c3, total;
@@ -1005,6 +953,17 @@ int moe_auto_block(int64_t M, int E, int topk) {
   if (rows <= 104) return 128;
   return 192;
 }
+// The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue, so what counts is how
+// few rows a tile pads: the shortest block that still holds a whole expert (its weights are streamed once).
+int moe_auto_block_rows(int64_t M, int E, int topk) {
+  static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;
+  if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
+  const double rows = (double)M * topk / (E > 0 ? E : 1);
+  if (rows <= 10) return 16;
+  if (rows <= 56) return 64;
+  if (rows <= 112) return 128;
+  return 192;
+}
 int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1); }
 }  // namespace
 
@@ -1014,11 +973,19 @@ extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, in
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
-extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E,
-                                          int topk, const void* w13, const float* w13_scale, const void* w2,
-                                          const float* w2_scale, const float* topk_weights, const void* topk_ids,
-                                          int ids_dtype, void* out, float routed_scaling_factor, int block_m,
-                                          void* workspace, int64_t workspace_bytes, void* stream) {
+extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk,
+                                                    int block_m) {
+  if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
+  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk) : moe_auto_block_rows(M, E, topk);
+  return moe_ws_layout(M, H, I, E, topk, block_m).total;
+}
+
+// `mode` is a GEMM_* mode: the two block-scaled ones with [E, 2I/128, H/128] and [E, H/128, I/128] scales, the two
+// row-scaled ones with one scale per output channel ([E, 2I], [E, H]) and optional biases of that shape in `dtype`.
+static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E, int topk,
+                     const void* w13, const float* w13_scale, const void* b13, const void* w2, const float* w2_scale,
+                     const void* b2, const float* topk_weights, const void* topk_ids, int ids_dtype, void* out,
+                     float routed_scaling_factor, int block_m, void* workspace, int64_t workspace_bytes, void* stream) {
   SGLAMD_REQUIRE(hidden && w13 && w13_scale && w2 && w2_scale && topk_weights && topk_ids && out && workspace,
                  SGLAMD_EINVAL, "fused_moe: null pointer");
   SGLAMD_REQUIRE(M > 0 && E > 0 && topk > 0, SGLAMD_EINVAL, "fused_moe: bad M/E/topk");
@@ -1026,7 +993,13 @@ extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t
                  "fused_moe: hidden (%lld) and intermediate (%lld) sizes must be multiples of 128", (long long)H,
                  (long long)I);
   SGLAMD_REQUIRE(dtype == SGLAMD_BF16 || dtype == SGLAMD_F16, SGLAMD_EINVAL, "fused_moe: dtype must be Half or BFloat16");
-  if (block_m == 0) block_m = moe_auto_block(M, E, topk);
+  const bool row = !gemm_is_block(mode), int8 = gemm_is_int8(mode);
+  SGLAMD_REQUIRE(!row || H <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: hidden size %lld is beyond %lld",
+                 (long long)H, (long long)ROW_QUANT_MAX_HIDDEN);
+  SGLAMD_REQUIRE(!row || I <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: intermediate size %lld is beyond %lld",
+                 (long long)I, (long long)ROW_QUANT_MAX_HIDDEN);
+  SGLAMD_REQUIRE(row || (!b13 && !b2), SGLAMD_ENOTSUP, "fused_moe: biases go with row-scaled weights");
+  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk) : moe_auto_block(M, E, topk);
   SGLAMD_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128 || block_m == 192, SGLAMD_EINVAL,
                  "fused_moe: block_m must be 16, 32, 64, 128 or 192");
   const MoeWs w = moe_ws_layout(M, H, I, E, topk, block_m);
@@ -1053,10 +1026,97 @@ extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t
   // bytes each would crowd the weight rings out of LDS: measured 150 against 120 us at two tokens).  Every variant produces the bits of the five-launch sequence.
   // SGLAMD_MOE_FUSE=1 keeps the launch in front, SGLAMD_MOE_FUSE=0 the whole sequence.
   static const int fuse_level = getenv("SGLAMD_MOE_FUSE") ? atoi(getenv("SGLAMD_MOE_FUSE")) : 2;
-  const bool fuse_act = fuse_level >= 1 && block_m == 16 && M <= 4 && T <= 32 && I % 256 == 0 &&
+  const bool fuse_act = mode == GEMM_BLOCK_FP8 && fuse_level >= 1 && block_m == 16 && M <= 4 && T <= 32 && I % 256 == 0 &&
                         M * H * 2 < 0x7ffffff0ll && 2 * I * H < 0x7ffffff0ll && T * I * 2 < 0x7ffffff0ll;
   // (T <= E: the in-kernel sort may open up to one block per pair, which is what the block bound then allows)
   const bool fuse_all = fuse_act && fuse_level >= 2 && M == 1 && T <= E;
+  if (row) {
+    const RowQuantArgs qa = {hidden, ws + w.xq, (float*)(ws + w.xs), H};
+    const int nb = E + 1;
+    const size_t lds = moe_align_lds_bytes(nb);
+    const int parts = moe_align_parts(T);
+    const unsigned blocks = (unsigned)(parts + M);
+    hipStream_t st = (hipStream_t)stream;
+#define SGLAMD_ROW_PROLOGUE(IDT, TT, Q, NV)                                                                            \
+  do {                                                                                                                 \
+    auto k = moe_row_prologue_kernel<IDT, TT, Q, NV>;                                                                  \
+    SGLAMD_RAISE_LDS(k, lds);                                                                                          \
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(1024), lds, st, (const IDT*)topk_ids, sorted, expert, post, cumsum, nb,   \
+                       block_m, (int)T, (int)w.max_padded, parts, qa);                                                 \
+  } while (0)
+#define SGLAMD_ROW_PROLOGUE_NV(IDT, TT, Q)                       \
+  do {                                                           \
+    if (H <= 8192) SGLAMD_ROW_PROLOGUE(IDT, TT, Q, 1);           \
+    else SGLAMD_ROW_PROLOGUE(IDT, TT, Q, 4);                     \
+  } while (0)
+#define SGLAMD_ROW_PROLOGUE_T(IDT, Q)                               \
+  do {                                                              \
+    if (dtype == SGLAMD_BF16) SGLAMD_ROW_PROLOGUE_NV(IDT, BF16, Q); \
+    else SGLAMD_ROW_PROLOGUE_NV(IDT, F16, Q);                       \
+  } while (0)
+    if (ids_dtype == SGLAMD_I32) {
+      if (int8) SGLAMD_ROW_PROLOGUE_T(int32_t, true);
+      else SGLAMD_ROW_PROLOGUE_T(int32_t, false);
+    } else {
+      if (int8) SGLAMD_ROW_PROLOGUE_T(int64_t, true);
+      else SGLAMD_ROW_PROLOGUE_T(int64_t, false);
+    }
+#undef SGLAMD_ROW_PROLOGUE_T
+#undef SGLAMD_ROW_PROLOGUE_NV
+#undef SGLAMD_ROW_PROLOGUE
+    rc = check_launch("moe_row_prologue");
+    if (rc) return rc;
+    GemmArgs g = {};
+    g.A = ws + w.xq;
+    g.lda = H;
+    g.sa = (const float*)(ws + w.xs);
+    g.sa_sm = 1;
+    g.B = (const uint8_t*)w13;
+    g.ldb = H;
+    g.b_expert_stride = 2 * I * H;
+    g.sb = w13_scale;
+    g.sb_se = 2 * I;
+    g.sb_sn = 1;
+    g.bias = b13;
+    g.sb_sk = 2 * I;
+    g.C = ws + w.c1;
+    g.ldc = 2 * I;
+    g.M = (int)T;
+    g.N = (int)(2 * I);
+    g.K = (int)H;
+    g.sorted_ids = sorted;
+    g.expert_ids = expert;
+    g.num_post_pad = post;
+    g.top_k = topk;
+    g.num_valid = (int)T;
+    g.max_blocks_m = (int)w.max_blocks;
+    GemmArgs h = g;
+    h.A = ws + w.aq;
+    h.lda = I;
+    h.sa = (const float*)(ws + w.as);
+    h.B = (const uint8_t*)w2;
+    h.ldb = I;
+    h.b_expert_stride = H * I;
+    h.sb = w2_scale;
+    h.sb_se = H;
+    h.bias = b2;
+    h.sb_sk = H;
+    h.C = ws + w.c3;
+    h.ldc = H;
+    h.N = (int)H;
+    h.K = (int)I;
+    h.topk_w = topk_weights;
+    h.top_k = 1;
+    h.mul_weight = 1;
+    SGLAMD_REQUIRE(moe_rows_ok(g) && moe_rows_ok(h), SGLAMD_ENOTSUP, "fused_moe: an operand of 2 GiB or more");
+    rc = moe_rows_gemm(mode, g, dtype, block_m, st);
+    if (rc) return rc;
+    rc = launch_row_quant(RowQuantArgs{ws + w.c1, ws + w.aq, (float*)(ws + w.as), I}, T, dtype, int8, true, st);
+    if (rc) return rc;
+    rc = moe_rows_gemm(mode, h, dtype, block_m, st);
+    if (rc) return rc;
+    return sglamd_moe_sum_reduce(ws + w.c3, out, dtype, M, topk, H, routed_scaling_factor, stream);
+  }
   if (!fuse_all) {
     GroupQuantArgs qa = {};
     qa.in = hidden;
@@ -1067,10 +1127,10 @@ extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t
     qa.layout = SGLAMD_SCALE_ROW_MAJOR;
     qa.scale_stride = 0;
     qa.eps = 1e-10f;
-    qa.min8 = -448.f;
-    qa.max8 = 448.f;
+    qa.min8 = int8 ? -128.f : -448.f;
+    qa.max8 = int8 ? 127.f : 448.f;
     qa.form = SGLAMD_QUANT_FORM_RECIPROCAL;
-    qa.q_is_fp8 = 1;
+    qa.q_is_fp8 = !int8;
     qa.fuse_silu_mul = 0;
     qa.hidden = H;
     const int nb = E + 1;
@@ -1186,7 +1246,7 @@ extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t
   // Where the persistent walk takes the first GEMM, its epilogue applies SiLU * up and the group quantisation
   // itself and writes the second GEMM's operand directly (same bits as the two launches it replaces).
   bool act_fused = false;
-  if ((block_m == 192 || (block_m == 128 && moe_persist128_enabled())) && moe_persist_enabled() && moe_actq_enabled() &&
+  if (!int8 && (block_m == 192 || (block_m == 128 && moe_persist128_enabled())) && moe_persist_enabled() && moe_actq_enabled() &&
       I % 128 == 0) {
     GemmArgs g = {};
     g.A = ws + w.xq;
@@ -1225,20 +1285,41 @@ extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t
     }
   }
   if (!act_fused) {
-    rc = sglamd_fused_moe_block_fp8_gemm(ws + w.xq, H, (const float*)(ws + w.xs), KB1, 1, w13, 2 * I * H, H, w13_scale,
-                                         (2 * I / 128) * KB1, KB1, 1, ws + w.c1, 2 * I, dtype, sorted, expert, post,
-                                         nullptr, T, topk, 0, block_m, w.max_blocks, 2 * I, H, stream);
+    rc = moe_block_gemm(mode, ws + w.xq, H, (const float*)(ws + w.xs), KB1, 1, w13, 2 * I * H, H, w13_scale,
+                        (2 * I / 128) * KB1, KB1, 1, ws + w.c1, 2 * I, dtype, sorted, expert, post, nullptr, T, topk, 0,
+                        block_m, w.max_blocks, 2 * I, H, stream);
     if (rc) return rc;
-    rc = sglamd_silu_mul_group_quant_8bit(ws + w.c1, dtype, ws + w.aq, SGLAMD_FP8_E4M3, ws + w.as, T, I, 128,
-                                          SGLAMD_SCALE_ROW_MAJOR, 0, 1e-10f, -448.f, 448.f,
-                                          SGLAMD_QUANT_FORM_RECIPROCAL, stream);
+    rc = sglamd_silu_mul_group_quant_8bit(ws + w.c1, dtype, ws + w.aq, int8 ? SGLAMD_I8 : SGLAMD_FP8_E4M3, ws + w.as, T,
+                                          I, 128, SGLAMD_SCALE_ROW_MAJOR, 0, 1e-10f, int8 ? -128.f : -448.f,
+                                          int8 ? 127.f : 448.f, SGLAMD_QUANT_FORM_RECIPROCAL, stream);
     if (rc) return rc;
   }
-  rc = sglamd_fused_moe_block_fp8_gemm(ws + w.aq, I, (const float*)(ws + w.as), KB2, 1, w2, H * I, I, w2_scale,
-                                       (H / 128) * KB2, KB2, 1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights,
-                                       T, 1, 1, block_m, w.max_blocks, H, I, stream);
+  rc = moe_block_gemm(mode, ws + w.aq, I, (const float*)(ws + w.as), KB2, 1, w2, H * I, I, w2_scale, (H / 128) * KB2, KB2,
+                      1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1, 1, block_m, w.max_blocks, H, I,
+                      stream);
   if (rc) return rc;
   return sglamd_moe_sum_reduce(ws + w.c3, out, dtype, M, topk, H, routed_scaling_factor, stream);
+}
+
+extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E,
+                                          int topk, const void* w13, const float* w13_scale, const void* w2,
+                                          const float* w2_scale, const float* topk_weights, const void* topk_ids,
+                                          int ids_dtype, void* out, float routed_scaling_factor, int block_m,
+                                          void* workspace, int64_t workspace_bytes, void* stream) {
+  return moe_layer(GEMM_BLOCK_FP8, hidden, dtype, M, H, I, E, topk, w13, w13_scale, nullptr, w2, w2_scale, nullptr,
+                   topk_weights, topk_ids, ids_dtype, out, routed_scaling_factor, block_m, workspace, workspace_bytes,
+                   stream);
+}
+
+extern "C" int sglamd_fused_moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E,
+                                      int topk, const void* w13, const float* w13_scale, const void* b13,
+                                      const void* w2, const float* w2_scale, const void* b2, const float* topk_weights,
+                                      const void* topk_ids, int ids_dtype, void* out, float routed_scaling_factor,
+                                      int block_m, void* workspace, int64_t workspace_bytes, void* stream) {
+  SGLAMD_REQUIRE(mode >= SGLAMD_MOE_BLOCK_FP8 && mode <= SGLAMD_MOE_BLOCK_INT8, SGLAMD_EINVAL, "fused_moe: bad mode %d",
+                 mode);
+  return moe_layer(mode, hidden, dtype, M, H, I, E, topk, w13, w13_scale, b13, w2, w2_scale, b2, topk_weights, topk_ids,
+                   ids_dtype, out, routed_scaling_factor, block_m, workspace, workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------------------

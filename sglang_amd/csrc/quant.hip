@@ -105,9 +105,49 @@ static int launch_group_quant(const GroupQuantArgs& a, int group, hipStream_t st
 }
 
 // ---------------------------------------------------------------------------------------
-// Per-token kernels: one 256-lane workgroup per row; the row is read twice (the second
-// read is served by L2), maxima meet through LDS.
+// Per-token kernels.  16-bit rows of a whole number of 8-value pieces, up to 32768 values: row_quant_kernel, one
+// workgroup per row, the row in registers between its maximum and its conversion.  The form below reads the row twice
+// (the second read is served by L2): 32-bit rows, other lengths.
+//
+// Bound by HBM with many rows, by one row's latency with few.  A row is cut into one 16-byte piece per lane while it
+// fits 1024 lanes and the launch has fewer rows than the chip keeps resident (two workgroups of 1024 lanes per CU);
+// with more rows than that up to four pieces per lane, so that more rows are in flight per CU.
 // ---------------------------------------------------------------------------------------
+template <typename T, bool INT8, bool SILU, int NT, int NV>
+__global__ __launch_bounds__(NT) void row_quant_kernel(RowQuantArgs a) {
+  __shared__ float red[NT / 64];
+  row_quant_body<T, INT8, SILU, NV>(a, blockIdx.x, red);
+}
+
+template <typename T, bool INT8, bool SILU>
+static void launch_row_quant_t(const RowQuantArgs& a, int64_t rows, hipStream_t st) {
+  const dim3 grid((unsigned)rows);
+  const int64_t nvec = a.hidden >> 3;
+  const bool many = rows >= 2 * (int64_t)device_cus();
+#define SGLAMD_ROWQ(NT, NV) hipLaunchKernelGGL((row_quant_kernel<T, INT8, SILU, NT, NV>), grid, dim3(NT), 0, st, a)
+  if (nvec <= 256) SGLAMD_ROWQ(256, 1);
+  else if (many && nvec <= 512) SGLAMD_ROWQ(256, 2);
+  else if (many && nvec <= 1024) SGLAMD_ROWQ(256, 4);
+  else if (nvec <= 1024) SGLAMD_ROWQ(1024, 1);
+  else if (nvec <= 2048) SGLAMD_ROWQ(1024, 2);
+  else SGLAMD_ROWQ(1024, 4);
+#undef SGLAMD_ROWQ
+}
+
+int launch_row_quant(const RowQuantArgs& a, int64_t rows, int in_dtype, bool int8, bool silu, hipStream_t st) {
+#define SGLAMD_ROWQ_T(TT)                                          \
+  do {                                                             \
+    if (int8 && silu) launch_row_quant_t<TT, true, true>(a, rows, st);   \
+    else if (int8) launch_row_quant_t<TT, true, false>(a, rows, st);     \
+    else if (silu) launch_row_quant_t<TT, false, true>(a, rows, st);     \
+    else launch_row_quant_t<TT, false, false>(a, rows, st);              \
+  } while (0)
+  if (in_dtype == SGLAMD_BF16) SGLAMD_ROWQ_T(BF16);
+  else SGLAMD_ROWQ_T(F16);
+#undef SGLAMD_ROWQ_T
+  return check_launch("row_quant");
+}
+
 __device__ __forceinline__ float block_max_256(float v, float* red) {
   v = group_max<64>(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
@@ -209,6 +249,8 @@ static void launch_per_token_t(const void* in, void* q, float* s, int64_t rows, 
 template <bool INT8>
 static int launch_per_token(const void* in, int in_dtype, void* q, float* s, int64_t rows, int64_t hidden,
                             hipStream_t st) {
+  if ((in_dtype == SGLAMD_BF16 || in_dtype == SGLAMD_F16) && hidden % 8 == 0 && hidden <= ROW_QUANT_MAX_HIDDEN)
+    return launch_row_quant(RowQuantArgs{in, q, s, hidden}, rows, in_dtype, INT8, false, st);
   switch (in_dtype) {
     case SGLAMD_BF16:
       launch_per_token_t<BF16, INT8>(in, q, s, rows, hidden, st);

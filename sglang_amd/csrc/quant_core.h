@@ -165,4 +165,102 @@ __device__ __forceinline__ void group_quant_body(const GroupQuantArgs& a, const 
   }
 }
 
+// Per-token (whole row) quantisation of one row by one workgroup of 64 * waves lanes: the row stays in registers
+// between the maximum and the conversion (NV pieces of 8 values per lane), so it is read once, all its loads in flight
+// together.  SILU: the row is [gate | up] (`up` points at the second half) and what is quantised is
+// T(silu(gate)) * up rounded to T, the bytes silu_and_mul would have stored.
+// INT8: amax = max(max|x|, 1e-10), s = amax / 127, q = round_half_away(x * (127 / amax));
+// FP8:  s = max|x| / 448, q = e4m3(clamp(x * (1 / s))), zeros for a row of zeros.
+struct RowQuantArgs {
+  const void* in;  // [rows, hidden], SILU: [rows, 2 * hidden]
+  void* q;         // [rows, hidden] bytes
+  float* s;        // [rows]
+  int64_t hidden;  // a multiple of 8
+};
+
+template <typename T, bool INT8, bool SILU, int NV>
+__device__ __forceinline__ void row_quant_body(const RowQuantArgs& a, int64_t row, float* red) {
+  typedef typename T::storage S;
+  static_assert(sizeof(S) == 2, "16-bit rows");
+  const int nt = (int)blockDim.x, tid = threadIdx.x;
+  const int nvec = (int)(a.hidden >> 3);
+  const S* src = (const S*)a.in + row * a.hidden * (SILU ? 2 : 1);
+  const S* up = src + a.hidden;
+  v4i raw[NV], rup[SILU ? NV : 1];
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    const int i = tid + k * nt;
+    raw[k] = v4i{0, 0, 0, 0};
+    if (SILU) rup[SILU ? k : 0] = v4i{0, 0, 0, 0};
+    if (i < nvec) {
+      raw[k] = *((const v4i*)src + i);
+      if (SILU) rup[SILU ? k : 0] = *((const v4i*)up + i);
+    }
+  }
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    S b[8];
+    __builtin_memcpy(b, &raw[k], 16);
+    if constexpr (SILU) {
+      S u[8];
+      __builtin_memcpy(u, &rup[k], 16);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float gv = T::to_f32(b[j]);
+        const float sv = T::to_f32(T::from_f32(gv / (1.0f + expf(-gv))));
+        b[j] = T::from_f32(sv * T::to_f32(u[j]));
+      }
+      __builtin_memcpy(&raw[k], b, 16);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(T::to_f32(b[j])));
+  }
+  amax = group_max<64>(amax);
+  if ((tid & 63) == 0) red[tid >> 6] = amax;
+  __syncthreads();
+  amax = red[0];
+  for (int w = 1; w < (nt >> 6); w++) amax = fmaxf(amax, red[w]);
+
+  float scale, mul;
+  if (INT8) {
+    amax = fmaxf(amax, 1e-10f);
+    scale = amax / 127.0f;
+    mul = 127.0f / amax;
+  } else {
+    scale = amax / 448.0f;
+    mul = (scale == 0.f) ? 0.f : 1.0f / scale;
+  }
+  if (tid == 0) a.s[row] = scale;
+  uint8_t* dst = (uint8_t*)a.q + row * a.hidden;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    const int i = tid + k * nt;
+    if (i >= nvec) break;
+    S b[8];
+    __builtin_memcpy(b, &raw[k], 16);
+    uint32_t w[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      float x[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) x[j] = T::to_f32(b[4 * h + j]) * mul;
+      if constexpr (INT8) {
+        w[h] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[h] |= ((uint32_t)(int)roundf(x[j]) & 0xff) << (8 * j);
+      } else {
+        w[h] = pack4_e4m3(clampf(x[0], -448.f, 448.f), clampf(x[1], -448.f, 448.f), clampf(x[2], -448.f, 448.f),
+                          clampf(x[3], -448.f, 448.f));
+      }
+    }
+    *((v2i*)dst + i) = v2i{(int)w[0], (int)w[1]};
+  }
+}
+
+constexpr int64_t ROW_QUANT_MAX_HIDDEN = 1024 * 8 * 4;  // the longest row that 1024 lanes keep in registers
+
+// Launches row_quant_body over `rows` rows of 16-bit values (quant.hip); hidden <= ROW_QUANT_MAX_HIDDEN, % 8 == 0.
+int launch_row_quant(const RowQuantArgs& a, int64_t rows, int in_dtype, bool int8, bool silu, hipStream_t st);
+
 }  // namespace sglamd

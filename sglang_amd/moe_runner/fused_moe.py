@@ -9,7 +9,7 @@ from typing import Any, Dict, List, Optional
 import torch
 
 from ..moe import gelu_and_mul, moe_sum_reduce, silu_and_mul
-from ..ops import fused_moe_block_fp8_, fused_moe_block_fp8_gemm_, fused_moe_gemm_any_
+from ..ops import _C, fused_moe_block_fp8_gemm_, fused_moe_gemm_any_
 from ..quantization.fp8_kernel import (
     sglang_per_token_group_quant_fp8,
     sglang_per_token_group_quant_int8,
@@ -146,6 +146,17 @@ def fused_experts_impl(
             "int8 quantization only supports channel-wise quantization except for block-wise quantization"
     # a1_scale / a2_scale only matter for FP8 without block_shape; the block and int8 configurations quantise the
     # activations themselves and, as in the reference, never look at them (fused_moe_triton_kernels.py:752-783)
+    clamped = gemm1_alpha is not None or gemm1_limit is not None or swiglu_limit is not None
+    block = block_shape is not None
+    if (activation == "silu" and is_gated and not clamped and not no_combine and not apply_router_weight_on_input
+            and (block_shape[0] == 128 and block_shape[1] == 128 if block
+                 else per_channel_quant and (use_int8_w8a8 or a1_scale is None and a2_scale is None))):
+        # the gated SiLU layer: its launches are issued back to back from one native call
+        out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids, block,
+                           use_int8_w8a8, inplace, 1.0 if routed_scaling_factor is None else routed_scaling_factor,
+                           0 if config is None else config["BLOCK_SIZE_M"])
+        if out is not None:
+            return out
     assert hidden_states.shape[1] == w1.shape[2], "Hidden size mismatch"
     assert topk_weights.shape == topk_ids.shape, "topk shape mismatch"
     assert hidden_states.is_contiguous(), "Hidden_states must be contiguous"
@@ -163,18 +174,6 @@ def fused_experts_impl(
     assert w1.dtype == wdt and w2.dtype == wdt, "expert weights do not have the dtype the flags name"
     plain = (block_shape is not None and list(block_shape) == [128, 128] and b1 is None and b2 is None
              and not apply_router_weight_on_input)
-    clamped = gemm1_alpha is not None or gemm1_limit is not None or swiglu_limit is not None
-    fusable = (plain and activation == "silu" and is_gated and not clamped and use_fp8_w8a8 and not no_combine
-               and hidden_states.shape[1] % 128 == 0 and N % 256 == 0
-               and num_tokens > 0 and w1_scale.is_contiguous() and w2_scale.is_contiguous())
-    if fusable:
-        # whole sequence from one host call: its (at most five) launches are issued back to back from C
-        out = hidden_states if inplace else torch.empty_like(hidden_states)
-        tw = topk_weights if topk_weights.dtype == torch.float32 else topk_weights.to(torch.float32)
-        fused_moe_block_fp8_(hidden_states, w1, w2, w1_scale, w2_scale, tw.contiguous(), topk_ids.contiguous(), out,
-                             1.0 if routed_scaling_factor is None else routed_scaling_factor,
-                             block_m=0 if config is None else config["BLOCK_SIZE_M"])
-        return out
     if config is None:
         config = get_default_config(num_tokens, E, topk)
     if not plain and config["BLOCK_SIZE_M"] > 128:
