@@ -60,9 +60,11 @@ __device__ __forceinline__ u16 f32_to_f16_bits(float f) {
   return h;
 }
 
-// 16-bit storage tags used to pick the conversion at compile time.
+// 16-bit storage tags used to pick the conversion at compile time.  DROPPED is the number of fp32 mantissa bits that
+// the rounding of a normal value drops.
 struct BF16 {
   static constexpr int tag = SGLAMD_BF16;
+  static constexpr int DROPPED = 16;
   typedef u16 storage;
   static __device__ __forceinline__ float to_f32(u16 h) { return bf16_bits_to_f32(h); }
   static __device__ __forceinline__ u16 from_f32(float f) { return f32_to_bf16_bits(f); }
@@ -70,6 +72,7 @@ struct BF16 {
 };
 struct F16 {
   static constexpr int tag = SGLAMD_F16;
+  static constexpr int DROPPED = 13;
   typedef u16 storage;
   static __device__ __forceinline__ float to_f32(u16 h) { return f16_bits_to_f32(h); }
   static __device__ __forceinline__ u16 from_f32(float f) { return f32_to_f16_bits(f); }
@@ -97,6 +100,39 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
 }
 
 __device__ __forceinline__ float clampf(float v, float lo, float hi) { return fminf(fmaxf(v, lo), hi); }
+
+// silu(x) = x / (1 + exp(-x)) rounded to the 16-bit type T, as fp32.  The value is defined through expf and the IEEE
+// division; together they are about 30 VALU instructions, and a kernel that reads 16-bit gates from HBM is then bound
+// by them and not by the memory.  The hardware's exp2 and reciprocal (1 ulp each) give the same 16-bit value unless
+// the fp32 result lies next to a rounding boundary: for |x| < X the two forms differ by at most
+//   |x| * 2^-23.7 (argument of the exponential) + 3 * 2^-23 (exp2, 1 +, rcp, *) + 2 * 2^-23 (the defined form),
+// 15 units in the last place for X = 4 and 30 for X = 16, so only results within D = 16 (32) units of a boundary --
+// 0.1 % of bf16 ones -- and the larger arguments take the defined form.
+template <typename T>
+__device__ __forceinline__ float silu_rounded(float x) {
+  constexpr uint32_t TIE = 1u << (T::DROPPED - 1), MASK = (1u << T::DROPPED) - 1, D = T::tag == SGLAMD_BF16 ? 32 : 16;
+  constexpr float X = T::tag == SGLAMD_BF16 ? 16.f : 4.f;
+  float y = x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504088896340736f));
+  const bool near_tie = ((__float_as_uint(y) - (TIE - D)) & MASK) <= 2 * D;
+  // (a half's subnormals drop more bits than DROPPED)
+  const bool small = T::tag == SGLAMD_F16 && !(fabsf(y) >= 6.2e-5f);
+  if (near_tie || small || !(fabsf(x) < X)) y = x / (1.0f + expf(-x));
+  return T::to_f32(T::from_f32(y));
+}
+
+// n / d for 0 <= n < 2^31 and a divisor known on the host: one 32 x 32 -> high 32 bit multiply, an add and a shift
+// (round-up method).  A 64-bit division by a kernel argument is over a hundred instructions.
+struct FastDiv {
+  uint32_t mul, shift;
+  static FastDiv of(uint32_t d) {
+    uint32_t s = 0;
+    while (s < 31 && (1u << s) < d) s++;
+    return {(uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << s) - d)) / d + 1), s};
+  }
+  __host__ __device__ uint32_t divide(uint32_t n) const {
+    return (uint32_t)((((uint64_t)n * mul) >> 32) + n) >> shift;
+  }
+};
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

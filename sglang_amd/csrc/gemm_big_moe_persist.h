@@ -430,7 +430,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
         for (int r = 0; r < 16; r++) {
           const float gv = OT::to_f32(OT::from_f32(acc[i][0][r] * wgt));
           const float uv = OT::to_f32(OT::from_f32(acc[i][1][r] * wgt));
-          const float sv = OT::to_f32(OT::from_f32(gv / (1.0f + expf(-gv))));
+          const float sv = silu_rounded<OT>(gv);
           const float y = OT::to_f32(OT::from_f32(sv * uv));
           acc[i][0][r] = y;
           m = fmaxf(m, fabsf(y));

@@ -469,13 +469,11 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const typename T::sto
 
 // ---------------------------------------------------------------------------------------
 // act_and_mul: out[t, j] = T(act_f32(x[t, j])) * x[t, d + j], product rounded to T.
-// ACT 0: silu x / (1 + exp(-x));  1: gelu x * 0.5 * (1 + erf(x / sqrt 2));  2: the tanh form of gelu.
+// ACT 0: silu x / (1 + exp(-x)) (silu_rounded);  1: gelu x * 0.5 * (1 + erf(x / sqrt 2));  2: the tanh form of gelu.
 // ---------------------------------------------------------------------------------------
 template <int ACT>
 __device__ __forceinline__ float act_f32(float x) {
-  if constexpr (ACT == 0) {
-    return x / (1.0f + expf(-x));
-  } else if constexpr (ACT == 1) {
+  if constexpr (ACT == 1) {
     return x * (0.5f * (1.0f + erff(x * 0.70710678118654752440f)));
   } else {
     const float cdf = 0.5f * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
@@ -495,7 +493,10 @@ __global__ __launch_bounds__(256) void act_and_mul_kernel(const u16* __restrict_
     __builtin_memcpy(ub, &uv, 16);
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      const float s = T::to_f32(T::from_f32(act_f32<ACT>(T::to_f32(gb[k]))));
+      const float x = T::to_f32(gb[k]);
+      float s;
+      if constexpr (ACT == 0) s = silu_rounded<T>(x);
+      else s = T::to_f32(T::from_f32(act_f32<ACT>(x)));
       ob[k] = T::from_f32(s * T::to_f32(ub[k]));
     }
     v4i ov;
@@ -1122,8 +1123,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     qa.in = hidden;
     qa.q = ws + w.xq;
     qa.s = ws + w.xs;
-    qa.groups_per_row = (int)KB1;
-    qa.num_groups = M * KB1;
+    qa.set_rows(M, H, 128);
     qa.layout = SGLAMD_SCALE_ROW_MAJOR;
     qa.scale_stride = 0;
     qa.eps = 1e-10f;
@@ -1131,8 +1131,6 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     qa.max8 = int8 ? 127.f : 448.f;
     qa.form = SGLAMD_QUANT_FORM_RECIPROCAL;
     qa.q_is_fp8 = !int8;
-    qa.fuse_silu_mul = 0;
-    qa.hidden = H;
     const int nb = E + 1;
     const size_t lds = moe_align_lds_bytes(nb);
     const int parts = moe_align_parts(T);

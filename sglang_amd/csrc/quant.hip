@@ -26,9 +26,9 @@ int check_launch(const char* what) {
   return SGLAMD_OK;
 }
 
-template <typename T, int GROUP>
+template <typename T, int GROUP, bool SILU>
 __global__ __launch_bounds__(256) void group_quant_kernel(GroupQuantArgs a) {
-  group_quant_body<T, GROUP>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  group_quant_body<T, GROUP, SILU>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 // Any group size (the divide-form operator accepts every divisor of the element count):
@@ -80,26 +80,27 @@ __global__ __launch_bounds__(256) void group_quant_generic_kernel(GroupQuantArgs
   }
 }
 
-template <typename T>
+template <typename T, bool SILU = false>
 static int launch_group_quant(const GroupQuantArgs& a, int group, hipStream_t st) {
   constexpr int ELEMS = 32 / (int)sizeof(typename T::storage);
   auto blocks_for = [&](int lpg) { return (unsigned)ceil_div(a.num_groups * lpg, 256); };
   switch (group) {
     case 128:
-      hipLaunchKernelGGL((group_quant_kernel<T, 128>), dim3(blocks_for(128 / ELEMS)), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((group_quant_kernel<T, 128, SILU>), dim3(blocks_for(128 / ELEMS)), dim3(256), 0, st, a);
       break;
     case 64:
-      hipLaunchKernelGGL((group_quant_kernel<T, 64>), dim3(blocks_for(64 / ELEMS)), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((group_quant_kernel<T, 64, SILU>), dim3(blocks_for(64 / ELEMS)), dim3(256), 0, st, a);
       break;
     case 32:
-      hipLaunchKernelGGL((group_quant_kernel<T, 32>), dim3(blocks_for(32 / ELEMS)), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((group_quant_kernel<T, 32, SILU>), dim3(blocks_for(32 / ELEMS)), dim3(256), 0, st, a);
       break;
     case 16:
-      hipLaunchKernelGGL((group_quant_kernel<T, 16>), dim3(blocks_for(16 / ELEMS)), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((group_quant_kernel<T, 16, SILU>), dim3(blocks_for(16 / ELEMS)), dim3(256), 0, st, a);
       break;
     default:
-      hipLaunchKernelGGL((group_quant_generic_kernel<T>), dim3((unsigned)ceil_div(a.num_groups, 4)), dim3(256), 0,
-                         st, a, group);
+      if constexpr (!SILU)
+        hipLaunchKernelGGL((group_quant_generic_kernel<T>), dim3((unsigned)ceil_div(a.num_groups, 4)), dim3(256), 0,
+                           st, a, group);
   }
   return check_launch("per_token_group_quant_8bit");
 }
@@ -489,8 +490,7 @@ extern "C" int sglamd_per_token_group_quant_8bit(const void* input, int in_dtype
   a.in = input;
   a.q = output_q;
   a.s = output_s;
-  a.groups_per_row = (int)(hidden / group_size);
-  a.num_groups = rows * a.groups_per_row;
+  a.set_rows(rows, hidden, group_size);
   a.layout = scale_layout;
   a.scale_stride = scale_stride;
   a.eps = eps;
@@ -498,8 +498,6 @@ extern "C" int sglamd_per_token_group_quant_8bit(const void* input, int in_dtype
   a.max8 = max_8bit;
   a.form = form;
   a.q_is_fp8 = q_dtype == SGLAMD_FP8_E4M3;
-  a.fuse_silu_mul = 0;
-  a.hidden = hidden;
   hipStream_t st = (hipStream_t)stream;
   switch (in_dtype) {
     case SGLAMD_BF16:
@@ -539,8 +537,7 @@ extern "C" int sglamd_silu_mul_group_quant_8bit(const void* input, int in_dtype,
   a.in = input;
   a.q = output_q;
   a.s = output_s;
-  a.groups_per_row = (int)(hidden / group_size);
-  a.num_groups = rows * a.groups_per_row;
+  a.set_rows(rows, hidden, group_size);
   a.layout = scale_layout;
   a.scale_stride = scale_stride;
   a.eps = eps;
@@ -548,11 +545,9 @@ extern "C" int sglamd_silu_mul_group_quant_8bit(const void* input, int in_dtype,
   a.max8 = max_8bit;
   a.form = form;
   a.q_is_fp8 = q_dtype == SGLAMD_FP8_E4M3;
-  a.fuse_silu_mul = 1;
-  a.hidden = hidden;
   hipStream_t st = (hipStream_t)stream;
-  if (in_dtype == SGLAMD_BF16) return launch_group_quant<BF16>(a, group_size, st);
-  return launch_group_quant<F16>(a, group_size, st);
+  if (in_dtype == SGLAMD_BF16) return launch_group_quant<BF16, true>(a, group_size, st);
+  return launch_group_quant<F16, true>(a, group_size, st);
 }
 
 extern "C" int sglamd_silu_mul_group_quant_8bit_masked(const void* input, int in_dtype, void* output_q, int q_dtype,
@@ -583,8 +578,7 @@ extern "C" int sglamd_silu_mul_group_quant_8bit_masked(const void* input, int in
   a.in = input;
   a.q = output_q;
   a.s = output_s;
-  a.groups_per_row = (int)(hidden / group_size);
-  a.num_groups = num_experts * tokens_per_expert * a.groups_per_row;
+  a.set_rows(num_experts * tokens_per_expert, hidden, group_size);
   a.layout = SGLAMD_SCALE_COL_MAJOR_UE8M0;
   a.scale_stride = scale_hidden_stride;
   a.eps = eps;
@@ -592,14 +586,12 @@ extern "C" int sglamd_silu_mul_group_quant_8bit_masked(const void* input, int in
   a.max8 = max_8bit;
   a.form = SGLAMD_QUANT_FORM_RECIPROCAL;
   a.q_is_fp8 = q_dtype == SGLAMD_FP8_E4M3;
-  a.fuse_silu_mul = 1;
-  a.hidden = hidden;
   a.masked_m = masked_m;
   a.tokens_per_expert = (int)tokens_per_expert;
   a.scale_expert_stride = scale_expert_stride;
   hipStream_t st = (hipStream_t)stream;
-  if (in_dtype == SGLAMD_BF16) return launch_group_quant<BF16>(a, group_size, st);
-  return launch_group_quant<F16>(a, group_size, st);
+  if (in_dtype == SGLAMD_BF16) return launch_group_quant<BF16, true>(a, group_size, st);
+  return launch_group_quant<F16, true>(a, group_size, st);
 }
 
 extern "C" int sglamd_per_token_quant_fp8(const void* input, int in_dtype, void* output_q, float* output_s,
