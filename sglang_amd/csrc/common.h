@@ -120,6 +120,51 @@ __device__ __forceinline__ float silu_rounded(float x) {
   return T::to_f32(T::from_f32(y));
 }
 
+// Maximum over each aligned group of N = 4, 8 or 16 lanes, in all of them, on the DPP data path.
+template <int N>
+__device__ __forceinline__ float lanes_max(float v) {
+  int x = __float_as_int(v);
+#define SGLAMD_DPP_MAX(ctrl) \
+  x = __float_as_int(fmaxf(__int_as_float(x), __int_as_float(__builtin_amdgcn_update_dpp(x, x, ctrl, 0xf, 0xf, false))))
+  SGLAMD_DPP_MAX(0xB1);               // quad_perm [1, 0, 3, 2]
+  SGLAMD_DPP_MAX(0x4E);               // quad_perm [2, 3, 0, 1]
+  if (N >= 8) SGLAMD_DPP_MAX(0x141);  // row_half_mirror
+  if (N >= 16) SGLAMD_DPP_MAX(0x140);  // row_mirror
+#undef SGLAMD_DPP_MAX
+  return __int_as_float(x);
+}
+
+// Maximum over the wave, in all lanes: within rows of 16 lanes by DPP, the four rows by v_readlane (a shuffle through
+// LDS costs a round trip of about 60 cycles for each of its six steps).
+__device__ __forceinline__ float wave_max(float v) {
+  const int x = __float_as_int(lanes_max<16>(v));
+  const float a = __int_as_float(__builtin_amdgcn_readlane(x, 0)), b = __int_as_float(__builtin_amdgcn_readlane(x, 16));
+  const float c = __int_as_float(__builtin_amdgcn_readlane(x, 32)), d = __int_as_float(__builtin_amdgcn_readlane(x, 48));
+  return fmaxf(fmaxf(a, b), fmaxf(c, d));
+}
+
+// One round of a router's top-k over scores v[j] of expert lane + 64 * j: the largest score, the lowest expert among
+// those that have it (`fallback` when nothing compares equal: NaN scores); its score is replaced by `taken`.
+template <int EPL>
+__device__ __forceinline__ float wave_pick(float (&v)[EPL], int fallback, float taken, int& expert) {
+  float best = v[0];
+#pragma unroll
+  for (int j = 1; j < EPL; j++) best = fmaxf(best, v[j]);
+  best = wave_max(best);
+  int e = -1;
+#pragma unroll
+  for (int j = 0; j < EPL; j++) {
+    const unsigned long long m = __ballot(v[j] == best);
+    if (e < 0 && m) e = (int)__builtin_ctzll(m) + 64 * j;
+  }
+  expert = e < 0 ? fallback : e;
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int j = 0; j < EPL; j++)
+    if (lane + 64 * j == expert) v[j] = taken;
+  return best;
+}
+
 // n / d for 0 <= n < 2^31 and a divisor known on the host: one 32 x 32 -> high 32 bit multiply, an add and a shift
 // (round-up method).  A 64-bit division by a kernel argument is over a hundred instructions.
 struct FastDiv {

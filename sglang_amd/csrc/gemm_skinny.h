@@ -81,20 +81,6 @@ constexpr int skinny_smem_bytes(int kw, int extra_bytes = 0) {
 // a lane with this offset fetches nothing and its LDS slot receives zeros.
 constexpr uint32_t SKINNY_NOWHERE = 0x7ffffff0u;
 
-// Maximum over each aligned group of N = 4, 8 or 16 lanes, in all of them, on the DPP data path.
-template <int N>
-__device__ __forceinline__ float lanes_max(float v) {
-  int x = __float_as_int(v);
-#define SGLAMD_DPP_MAX(ctrl) \
-  x = __float_as_int(fmaxf(__int_as_float(x), __int_as_float(__builtin_amdgcn_update_dpp(x, x, ctrl, 0xf, 0xf, false))))
-  SGLAMD_DPP_MAX(0xB1);               // quad_perm [1, 0, 3, 2]
-  SGLAMD_DPP_MAX(0x4E);               // quad_perm [2, 3, 0, 1]
-  if (N >= 8) SGLAMD_DPP_MAX(0x141);  // row_half_mirror
-  if (N >= 16) SGLAMD_DPP_MAX(0x140);  // row_mirror
-#undef SGLAMD_DPP_MAX
-  return __int_as_float(x);
-}
-
 template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int PD, int AQ = 0>
 __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub

@@ -33,7 +33,7 @@ static int generic_out(const GemmArgsX& g, int bm, int out_dtype, hipStream_t st
 // ---------------------------------------------------------------------------------------
 // topk_sigmoid: one wavefront per token, lane l holds experts l, l + 64, ...  score = 1 / (1 + exp(-x)) (+ bias for
 // the choice only: the written weight is the biased score minus the bias, as the reference computes it); k rounds
-// of (value, lower index wins) arg-max by butterfly shuffles; optional division by the sum of the picked weights.
+// of (value, lower index wins) arg-max (wave_pick); optional division by the sum of the picked weights.
 // ---------------------------------------------------------------------------------------
 template <typename T, int EPL>
 __global__ __launch_bounds__(256) void topk_sigmoid_kernel(const typename T::storage* __restrict__ gating,
@@ -59,29 +59,8 @@ __global__ __launch_bounds__(256) void topk_sigmoid_kernel(const typename T::sto
   int picked_id = 0;
   float total = 0.f;
   for (int k = 0; k < topk; k++) {
-    float best = v[0];
-    int best_e = lane;
-#pragma unroll
-    for (int j = 1; j < EPL; j++) {
-      if (v[j] > best) {
-        best = v[j];
-        best_e = lane + 64 * j;
-      }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      const float ob = __shfl_xor(best, off, 64);
-      const int oe = __shfl_xor(best_e, off, 64);
-      if (ob > best || (ob == best && oe < best_e)) {
-        best = ob;
-        best_e = oe;
-      }
-    }
-    if ((best_e & 63) == lane) {
-#pragma unroll
-      for (int j = 0; j < EPL; j++)
-        if (j == (best_e >> 6)) v[j] = -20000.f;
-    }
+    int best_e;
+    const float best = wave_pick<EPL>(v, k, -20000.f, best_e);
     const float w = bias ? best - bias[best_e] : best;
     if (lane == (k & 63)) {
       picked = w;
@@ -91,12 +70,13 @@ __global__ __launch_bounds__(256) void topk_sigmoid_kernel(const typename T::sto
     if ((k & 63) == 63 || k == topk - 1) {
       const int base = k & ~63;
       if (base + lane <= k) {
+        if (renormalize && topk <= 64) picked *= 1.f / total;  // the only flush: all picks are in
         weights[(int64_t)row * topk + base + lane] = picked;
         ids[(int64_t)row * topk + base + lane] = picked_id;
       }
     }
   }
-  if (renormalize) {
+  if (renormalize && topk > 64) {
     // every lane holds the same total; lane l re-reads exactly the entries it wrote itself (l, l + 64, ...)
     const float inv = 1.f / total;
     for (int k = lane; k < topk; k += 64) weights[(int64_t)row * topk + k] *= inv;
