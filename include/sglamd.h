@@ -115,6 +115,15 @@ int sglamd_per_token_quant_int8(const void* input, int in_dtype, int8_t* output_
 int sglamd_ue8m0_unpack(const void* packed, int64_t row_stride, int64_t word_stride, int64_t row_step, float* out,
                         int64_t rows, int64_t groups, void* stream);
 
+/* Operands of a linear layer whose weight scales are packed UE8M0 (fp8_utils.py:645-696), in one launch: input
+ * [rows, hidden] (F16 or BF16, hidden % 128 == 0) quantised per 1x128 group to e4m3fn with power-of-two scales
+ * (reciprocal form), output_s[g * rows + m] the scales as floats; weight_s [weight_blocks, hidden/128] the weight's
+ * scales expanded from words packed[(128 * b) * row_stride + (g / 4) * word_stride]. */
+int sglamd_ue8m0_linear_operands(const void* input, int in_dtype, void* output_q, float* output_s, int64_t rows,
+                                 int64_t hidden, const void* packed, int64_t row_stride, int64_t word_stride,
+                                 float* weight_s, int64_t weight_blocks, void* stream);
+
+
 /* ------------------------------------------------------------------------------------
  * W8A8 block-scaled FP8 GEMM:
  *   out[m, n] = cast( sum_kb ( sum_{k in kb} a[m, k] * b[n, k] ) * sa[m, kb] * sb[n/128, kb] )

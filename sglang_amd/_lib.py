@@ -37,6 +37,7 @@ SIGNATURES = {
     "sglamd_last_streaming_shape": [],
     "sglamd_streaming_piece_offset": [_i, _i, _i64, _p],
     "sglamd_ue8m0_unpack": [_p, _i64, _i64, _i64, _p, _i64, _i64, _p],
+    "sglamd_ue8m0_linear_operands": [_p, _i, _p, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _p],
     "sglamd_ceiling_mfma": [_i, _i, _i, _p, _p],
     "sglamd_ceiling_hbm": [_p, _p, _i64, _p, _p],
     "sglamd_ceiling_hbm_lds": [_p, _i64, _p],

@@ -534,30 +534,25 @@ optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws
   const c10::DeviceGuard guard(x.device());
   Tensor out = empty({m, n}, t, x);
   Scratch sc;
-  const int64_t words = cdiv(kb, 4), pad = up(m, 4);
-  const int64_t q = sc.take(m * k), sa = sc.take(4 * m * kb);
-  const int64_t packed = ue8m0 ? sc.take(4 * words * pad) : 0, sb = ue8m0 ? sc.take(4 * cdiv(n, 128) * kb) : 0;
+  const int64_t q = sc.take(m * k), sa = sc.take(4 * m * kb), sb = ue8m0 ? sc.take(4 * cdiv(n, 128) * kb) : 0;
   const int64_t wb = sglamd_gemm_workspace_bytes(m, n, k), wp = sc.take(wb > 0 ? wb : 0);
   sc.allocate(x);
   void* st = stream_of(x);
-  const void* xp = x.data_ptr();
+  const float* wsp;
+  int64_t ws_n, ws_k;
   if (ue8m0) {
-    check(sglamd_per_token_group_quant_8bit(xp, tag(t), sc.at(q), SGLAMD_FP8_E4M3, sc.at(packed), m, k, 128,
-                                            SGLAMD_SCALE_COL_MAJOR_UE8M0, pad, 1e-10f, -448.f, 448.f,
-                                            SGLAMD_QUANT_FORM_RECIPROCAL, st));
-    check(sglamd_ue8m0_unpack(sc.at(packed), 1, pad, 1, (float*)sc.at(sa), m, kb, st));
-    check(sglamd_ue8m0_unpack(ws.data_ptr(), ws.stride(0), ws.stride(1), 128, (float*)sc.at(sb), cdiv(n, 128), kb, st));
-    check(sglamd_fp8_blockwise_scaled_mm_pow2(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), kb, 1, (float*)sc.at(sb),
-                                              kb, 1, out.data_ptr(), n, tag(t), m, n, k, wb > 0 ? sc.at(wp) : nullptr,
-                                              wb, st));
+    check(sglamd_ue8m0_linear_operands(x.data_ptr(), tag(t), sc.at(q), (float*)sc.at(sa), m, k, ws.data_ptr(),
+                                       ws.stride(0), ws.stride(1), (float*)sc.at(sb), cdiv(n, 128), st));
+    wsp = (const float*)sc.at(sb), ws_n = kb, ws_k = 1;
   } else {
-    check(sglamd_per_token_group_quant_8bit(xp, tag(t), sc.at(q), SGLAMD_FP8_E4M3, sc.at(sa), m, k, 128,
+    check(sglamd_per_token_group_quant_8bit(x.data_ptr(), tag(t), sc.at(q), SGLAMD_FP8_E4M3, sc.at(sa), m, k, 128,
                                             SGLAMD_SCALE_COL_MAJOR, m, 1e-10f, -448.f, 448.f,
                                             SGLAMD_QUANT_FORM_RECIPROCAL, st));
-    check(sglamd_fp8_blockwise_scaled_mm(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, ws.data_ptr<float>(),
-                                         ws.stride(0), ws.stride(1), out.data_ptr(), n, tag(t), m, n, k,
-                                         wb > 0 ? sc.at(wp) : nullptr, wb, st));
+    wsp = ws.data_ptr<float>(), ws_n = ws.stride(0), ws_k = ws.stride(1);
   }
+  auto fn = ue8m0 ? sglamd_fp8_blockwise_scaled_mm_pow2 : sglamd_fp8_blockwise_scaled_mm;
+  check(fn(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, out.data_ptr(), n, tag(t), m, n, k,
+           wb > 0 ? sc.at(wp) : nullptr, wb, st));
   if (bias) out.add_(*bias);
   return out;
 }

@@ -31,6 +31,36 @@ __global__ __launch_bounds__(256) void group_quant_kernel(GroupQuantArgs a) {
   group_quant_body<T, GROUP, SILU>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
+// Packed UE8M0 scales -> fp32: element idx of [rows, groups] is the float with exponent byte (g % 4) of word
+// in[(r * row_step) * row_stride + (g / 4) * word_stride] and zero mantissa.
+struct Ue8m0Args {
+  const uint32_t* in;
+  int64_t row_stride, word_stride, row_step;
+  float* out;
+  int64_t rows;
+  int groups;
+};
+__device__ __forceinline__ void ue8m0_unpack_one(const Ue8m0Args& u, int64_t idx) {
+  const int64_t r = idx / u.groups;
+  const int g = (int)(idx - r * u.groups);
+  const uint32_t w = u.in[r * u.row_step * u.row_stride + (int64_t)(g >> 2) * u.word_stride];
+  u.out[idx] = __uint_as_float(((w >> ((g & 3) * 8)) & 0xffu) << 23);
+}
+
+// Both operands' scales of a linear layer with packed UE8M0 weight scales, ready for the GEMM, in one launch: the first
+// `quant_blocks` workgroups quantise the activations (power-of-two scales as floats), the others expand the weights'.
+// In place of three launches (quantise to packed words, expand those, expand the weights'): 300 x 18432 rows against a
+// 7168 x 18432 weight 12.6 -> 6 us.
+template <typename T>
+__global__ __launch_bounds__(256) void group_quant_unpack_kernel(GroupQuantArgs a, unsigned quant_blocks, Ue8m0Args u) {
+  if (blockIdx.x < quant_blocks) {
+    group_quant_body<T, 128>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
+    return;
+  }
+  const int64_t idx = (int64_t)(blockIdx.x - quant_blocks) * 256 + threadIdx.x;
+  if (idx < u.rows * u.groups) ue8m0_unpack_one(u, idx);
+}
+
 // Any group size (the divide-form operator accepts every divisor of the element count):
 // one wavefront per group, scalar element loop.
 template <typename T>
@@ -423,18 +453,10 @@ static int launch_rms_quant(const RmsQuantArgs& a, int w_dtype, int64_t M, hipSt
   return fail(SGLAMD_EINVAL, "fused_rms_fp8_group_quant: weight dtype must be F32, F16 or BF16");
 }
 
-// Packed UE8M0 scales -> fp32: out[r, g] = float with exponent byte (g % 4) of word
-// in[(r * row_step) * row_stride + (g / 4) * word_stride] and zero mantissa.
-__global__ __launch_bounds__(256) void ue8m0_unpack_kernel(const uint32_t* __restrict__ in, int64_t row_stride,
-                                                           int64_t word_stride, int64_t row_step,
-                                                           float* __restrict__ out, int64_t rows, int groups) {
-  const int64_t total = rows * groups;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
-    const int64_t r = idx / groups;
-    const int g = (int)(idx - r * groups);
-    const uint32_t w = in[r * row_step * row_stride + (int64_t)(g >> 2) * word_stride];
-    out[idx] = __uint_as_float(((w >> ((g & 3) * 8)) & 0xffu) << 23);
-  }
+__global__ __launch_bounds__(256) void ue8m0_unpack_kernel(Ue8m0Args u) {
+  const int64_t total = u.rows * u.groups;
+  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256)
+    ue8m0_unpack_one(u, idx);
 }
 
 }  // namespace sglamd
@@ -450,13 +472,50 @@ extern "C" int sglamd_ue8m0_unpack(const void* packed, int64_t row_stride, int64
   if (rows == 0) return SGLAMD_OK;
   const int64_t total = rows * groups;
   const unsigned blocks = (unsigned)(total / 256 + 1 < 4096 ? total / 256 + 1 : 4096);
-  hipLaunchKernelGGL(ue8m0_unpack_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (const uint32_t*)packed,
-                     row_stride, word_stride, row_step, out, rows, (int)groups);
+  const Ue8m0Args u = {(const uint32_t*)packed, row_stride, word_stride, row_step, out, rows, (int)groups};
+  hipLaunchKernelGGL(ue8m0_unpack_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, u);
   return check_launch("ue8m0_unpack");
 }
 
+extern "C" int sglamd_ue8m0_linear_operands(const void* input, int in_dtype, void* output_q, float* output_s, int64_t rows,
+                                            int64_t hidden, const void* packed, int64_t row_stride,
+                                            int64_t word_stride, float* weight_s, int64_t weight_blocks, void* stream) {
+  SGLAMD_REQUIRE(input && output_q && output_s && packed && weight_s, SGLAMD_EINVAL,
+                 "ue8m0_linear_operands: null pointer");
+  SGLAMD_REQUIRE(rows > 0 && hidden > 0 && hidden % 128 == 0 && weight_blocks > 0, SGLAMD_EINVAL,
+                 "ue8m0_linear_operands: bad sizes");
+  SGLAMD_REQUIRE(in_dtype == SGLAMD_F16 || in_dtype == SGLAMD_BF16, SGLAMD_EINVAL,
+                 "ue8m0_linear_operands: input must be F16 or BF16");
+  SGLAMD_REQUIRE(((uintptr_t)input % 16) == 0 && ((uintptr_t)output_q % 16) == 0 && ((uintptr_t)packed % 4) == 0,
+                 SGLAMD_EINVAL, "ue8m0_linear_operands: misaligned pointer");
+  GroupQuantArgs a = {};
+  a.in = input;
+  a.q = output_q;
+  a.s = output_s;
+  a.set_rows(rows, hidden, 128);
+  a.layout = SGLAMD_SCALE_COL_MAJOR;
+  a.scale_stride = rows;
+  a.eps = 1e-10f;
+  a.min8 = -448.f;
+  a.max8 = 448.f;
+  a.form = SGLAMD_QUANT_FORM_RECIPROCAL;
+  a.q_is_fp8 = 1;
+  a.pow2 = 1;
+  const Ue8m0Args u = {(const uint32_t*)packed, row_stride, word_stride, 128, weight_s, weight_blocks, (int)(hidden / 128)};
+  const int64_t quant_blocks = ceil_div(a.num_groups * 8, 256);
+  const int64_t blocks = quant_blocks + ceil_div(weight_blocks * (hidden / 128), 256);
+  SGLAMD_REQUIRE(blocks < 0x7fffffff, SGLAMD_EINVAL, "ue8m0_linear_operands: grid too large");
+  if (in_dtype == SGLAMD_BF16)
+    hipLaunchKernelGGL(group_quant_unpack_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a,
+                       (unsigned)quant_blocks, u);
+  else
+    hipLaunchKernelGGL(group_quant_unpack_kernel<F16>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a,
+                       (unsigned)quant_blocks, u);
+  return check_launch("ue8m0_linear_operands");
+}
+
 extern "C" const char* sglamd_last_error(void) { return g_err; }
-extern "C" int sglamd_abi_version(void) { return 6; }
+extern "C" int sglamd_abi_version(void) { return 7; }
 
 extern "C" int sglamd_per_token_group_quant_8bit(const void* input, int in_dtype, void* output_q, int q_dtype,
                                                  void* output_s, int64_t rows, int64_t hidden, int group_size,
