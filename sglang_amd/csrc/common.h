@@ -60,11 +60,9 @@ __device__ __forceinline__ u16 f32_to_f16_bits(float f) {
   return h;
 }
 
-// 16-bit storage tags used to pick the conversion at compile time.  DROPPED is the number of fp32 mantissa bits that
-// the rounding of a normal value drops.
+// 16-bit storage tags used to pick the conversion at compile time.
 struct BF16 {
   static constexpr int tag = SGLAMD_BF16;
-  static constexpr int DROPPED = 16;
   typedef u16 storage;
   static __device__ __forceinline__ float to_f32(u16 h) { return bf16_bits_to_f32(h); }
   static __device__ __forceinline__ u16 from_f32(float f) { return f32_to_bf16_bits(f); }
@@ -72,7 +70,6 @@ struct BF16 {
 };
 struct F16 {
   static constexpr int tag = SGLAMD_F16;
-  static constexpr int DROPPED = 13;
   typedef u16 storage;
   static __device__ __forceinline__ float to_f32(u16 h) { return f16_bits_to_f32(h); }
   static __device__ __forceinline__ u16 from_f32(float f) { return f32_to_f16_bits(f); }
@@ -101,23 +98,32 @@ __device__ __forceinline__ uint32_t pack4_e4m3(float a, float b, float c, float 
 
 __device__ __forceinline__ float clampf(float v, float lo, float hi) { return fminf(fmaxf(v, lo), hi); }
 
-// silu(x) = x / (1 + exp(-x)) rounded to the 16-bit type T, as fp32.  The value is defined through expf and the IEEE
-// division; together they are about 30 VALU instructions, and a kernel that reads 16-bit gates from HBM is then bound
-// by them and not by the memory.  The hardware's exp2 and reciprocal (1 ulp each) give the same 16-bit value unless
-// the fp32 result lies next to a rounding boundary: for |x| < X the two forms differ by at most
-//   |x| * 2^-23.7 (argument of the exponential) + 3 * 2^-23 (exp2, 1 +, rcp, *) + 2 * 2^-23 (the defined form),
-// 15 units in the last place for X = 4 and 30 for X = 16, so only results within D = 16 (32) units of a boundary --
-// 0.1 % of bf16 ones -- and the larger arguments take the defined form.
+// silu(x) = x / (1 + exp(-x)) rounded to the 16-bit type T, as fp32.
+//
+// The value is defined through expf and the IEEE division, about 30 VALU instructions, and a kernel that reads 16-bit
+// gates from HBM is then bound by them and not by the memory.  For bfloat16 the hardware's exp2 (its argument split in
+// two, so that its error does not grow with x) and reciprocal, 1 ulp each, give the same 16-bit value unless the fp32
+// result lies next to a rounding boundary: the two forms differ by at most 1 + 1/2 (exp2 and its correction) + 1/2 (1 +)
+// + 1 (rcp) + 1/2 (*) and 1 + 1/2 + 1/2 (the defined form) times 2^-23, eleven units in the last place, so results within
+// D = 16 units of a boundary, one in two thousand, take the defined form.  So do the ranges where that count does not
+// hold: below -60 (the reciprocal's subnormals), above 1e30 (the product with log2 e overflows), NaN.
+// A half lies next to a boundary eight times as often, and the sign of its zeros is decided by which instruction the
+// compiler picks for the product behind it (v_fma_mixlo_f16 adds a +0), so it keeps the defined form.
 template <typename T>
 __device__ __forceinline__ float silu_rounded(float x) {
-  constexpr uint32_t TIE = 1u << (T::DROPPED - 1), MASK = (1u << T::DROPPED) - 1, D = T::tag == SGLAMD_BF16 ? 32 : 16;
-  constexpr float X = T::tag == SGLAMD_BF16 ? 16.f : 4.f;
-  float y = x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504088896340736f));
-  const bool near_tie = ((__float_as_uint(y) - (TIE - D)) & MASK) <= 2 * D;
-  // (a half's subnormals drop more bits than DROPPED)
-  const bool small = T::tag == SGLAMD_F16 && !(fabsf(y) >= 6.2e-5f);
-  if (near_tie || small || !(fabsf(x) < X)) y = x / (1.0f + expf(-x));
-  return T::to_f32(T::from_f32(y));
+  if constexpr (T::tag == SGLAMD_BF16) {
+    constexpr uint32_t TIE = 0x8000u, MASK = 0xffffu, D = 16;
+    constexpr float L2E_HI = 1.44269502162933349609375f, L2E_LO = 1.9259629911e-8f, LN2 = 0.69314718055994530942f;
+    const float p = x * -L2E_HI;
+    const float rest = fmaf(x, -L2E_LO, fmaf(x, -L2E_HI, -p));
+    const float t = __builtin_amdgcn_exp2f(p);
+    float y = x * __builtin_amdgcn_rcpf(1.0f + fmaf(t, rest * LN2, t));
+    const bool near_tie = ((__float_as_uint(y) - (TIE - D)) & MASK) <= 2 * D;
+    if (near_tie || !(x > -60.f && x < 1e30f)) y = x / (1.0f + expf(-x));
+    return T::to_f32(T::from_f32(y));
+  } else {
+    return T::to_f32(T::from_f32(x / (1.0f + expf(-x))));
+  }
 }
 
 // Maximum over each aligned group of N = 4, 8 or 16 lanes, in all of them, on the DPP data path.
