@@ -420,6 +420,16 @@ int sglamd_fused_moe_layer(int mode, const void* hidden, int dtype, int64_t M, i
                            int ids_dtype, void* out, float routed_scaling_factor, int block_m, void* workspace,
                            int64_t workspace_bytes, void* stream);
 
+/* The block-FP8 layer behind the expert-major interface (cutlass_moe.py:29-341) in one call: the routing weights are
+ * rounded to `dtype` and applied in the final sum, and the caller's tables are filled as sglamd_prepare_moe_input fills
+ * them (expert_offsets [E+1], problem_sizes1/2 [E,3]).  w13 [E, 2I, H], w2 [E, H, I] and their scales contiguous;
+ * workspace as for mode SGLAMD_MOE_BLOCK_FP8, block_m 0. */
+int sglamd_fused_moe_grouped_layer(const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E, int topk,
+                                   const void* w13, const float* w13_scale, const void* w2, const float* w2_scale,
+                                   const float* topk_weights, const int32_t* topk_ids, int32_t* expert_offsets,
+                                   int32_t* problem_sizes1, int32_t* problem_sizes2, void* out, void* workspace,
+                                   int64_t workspace_bytes, void* stream);
+
 /* sglamd_fused_moe_block_fp8 for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and results
  * as sglamd_fused_moe_block_fp8, without the workspace: the intermediates live in a 16 MiB device array that is

@@ -72,6 +72,8 @@ SIGNATURES = {
     "sglamd_fused_moe_block_fp8_static_max_bytes": [],
     "sglamd_fused_moe_block_fp8_static": [_p, _i, _i64, _i64, _i64, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p, _f, _i, _p],
     "sglamd_fused_moe_layer_workspace": [_i, _i64, _i64, _i64, _i, _i, _i],
+    "sglamd_fused_moe_grouped_layer": [_p, _i, _i64, _i64, _i64, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64,
+                                       _p],
     "sglamd_fused_moe_layer": [_i, _p, _i, _i64, _i64, _i64, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _f, _i, _p,
                                _i64, _p],
     "sglamd_fused_moe_block_fp8": [_p, _i, _i64, _i64, _i64, _i, _i, _p, _p, _p, _p, _p, _p, _i, _p, _f, _i, _p, _i64,

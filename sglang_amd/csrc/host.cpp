@@ -1020,6 +1020,52 @@ optional<Tensor> moe_layer(const Tensor& hidden, const Tensor& w1, const Tensor&
   return out;
 }
 
+// cutlass_fused_experts_fp8 (cutlass_moe.py:29-341) in its block-scaled configuration: w1 [E, k, 2n] and w2 [E, n, k] as
+// column-major views of contiguous [E, 2n, k] / [E, k, n] weights, the scales as the matching views.
+optional<Tensor> moe_grouped_layer(const Tensor& a, const Tensor& w1, const Tensor& w2, const Tensor& w1_scale,
+                                   const Tensor& w2_scale, const Tensor& topk_weights, const Tensor& topk_ids,
+                                   const Tensor& offsets, const Tensor& sizes1, const Tensor& sizes2,
+                                   const optional<Tensor>& output) {
+  const ScalarType t = a.scalar_type();
+  if (a.dim() != 2 || !a.is_cuda() || !is_half(t) || !a.is_contiguous() || a.size(0) == 0) return {};
+  const int64_t m = a.size(0), k = a.size(1);
+  // a [E, c, r] view of contiguous [E, r, c] memory
+  auto column_major = [&](const Tensor& v, int64_t e, int64_t r, int64_t c, ScalarType vt) {
+    return v.dim() == 3 && v.scalar_type() == vt && v.device() == a.device() && v.size(0) == e && v.size(1) == c &&
+           v.size(2) == r && v.transpose(1, 2).is_contiguous();
+  };
+  if (w1.dim() != 3) return {};
+  const int64_t e = w1.size(0), n = w1.size(2) / 2;
+  if (k == 0 || n == 0 || k % 128 || n % 128 || w1.size(2) % 2 || e + 1 > 2048) return {};
+  if (!column_major(w1, e, 2 * n, k, kFp8) || !column_major(w2, e, k, n, kFp8) ||
+      !column_major(w1_scale, e, 2 * n / 128, k / 128, at::kFloat) ||
+      !column_major(w2_scale, e, k / 128, n / 128, at::kFloat))
+    return {};
+  if (topk_ids.dim() != 2 || topk_ids.scalar_type() != at::kInt || !topk_ids.is_contiguous() || topk_ids.size(0) != m ||
+      topk_ids.size(1) == 0 || topk_ids.sizes() != topk_weights.sizes() || topk_ids.device() != a.device() ||
+      topk_weights.device() != a.device() || m * topk_ids.size(1) >= (1ll << 30))
+    return {};
+  auto table = [&](const Tensor& v, int64_t need) {
+    return v.scalar_type() == at::kInt && v.is_contiguous() && v.numel() >= need && v.device() == a.device();
+  };
+  if (!table(offsets, e + 1) || !table(sizes1, 3 * e) || !table(sizes2, 3 * e)) return {};
+  if (output && !(output->sizes() == a.sizes() && output->scalar_type() == t && output->is_contiguous() &&
+                  output->device() == a.device()))
+    return {};
+  const int64_t topk = topk_ids.size(1);
+  const c10::DeviceGuard guard(a.device());
+  const Tensor tw = topk_weights.to(at::kFloat).contiguous();
+  Tensor out = output ? *output : empty({m, k}, t, a);
+  const int64_t need = sglamd_fused_moe_layer_workspace(SGLAMD_MOE_BLOCK_FP8, m, k, n, (int)e, (int)topk, 0);
+  const Tensor ws = empty({need}, at::kByte, a);
+  check(sglamd_fused_moe_grouped_layer(a.data_ptr(), tag(t), m, k, n, (int)e, (int)topk, w1.data_ptr(),
+                                       w1_scale.data_ptr<float>(), w2.data_ptr(), w2_scale.data_ptr<float>(),
+                                       tw.data_ptr<float>(), topk_ids.data_ptr<int32_t>(), offsets.data_ptr<int32_t>(),
+                                       sizes1.data_ptr<int32_t>(), sizes2.data_ptr<int32_t>(), out.data_ptr(),
+                                       ws.data_ptr(), need, stream_of(a)));
+  return out;
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(sgl_kernel, m) {
@@ -1120,6 +1166,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("w1_scale"), py::arg("w2_scale"), py::arg("topk_weights"), py::arg("topk_ids"), py::arg("out"),
         py::arg("routed_scaling_factor"), py::arg("block_m") = 0, py::arg("workspace") = py::none());
   m.def("moe_layer", &moe_layer, Unlocked());
+  m.def("moe_grouped_layer", &moe_grouped_layer, Unlocked());
   m.def("fused_moe_block_fp8_workspace_bytes",
         [](int64_t m_, int64_t h, int64_t i, int64_t e, int64_t topk, int64_t block_m) {
           return sglamd_fused_moe_block_fp8_workspace(m_, h, i, (int)e, (int)topk, (int)block_m);

@@ -31,7 +31,7 @@ struct MoePrepArgs {
   int32_t* blockscale_offsets;  // [E + 1] or null: offsets with every expert's rows rounded up to 128
   int32_t* problem_sizes1;      // [E, 3] = (rows, 2n, k)
   int32_t* problem_sizes2;      // [E, 3] = (rows, k, n)
-  int32_t* input_permutation;   // [numel]: expert-major position -> token
+  int32_t* input_permutation;   // [numel]: expert-major position -> token; null: no permutations are written
   int32_t* output_permutation;  // [numel]: flat (token, j) -> expert-major position
   int topk, n, k;
 };
@@ -179,6 +179,7 @@ __device__ __forceinline__ void moe_align_body(const IdT* __restrict__ topk_ids,
       pa.blockscale_offsets[nb - 1] = rounded;
     }
   }
+  if (PREP && !pa.input_permutation) return;  // offsets and sizes only
   const int prep_base = PREP ? prefix[1] : 0;
   if (pad_fill)
     for (int j = post_pad + part * 1024 + tid; j < max_padded; j += 1024 * parts) sorted_ids[j] = numel;
@@ -233,20 +234,24 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const IdT* __restrict__
                       max_padded, (int)blockIdx.x, (int)gridDim.x);
 }
 
-// First launch of the fused MoE layer: workgroup 0 sorts the tokens, the others quantise the hidden
-// states (group 128, reciprocal form).  The two jobs are independent, so sharing a launch only removes
-// one launch latency from the decode path.
-template <typename IdT, typename T>
+// First launch of the fused MoE layer: the first `parts` workgroups sort the tokens, the others quantise the hidden
+// states (group 128, reciprocal form).  The jobs are independent, so sharing a launch only removes one launch latency
+// from the decode path.  TABLES: one more workgroup behind the sorting ones writes the expert offsets and problem sizes
+// that callers of the expert-major interface hand in.
+template <typename IdT, typename T, bool TABLES = false>
 __global__ __launch_bounds__(1024) void moe_prologue_kernel(const IdT* __restrict__ topk_ids, int32_t* sorted_ids,
                                                             int32_t* expert_ids, int32_t* post_pad_out,
                                                             int32_t* cumsum_out, int nb, int block_size, int numel,
-                                                            int max_padded, int parts, GroupQuantArgs qa) {
-  if ((int)blockIdx.x < parts) {
+                                                            int max_padded, int parts, GroupQuantArgs qa,
+                                                            MoePrepArgs pa) {
+  const int wg = (int)blockIdx.x - parts;
+  if (wg < 0)
     moe_align_body<IdT>(topk_ids, sorted_ids, expert_ids, post_pad_out, cumsum_out, nb, block_size, numel, 1, max_padded,
                         (int)blockIdx.x, parts);
-  } else {
-    group_quant_body<T, 128>(qa, (int64_t)((int)blockIdx.x - parts) * 1024 + threadIdx.x);
-  }
+  else if (TABLES && wg == 0)
+    moe_align_body<IdT, true>(topk_ids, nullptr, nullptr, nullptr, nullptr, nb, 1, numel, 0, 0, 0, 1, pa);
+  else
+    group_quant_body<T, 128>(qa, (int64_t)(wg - (TABLES ? 1 : 0)) * 1024 + threadIdx.x);
 }
 
 // The same for the row-scaled layers: one row of hidden states per workgroup behind the sorting ones.
@@ -320,9 +325,37 @@ __global__ __launch_bounds__(256) void shuffle_mul_sum_kernel(const u16* __restr
   }
 }
 
+// The same sum over rows that lie in (token, k) order already, factors as floats that are rounded to T first.
+template <typename T>
+__global__ __launch_bounds__(256) void weighted_sum_kernel(const u16* __restrict__ in, u16* __restrict__ out,
+                                                           const float* __restrict__ factors, int topk, int d) {
+  const int64_t i = blockIdx.x;
+  const u16* src = in + i * topk * d;
+  const float* f = factors + i * topk;
+  for (int j = (blockIdx.y * 256 + threadIdx.x) * 8; j < d; j += gridDim.y * 2048) {
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < topk; k++) {
+      const float w = T::to_f32(T::from_f32(f[k]));
+      const v4i v = *(const v4i*)(src + (int64_t)k * d + j);
+      u16 b[8];
+      __builtin_memcpy(b, &v, 16);
+#pragma unroll
+      for (int e = 0; e < 8; e++) acc[e] = fmaf(w, T::to_f32(b[e]), acc[e]);
+    }
+    u16 ob[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) ob[e] = T::from_f32(acc[e]);
+    v4i ov;
+    __builtin_memcpy(&ov, ob, 16);
+    *(v4i*)(out + i * d + j) = ov;
+  }
+}
+
 // Sorted-block schedule of a grouped GEMM whose rows are already expert-major: expert e owns rows
 // [offsets[e], offsets[e] + problem_sizes[e][0]).  Every expert gets ceil(rows / block_m) blocks; slot values
-// are row numbers, slots past an expert's last row hold num_rows (the "no row" value of the GEMM kernels).
+// are row numbers, slots past an expert's last row hold num_rows (the "no row" value of the GEMM kernels).  Every
+// workgroup forms the prefix over the experts itself (a few KB from L2) and fills its share of the slots: one workgroup
+// alone took 31 us for the 36000 slots of 4096 rows over 256 experts.
 __global__ __launch_bounds__(1024) void grouped_schedule_kernel(const int32_t* __restrict__ problem_sizes,
                                                                 const int32_t* __restrict__ offsets, int num_experts,
                                                                 int block_m, int num_rows, int max_blocks,
@@ -358,10 +391,10 @@ __global__ __launch_bounds__(1024) void grouped_schedule_kernel(const int32_t* _
   const int total = min(s_carry, max_blocks);
   if (tid == 0) {
     lds[num_experts] = s_carry;
-    *post_pad = total * block_m;
+    if (blockIdx.x == 0) *post_pad = total * block_m;
   }
   __syncthreads();
-  for (int idx = tid; idx < total * block_m; idx += 1024) {
+  for (int idx = (int)blockIdx.x * 1024 + tid; idx < total * block_m; idx += 1024 * (int)gridDim.x) {
     const int blk = idx / block_m, r = idx - blk * block_m;
     int lo = 0, hi = num_experts - 1;  // last expert whose first block is <= blk (experts without rows share a value)
     while (lo < hi) {
@@ -866,7 +899,8 @@ extern "C" int sglamd_fp8_blockwise_scaled_grouped_mm(void* output, int out_dtyp
   int32_t* expert = (int32_t*)(ws + w.expert);
   int32_t* post = (int32_t*)(ws + w.post);
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(grouped_schedule_kernel, dim3(1), dim3(1024), (size_t)(num_experts + 1) * sizeof(int32_t), st,
+  const int64_t parts = ceil_div(w.max_padded, 2048);
+  hipLaunchKernelGGL(grouped_schedule_kernel, dim3((unsigned)(parts < 64 ? parts : 64)), dim3(1024), (size_t)(num_experts + 1) * sizeof(int32_t), st,
                      problem_sizes, expert_offsets, num_experts, block_m, (int)total_rows, (int)w.max_blocks, sorted,
                      expert, post);
   int rc = check_launch("grouped_schedule");
@@ -962,12 +996,19 @@ extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
+// What the expert-major form of the layer adds: the caller's tables, and routing weights that are rounded to the layer's
+// type and applied in the final sum, not in the second GEMM.
+struct MoeGroupedOut {
+  int32_t *expert_offsets, *problem_sizes1, *problem_sizes2;
+};
+
 // `mode` is a GEMM_* mode: the two block-scaled ones with [E, 2I/128, H/128] and [E, H/128, I/128] scales, the two
 // row-scaled ones with one scale per output channel ([E, 2I], [E, H]) and optional biases of that shape in `dtype`.
 static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E, int topk,
                      const void* w13, const float* w13_scale, const void* b13, const void* w2, const float* w2_scale,
                      const void* b2, const float* topk_weights, const void* topk_ids, int ids_dtype, void* out,
-                     float routed_scaling_factor, int block_m, void* workspace, int64_t workspace_bytes, void* stream) {
+                     float routed_scaling_factor, int block_m, void* workspace, int64_t workspace_bytes, void* stream,
+                     const MoeGroupedOut* grouped = nullptr) {
   SGLAMD_REQUIRE(hidden && w13 && w13_scale && w2 && w2_scale && topk_weights && topk_ids && out && workspace,
                  SGLAMD_EINVAL, "fused_moe: null pointer");
   SGLAMD_REQUIRE(M > 0 && E > 0 && topk > 0, SGLAMD_EINVAL, "fused_moe: bad M/E/topk");
@@ -999,6 +1040,19 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   SGLAMD_REQUIRE(E + 1 <= 2048 && T < (1ll << 30), SGLAMD_EINVAL, "fused_moe: too many experts or tokens");
   SGLAMD_REQUIRE(((uintptr_t)hidden % 16) == 0, SGLAMD_EINVAL, "fused_moe: hidden must be 16-byte aligned");
   int rc = SGLAMD_OK;
+  // the last launch: the k rows of every token summed
+  auto finish = [&]() -> int {
+    if (!grouped) return sglamd_moe_sum_reduce(ws + w.c3, out, dtype, M, topk, H, routed_scaling_factor, stream);
+    const int64_t slices = ceil_div(H, 2048);
+    const dim3 grid((unsigned)M, (unsigned)(slices < 64 ? slices : 64));
+    if (dtype == SGLAMD_BF16)
+      hipLaunchKernelGGL(weighted_sum_kernel<BF16>, grid, dim3(256), 0, (hipStream_t)stream, (const u16*)(ws + w.c3),
+                         (u16*)out, topk_weights, topk, (int)H);
+    else
+      hipLaunchKernelGGL(weighted_sum_kernel<F16>, grid, dim3(256), 0, (hipStream_t)stream, (const u16*)(ws + w.c3),
+                         (u16*)out, topk_weights, topk, (int)H);
+    return check_launch("weighted_sum");
+  };
   // Decode-sized calls run with fewer launches.  Up to four tokens the activation kernel goes: the first GEMM's
   // tiles pair gate and up rows and write silu(gate) * up, the second GEMM quantises those 16-bit rows itself, at
   // most four per tile -- so these calls align the routing to blocks of 4 (a tile then holds one such block; an
@@ -1011,7 +1065,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   const bool fuse_act = mode == GEMM_BLOCK_FP8 && fuse_level >= 1 && block_m == 16 && M <= 4 && T <= 32 && I % 256 == 0 &&
                         M * H * 2 < 0x7ffffff0ll && 2 * I * H < 0x7ffffff0ll && T * I * 2 < 0x7ffffff0ll;
   // (T <= E: the in-kernel sort may open up to one block per pair, which is what the block bound then allows)
-  const bool fuse_all = fuse_act && fuse_level >= 2 && M == 1 && T <= E;
+  const bool fuse_all = fuse_act && fuse_level >= 2 && M == 1 && T <= E && !grouped;
   if (row) {
     const RowQuantArgs qa = {hidden, ws + w.xq, (float*)(ws + w.xs), H};
     const int nb = E + 1;
@@ -1115,21 +1169,33 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     const int nb = E + 1;
     const size_t lds = moe_align_lds_bytes(nb);
     const int parts = moe_align_parts(T);
-    const unsigned blocks = (unsigned)parts + (unsigned)ceil_div(qa.num_groups * 8, 1024);
+    const unsigned blocks = (unsigned)parts + (grouped ? 1 : 0) + (unsigned)ceil_div(qa.num_groups * 8, 1024);
+    MoePrepArgs pa = {};
+    if (grouped) {
+      pa.expert_offsets = grouped->expert_offsets;
+      pa.problem_sizes1 = grouped->problem_sizes1;
+      pa.problem_sizes2 = grouped->problem_sizes2;
+      pa.topk = topk;
+      pa.n = (int)I;
+      pa.k = (int)H;
+    }
     hipStream_t st = (hipStream_t)stream;
-#define SGLAMD_PROLOGUE(IDT, TT)                                                                                       \
+#define SGLAMD_PROLOGUE(IDT, TT, TABLES)                                                                               \
   do {                                                                                                                 \
-    auto k = moe_prologue_kernel<IDT, TT>;                                                                             \
+    auto k = moe_prologue_kernel<IDT, TT, TABLES>;                                                                     \
     SGLAMD_RAISE_LDS(k, lds);                                                                                          \
     hipLaunchKernelGGL(k, dim3(blocks), dim3(1024), lds, st, (const IDT*)topk_ids, sorted, expert, post, cumsum, nb,   \
-                       fuse_act ? 4 : block_m, (int)T, (int)(fuse_act ? w.few_padded : w.max_padded), parts, qa);      \
+                       fuse_act ? 4 : block_m, (int)T, (int)(fuse_act ? w.few_padded : w.max_padded), parts, qa, pa);  \
   } while (0)
-    if (ids_dtype == SGLAMD_I32) {
-      if (dtype == SGLAMD_BF16) SGLAMD_PROLOGUE(int32_t, BF16);
-      else SGLAMD_PROLOGUE(int32_t, F16);
+    if (grouped) {
+      if (dtype == SGLAMD_BF16) SGLAMD_PROLOGUE(int32_t, BF16, true);
+      else SGLAMD_PROLOGUE(int32_t, F16, true);
+    } else if (ids_dtype == SGLAMD_I32) {
+      if (dtype == SGLAMD_BF16) SGLAMD_PROLOGUE(int32_t, BF16, false);
+      else SGLAMD_PROLOGUE(int32_t, F16, false);
     } else {
-      if (dtype == SGLAMD_BF16) SGLAMD_PROLOGUE(int64_t, BF16);
-      else SGLAMD_PROLOGUE(int64_t, F16);
+      if (dtype == SGLAMD_BF16) SGLAMD_PROLOGUE(int64_t, BF16, false);
+      else SGLAMD_PROLOGUE(int64_t, F16, false);
     }
 #undef SGLAMD_PROLOGUE
     rc = check_launch("moe_prologue");
@@ -1209,7 +1275,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     h.topk_w = topk_weights;
     h.top_k = 1;
     h.num_valid = (int)T;
-    h.mul_weight = 1;
+    h.mul_weight = grouped ? 0 : 1;
     h.max_blocks_m = (int)(fuse_all ? w.max_blocks : w.few_blocks);
     h.sorted_stride = fuse_all ? 0 : 4;
     if (fuse_all) {
@@ -1220,7 +1286,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     rc = dtype == SGLAMD_BF16 ? gemm8_skinny_launch_actquant<BF16>(h, (hipStream_t)stream, expect)
                               : gemm8_skinny_launch_actquant<F16>(h, (hipStream_t)stream, expect);
     if (rc) return rc;
-    return sglamd_moe_sum_reduce(ws + w.c3, out, dtype, M, topk, H, routed_scaling_factor, stream);
+    return finish();
   }
   // Where the persistent walk takes the first GEMM, its epilogue applies SiLU * up and the group quantisation
   // itself and writes the second GEMM's operand directly (same bits as the two launches it replaces).
@@ -1274,10 +1340,10 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     if (rc) return rc;
   }
   rc = moe_block_gemm(mode, ws + w.aq, I, (const float*)(ws + w.as), KB2, 1, w2, H * I, I, w2_scale, (H / 128) * KB2, KB2,
-                      1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1, 1, block_m, w.max_blocks, H, I,
-                      stream);
+                      1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1, grouped ? 0 : 1, block_m,
+                      w.max_blocks, H, I, stream);
   if (rc) return rc;
-  return sglamd_moe_sum_reduce(ws + w.c3, out, dtype, M, topk, H, routed_scaling_factor, stream);
+  return finish();
 }
 
 extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E,
@@ -1288,6 +1354,18 @@ extern "C" int sglamd_fused_moe_block_fp8(const void* hidden, int dtype, int64_t
   return moe_layer(GEMM_BLOCK_FP8, hidden, dtype, M, H, I, E, topk, w13, w13_scale, nullptr, w2, w2_scale, nullptr,
                    topk_weights, topk_ids, ids_dtype, out, routed_scaling_factor, block_m, workspace, workspace_bytes,
                    stream);
+}
+
+extern "C" int sglamd_fused_moe_grouped_layer(const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E,
+                                              int topk, const void* w13, const float* w13_scale, const void* w2,
+                                              const float* w2_scale, const float* topk_weights, const int32_t* topk_ids,
+                                              int32_t* expert_offsets, int32_t* problem_sizes1, int32_t* problem_sizes2,
+                                              void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  SGLAMD_REQUIRE(expert_offsets && problem_sizes1 && problem_sizes2, SGLAMD_EINVAL, "fused_moe_grouped: null pointer");
+  SGLAMD_REQUIRE(((uintptr_t)out % 16) == 0, SGLAMD_EINVAL, "fused_moe_grouped: out must be 16-byte aligned");
+  const MoeGroupedOut tables = {expert_offsets, problem_sizes1, problem_sizes2};
+  return moe_layer(GEMM_BLOCK_FP8, hidden, dtype, M, H, I, E, topk, w13, w13_scale, nullptr, w2, w2_scale, nullptr,
+                   topk_weights, topk_ids, SGLAMD_I32, out, 1.f, 0, workspace, workspace_bytes, stream, &tables);
 }
 
 extern "C" int sglamd_fused_moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t H, int64_t I, int E,
