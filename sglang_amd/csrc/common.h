@@ -187,11 +187,29 @@ struct FastDiv {
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// The current device, asked for once per entry point: while a DeviceScope is alive on a thread its launches share one
+// hipGetDevice (the cost models of a single decode GEMM used to make about a hundred of them, 2 us).  Nothing between an
+// entry point's first and last launch changes the device.
+inline thread_local int scoped_device = -1;
+struct DeviceScope {
+  const int outer;
+  DeviceScope() : outer(scoped_device) {
+    if (outer < 0 && hipGetDevice(&scoped_device) != hipSuccess) scoped_device = -1;
+  }
+  ~DeviceScope() { scoped_device = outer; }
+  DeviceScope(const DeviceScope&) = delete;
+};
+static inline int current_device() {  // -1 when the query fails
+  if (scoped_device >= 0) return scoped_device;
+  int dev = 0;
+  return hipGetDevice(&dev) == hipSuccess ? dev : -1;
+}
+
 // Compute units of the current device (cached per device; 256 when the query fails, the MI355X count).
 static inline int device_cus() {
   static int cus[32] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 32) return 256;
+  const int dev = current_device();
+  if (dev < 0 || dev >= 32) return 256;
   if (!cus[dev]) {
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
@@ -206,8 +224,8 @@ struct SmemAttrOnce {
   int bytes[32] = {};
 };
 static inline hipError_t raise_dynamic_smem(SmemAttrOnce& state, const void* kern, int bytes) {
-  int dev = 0;
-  const bool cached = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 32;
+  const int dev = current_device();
+  const bool cached = dev >= 0 && dev < 32;
   if (cached && state.bytes[dev] >= bytes) return hipSuccess;
   const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e == hipSuccess && cached) state.bytes[dev] = bytes;

@@ -34,6 +34,7 @@ static int blockwise(int mode, const char* op, const void* a, int64_t lda, const
                      int64_t sa_stride_m, int64_t sa_stride_k, const float* sb, int64_t sb_stride_n,
                      int64_t sb_stride_k, void* out, int64_t ldc, int out_dtype, int64_t M, int64_t N, int64_t K,
                      void* workspace, int64_t workspace_bytes, void* stream, bool scales_pow2 = false) {
+  const DeviceScope scope;
   int rc = check_common(op, a, b, out, M, N, K, lda, ldb, ldc);
   if (rc) return rc;
   SGLAMD_REQUIRE(sa && sb, SGLAMD_EINVAL, "%s: null scale pointer", op);
@@ -90,6 +91,7 @@ extern "C" int sglamd_int8_blockwise_scaled_mm(const void* a, int64_t lda, const
 static int rowwise(int mode, const char* op, const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
                    const float* sb, const void* bias, void* out, int64_t ldc, int out_dtype, int64_t M, int64_t N,
                    int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
+  const DeviceScope scope;
   int rc = check_common(op, a, b, out, M, N, K, lda, ldb, ldc);
   if (rc) return rc;
   SGLAMD_REQUIRE(sa && sb, SGLAMD_EINVAL, "%s: null scale pointer", op);
@@ -139,6 +141,7 @@ extern "C" int sglamd_streaming_piece_offset(int kb, int lchunk, int64_t K, int6
 // Bytes of fp32 scratch with which the GEMM entry points above can split K for this shape (0: no use for it).
 extern "C" int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M >= (1ll << 31) || N <= 0 || K <= 0 || (K % 128) != 0) return 0;
+  const DeviceScope scope;
   if (M <= 64 && !small_m_uses_tile(M, N, K)) return 0;
   const BigConfig cfg = gemm8_big_config(M, N, K);
   int64_t need = cfg.slices > 1 ? (int64_t)cfg.slices * M * N * 4 : 0;

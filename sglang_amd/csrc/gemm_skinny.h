@@ -800,28 +800,41 @@ static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expec
   GemmArgs g = g0;
   int fn = (g.N % 32 == 0 && g.N >= 2048) ? 2 : 1;
   if constexpr (!MOE) {
-    if (g.N >= 1024) {
-      double best = -1.0;
-      int best_rows = 16 * fn;
-      auto consider = [&](int f, double (*cost)(const GemmArgs&, int)) {
-        if (force_fn && force_fn != f) return;
-        for (int rows = 16 * f; rows > 16 * f - 16 && rows >= 12; rows -= 4) {
-          if (force_rows && force_rows != rows) continue;
-          const double c = cost(g, rows);
-          if (best < 0 || c < best - 1e-9) {
-            best = c;
-            best_rows = rows;
-            fn = f;
+    // the search is a few microseconds of host time, as much as the launch itself: a thread remembers its last shapes
+    struct Plan {
+      int M, N, K, cus, fn, rows;
+    };
+    static thread_local Plan plans[32] = {};
+    const int cus = device_cus();
+    Plan& plan = plans[((uint32_t)g.M * 31u + (uint32_t)(g.N >> 3) * 7u + (uint32_t)(g.K >> 4)) & 31u];
+    if (plan.M == g.M && plan.N == g.N && plan.K == g.K && plan.cus == cus) {
+      fn = plan.fn;
+      g.rows_per_wg = plan.rows;
+    } else {
+      if (g.N >= 1024) {
+        double best = -1.0;
+        int best_rows = 16 * fn;
+        auto consider = [&](int f, double (*cost)(const GemmArgs&, int)) {
+          if (force_fn && force_fn != f) return;
+          for (int rows = 16 * f; rows > 16 * f - 16 && rows >= 12; rows -= 4) {
+            if (force_rows && force_rows != rows) continue;
+            const double c = cost(g, rows);
+            if (best < 0 || c < best - 1e-9) {
+              best = c;
+              best_rows = rows;
+              fn = f;
+            }
           }
+        };
+        if constexpr (FM <= 2) {
+          consider(4, skinny_cost<FM, 4>);
+          consider(3, skinny_cost<FM, 3>);
         }
-      };
-      if constexpr (FM <= 2) {
-        consider(4, skinny_cost<FM, 4>);
-        consider(3, skinny_cost<FM, 3>);
+        consider(2, skinny_cost<FM, 2>);
+        consider(1, skinny_cost<FM, 1>);
+        g.rows_per_wg = best_rows == 16 * fn ? 0 : best_rows;
       }
-      consider(2, skinny_cost<FM, 2>);
-      consider(1, skinny_cost<FM, 1>);
-      g.rows_per_wg = best_rows == 16 * fn ? 0 : best_rows;
+      plan = Plan{g.M, g.N, g.K, cus, fn, g.rows_per_wg};
     }
   } else if (force_fn == 1 || force_fn == 2) {
     fn = force_fn;

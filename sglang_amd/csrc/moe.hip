@@ -602,6 +602,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
                           const int32_t* num_tokens_post_padded, const float* topk_weights, int64_t num_valid_tokens,
                           int top_k, int mul_routed_weight, int block_m, int64_t max_m_blocks, int64_t N, int64_t K,
                           void* stream) {
+  const DeviceScope scope;
   SGLAMD_REQUIRE(a && a_scale && w && w_scale && c && sorted_token_ids && expert_ids && num_tokens_post_padded,
                  SGLAMD_EINVAL, "fused_moe_gemm: null pointer");
   SGLAMD_REQUIRE(!mul_routed_weight || topk_weights, SGLAMD_EINVAL, "fused_moe_gemm: topk_weights missing");
@@ -1009,6 +1010,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
                      const void* b2, const float* topk_weights, const void* topk_ids, int ids_dtype, void* out,
                      float routed_scaling_factor, int block_m, void* workspace, int64_t workspace_bytes, void* stream,
                      const MoeGroupedOut* grouped = nullptr) {
+  const DeviceScope scope;
   SGLAMD_REQUIRE(hidden && w13 && w13_scale && w2 && w2_scale && topk_weights && topk_ids && out && workspace,
                  SGLAMD_EINVAL, "fused_moe: null pointer");
   SGLAMD_REQUIRE(M > 0 && E > 0 && topk > 0, SGLAMD_EINVAL, "fused_moe: bad M/E/topk");

@@ -16,6 +16,7 @@ bool moe_rows_ok(const GemmArgs& g) {
 int moe_rows_gemm(int mode, const GemmArgs& g, int out_dtype, int block_m, hipStream_t st) {
   SGLAMD_REQUIRE(out_dtype == SGLAMD_BF16 || out_dtype == SGLAMD_F16, SGLAMD_EINVAL,
                  "fused_moe_gemm: out_dtype must be Half or BFloat16");
+  const DeviceScope scope;
   const bool bf16 = out_dtype == SGLAMD_BF16;
   if (mode == GEMM_ROW_INT8)
     return bf16 ? dispatch_moe_gemm<GEMM_ROW_INT8, BF16>(g, block_m, st)

@@ -93,6 +93,20 @@ def invoke_fused_moe_kernel(A, B, C, B_scale, topk_weights, sorted_token_ids, ex
                         block_shape=block_shape, bias=bias)
 
 
+def _plain_gated_silu(activation, is_gated, router_weight_on_input, no_combine, gemm1_alpha, gemm1_limit, swiglu_limit,
+                      use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16, per_channel_quant, a1_scale, a2_scale,
+                      block_shape) -> bool:
+    """The configurations that _C.moe_layer runs: gated SiLU experts, one of the two 8-bit types, 128x128 scale blocks or
+    per-channel scales with dynamic per-token activation scales."""
+    if (activation != "silu" or not is_gated or router_weight_on_input or no_combine or use_fp8_w8a8 == use_int8_w8a8
+            or use_int8_w8a16 or use_int4_w4a16 or gemm1_alpha is not None or gemm1_limit is not None
+            or swiglu_limit is not None):
+        return False
+    if block_shape is not None:
+        return len(block_shape) == 2 and block_shape[0] == 128 and block_shape[1] == 128
+    return per_channel_quant and (use_int8_w8a8 or (a1_scale is None and a2_scale is None))
+
+
 def fused_experts_impl(
     hidden_states: torch.Tensor,
     w1: torch.Tensor,
@@ -146,13 +160,12 @@ def fused_experts_impl(
             "int8 quantization only supports channel-wise quantization except for block-wise quantization"
     # a1_scale / a2_scale only matter for FP8 without block_shape; the block and int8 configurations quantise the
     # activations themselves and, as in the reference, never look at them (fused_moe_triton_kernels.py:752-783)
-    clamped = gemm1_alpha is not None or gemm1_limit is not None or swiglu_limit is not None
-    block = block_shape is not None
-    if (activation == "silu" and is_gated and not clamped and not no_combine and not apply_router_weight_on_input
-            and (block_shape[0] == 128 and block_shape[1] == 128 if block
-                 else per_channel_quant and (use_int8_w8a8 or a1_scale is None and a2_scale is None))):
+    if _plain_gated_silu(activation, is_gated, apply_router_weight_on_input, no_combine, gemm1_alpha, gemm1_limit,
+                         swiglu_limit, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16, per_channel_quant,
+                         a1_scale, a2_scale, block_shape):
         # the gated SiLU layer: its launches are issued back to back from one native call
-        out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids, block,
+        out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids,
+                           block_shape is not None,
                            use_int8_w8a8, inplace, 1.0 if routed_scaling_factor is None else routed_scaling_factor,
                            0 if config is None else config["BLOCK_SIZE_M"])
         if out is not None:
@@ -365,17 +378,27 @@ def fused_experts(
     configuration picks the in-place or the out-of-place operator."""
     topk_weights, topk_ids, _ = topk_output
     c = moe_runner_config
+    operator = _needs_operator(hidden_states)
+    if not operator and _plain_gated_silu(c.activation, c.is_gated, c.apply_router_weight_on_input, c.no_combine,
+                                          c.gemm1_alpha, c.gemm1_clamp_limit, c.swiglu_limit, use_fp8_w8a8, use_int8_w8a8,
+                                          use_int8_w8a16, use_int4_w4a16, per_channel_quant, a1_scale, a2_scale,
+                                          block_shape):
+        out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids,
+                           block_shape is not None, use_int8_w8a8, c.inplace,
+                           1.0 if c.routed_scaling_factor is None else c.routed_scaling_factor, 0)
+        if out is not None:
+            return hidden_states if c.inplace else out
     filter_expert = c.num_experts is None or c.num_experts != c.num_local_experts
     if c.inplace:
         assert not c.no_combine, "no combine + inplace makes no sense"
-        layer = _inplace_op if _needs_operator(hidden_states) else inplace_fused_experts
+        layer = _inplace_op if operator else inplace_fused_experts
         layer(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
               c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
               per_channel_quant, w1_scale, w2_scale, w1_zp, w2_zp, a1_scale, a2_scale, block_shape,
               c.routed_scaling_factor, c.gemm1_alpha, c.gemm1_clamp_limit, filter_expert,
               swiglu_limit=c.swiglu_limit)
         return hidden_states
-    layer = _outplace_op if _needs_operator(hidden_states) else outplace_fused_experts
+    layer = _outplace_op if operator else outplace_fused_experts
     return layer(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
                  c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
                  per_channel_quant, w1_scale, w2_scale, w1_zp, w2_zp, a1_scale, a2_scale, block_shape,
