@@ -588,6 +588,9 @@ static inline bool gemm8_big_ok(const GemmArgs& g) {
 }
 
 // out[m, n] = cast(sum_s slab[s][m][n]) for block mode; row mode applies sa[m] * sb[n] (+ bias) to the sum.
+// Row mode was bound by issuing its loads, not by the slabs: four scales and four biases as single loads per lane beside
+// two or three 16-byte pieces of the slabs.  One load each where they are aligned: 1000 x 8192, two slices, INT8 with a
+// bias 24.8 -> 15.8 us.
 template <int MODE, typename OT>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int slices, GemmArgs g) {
   typedef typename OT::storage OS;
@@ -610,11 +613,32 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     const int n = (int)(e % g.N);
     if (!gemm_is_block(MODE)) {
       const float sam = g.sa[m];
+      float sbn[4], bia[4] = {0.f, 0.f, 0.f, 0.f};
+      if ((((uintptr_t)g.sb) & 15) == 0) {
+        const v4f s4 = *(const v4f*)(g.sb + n);
+#pragma unroll
+        for (int r = 0; r < 4; r++) sbn[r] = s4[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) sbn[r] = g.sb[n + r];
+      }
+      if (g.bias) {
+        OS b4[4];
+        if ((((uintptr_t)g.bias) & 7) == 0) {
+          const v2i b2 = *(const v2i*)((const OS*)g.bias + n);
+          __builtin_memcpy(b4, &b2, 8);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; r++) b4[r] = ((const OS*)g.bias)[n + r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) bia[r] = OT::to_f32(b4[r]);
+      }
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        if constexpr (MODE == GEMM_ROW_FP8) v[r] = v[r] * g.sb[n + r] * sam;
-        else v[r] = v[r] * (g.sb[n + r] * sam);
-        if (g.bias) v[r] += OT::to_f32(((const OS*)g.bias)[n + r]);
+        if constexpr (MODE == GEMM_ROW_FP8) v[r] = v[r] * sbn[r] * sam;
+        else v[r] = v[r] * (sbn[r] * sam);
+        if (g.bias) v[r] += bia[r];
       }
     }
     OS* crow = (OS*)g.C + m * g.ldc + n;
