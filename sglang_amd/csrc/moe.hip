@@ -951,7 +951,10 @@ MoeWs moe_ws_layout(int64_t M, int64_t H, int64_t I, int E, int topk, int block_
   w.total = o;
   return w;
 }
-int moe_auto_block(int64_t M, int E, int topk) {
+// Whether the first GEMM of a layer leaves CUs idle while every expert owns one block (0: intermediate size unknown).
+bool moe_small_launch(int E, int64_t I) { return I > 0 && (int64_t)E * ceil_div(2 * I, 256) <= device_cus(); }
+
+int moe_auto_block(int64_t M, int E, int topk, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;  // tuning knob
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
@@ -965,35 +968,44 @@ int moe_auto_block(int64_t M, int E, int topk) {
   // blocks for a few more rows, then 128-slot blocks (from there on a launch has more tiles than CUs and runs the
   // persistent walk, whose first GEMM also applies the activation), and 192-slot blocks once experts start to
   // overflow 128 slots (an expert's second block streams nothing new but still costs a tile).
+  // Layers whose tiles do not fill the chip take one round whatever the height, so the shorter block wins where it holds
+  // an expert, and two full blocks of 128 beat 192 where half of the experts overflow those.  Seven layers of 8 to 64
+  // experts: 64 at 20..48 rows 4-14 % faster on each, 128 at 176..208 rows 15-29 %; in the bands between, the layers
+  // disagree by as much in both directions.
+  const bool small = moe_small_launch(E, I);
   if (rows < 10) return 16;
-  if (rows < 14) return 64;
-  if (rows <= 104) return 128;
+  if (rows < 14 || (small && rows <= 52)) return 64;
+  if (rows <= 104 || (small && rows >= 170 && rows <= 215)) return 128;
   return 192;
 }
 // The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue, so what counts is how
-// few rows a tile pads: the shortest block that still holds a whole expert (its weights are streamed once).
-int moe_auto_block_rows(int64_t M, int E, int topk) {
+// few rows a tile pads: the shortest block that still holds a whole expert (its weights are streamed once).  A layer that
+// fills the chip moves on sooner, since an expert that overflows adds a tile to a full round: measured on three layers
+// of 64 to 256 experts, 128 at 48 rows 1-9 % faster, 192 at 112 rows 2-10 %; on seven smaller ones 64 stays the faster one
+// at 48 rows by 4-15 %, and 128 at 176..208 rows is 12 % ahead of 192.
+int moe_auto_block_rows(int64_t M, int E, int topk, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
+  const bool small = moe_small_launch(E, I);
   if (rows <= 10) return 16;
-  if (rows <= 56) return 64;
-  if (rows <= 112) return 128;
+  if (rows <= (small ? 56 : 42)) return 64;
+  if (rows <= (small ? 112 : 104) || (small && rows >= 170 && rows <= 215)) return 128;
   return 192;
 }
-int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1); }
+int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1, 0); }
 }  // namespace
 
 extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, int64_t I, int E, int topk, int block_m) {
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
-  if (block_m == 0) block_m = moe_auto_block(M, E, topk);
+  if (block_m == 0) block_m = moe_auto_block(M, E, topk, I);
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
 extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk,
                                                     int block_m) {
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
-  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk) : moe_auto_block_rows(M, E, topk);
+  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk, I) : moe_auto_block_rows(M, E, topk, I);
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
@@ -1024,7 +1036,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   SGLAMD_REQUIRE(!row || I <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: intermediate size %lld is beyond %lld",
                  (long long)I, (long long)ROW_QUANT_MAX_HIDDEN);
   SGLAMD_REQUIRE(row || (!b13 && !b2), SGLAMD_ENOTSUP, "fused_moe: biases go with row-scaled weights");
-  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk) : moe_auto_block(M, E, topk);
+  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk, I) : moe_auto_block(M, E, topk, I);
   SGLAMD_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128 || block_m == 192, SGLAMD_EINVAL,
                  "fused_moe: block_m must be 16, 32, 64, 128 or 192");
   const MoeWs w = moe_ws_layout(M, H, I, E, topk, block_m);
