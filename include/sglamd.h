@@ -208,7 +208,7 @@ int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 #define SGLAMD_KERNEL_TILE128 3       /* tile kernel, 128-row tiles */
 #define SGLAMD_KERNEL_TILE256 4       /* tile kernel, 256-row tiles, one tile per workgroup */
 #define SGLAMD_KERNEL_PERSISTENT256 5 /* 256x256 tiles, one workgroup per CU walking several tiles */
-#define SGLAMD_KERNEL_GENERIC 6       /* register-staged fallback (K % 128 != 0, operands of 2 GiB and more) */
+#define SGLAMD_KERNEL_GENERIC 6       /* register-staged fallback (operands of 2 GiB and more; K % 128 != 0 in block modes or below 512) */
 #define SGLAMD_KERNEL_PERSISTENT256_POW2 7 /* the persistent kernel applying power-of-two scales inside the MFMA */
 #define SGLAMD_KERNEL_STREAMING_WIDE 8  /* weight-streaming kernel, 33..64 rows x 96..144 weight rows per workgroup */
 int sglamd_last_gemm_kernel(void);

@@ -140,7 +140,7 @@ extern "C" int sglamd_streaming_piece_offset(int kb, int lchunk, int64_t K, int6
 
 // Bytes of fp32 scratch with which the GEMM entry points above can split K for this shape (0: no use for it).
 extern "C" int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M >= (1ll << 31) || N <= 0 || K <= 0 || (K % 128) != 0) return 0;
+  if (M >= (1ll << 31) || N <= 0 || K <= 0) return 0;
   const DeviceScope scope;
   if (M <= 64 && !small_m_uses_tile(M, N, K)) return 0;
   const BigConfig cfg = gemm8_big_config(M, N, K);

@@ -54,7 +54,10 @@ constexpr int gemm8_big_smem() {
 // MOE: the row tiles are the sorted blocks of the fused-MoE schedule (block height = 64*MT): activation rows
 // are gathered through sorted_token_ids (row = id / top_k, padding slots read zeros), the weight matrix and
 // its scales are those of expert_ids[block], results are scattered to row id with the routing weight applied.
-template <int MODE, typename OT, int WGN, int MT, bool MOE = false>
+// RAGGED: K is not a multiple of 128.  The last K block's 16-byte pieces past the end of a row are requested outside the
+// descriptor's range by both operands (zeros; a row's neighbour may hold NaN), which is a select per load: the row
+// modes only, which have no fold and so registers and issue slots to spare.
+template <int MODE, typename OT, int WGN, int MT, bool MOE = false, bool RAGGED = false>
 __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub; buffer-resource builtins are device-only
   constexpr int BM = 64 * MT, BN = 64 * WGN, NW = 2 * WGN, WTM = 32 * MT;
@@ -158,6 +161,16 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     b_voff[l] = (uint32_t)((n0 + row) * (int)g.ldb + chunk * 16);
   }
+  // RAGGED: whether a load's piece lies past K in the last block; a lane's chunk is its a_voff's / b_voff's
+  bool a_dead[APT] = {}, b_dead[2] = {};
+  if constexpr (RAGGED) {
+    const int tail_chunks = (g.K & 127) >> 4;
+#pragma unroll
+    for (int u = 0; u < APT; u++)
+      a_dead[u] = ((lane & 7) ^ (((wave * APT + u) * 4 + (lane >> 4)) & 7)) >= tail_chunks;
+#pragma unroll
+    for (int l = 0; l < 2; l++) b_dead[l] = ((lane & 7) ^ ((l * 4 + (lane >> 4)) & 7)) >= tail_chunks;
+  }
   // activation scales of the tile rows: waves 0..BM/64-1 fetch 64 rows each (block mode)
   int srow;
   if (MOE) {
@@ -171,7 +184,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       BLK ? (int)min(((a_rows - 1) * g.sa_sm + (int64_t)((g.K >> 7) - 1) * g.sa_sk + 1) * 4, (int64_t)0x7fffffff) : 0;
 
   // K blocks of this split-K slice
-  const int nkb_all = g.K >> 7;
+  const int nkb_all = RAGGED ? (g.K + 127) >> 7 : g.K >> 7;
   const int kb_begin = (int)((int64_t)nkb_all * blockIdx.y / gridDim.y);
   const int kb_end = (int)((int64_t)nkb_all * (blockIdx.y + 1) / gridDim.y);
   const int nkb = kb_end - kb_begin;
@@ -202,11 +215,13 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   auto issue_piece = [&](int kb, int stage, int t, int part) {
     const bool live = kb < nkb;
     const int koff = (kb_begin + kb) << 7;
+    const bool tail = RAGGED && kb_begin + kb == nkb_all - 1;
     if (part == 0) {
 #pragma unroll
       for (int u = 0; u < APT; u++) {
         const int gi = wave * APT + u;
-        const uint32_t vo = MOE ? a_voff[t * APT + u] : a_voff[u] + (uint32_t)(t * 32 * (int)g.lda);
+        uint32_t vo = MOE ? a_voff[t * APT + u] : a_voff[u] + (uint32_t)(t * 32 * (int)g.lda);
+        if (tail && a_dead[u]) vo = 0x7ffffff0u;
         dma16(g.A, live ? a_bytes : 0, vo, koff, stage * A_STAGE + ((gi >> 2) * WTM + t * 32 + (gi & 3) * 8) * 128);
       }
       return;
@@ -214,7 +229,9 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
 #pragma unroll
     for (int l = 0; l < 4; l++) {
       if (l % MT != t) continue;
-      dma16(Bmat, live ? b_bytes : 0, b_voff[l & 1] + (uint32_t)((l & 2) * 8 * (int)g.ldb), koff,
+      uint32_t vo = b_voff[l & 1] + (uint32_t)((l & 2) * 8 * (int)g.ldb);
+      if (tail && b_dead[l & 1]) vo = 0x7ffffff0u;
+      dma16(Bmat, live ? b_bytes : 0, vo, koff,
             B_BASE + stage * B_STAGE + (wave * 4 + l) * 1024);
     }
     if (BLK && t == MT - 1) {
@@ -580,10 +597,10 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
 #endif
 }
 
-// Preconditions beyond the generic kernel's: K % 128 == 0 and both operands smaller than 2 GiB
+// Preconditions beyond the generic kernel's: K % 128 == 0 (row modes take any K) and both operands smaller than 2 GiB
 // (buffer descriptors carry 32-bit ranges and offsets).
-static inline bool gemm8_big_ok(const GemmArgs& g) {
-  return (g.K % 128) == 0 && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)g.M * g.lda < 0x7fffffffll &&
+static inline bool gemm8_big_ok(const GemmArgs& g, bool any_k = false) {
+  return (any_k || (g.K % 128) == 0) && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)g.M * g.lda < 0x7fffffffll &&
          (int64_t)g.N * g.ldb < 0x7fffffffll;
 }
 
@@ -715,9 +732,12 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool p
   return best;
 }
 
-template <int MODE, typename OT, int WGN, int MT>
+template <int MODE, typename OT, int WGN, int MT, bool RAGGED = false>
 static int gemm8_big_launch(const GemmArgs& g, hipStream_t st, int slices, void* workspace) {
-  auto kern = gemm8_big_kernel<MODE, OT, WGN, MT>;
+  if constexpr (!gemm_is_block(MODE) && !RAGGED) {
+    if (g.K & 127) return gemm8_big_launch<MODE, OT, WGN, MT, true>(g, st, slices, workspace);
+  }
+  auto kern = gemm8_big_kernel<MODE, OT, WGN, MT, false, RAGGED>;
   constexpr int smem = gemm8_big_smem<WGN, MT>();
   static SmemAttrOnce attr;
   hipError_t e = raise_dynamic_smem(attr, (const void*)kern, smem);

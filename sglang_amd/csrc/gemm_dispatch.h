@@ -28,9 +28,13 @@ static int tile_min_m() {
 // 50.6).  Its four-tile form for 33..64 rows re-reads the activations too often for large weights (gate_up at 48
 // rows: 83.9 us against 63.5), but a launch of the tile kernel costs more (a second kernel when K is split) and it
 // needs about a hundred workgroups to hide its per-block latency, so small weights stay with the streaming kernel.
+// Rows of a ragged K start anywhere in a 128-byte line, which the tile kernel's loads (8 rows each) pay for more than
+// the streaming kernel's: there it takes 80 column tiles, or 48 of a long K (8192 x 4112 at 40 rows 20 us in tiles, 17
+// streamed; 12288 20 against 24, 20480 25 against 35, 28672 29 against 46).
 static bool small_m_uses_tile(int64_t M, int64_t N, int64_t K) {
   if (M < tile_min_m() || M <= 32) return false;
   const int64_t tiles = (N + 255) / 256;
+  if (K & 127) return tiles >= 80 || (tiles >= 48 && K >= 4096);
   const int slices = gemm8_big_slices(tiles, N, K);
   if (tiles * slices >= 96) return true;
   return (slices == 1 && tiles >= 32) || K >= 6144;
@@ -71,11 +75,14 @@ static int64_t column_split(int64_t M, int64_t N, int64_t K) {
   return first * 256;
 }
 
+// The row modes' tile kernel also takes a K that is not a multiple of 128, from 512 up: 8192 x 4112 at 100 / 300 / 1000 rows
+// 43 / 45 / 60 -> 21 / 32 / 46 us (4096: 20 / 23 / 39), 28672 x 4112 at 2048 rows 407 -> 281.  Shorter sums are a launch of
+// 12 to 17 us either way and stay with the generic kernel.
 template <int MODE, typename OT>
 static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, int64_t workspace_bytes,
                           bool may_split = true) {
   RAN(SGLAMD_KERNEL_STREAMING);
-  const bool big = gemm8_big_ok(g);
+  const bool big = gemm8_big_ok(g, !gemm_is_block(MODE) && g.K >= 512);
   const int wgs = gemm_is_block(MODE) ? persist_workgroups() : 0;
   const int nkb = g.K >> 7;
   const bool persistent = wgs > 0 && (wgs & 7) == 0 && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;

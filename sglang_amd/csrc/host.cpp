@@ -355,8 +355,9 @@ std::tuple<Tensor, Tensor, optional<Tensor>, optional<Tensor>, optional<Tensor>>
 // ---------------------------------------------------------------------------------------
 // fp32 split-K scratch when the library can use one for this shape; from the caching allocator, so calls on other
 // streams and threads have their own.
-Tensor gemm_workspace(int64_t m, int64_t n, int64_t k, const Tensor& like, void** ptr, int64_t* bytes) {
-  *bytes = sglamd_gemm_workspace_bytes(m, n, k);
+Tensor gemm_workspace(int64_t m, int64_t n, int64_t k, bool row_scaled, const Tensor& like, void** ptr,
+                      int64_t* bytes) {
+  *bytes = row_scaled || k % 128 == 0 ? sglamd_gemm_workspace_bytes(m, n, k) : 0;
   *ptr = nullptr;
   if (*bytes <= 0) return Tensor();
   Tensor ws = empty({*bytes}, at::kByte, like);
@@ -407,7 +408,7 @@ Tensor fp8_blockwise_scaled_mm(const Tensor& a, const Tensor& b, const Tensor& s
   if (m == 0) return out;
   void* wp;
   int64_t wb;
-  const Tensor ws = gemm_workspace(m, n, k, a, &wp, &wb);
+  const Tensor ws = gemm_workspace(m, n, k, false, a, &wp, &wb);
   check(sglamd_fp8_blockwise_scaled_mm(a.data_ptr(), ld(a, 0), b.data_ptr(), ld(b, 1), sa.data_ptr<float>(),
                                        sa.stride(0), sa.stride(1), sb.data_ptr<float>(), sb.stride(1), sb.stride(0),
                                        out.data_ptr(), n, tag(out_dtype), m, n, k, wp, wb, stream_of(a)));
@@ -424,7 +425,7 @@ void block_matmul_(const Tensor& a, const Tensor& b, const Tensor& sa, const Ten
   const c10::DeviceGuard guard(a.device());
   void* wp;
   int64_t wb;
-  const Tensor ws = gemm_workspace(m, n, k, a, &wp, &wb);
+  const Tensor ws = gemm_workspace(m, n, k, false, a, &wp, &wb);
   auto fn = int8 ? sglamd_int8_blockwise_scaled_mm
                  : pow2 ? sglamd_fp8_blockwise_scaled_mm_pow2 : sglamd_fp8_blockwise_scaled_mm;
   check(fn(a.data_ptr(), ld(a, 0), b.data_ptr(), ld(b, 0), (float*)sa.data_ptr(), sa.stride(0), sa.stride(1),
@@ -475,7 +476,7 @@ Tensor rowwise_mm(bool int8, const Tensor& a, const Tensor& b, const Tensor& sa,
   if (m == 0) return out;
   void* wp;
   int64_t wb;
-  const Tensor ws = gemm_workspace(m, n, k, a, &wp, &wb);
+  const Tensor ws = gemm_workspace(m, n, k, true, a, &wp, &wb);
   auto fn = int8 ? sglamd_int8_scaled_mm : sglamd_fp8_scaled_mm;
   check(fn(a.data_ptr(), ld(a, 0), b.data_ptr(), ld(b, 1), sa.data_ptr<float>(), sb.data_ptr<float>(),
            bias ? bias->data_ptr() : nullptr, out.data_ptr(), n, tag(out_dtype), m, n, k, wp, wb, stream_of(a)));
