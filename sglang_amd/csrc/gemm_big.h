@@ -47,6 +47,18 @@ constexpr int gemm8_big_smem() {
          (64 * WGN / 128) * GEMM8_BIG_MAX_KB * 4;
 }
 
+// The K block at which a MoE tile starts its walk (it wraps round).  Weight rows whose pitch is a multiple of 4096 bytes
+// put the same K offset of all rows on a few memory channels, and workgroups that start together stay at the same
+// offset: 64 experts of [3072, 4096] at 28 rows stream at 4.2 TB/s, of [3072, 3968] at 5.2.  So every expert starts
+// elsewhere.  By the expert and nothing else: an expert's blocks share their weights through L2, and a gate column sums
+// in the order of its up column however the columns are tiled.  First GEMM of that layer 191 -> 154 us, [4096, 8192] 459
+// -> 399; layers of 8 to 32 experts with K = 4096 or 8192 gain 4-20 % in every scaling mode; pitches of 1024, 2048, 3072,
+// 5120, 6144, 7168 bytes do not change and keep their order of summation.
+__device__ __forceinline__ int moe_k_rotation(int64_t pitch, int expert, int nkb) {
+  if (pitch & 4095) return 0;
+  return __builtin_amdgcn_readfirstlane((int)((unsigned)(expert * 5) % (unsigned)nkb));
+}
+
 // MT = 32-row tiles per wave along M (4 -> 256-row workgroup tile, 2 -> 128-row tile).
 // Split-K: gridDim.y slices of the K blocks; with more than one slice every workgroup stores its fp32
 // partial tile (block mode: already scaled; row mode: raw accumulators) to slab blockIdx.y of g.C, which
@@ -188,6 +200,9 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   const int kb_begin = (int)((int64_t)nkb_all * blockIdx.y / gridDim.y);
   const int kb_end = (int)((int64_t)nkb_all * (blockIdx.y + 1) / gridDim.y);
   const int nkb = kb_end - kb_begin;
+  // MoE: up to three rounds of one tile per CU; in a longer launch the workgroups have drifted apart by themselves and
+  // the rotation gives nothing (-6 to +3 % at 1024 to 1536 tiles)
+  const int rot = MOE && moe_tiles <= 768 ? moe_k_rotation(g.ldb, max(expert, 0), nkb) : 0;
 
   // The loads are written as assembly so that the compiler's own wait-count bookkeeping does not know them:
   // it treats a direct-to-LDS load as a store every later LDS read might alias and would wait for all of them
@@ -212,9 +227,19 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   // piece t of K block kb of this slice into a stage; the scalar offset operand is not range-checked, so it
   // only carries the K offset (which stays inside a row); everything that selects the row is per lane
   // (part 0: the A loads; part 1: the B loads and the activation scales -- always issued in this order)
-  auto issue_piece = [&](int kb, int stage, int t, int part) {
+  // where block kb of the walk lies (moe_k_rotation)
+  auto block_at = [&](int kb) -> int {
+    int kq = kb_begin + kb;
+    if constexpr (MOE) {
+      kq += rot - nkb;
+      asm volatile("" : "+s"(kq));  // (seen as a function of kb, the wrap makes the compiler split the K loop, and spill)
+      kq += nkb & (kq >> 31);
+    }
+    return kq;
+  };
+  auto issue_piece = [&](int kb, int kq, int stage, int t, int part) {
     const bool live = kb < nkb;
-    const int koff = (kb_begin + kb) << 7;
+    const int koff = kq << 7;
     const bool tail = RAGGED && kb_begin + kb == nkb_all - 1;
     if (part == 0) {
 #pragma unroll
@@ -238,7 +263,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       // waves past the last 64-row group take part with an empty range and a scratch destination, so every
       // wave issues the same number of loads
       const bool mine = wave < BM / 64;
-      dma4(g.sa, (live && mine) ? s_bytes : 0, s_voff, ((kb_begin + kb) * (int)g.sa_sk) << 2,
+      dma4(g.sa, (live && mine) ? s_bytes : 0, s_voff, (kq * (int)g.sa_sk) << 2,
            mine ? S_BASE + stage * S_STAGE + wave * 256 : S_BASE + NS * S_STAGE);
     }
   };
@@ -287,8 +312,13 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     const float* sb_tile = g.sb + (MOE ? (int64_t)max(expert, 0) * g.sb_se : 0);
     for (int idx = tid; idx < (BN / 128) * nkb; idx += 128 * WGN) {
       const int cb = idx / nkb, kb = idx - cb * nkb;
+      int kq = kb_begin + kb;
+      if constexpr (MOE) {
+        kq += rot;
+        if (kq >= nkb) kq -= nkb;
+      }
       sb_lds_all[cb * GEMM8_BIG_MAX_KB + kb] =
-          sb_tile[(int64_t)(min(n0 + cb * 128, g.N - 1) >> 7) * g.sb_sn + (int64_t)(kb_begin + kb) * g.sb_sk];
+          sb_tile[(int64_t)(min(n0 + cb * 128, g.N - 1) >> 7) * g.sb_sn + (int64_t)kq * g.sb_sk];
     }
   }
   const float* sb_mine = sb_lds_all + ((wn * 64) >> 7) * GEMM8_BIG_MAX_KB;
@@ -312,7 +342,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
 #pragma unroll
   for (int st = 0; st < NS; st++)
 #pragma unroll
-    for (int t = 0; t < MT; t++) issue_piece(st, st, t, 0), issue_piece(st, st, t, 1);
+    for (int t = 0; t < MT; t++) issue_piece(st, block_at(st), st, t, 0), issue_piece(st, block_at(st), st, t, 1);
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
   __syncthreads();
   v8i wf[2][2];  // [column tile j][K half h]
@@ -358,7 +388,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   // One tile step of one K block; stage and tile are compile-time constants (the K loop is unrolled NS times).
   constexpr int MPH = gemm_is_int8(MODE) ? 2 : 1;  // MFMA instructions per mm_half
   constexpr int FOLDN = gemm_is_int8(MODE) ? 32 : 16;  // VALU instructions of one fold (int32 products convert first)
-  auto tile_step = [&](int kb, auto stage_c, auto tile_c) {
+  auto tile_step = [&](int kb, int kq, auto stage_c, auto tile_c) {
     constexpr int cur = decltype(stage_c)::value, i = decltype(tile_c)::value;
     constexpr int nxt = (cur + 1) % NS;
     constexpr bool last = i == MT - 1;
@@ -413,7 +443,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     // and the vector memory pipe takes 16 cycles per load, so a wave can wait at a load for a hundred cycles
     // and more; behind an MFMA the matrix pipe's queue covers that wait.
     __builtin_amdgcn_sched_barrier(0);
-    issue_piece(kb + NS, cur, i, 0);
+    issue_piece(kb + NS, kq, cur, i, 0);
     __builtin_amdgcn_sched_barrier(0);
     float sa_nxt = 1.f, sb_nxt = sb_cur;
     if (!last) {
@@ -433,7 +463,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     else acc[i][1] = mm_half(wf[1][1], x1, acc[i][1]);
     __builtin_amdgcn_sched_group_barrier(0x8, MPH, 0);
     __builtin_amdgcn_sched_barrier(0);
-    issue_piece(kb + NS, cur, i, 1);
+    issue_piece(kb + NS, kq, cur, i, 1);
     __builtin_amdgcn_sched_barrier(0);
     if (!last) {
       x1 = xfrag(cur, i + 1, 1);
@@ -453,10 +483,11 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     }
   };
   auto k_block = [&](int kb, auto stage_c) {
-    tile_step(kb, stage_c, std::integral_constant<int, 0>{});
-    if constexpr (MT > 1) tile_step(kb, stage_c, std::integral_constant<int, 1>{});
-    if constexpr (MT > 2) tile_step(kb, stage_c, std::integral_constant<int, 2>{});
-    if constexpr (MT > 3) tile_step(kb, stage_c, std::integral_constant<int, 3>{});
+    const int kq = block_at(kb + NS);
+    tile_step(kb, kq, stage_c, std::integral_constant<int, 0>{});
+    if constexpr (MT > 1) tile_step(kb, kq, stage_c, std::integral_constant<int, 1>{});
+    if constexpr (MT > 2) tile_step(kb, kq, stage_c, std::integral_constant<int, 2>{});
+    if constexpr (MT > 3) tile_step(kb, kq, stage_c, std::integral_constant<int, 3>{});
   };
   for (int kb = 0; kb < nkb; kb += NS) {
     k_block(kb, std::integral_constant<int, 0>{});

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   };
 
   // ---- state of the tile whose K loop runs (or is about to) ----------------------------------------------
-  int n0 = 0, expert = 0, buf = 0;
+  int n0 = 0, expert = 0, buf = 0, rot = 0;
   const uint8_t* Bmat = g.B;
   uint32_t a_voff[MT], b_voff[2], s_voff = 0;
   // Row offsets, weight base and scale table of tile `p`, whose ids sit in s_rows[b]; requests the table.
@@ -130,6 +130,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     expert = p_expert;
     const int ex = max(expert, 0);
     Bmat = g.B + (int64_t)ex * g.b_expert_stride;
+    rot = moe_k_rotation(g.ldb, ex, nkb);
 #pragma unroll
     for (int t = 0; t < MT; t++) {
       const int row = (wave >> 2) * WTM + t * 32 + (wave & 3) * 8 + (lane >> 3);
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     }
     // weight-block scales: entry e = cb * nkb + kb, 64 entries per wave
     const int e = wave * 64 + lane;
-    const int cb = e / nkb, kbb = e - cb * nkb;
+    const int cb = e / nkb, kbl = e - cb * nkb + rot, kbb = kbl >= nkb ? kbl - nkb : kbl;
     // (ACTQ: column block 0 is the gate rows' scale block, column block 1 the up rows')
     const int sbrow = ACTQ ? (cb * half_n + n0) >> 7 : min(n0 + cb * 128, g.N - 1) >> 7;
     const uint32_t tv = cb < BN / 128 ? (uint32_t)(sbrow * (int)g.sb_sn + kbb * (int)g.sb_sk) << 2 : 0x7ffffff0u;
@@ -163,9 +164,16 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   // the last piece, the activation scales)
   auto piece_loads = [](int t) constexpr { return APT + (4 / MT + ((4 % MT) > t ? 1 : 0)) + (t == MT - 1 ? 1 : 0); };
   constexpr int LPB = A_LOADS + 4 + 1;
-  auto issue_piece = [&](int kb, int stage, int t, int part) {
+  // where block kb of the walk lies (moe_k_rotation)
+  auto block_at = [&](int kb) -> int {
+    int kq = kb + rot - nkb;
+    asm volatile("" : "+s"(kq));
+    kq += nkb & (kq >> 31);
+    return kq;
+  };
+  auto issue_piece = [&](int kb, int kq, int stage, int t, int part) {
     const bool live = kb < nkb;
-    const int koff = kb << 7;
+    const int koff = kq << 7;
     if (part == 0) {
       dma16(g.A, live ? a_bytes : 0, a_voff[t], koff, stage * A_STAGE + ((wave >> 2) * WTM + t * 32 + (wave & 3) * 8) * 128);
       return;
@@ -178,7 +186,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     }
     if (t == MT - 1) {
       const bool mine = wave < BM / 64;
-      dma4(g.sa, (live && mine) ? s_bytes : 0, s_voff, (kb * (int)g.sa_sk) << 2,
+      dma4(g.sa, (live && mine) ? s_bytes : 0, s_voff, (kq * (int)g.sa_sk) << 2,
            mine ? S_BASE + stage * S_STAGE + wave * 256 : NOWHERE);
     }
   };
@@ -187,8 +195,8 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     for (int st = 0; st < NS; st++)
 #pragma unroll
       for (int t = 0; t < MT; t++) {
-        issue_piece(st, st, t, 0);
-        issue_piece(st, st, t, 1);
+        issue_piece(st, block_at(st), st, t, 0);
+        issue_piece(st, block_at(st), st, t, 1);
       }
   };
   // ids of sorted block pm for this thread's slot, or a padding id when there is no such block
@@ -274,7 +282,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   constexpr int MPH = gemm_is_int8(MODE) ? 2 : 1;
   constexpr int FOLDN = gemm_is_int8(MODE) ? 32 : 16;
   // One row tile step of one K block: the schedule of gemm8_big_kernel's block mode.
-  auto tile_step = [&](int kb, auto stage_c, auto tile_c) {
+  auto tile_step = [&](int kb, int kq, auto stage_c, auto tile_c) {
     constexpr int cur = decltype(stage_c)::value, i = decltype(tile_c)::value;
     constexpr int nxt = (cur + 1) % NS;
     constexpr bool last = i == MT - 1;
@@ -313,7 +321,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     qb = mm_half(wf[1][0], x0, zero16);
     __builtin_amdgcn_sched_group_barrier(0x8, MPH, 0);
     __builtin_amdgcn_sched_barrier(0);
-    issue_piece(kb + NS, cur, i, 0);
+    issue_piece(kb + NS, kq, cur, i, 0);
     __builtin_amdgcn_sched_barrier(0);
     float sa_nxt, sb_nxt = sb_cur, sb1_nxt = sb1_cur;
     if (!last) {
@@ -331,7 +339,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     qb = mm_half(wf[1][1], x1, qb);
     __builtin_amdgcn_sched_group_barrier(0x8, MPH, 0);
     __builtin_amdgcn_sched_barrier(0);
-    issue_piece(kb + NS, cur, i, 1);
+    issue_piece(kb + NS, kq, cur, i, 1);
     __builtin_amdgcn_sched_barrier(0);
     if (!last) {
       x1 = xfrag(cur, i + 1, 1);
@@ -351,10 +359,11 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     __builtin_amdgcn_sched_group_barrier(0x2, FOLDN, 0);
   };
   auto k_block = [&](int kb, auto stage_c) {
-    tile_step(kb, stage_c, std::integral_constant<int, 0>{});
-    if constexpr (MT > 1) tile_step(kb, stage_c, std::integral_constant<int, 1>{});
-    if constexpr (MT > 2) tile_step(kb, stage_c, std::integral_constant<int, 2>{});
-    if constexpr (MT > 3) tile_step(kb, stage_c, std::integral_constant<int, 3>{});
+    const int kq = block_at(kb + NS);
+    tile_step(kb, kq, stage_c, std::integral_constant<int, 0>{});
+    if constexpr (MT > 1) tile_step(kb, kq, stage_c, std::integral_constant<int, 1>{});
+    if constexpr (MT > 2) tile_step(kb, kq, stage_c, std::integral_constant<int, 2>{});
+    if constexpr (MT > 3) tile_step(kb, kq, stage_c, std::integral_constant<int, 3>{});
   };
 
   uint8_t* stg = smem + STG_BASE + wave * (32 * STG_ROW);
