@@ -157,6 +157,15 @@ int sglamd_fp8_blockwise_scaled_mm_pow2(const void* a, int64_t lda, const void* 
                                         int64_t sb_stride_k, void* out, int64_t ldc, int out_dtype, int64_t M,
                                         int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* sglamd_fp8_blockwise_scaled_mm (scales_pow2 != 0: its _pow2 form) for a linear layer with a bias [N] of the output's
+ * type: out = round(round(a b^T) + bias), what adding the bias to that operator's output gives
+ * (fp8_utils.py:639-641), in one pass.  Any even bias address. */
+int sglamd_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
+                                        int64_t sa_stride_m, int64_t sa_stride_k, const float* sb, int64_t sb_stride_n,
+                                        int64_t sb_stride_k, int scales_pow2, const void* bias, void* out, int64_t ldc,
+                                        int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
+                                        int64_t workspace_bytes, void* stream);
+
 /* The block-scaled GEMM on int8 operands: the int32 partial product of every 128-wide K block is exact and is
  * folded as float(p) * (sa[m, kb] * sb[n/128, kb]) into the fp32 accumulator.  Same arguments as above.
  * Stands in for w8a8_block_int8_matmul (python/sglang/srt/layers/quantization/int8_kernel.py:228-441, a Triton

@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB_PATH = os.path.join(PKG, "libsglamd.so")
 HOST_PATH = os.path.join(PKG, "_C.so")
-SOURCES = ["gemm_mode_block_fp8.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
+SOURCES = ["gemm_mode_block_fp8.hip", "gemm_mode_block_fp8_bias.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
            "moe.hip", "moe_rows.hip", "quant.hip", "gemm.hip", "generic.hip", "ceilings.hip"]
 # packed fp32 ALU forms are switched off on purpose (the -Xclang -target-feature pair below)
 HIPCC_FLAGS = [
@@ -30,7 +30,7 @@ HIPCC_FLAGS = [
 # The GEMM kernels sit at the edge of the 256-VGPR budget their two waves per SIMD leave: a few more live values
 # and the compiler spills accumulators into scratch memory, which still computes the right result, two to ten
 # times slower.  A build in which a kernel of these files uses scratch memory therefore fails.
-NO_SCRATCH = {"gemm_mode_block_fp8.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
+NO_SCRATCH = {"gemm_mode_block_fp8.hip", "gemm_mode_block_fp8_bias.hip", "gemm_mode_row_fp8.hip", "gemm_mode_row_int8.hip", "gemm_mode_block_int8.hip",
               "moe.hip", "moe_rows.hip"}
 
 

@@ -8,6 +8,7 @@ thread_local int last_kernel = 0;
 thread_local int skinny_last_shape = 0;
 
 extern template int dispatch_out<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
+extern template int dispatch_out_biased<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out<GEMM_ROW_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out<GEMM_ROW_INT8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out<GEMM_BLOCK_INT8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
@@ -33,7 +34,8 @@ using namespace sglamd;
 static int blockwise(int mode, const char* op, const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
                      int64_t sa_stride_m, int64_t sa_stride_k, const float* sb, int64_t sb_stride_n,
                      int64_t sb_stride_k, void* out, int64_t ldc, int out_dtype, int64_t M, int64_t N, int64_t K,
-                     void* workspace, int64_t workspace_bytes, void* stream, bool scales_pow2 = false) {
+                     void* workspace, int64_t workspace_bytes, void* stream, bool scales_pow2 = false,
+                     const void* bias = nullptr) {
   const DeviceScope scope;
   int rc = check_common(op, a, b, out, M, N, K, lda, ldb, ldc);
   if (rc) return rc;
@@ -56,6 +58,9 @@ static int blockwise(int mode, const char* op, const void* a, int64_t lda, const
   g.M = (int)M;
   g.N = (int)N;
   g.K = (int)K;
+  g.bias = bias;
+  if (mode == GEMM_BLOCK_FP8 && bias)
+    return dispatch_out_biased<GEMM_BLOCK_FP8>(g, out_dtype, (hipStream_t)stream, workspace, workspace_bytes);
   if (mode == GEMM_BLOCK_FP8)
     return dispatch_out<GEMM_BLOCK_FP8>(g, out_dtype, (hipStream_t)stream, workspace, workspace_bytes);
   return dispatch_out<GEMM_BLOCK_INT8>(g, out_dtype, (hipStream_t)stream, workspace, workspace_bytes);
@@ -77,6 +82,18 @@ extern "C" int sglamd_fp8_blockwise_scaled_mm_pow2(const void* a, int64_t lda, c
                                                    void* workspace, int64_t workspace_bytes, void* stream) {
   return blockwise(GEMM_BLOCK_FP8, "fp8_blockwise_scaled_mm_pow2", a, lda, b, ldb, sa, sa_stride_m, sa_stride_k, sb,
                    sb_stride_n, sb_stride_k, out, ldc, out_dtype, M, N, K, workspace, workspace_bytes, stream, true);
+}
+
+extern "C" int sglamd_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                                   const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
+                                                   const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,
+                                                   int scales_pow2, const void* bias, void* out, int64_t ldc,
+                                                   int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
+                                                   int64_t workspace_bytes, void* stream) {
+  SGLAMD_REQUIRE(bias && ((uintptr_t)bias & 1) == 0, SGLAMD_EINVAL, "fp8_blockwise_scaled_mm_bias: null or odd bias pointer");
+  return blockwise(GEMM_BLOCK_FP8, "fp8_blockwise_scaled_mm_bias", a, lda, b, ldb, sa, sa_stride_m, sa_stride_k, sb,
+                   sb_stride_n, sb_stride_k, out, ldc, out_dtype, M, N, K, workspace, workspace_bytes, stream,
+                   scales_pow2 != 0, bias);
 }
 
 extern "C" int sglamd_int8_blockwise_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,

@@ -603,6 +603,13 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   constexpr int RPI = 64 / LPR;       // rows per wave-wide store
   const int cl = (lane % LPR) * 8;
   const int n = n0 + cl;
+  v4i bias8 = {};
+  if constexpr (out_biased<OT>) {
+    OS b[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) b[r] = ((const OS*)g.bias)[min(n + r, (int)g.N - 1)];
+    __builtin_memcpy(&bias8, b, 16);
+  }
 #pragma unroll 4
   for (int rl = wave * RPI + lane / LPR; rl < BM; rl += NW * RPI) {
     int m = m0 + rl;
@@ -614,7 +621,12 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     }
     if (n >= g.N) continue;
     const uint8_t* src = smem + rl * CROW + cl * 2;
-    const v2i lo = *(const v2i*)src, hi = *(const v2i*)(src + 8);
+    v2i lo = *(const v2i*)src, hi = *(const v2i*)(src + 8);
+    if constexpr (out_biased<OT>) {
+      const v4i w = add_bias8<OT>(v4i{lo[0], lo[1], hi[0], hi[1]}, bias8);
+      lo = v2i{w[0], w[1]};
+      hi = v2i{w[2], w[3]};
+    }
     OS* dst = (OS*)g.C + (int64_t)m * g.ldc + n;
     if (n + 8 <= g.N && ((((uintptr_t)dst) & 15) == 0)) {
       *(v4i*)dst = v4i{lo[0], lo[1], hi[0], hi[1]};
@@ -659,6 +671,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
     const int64_t m = e / g.N;
     const int n = (int)(e % g.N);
+    if constexpr (out_biased<OT>) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[r] = add_bias<OT>(v[r], ((const OS*)g.bias)[n + r]);
+    }
     if (!gemm_is_block(MODE)) {
       const float sam = g.sa[m];
       float sbn[4], bia[4] = {0.f, 0.f, 0.f, 0.f};

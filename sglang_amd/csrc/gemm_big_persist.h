@@ -472,6 +472,21 @@ __global__ __launch_bounds__(512) void gemm8_big_persist_kernel(GemmArgs g0) {
     // 32-row form does not fit beside the operand stages) were measured on the same chip in alternation: 0.2-0.7 %
     // slower, the half-masked staging writes cost more than the fuller lines save.
     __builtin_amdgcn_sched_barrier(0);
+    // Biased: this lane's eight columns of either patch.  Through scalar loads: a vector load would have to wait, in
+    // issue order, for the next tile's first blocks in flight.
+    v4i bias8[2];
+    if constexpr (out_biased<OT>) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int nb = n0 + wn * 64 + j * 32, start = __builtin_amdgcn_readfirstlane(min(nb, g.N - 32));
+        const uint8_t* p = (const uint8_t*)g.bias + (int64_t)start * 2;
+        v16i s;
+        asm volatile("s_nop 4\n\ts_load_dwordx16 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(s) : "s"(p) : "memory");
+        const int piece = ((lane & 3) + ((nb - start) >> 3)) & 3;
+#pragma unroll
+        for (int w = 0; w < 4; w++) bias8[j][w] = piece < 2 ? (piece == 0 ? s[w] : s[4 + w]) : (piece == 2 ? s[8 + w] : s[12 + w]);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < MT; i++) {
 #pragma unroll
@@ -485,7 +500,8 @@ __global__ __launch_bounds__(512) void gemm8_big_persist_kernel(GemmArgs g0) {
 #pragma unroll
         for (int half = 0; half < 2; half++) {
           const int row = (lane >> 2) + 16 * half, piece = lane & 3;
-          const v4i v = *(const v4i*)(stg + row * STG_ROW + piece * 16);
+          v4i v = *(const v4i*)(stg + row * STG_ROW + piece * 16);
+          if constexpr (out_biased<OT>) v = add_bias8<OT>(v, bias8[j]);
           const int m = (L2RES ? om0 : m0) + wm * WTM + i * 32 + row;
           const int n = (L2RES ? on0 : n0) + wn * 64 + j * 32 + piece * 8;
           // rows past M fall outside the descriptor's range and are dropped, columns past N are sent there

@@ -26,6 +26,29 @@ enum { GEMM_BLOCK_FP8 = 0, GEMM_ROW_FP8 = 1, GEMM_ROW_INT8 = 2, GEMM_BLOCK_INT8 
 constexpr bool gemm_is_block(int mode) { return mode == GEMM_BLOCK_FP8 || mode == GEMM_BLOCK_INT8; }
 constexpr bool gemm_is_int8(int mode) { return mode == GEMM_ROW_INT8 || mode == GEMM_BLOCK_INT8; }
 
+// Output type of a dense block-scaled GEMM that adds a bias to its rounded result and rounds again, what out.add_(bias)
+// behind it computes, without that pass over the output.  A type and not an argument: the kernels without a bias are at
+// the edge of their registers and stay as they are.
+template <typename T>
+struct Biased : T {};
+template <typename T>
+constexpr bool out_biased = false;
+template <typename T>
+constexpr bool out_biased<Biased<T>> = true;
+template <typename OT>
+__device__ __forceinline__ float add_bias(float v, typename OT::storage b) {
+  return OT::to_f32(OT::from_f32(v)) + OT::to_f32(b);
+}
+// The same for eight rounded results and eight biases, packed.
+template <typename OT>
+__device__ __forceinline__ v4i add_bias8(v4i v, v4i b) {
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    v[i] = (int)OT::pack2(OT::to_f32((u16)(v[i] & 0xffff)) + OT::to_f32((u16)(b[i] & 0xffff)),
+                          OT::to_f32((u16)((uint32_t)v[i] >> 16)) + OT::to_f32((u16)((uint32_t)b[i] >> 16)));
+  return v;
+}
+
 struct GemmArgs {
   const uint8_t* A;
   int64_t lda;
@@ -38,7 +61,7 @@ struct GemmArgs {
   int64_t sb_sn, sb_sk, sb_se;
   // rowwise MoE: sa[(slot / top_k) * sa_sm] (0: per tensor), sb[e*sb_se + n*sb_sn] (sb_sn 0: per expert), and the
   // bias rows of the experts lie sb_sk elements apart
-  const void* bias;         // rowwise, optional, [N] in the output dtype
+  const void* bias;         // rowwise: optional, [N] in the output dtype; block modes: with a Biased output type
   void* C;
   int64_t ldc;
   int M, N, K;
@@ -371,6 +394,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm8_kernel(GA ga) {
         if constexpr (gemm_is_block(MODE)) {
           v[r] = acc[i][j][r];
           if (MOE && bias) v[r] += OT::to_f32(bias[(n + r) < g.N ? n + r : 0]);
+          if constexpr (out_biased<OT>) v[r] = add_bias<OT>(v[r], bias[(n + r) < g.N ? n + r : 0]);
         } else {
           const float sbn = (n + r) < g.N ? (MOE ? sb_base[(int64_t)(n + r) * gx.row_sb_stride] : g.sb[n + r]) : 0.f;
           if constexpr (MODE == GEMM_ROW_FP8) {

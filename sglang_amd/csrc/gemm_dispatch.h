@@ -127,7 +127,8 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
       if (bm == 128) return gemm8_big_launch<MODE, OT, 4, 2>(g, st, slices, workspace);
       if (big_wgn() == 2) return gemm8_big_launch<MODE, OT, 2, 4>(g, st, slices, workspace);
       if constexpr (gemm_is_block(MODE)) {
-        if (slices == 1 && wgs > 0 && (wgs & 7) == 0 && gemm8_big_persist_ok(g, wgs)) {
+        const bool bias_ok = !out_biased<OT> || (g.N >= 32 && ((uintptr_t)g.bias & 3) == 0);
+        if (slices == 1 && wgs > 0 && (wgs & 7) == 0 && bias_ok && gemm8_big_persist_ok(g, wgs)) {
           if constexpr (MODE == GEMM_BLOCK_FP8) {
             if (g.scales_pow2) {
               RAN(SGLAMD_KERNEL_PERSISTENT256_POW2);
@@ -149,6 +150,14 @@ template <int MODE>
 int dispatch_out(const GemmArgs& g, int out_dtype, hipStream_t st, void* ws, int64_t ws_bytes) {
   if (out_dtype == SGLAMD_BF16) return dispatch_dense<MODE, BF16>(g, st, ws, ws_bytes);
   if (out_dtype == SGLAMD_F16) return dispatch_dense<MODE, F16>(g, st, ws, ws_bytes);
+  return fail(SGLAMD_EINVAL, "out_dtype must be Half or BFloat16");
+}
+
+// The same with a bias: block-scaled modes only (gemm_mode_block_fp8_bias.hip).
+template <int MODE>
+int dispatch_out_biased(const GemmArgs& g, int out_dtype, hipStream_t st, void* ws, int64_t ws_bytes) {
+  if (out_dtype == SGLAMD_BF16) return dispatch_dense<MODE, Biased<BF16>>(g, st, ws, ws_bytes);
+  if (out_dtype == SGLAMD_F16) return dispatch_dense<MODE, Biased<F16>>(g, st, ws, ws_bytes);
   return fail(SGLAMD_EINVAL, "out_dtype must be Half or BFloat16");
 }
 

@@ -630,6 +630,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       for (int r = 0; r < 4; r++) {
         if constexpr (gemm_is_block(MODE)) {
           v[r] = a[r];
+          if constexpr (out_biased<OT>) v[r] = add_bias<OT>(v[r], bias[(n + r) < g.N ? n + r : 0]);
         } else {
           const float sbn = (n + r) < g.N ? sb_row[MOE ? (int64_t)(n + r) * g.sb_sn : n + r] : 0.f;
           if constexpr (MODE == GEMM_ROW_FP8) {

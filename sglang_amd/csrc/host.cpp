@@ -551,10 +551,15 @@ optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws
                                             SGLAMD_QUANT_FORM_RECIPROCAL, st));
     wsp = ws.data_ptr<float>(), ws_n = ws.stride(0), ws_k = ws.stride(1);
   }
+  if (bias) {
+    check(sglamd_fp8_blockwise_scaled_mm_bias(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, ue8m0,
+                                              bias->data_ptr(), out.data_ptr(), n, tag(t), m, n, k,
+                                              wb > 0 ? sc.at(wp) : nullptr, wb, st));
+    return out;
+  }
   auto fn = ue8m0 ? sglamd_fp8_blockwise_scaled_mm_pow2 : sglamd_fp8_blockwise_scaled_mm;
   check(fn(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, out.data_ptr(), n, tag(t), m, n, k,
            wb > 0 ? sc.at(wp) : nullptr, wb, st));
-  if (bias) out.add_(*bias);
   return out;
 }
 
@@ -572,6 +577,16 @@ optional<Tensor> block_matmul(const Tensor& a, const Tensor& b, const Tensor& sa
     return {};
   const c10::DeviceGuard guard(a.device());
   Tensor out = empty({m, n}, out_dtype, a);
+  if (bias && t == kFp8) {
+    void* wp;
+    int64_t wb;
+    const Tensor ws = gemm_workspace(m, n, k, false, a, &wp, &wb);
+    check(sglamd_fp8_blockwise_scaled_mm_bias(a.data_ptr(), k, b.data_ptr(), k, sa.data_ptr<float>(), sa.stride(0),
+                                              sa.stride(1), sb.data_ptr<float>(), sb.stride(0), sb.stride(1), 0,
+                                              bias->data_ptr(), out.data_ptr(), n, tag(out_dtype), m, n, k, wp, wb,
+                                              stream_of(a)));
+    return out;
+  }
   block_matmul_(a, b, sa, sb, out, t == at::kChar, false);
   if (bias) out.add_(*bias);
   return out;
