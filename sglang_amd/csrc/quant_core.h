@@ -214,14 +214,19 @@ struct RowQuantArgs {
   void* q;         // [rows, hidden] bytes
   float* s;        // [rows]
   int64_t hidden;  // a multiple of 8
+  int64_t rows;
 };
 
-template <typename T, bool INT8, bool SILU, int NV>
+// TEAM: lanes that share a row, 32 or 64 (no barrier), a multiple of 64, or 0 for the whole workgroup; `row` is the lane's
+// own and may be past the end, since every lane takes part in the barrier.
+// A row of the experts' activations is 256 to 2048 values: a workgroup per row leaves most of its lanes without work, and
+// the launch is bound by starting workgroups (20025 rows of [256 | 256] 34 us, the 25 MB are worth 5).
+template <typename T, bool INT8, bool SILU, int NV, int TEAM = 0>
 __device__ __forceinline__ void row_quant_body(const RowQuantArgs& a, int64_t row, float* red) {
   typedef typename T::storage S;
   static_assert(sizeof(S) == 2, "16-bit rows");
-  const int nt = (int)blockDim.x, tid = threadIdx.x;
-  const int nvec = (int)(a.hidden >> 3);
+  const int nt = TEAM ? TEAM : (int)blockDim.x, tid = TEAM ? (int)threadIdx.x % (TEAM ? TEAM : 1) : (int)threadIdx.x;
+  const int nvec = row < a.rows ? (int)(a.hidden >> 3) : 0;
   const S* src = (const S*)a.in + row * a.hidden * (SILU ? 2 : 1);
   const S* up = src + a.hidden;
   v4i raw[NV], rup[SILU ? NV : 1];
@@ -250,11 +255,14 @@ __device__ __forceinline__ void row_quant_body(const RowQuantArgs& a, int64_t ro
 #pragma unroll
     for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(T::to_f32(b[j])));
   }
-  amax = group_max<64>(amax);
-  if ((tid & 63) == 0) red[tid >> 6] = amax;
-  __syncthreads();
-  amax = red[0];
-  for (int w = 1; w < (nt >> 6); w++) amax = fmaxf(amax, red[w]);
+  amax = group_max<TEAM == 32 ? 32 : 64>(amax);
+  if constexpr (TEAM != 32 && TEAM != 64) {
+    float* mine = red + ((int)threadIdx.x - tid) / 64;
+    if ((tid & 63) == 0) mine[tid >> 6] = amax;
+    __syncthreads();
+    amax = mine[0];
+    for (int w = 1; w < (nt >> 6); w++) amax = fmaxf(amax, mine[w]);
+  }
 
   float scale, mul;
   if (INT8) {
@@ -265,7 +273,7 @@ __device__ __forceinline__ void row_quant_body(const RowQuantArgs& a, int64_t ro
     scale = amax / 448.0f;
     mul = (scale == 0.f) ? 0.f : 1.0f / scale;
   }
-  if (tid == 0) a.s[row] = scale;
+  if (tid == 0 && row < a.rows) a.s[row] = scale;
   uint8_t* dst = (uint8_t*)a.q + row * a.hidden;
 #pragma unroll
   for (int k = 0; k < NV; k++) {
