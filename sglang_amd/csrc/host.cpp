@@ -58,6 +58,9 @@ void check_input(const Tensor& t, const char* name) {
   TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
 }
 
+// A size that a division below is by: an integer division by zero ends the process with SIGFPE.
+void check_positive(int64_t v, const char* name) { TORCH_CHECK(v > 0, name, " must be positive, but got ", v); }
+
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int64_t up(int64_t a, int64_t b) { return cdiv(a, b) * b; }
 
@@ -91,6 +94,7 @@ int64_t ld(const Tensor& t, int64_t dim) {
 void group_quant(const Tensor& input, const Tensor& q, const Tensor& s, int64_t group, double eps, double lo, double hi,
                  bool ue8m0, int form, bool col_major, bool silu) {
   int64_t hidden = input.size(-1);
+  check_positive(hidden, "hidden size");
   const int64_t rows = input.numel() / hidden;
   if (silu) {  // input rows are [gate | up], the quantised row has half the width (v2.cu:412-424)
     TORCH_CHECK(hidden % 2 == 0 && q.size(-1) == hidden / 2, "output_q must have half of input's last dim");
@@ -126,6 +130,7 @@ void sgl_per_token_group_quant_8bit(const Tensor& input, const Tensor& q, const 
                                     double lo, double hi, bool ue8m0) {
   check_input(input, "input");
   check_input(q, "output_q");
+  check_positive(group, "group_size");
   TORCH_CHECK(input.numel() % group == 0, "input.numel() % group_size must be 0");
   TORCH_CHECK(s.dim() == 2, "output_s.dim() must be 2");
   TORCH_CHECK(input.size(-1) % group == 0, "hidden size must be a multiple of group_size");
@@ -139,6 +144,7 @@ void sgl_per_token_group_quant_8bit_v2(const Tensor& input, const Tensor& q, con
   check_input(q, "output_q");
   TORCH_CHECK(input.numel() > 0, "input.numel() must be > 0");
   TORCH_CHECK(std::abs(1e-10 - eps) < 1e-13, "eps must be 1e-10");
+  check_positive(group, "group_size");
   TORCH_CHECK(input.numel() % group == 0, "input.numel() % group_size must be 0");
   const bool masked = masked_m.has_value();
   TORCH_CHECK(s.dim() == (masked ? 3 : 2), "output_s.dim() must be ", masked ? 3 : 2);
@@ -887,7 +893,10 @@ void fused_moe_block_fp8_gemm_(const Tensor& a, const Tensor& a_scale, const Ten
                                const Tensor& c, const optional<Tensor>& topk_weights, const Tensor& sorted,
                                const Tensor& experts, const Tensor& post_pad, bool mul_routed_weight, int64_t top_k,
                                int64_t block_m) {
-  const int64_t n = b.size(1), k = b.size(2), num_valid = c.numel() / n;
+  const int64_t n = b.size(1), k = b.size(2);
+  check_positive(n, "N");
+  check_positive(block_m, "block_m");
+  const int64_t num_valid = c.numel() / n;
   const bool int8 = a.scalar_type() == at::kChar;
   TORCH_CHECK((int8 || a.scalar_type() == kFp8) && b.scalar_type() == a.scalar_type(),
               "A and B must both be Float8_e4m3fn or both Int8");
@@ -914,7 +923,10 @@ void fused_moe_gemm_any_(const Tensor& a, const Tensor& a_scale, const Tensor& b
                          const optional<Tensor>& topk_weights, const Tensor& sorted, const Tensor& experts,
                          const Tensor& post_pad, bool mul_routed_weight, int64_t top_k, int64_t block_m,
                          const optional<std::vector<int64_t>>& block_shape, const optional<Tensor>& bias) {
-  const int64_t e = b.size(0), n = b.size(1), k = b.size(2), num_valid = c.numel() / n;
+  const int64_t e = b.size(0), n = b.size(1), k = b.size(2);
+  check_positive(n, "N");
+  check_positive(block_m, "block_m");
+  const int64_t num_valid = c.numel() / n;
   TORCH_CHECK((a.scalar_type() == kFp8 || a.scalar_type() == at::kChar) && b.scalar_type() == a.scalar_type(),
               "A and B must both be Float8_e4m3fn or both Int8");
   TORCH_CHECK(a.stride(-1) == 1 && b.stride(-1) == 1 && c.is_contiguous(), "A, B rows and C must be contiguous");
@@ -922,7 +934,10 @@ void fused_moe_gemm_any_(const Tensor& a, const Tensor& a_scale, const Tensor& b
   Tensor as = a_scale, bs = b_scale;
   int64_t bn = 0, bk = 0, a_m, a_k, b_e, b_n, b_k;
   if (block_shape) {
-    bn = block_shape->at(0), bk = block_shape->at(1);
+    TORCH_CHECK(block_shape->size() == 2, "block_shape must be [block_n, block_k]");
+    bn = (*block_shape)[0], bk = (*block_shape)[1];
+    check_positive(bn, "block_n");
+    check_positive(bk, "block_k");
     TORCH_CHECK(as.size(-1) == cdiv(k, bk) && bs.size(-1) == cdiv(k, bk) && bs.size(-2) == cdiv(n, bn),
                 "scale shapes do not match the scale blocks");
     a_m = as.stride(0), a_k = as.stride(1);
