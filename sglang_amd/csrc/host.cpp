@@ -12,6 +12,7 @@
 //   * calls that stand for a whole Python wrapper (quantise + GEMM, a MoE layer).  They take the plain configurations
 //     and answer "not mine" (an empty optional, None in Python) for anything else, before any work: the wrapper then
 //     goes through its steps one by one, which also raise the errors for arguments that are wrong.
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
@@ -63,6 +64,26 @@ void check_positive(int64_t v, const char* name) { TORCH_CHECK(v > 0, name, " mu
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int64_t up(int64_t a, int64_t b) { return cdiv(a, b) * b; }
+
+// Whether somebody between the dispatcher and the kernels has to see the operators that a whole-call function stands for: a
+// dispatch mode (fake tensors, a tracer, functorch) is active on this thread, or a tensor is not a plain dense one (a
+// subclass with its own dispatch, a transform's wrapper, a lazy conjugate or negation).  Then the call is not ours.
+bool is_observed() {
+  const uint64_t usual = c10::default_included_set.raw_repr();
+  return (c10::impl::tls_local_dispatch_key_set().included_.raw_repr() & ~usual) != 0;
+}
+bool is_observed(const Tensor& t) {
+  static const uint64_t plain =
+      c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView,
+                           c10::DispatchKey::AutocastCUDA})
+          .raw_repr();
+  return (t.key_set().raw_repr() & ~plain) != 0;
+}
+bool is_observed(const optional<Tensor>& t) { return t && is_observed(*t); }
+template <typename... Tensors>
+bool any_observed(const Tensors&... tensors) {
+  return is_observed() || (is_observed(tensors) || ...);
+}
 
 Tensor empty(at::IntArrayRef shape, ScalarType t, const Tensor& like) {
   return at::empty(shape, at::TensorOptions().dtype(t).device(like.device()));
@@ -285,6 +306,7 @@ Tensor scale_buffer(const Tensor& like, int64_t rows, int64_t cols, int64_t grou
 // sglang_per_token_group_quant_fp8 / _int8 for a 2-D half-precision input in the reciprocal arithmetic.
 optional<std::tuple<Tensor, Tensor>> group_quant_2d(const Tensor& x, int64_t group, double eps, bool col_major,
                                                     bool aligned, bool ue8m0, bool silu, bool int8) {
+  if (any_observed(x)) return {};
   if (x.dim() != 2 || !x.is_cuda() || !is_half(x.scalar_type()) || !x.is_contiguous()) return {};
   if (group != 16 && group != 32 && group != 64 && group != 128) return {};
   const int64_t rows = x.size(0), width = silu ? x.size(1) / 2 : x.size(1);
@@ -303,6 +325,7 @@ optional<std::tuple<Tensor, Tensor>> group_quant_2d(const Tensor& x, int64_t gro
 
 // sglang_per_token_quant_fp8 / per_token_quant_int8 for a contiguous device tensor.
 optional<std::tuple<Tensor, Tensor>> per_token_quant(const Tensor& x, bool int8) {
+  if (any_observed(x)) return {};
   if (x.dim() < 1 || !x.is_cuda() || !x.is_contiguous() || x.numel() == 0) return {};
   const ScalarType t = x.scalar_type();
   if (!(t == at::kFloat || is_half(t)) || (!int8 && (x.dim() != 2 || x.size(1) % 4))) return {};
@@ -532,6 +555,7 @@ bool plain_bias(const optional<Tensor>& bias, const Tensor& out_like, int64_t n,
 // The block-scaled linear layer (fp8_utils.py:612-642,645-696,814-834): quantise x [m, k] per 1x128 group, multiply by
 // weight [n, k] with 128x128 block scales, add the bias.
 optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws, const optional<Tensor>& bias) {
+  if (any_observed(x, w, ws, bias)) return {};
   const ScalarType t = x.scalar_type();
   if (x.dim() != 2 || !x.is_cuda() || !is_half(t) || !x.is_contiguous() || x.size(0) == 0) return {};
   if (!plain_weight(w, x, kFp8) || w.size(1) != x.size(1) || !plain_block_scale(ws, w)) return {};
@@ -573,6 +597,7 @@ optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws
 // scales, [m, k] x [n, k]; with an optional bias for the linear layers that take quantised inputs.
 optional<Tensor> block_matmul(const Tensor& a, const Tensor& b, const Tensor& sa, const Tensor& sb, ScalarType out_dtype,
                               const optional<Tensor>& bias) {
+  if (any_observed(a, b, sa, sb, bias)) return {};
   const ScalarType t = a.scalar_type();
   if (a.dim() != 2 || !a.is_cuda() || (t != kFp8 && t != at::kChar) || !a.is_contiguous() || a.size(0) == 0) return {};
   if (!plain_weight(b, a, t) || b.size(1) != a.size(1) || !is_half(out_dtype)) return {};
@@ -601,6 +626,7 @@ optional<Tensor> block_matmul(const Tensor& a, const Tensor& b, const Tensor& sa
 // The per-channel FP8 linear layer with per-token activation scales (fp8_utils.py:1458-1560): weight is the [k, n]
 // view of the [n, k] parameter, weight_scale one value per output column.
 optional<Tensor> row_linear(const Tensor& x, const Tensor& weight, const Tensor& ws, const optional<Tensor>& bias) {
+  if (any_observed(x, weight, ws, bias)) return {};
   const ScalarType t = x.scalar_type();
   if (x.dim() != 2 || !x.is_cuda() || !is_half(t) || !x.is_contiguous() || x.size(0) == 0) return {};
   if (weight.dim() != 2 || weight.device() != x.device() || weight.scalar_type() != kFp8 || weight.stride(0) != 1)
@@ -1005,6 +1031,7 @@ optional<Tensor> moe_layer(const Tensor& hidden, const Tensor& w1, const Tensor&
                            const optional<Tensor>& w2_scale, const optional<Tensor>& b1, const optional<Tensor>& b2,
                            const Tensor& topk_weights, const Tensor& topk_ids, bool block, bool int8, bool inplace,
                            double routed_scaling_factor, int64_t block_m) {
+  if (any_observed(hidden, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids)) return {};
   const ScalarType t = hidden.scalar_type(), wt = int8 ? at::kChar : kFp8;
   if (hidden.dim() != 2 || !hidden.is_cuda() || !is_half(t) || !hidden.is_contiguous() || hidden.size(0) == 0) return {};
   const int64_t m = hidden.size(0), h = hidden.size(1);
@@ -1057,6 +1084,7 @@ optional<Tensor> moe_grouped_layer(const Tensor& a, const Tensor& w1, const Tens
                                    const Tensor& w2_scale, const Tensor& topk_weights, const Tensor& topk_ids,
                                    const Tensor& offsets, const Tensor& sizes1, const Tensor& sizes2,
                                    const optional<Tensor>& output) {
+  if (any_observed(a, w1, w2, w1_scale, w2_scale, topk_weights, topk_ids, offsets, sizes1, sizes2, output)) return {};
   const ScalarType t = a.scalar_type();
   if (a.dim() != 2 || !a.is_cuda() || !is_half(t) || !a.is_contiguous() || a.size(0) == 0) return {};
   const int64_t m = a.size(0), k = a.size(1);

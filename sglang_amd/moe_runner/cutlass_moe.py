@@ -18,7 +18,7 @@ from ..moe import (
     shuffle_rows,
     silu_and_mul,
 )
-from ..ops import _C
+from ..ops import _C, eager
 from ..quantization.fp8_kernel import sglang_per_token_group_quant_fp8
 
 
@@ -71,10 +71,11 @@ def cutlass_fused_experts_fp8(
 
     # the whole layer from one native call: the grouped GEMMs gather their rows themselves, so nothing is permuted in
     # memory; offsets and sizes are filled in all the same
-    out = _C.moe_grouped_layer(a, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids, expert_offsets, problem_sizes1,
-                               problem_sizes2, output)
-    if out is not None:
-        return out
+    if eager(a):
+        out = _C.moe_grouped_layer(a, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids, expert_offsets,
+                                   problem_sizes1, problem_sizes2, output)
+        if out is not None:
+            return out
 
     m, topk = topk_ids.shape
     rows = m * topk

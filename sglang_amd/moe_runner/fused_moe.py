@@ -9,7 +9,7 @@ from typing import Any, Dict, List, Optional
 import torch
 
 from ..moe import gelu_and_mul, moe_sum_reduce, silu_and_mul
-from ..ops import _C, fused_moe_block_fp8_gemm_, fused_moe_gemm_any_
+from ..ops import _C, eager, fused_moe_block_fp8_gemm_, fused_moe_gemm_any_
 from ..quantization.fp8_kernel import (
     sglang_per_token_group_quant_fp8,
     sglang_per_token_group_quant_int8,
@@ -160,9 +160,10 @@ def fused_experts_impl(
             "int8 quantization only supports channel-wise quantization except for block-wise quantization"
     # a1_scale / a2_scale only matter for FP8 without block_shape; the block and int8 configurations quantise the
     # activations themselves and, as in the reference, never look at them (fused_moe_triton_kernels.py:752-783)
-    if _plain_gated_silu(activation, is_gated, apply_router_weight_on_input, no_combine, gemm1_alpha, gemm1_limit,
-                         swiglu_limit, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16, per_channel_quant,
-                         a1_scale, a2_scale, block_shape):
+    if eager(hidden_states) and _plain_gated_silu(activation, is_gated, apply_router_weight_on_input, no_combine,
+                                                  gemm1_alpha, gemm1_limit, swiglu_limit, use_fp8_w8a8, use_int8_w8a8,
+                                                  use_int8_w8a16, use_int4_w4a16, per_channel_quant, a1_scale, a2_scale,
+                                                  block_shape):
         # the gated SiLU layer: its launches are issued back to back from one native call
         out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids,
                            block_shape is not None,

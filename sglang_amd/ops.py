@@ -50,3 +50,10 @@ shuffle_rows = _K.shuffle_rows.default
 apply_shuffle_mul_sum = _K.apply_shuffle_mul_sum.default
 fp8_blockwise_scaled_grouped_mm = _K.fp8_blockwise_scaled_grouped_mm.default
 es_fp8_blockwise_scaled_grouped_mm = _K.es_fp8_blockwise_scaled_grouped_mm.default
+
+
+def eager(x: torch.Tensor) -> bool:
+    """Whether the whole-call functions of _C may be tried on `x` at all: a compiler that traces the caller cannot follow
+    them, and a tensor subclass would not get its own type back.  They look at the rest themselves (dispatch modes,
+    transforms, autograd) and answer None; the caller then goes through the operators."""
+    return not torch.compiler.is_compiling() and type(x) is torch.Tensor

@@ -9,7 +9,15 @@ from ..gemm import (
     sgl_per_token_group_quant_8bit,
     sgl_per_token_quant_fp8,
 )
-from ..ops import _C, block_scaled_mm_any_, static_quant_fp8_, tensor_absmax_scale_, ue8m0_unpack_, w8a8_block_fp8_matmul_
+from ..ops import (
+    _C,
+    block_scaled_mm_any_,
+    eager,
+    static_quant_fp8_,
+    tensor_absmax_scale_,
+    ue8m0_unpack_,
+    w8a8_block_fp8_matmul_,
+)
 
 fp8_dtype = torch.float8_e4m3fn
 fp8_max = 448.0
@@ -72,7 +80,7 @@ def sglang_per_token_group_quant_fp8(
     half its width.  `enable_v2=None` picks the second arithmetic for the group sizes it supports."""
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
-    if masked_m is None and enable_v2 is not False:
+    if masked_m is None and enable_v2 is not False and eager(x):
         quantised = _C.group_quant_2d(x, group_size, eps, column_major_scales, scale_tma_aligned, scale_ue8m0,
                                       fuse_silu_and_mul, False)
         if quantised is not None:
@@ -104,7 +112,7 @@ def sglang_per_token_group_quant_int8(x: torch.Tensor, group_size: int, eps: flo
     """int8 sibling (python/sglang/srt/layers/quantization/int8_kernel.py:184-225): row-major fp32 scales."""
     assert x.shape[-1] % group_size == 0
     assert x.is_contiguous()
-    if dtype == torch.int8 and enable_v2 is not False:
+    if dtype == torch.int8 and enable_v2 is not False and eager(x):
         quantised = _C.group_quant_2d(x, group_size, eps, False, False, False, False, True)
         if quantised is not None:
             return quantised
@@ -140,7 +148,7 @@ def sglang_per_token_group_quant_8bit(
 def sglang_per_token_quant_fp8(x: torch.Tensor, dtype: torch.dtype = fp8_dtype):
     """fp8_kernel.py:656-672: one scale per row, shape [rows, 1]."""
     assert x.is_contiguous(), "`x` is not contiguous"
-    if dtype == fp8_dtype:
+    if dtype == fp8_dtype and eager(x):
         quantised = _C.per_token_quant(x, False)
         if quantised is not None:
             return quantised
@@ -236,7 +244,7 @@ def w8a8_block_fp8_matmul(A, B, As, Bs, block_size: List[int], output_dtype: tor
     (what the quantiser writes with scale_ue8m0=True; for the weights the same words on every row of a block)
     are expanded to the fp32 powers of two they stand for by one small launch each; when both operands came with
     such scales the GEMM is told so (the large-tile kernel then applies them inside the MFMA)."""
-    if block_size[0] == 128 and block_size[1] == 128 and A.dtype == fp8_dtype:
+    if block_size[0] == 128 and block_size[1] == 128 and A.dtype == fp8_dtype and eager(A):
         out = _C.block_matmul(A, B, As, Bs, output_dtype, None)
         if out is not None:
             return out

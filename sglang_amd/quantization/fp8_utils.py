@@ -5,7 +5,7 @@ from typing import Callable, List, Optional
 import torch
 
 from ..gemm import fp8_blockwise_scaled_mm, fp8_scaled_mm
-from ..ops import _C, tensor_absmax_scale_
+from ..ops import _C, eager, tensor_absmax_scale_
 from .fp8_kernel import (
     per_token_group_quant_fp8,
     sglang_per_token_group_quant_fp8,
@@ -31,7 +31,7 @@ def _finish(out_2d: torch.Tensor, input: torch.Tensor, bias, dtype: torch.dtype)
 def _plain_block_linear(x, weight, block_size, weight_scale, bias):
     """The layer in one native call where its configuration is the plain one (128x128 scale blocks, whole groups of
     128 columns); None otherwise."""
-    if block_size[0] != 128 or block_size[1] != 128:
+    if block_size[0] != 128 or block_size[1] != 128 or not eager(x):
         return None
     return _C.block_linear(x, weight, weight_scale, bias)
 
@@ -109,9 +109,10 @@ def aiter_w8a8_block_fp8_linear(input, weight, block_size: List[int], weight_sca
     if input_scale.numel() != x_q.shape[0] * (-(-x_q.shape[1] // 128)):
         raise NotImplementedError("the input scale must hold one value per row and 128 columns")
     input_scale = input_scale.view(x_q.shape[0], -1)
-    out = _C.block_matmul(x_q, weight, input_scale, weight_scale, torch.bfloat16, bias)
-    if out is not None:
-        return _finish(out, input, None, torch.bfloat16)
+    if eager(x_q):
+        out = _C.block_matmul(x_q, weight, input_scale, weight_scale, torch.bfloat16, bias)
+        if out is not None:
+            return _finish(out, input, None, torch.bfloat16)
     out = w8a8_block_fp8_matmul(x_q, weight, input_scale, weight_scale, block_size, output_dtype=torch.bfloat16)
     return _finish(out, input, bias, torch.bfloat16)
 
@@ -153,7 +154,7 @@ def apply_fp8_linear(input, weight, weight_scale, input_scale=None, input_scale_
         tensor_absmax_scale_(x if x.is_contiguous() else x.contiguous(), scale)
         x_q, x_scale = static_quant_fp8(x, scale, repeat_scale=True)
     else:
-        out = _C.row_linear(x, weight, weight_scale, bias)
+        out = _C.row_linear(x, weight, weight_scale, bias) if eager(x) else None
         if out is not None:
             return _finish(out, input, None, input.dtype)
         x_q, x_scale = sglang_per_token_quant_fp8(x)

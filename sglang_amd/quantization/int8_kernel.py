@@ -4,7 +4,7 @@ from typing import List
 
 import torch
 
-from ..ops import _C, per_token_quant_int8_, w8a8_block_int8_matmul_
+from ..ops import _C, eager, per_token_quant_int8_, w8a8_block_int8_matmul_
 from .fp8_kernel import sglang_per_token_group_quant_int8
 
 
@@ -12,7 +12,7 @@ def per_token_quant_int8(x: torch.Tensor, scale_dtype=torch.float32, cal_sum: bo
     """Returns (x_q int8 like x, scales [..., 1]); cal_sum additionally returns the row sums."""
     assert x.is_contiguous()
     assert scale_dtype == torch.float32, "only fp32 scales are produced"
-    quantised = _C.per_token_quant(x, True)
+    quantised = _C.per_token_quant(x, True) if eager(x) else None
     if quantised is None:
         x_q = torch.empty_like(x, dtype=torch.int8)
         scales = torch.empty(x.shape[:-1] + (1,), device=x.device, dtype=torch.float32)
@@ -53,7 +53,7 @@ def w8a8_block_int8_matmul(A, B, As, Bs, block_size: List[int], output_dtype: to
     assert A.dtype == torch.int8 and B.dtype == torch.int8
     assert As.dtype == torch.float32 and Bs.dtype == torch.float32
     assert output_dtype in (torch.float16, torch.bfloat16)
-    if block_n == 128 and block_k == 128:
+    if block_n == 128 and block_k == 128 and eager(A):
         out = _C.block_matmul(A, B, As, Bs, output_dtype, None)
         if out is not None:
             return out

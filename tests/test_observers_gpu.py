@@ -1,0 +1,57 @@
+"""Callers that a whole-layer native call must not hide its operators from: transforms, tensor subclasses, autograd."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FP8 = torch.float8_e4m3fn
+M, N, K = 6, 384, 256
+
+
+@pytest.fixture(scope="module")
+def linears(dev):
+    """name -> f(x, bias): every linear layer that has a whole-layer call."""
+    from sglang_amd.quantization import fp8_utils as fu
+    from sglang_amd.quantization.fp8_kernel import sglang_per_token_group_quant_fp8
+
+    g = torch.Generator().manual_seed(0)
+    w = torch.randn(N, K, generator=g).to(FP8).to(dev)
+    ws = (torch.rand(N // 128, K // 128, generator=g) + 0.1).to(dev)
+    packed = torch.full((N, 4), 120, dtype=torch.uint8).view(torch.int32).to(dev)
+    rows = torch.ones(N, 1, device=dev)
+    block = [128, 128]
+
+    def quantised(x, bias):
+        q, s = sglang_per_token_group_quant_fp8(x, 128)
+        return fu.aiter_w8a8_block_fp8_linear(q, w, block, ws, s, bias)
+
+    return {
+        "cutlass": lambda x, b: fu.cutlass_w8a8_block_fp8_linear_with_fallback(x, w, block, ws, None, b),
+        "triton": lambda x, b: fu.triton_w8a8_block_fp8_linear(x, w, block, ws, None, b),
+        "deepgemm": lambda x, b: fu.deepgemm_w8a8_block_fp8_linear_with_fallback(x, w, block, packed, None, b),
+        "aiter": lambda x, b: fu.aiter_w8a8_block_fp8_linear(x, w, block, ws, None, b),
+        "quantised": quantised,
+        "rows": lambda x, b: fu.apply_fp8_linear(x, w.t(), rows, bias=b, use_per_token_if_dynamic=True),
+    }
+
+
+def _operands(dev):
+    g = torch.Generator().manual_seed(1)
+    return torch.randn(M, K, generator=g).bfloat16().to(dev), torch.randn(N, generator=g).bfloat16().to(dev)
+
+
+def test_vmap_over_the_bias(dev, linears):
+    x, bias = _operands(dev)
+    out = torch.func.vmap(lambda b: linears["rows"](x, b))(torch.stack([bias, -bias]))
+    assert torch.equal(out, torch.stack([linears["rows"](x, bias), linears["rows"](x, -bias)]))
+
+
+def test_a_subclass_gets_its_own_type_back(dev, linears):
+    from sglang_amd.quantization.fp8_kernel import sglang_per_token_group_quant_fp8
+
+    class Tagged(torch.Tensor):
+        pass
+
+    x, _ = _operands(dev)
+    q, _ = sglang_per_token_group_quant_fp8(x.as_subclass(Tagged), 128)
+    assert type(q) is Tagged and type(linears["cutlass"](x.as_subclass(Tagged), None)) is Tagged
