@@ -66,8 +66,10 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int64_t up(int64_t a, int64_t b) { return cdiv(a, b) * b; }
 
 // Whether somebody between the dispatcher and the kernels has to see the operators that a whole-call function stands for: a
-// dispatch mode (fake tensors, a tracer, functorch) is active on this thread, or a tensor is not a plain dense one (a
-// subclass with its own dispatch, a transform's wrapper, a lazy conjugate or negation).  Then the call is not ours.
+// dispatch mode (fake tensors, a tracer, functorch) is active on this thread, a tensor is not a plain dense one (a
+// subclass with its own dispatch, a transform's wrapper, a lazy conjugate or negation), or autograd records it, backward
+// or forward (the addition of a bias carries its gradient; the operators say that they have none).  Then the call is not
+// ours.  Below autograd, where a custom operator's implementation runs, nothing is recorded.
 bool is_observed() {
   const uint64_t usual = c10::default_included_set.raw_repr();
   return (c10::impl::tls_local_dispatch_key_set().included_.raw_repr() & ~usual) != 0;
@@ -77,7 +79,9 @@ bool is_observed(const Tensor& t) {
       c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView,
                            c10::DispatchKey::AutocastCUDA})
           .raw_repr();
-  return (t.key_set().raw_repr() & ~plain) != 0;
+  if ((t.key_set().raw_repr() & ~plain) != 0) return true;
+  if (c10::impl::tls_local_dispatch_key_set().excluded_.has_any(c10::autograd_dispatch_keyset)) return false;
+  return (c10::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined();
 }
 bool is_observed(const optional<Tensor>& t) { return t && is_observed(*t); }
 template <typename... Tensors>

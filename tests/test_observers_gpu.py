@@ -55,3 +55,34 @@ def test_a_subclass_gets_its_own_type_back(dev, linears):
     x, _ = _operands(dev)
     q, _ = sglang_per_token_group_quant_fp8(x.as_subclass(Tagged), 128)
     assert type(q) is Tagged and type(linears["cutlass"](x.as_subclass(Tagged), None)) is Tagged
+
+
+LINEARS = ["cutlass", "triton", "deepgemm", "aiter", "quantised", "rows"]
+
+
+@pytest.mark.parametrize("name", LINEARS)
+def test_a_bias_that_requires_grad(dev, linears, name):
+    """Adding the bias to the GEMM's output records it: its gradient is the number of rows.  The row-scaled operator adds
+    it inside and has no backward: its output says that it needs one."""
+    x, bias = _operands(dev)
+    plain = linears[name](x, bias)
+    assert not plain.requires_grad
+    bias.requires_grad_()
+    out = linears[name](x, bias)
+    assert out.requires_grad and torch.equal(out.detach(), plain)
+    if name != "rows":
+        out.sum().backward()
+        assert torch.equal(bias.grad, torch.full_like(bias, M))
+    with torch.no_grad():
+        assert not linears[name](x, bias).requires_grad
+
+
+@pytest.mark.parametrize("name", LINEARS[:-1])
+def test_forward_mode_over_the_bias(dev, linears, name):
+    import torch.autograd.forward_ad as forward_ad
+
+    x, bias = _operands(dev)
+    tangent = torch.arange(N, device=dev).bfloat16()
+    with forward_ad.dual_level():
+        out = linears[name](x, forward_ad.make_dual(bias, tangent))
+        assert torch.equal(forward_ad.unpack_dual(out).tangent, tangent.expand(M, N))
