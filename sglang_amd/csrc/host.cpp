@@ -1210,6 +1210,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("fp8_max") = 448.0);
   m.def("per_token_quant_int8_", &per_token_quant_int8_, Unlocked());
   m.def("ue8m0_unpack_", &ue8m0_unpack_, Unlocked(), py::arg("packed"), py::arg("rows"), py::arg("groups"), py::arg("row_step") = 1);
+  m.def("any_observed", [](const std::vector<optional<Tensor>>& tensors) {
+    return is_observed() || std::any_of(tensors.begin(), tensors.end(), [](const auto& t) { return is_observed(t); });
+  });
   m.def("group_quant_2d", &group_quant_2d, Unlocked());
   m.def("per_token_quant", &per_token_quant, Unlocked());
   m.def("fused_rms_group_quant", &fused_rms_group_quant, Unlocked());

@@ -345,13 +345,11 @@ _inplace_op = _register_custom_op(inplace_fused_experts, ["hidden_states"])
 _outplace_op = _register_custom_op(outplace_fused_experts, [])
 
 
-def _needs_operator(hidden_states: torch.Tensor) -> bool:
+def _needs_operator(hidden_states: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
     """Whether somebody has to see the layer as one operator node: a compiler or another tracing mode, a tensor
-    subclass, autograd.  Otherwise the function behind the operator is called as it is (the Python side of a custom
-    operator costs about 20 us a call, as much as a quarter of a one-token layer)."""
-    return (torch.compiler.is_compiling() or type(hidden_states) is not torch.Tensor
-            or torch._C._len_torch_dispatch_stack() > 0
-            or (hidden_states.requires_grad and torch.is_grad_enabled()))
+    subclass, autograd through any of the tensors.  Otherwise the function behind the operator is called as it is (the
+    Python side of a custom operator costs about 20 us a call, as much as a quarter of a one-token layer)."""
+    return not eager(hidden_states) or _C.any_observed([hidden_states, *others])
 
 
 def fused_experts(
@@ -379,16 +377,18 @@ def fused_experts(
     configuration picks the in-place or the out-of-place operator."""
     topk_weights, topk_ids, _ = topk_output
     c = moe_runner_config
-    operator = _needs_operator(hidden_states)
-    if not operator and _plain_gated_silu(c.activation, c.is_gated, c.apply_router_weight_on_input, c.no_combine,
-                                          c.gemm1_alpha, c.gemm1_clamp_limit, c.swiglu_limit, use_fp8_w8a8, use_int8_w8a8,
-                                          use_int8_w8a16, use_int4_w4a16, per_channel_quant, a1_scale, a2_scale,
-                                          block_shape):
+    if eager(hidden_states) and _plain_gated_silu(c.activation, c.is_gated, c.apply_router_weight_on_input, c.no_combine,
+                                                  c.gemm1_alpha, c.gemm1_clamp_limit, c.swiglu_limit, use_fp8_w8a8,
+                                                  use_int8_w8a8, use_int8_w8a16, use_int4_w4a16, per_channel_quant,
+                                                  a1_scale, a2_scale, block_shape):
+        # (declines what _needs_operator is for)
         out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids,
                            block_shape is not None, use_int8_w8a8, c.inplace,
                            1.0 if c.routed_scaling_factor is None else c.routed_scaling_factor, 0)
         if out is not None:
             return hidden_states if c.inplace else out
+    operator = _needs_operator(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, w1_scale, w2_scale, w1_zp, w2_zp,
+                               a1_scale, a2_scale)
     filter_expert = c.num_experts is None or c.num_experts != c.num_local_experts
     if c.inplace:
         assert not c.no_combine, "no combine + inplace makes no sense"

@@ -86,3 +86,38 @@ def test_forward_mode_over_the_bias(dev, linears, name):
     with forward_ad.dual_level():
         out = linears[name](x, forward_ad.make_dual(bias, tangent))
         assert torch.equal(forward_ad.unpack_dual(out).tangent, tangent.expand(M, N))
+
+
+def _moe(dev):
+    """(hidden, tensors by name, f(hidden, tensors, **runner options)) of a small block-scaled layer."""
+    from sglang_amd.moe_runner import MoeRunnerConfig, fused_moe
+
+    g = torch.Generator().manual_seed(2)
+    experts, hidden, inner, topk = 4, 256, 128, 2
+    t = dict(w1=torch.randn(experts, 2 * inner, hidden, generator=g).to(FP8),
+             w2=torch.randn(experts, hidden, inner, generator=g).to(FP8),
+             w1_scale=torch.rand(experts, 2, 2, generator=g) + 0.1, w2_scale=torch.rand(experts, 2, 1, generator=g) + 0.1,
+             topk_weights=torch.rand(M, topk, generator=g))
+    t = {name: v.to(dev) for name, v in t.items()}
+    ids = torch.stack([torch.randperm(experts, generator=g)[:topk] for _ in range(M)]).int().to(dev)
+
+    def layer(h, t, **runner):
+        return fused_moe(h, t["w1"], t["w2"], (t["topk_weights"], ids, None), MoeRunnerConfig(**runner), use_fp8_w8a8=True,
+                         w1_scale=t["w1_scale"], w2_scale=t["w2_scale"], block_shape=[128, 128])
+
+    return torch.randn(M, hidden, generator=g).bfloat16().to(dev), t, layer
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu"])  # the layer as one native call, and step by step
+@pytest.mark.parametrize("name", ["topk_weights", "w1", "w2_scale", "hidden"])
+def test_moe_layer_says_that_it_has_no_backward(dev, name, activation):
+    h, t, layer = _moe(dev)
+    plain = layer(h, t, inplace=False, activation=activation)
+    assert not plain.requires_grad
+    (h if name == "hidden" else t[name]).requires_grad_()
+    out = layer(h, t, inplace=False, activation=activation)
+    assert torch.equal(out.detach(), plain)
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        out.sum().backward()
+    with torch.no_grad():
+        assert not layer(h, t, inplace=False, activation=activation).requires_grad
