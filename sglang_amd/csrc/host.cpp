@@ -89,6 +89,12 @@ bool any_observed(const Tensors&... tensors) {
   return is_observed() || (is_observed(tensors) || ...);
 }
 
+// What an operator that declares the write does for autograd: a tensor saved before it no longer counts as unchanged.
+// (Inference tensors have no version.)
+void written_in_place(const Tensor& t) {
+  if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+}
+
 Tensor empty(at::IntArrayRef shape, ScalarType t, const Tensor& like) {
   return at::empty(shape, at::TensorOptions().dtype(t).device(like.device()));
 }
@@ -1079,6 +1085,7 @@ optional<Tensor> moe_layer(const Tensor& hidden, const Tensor& w1, const Tensor&
                                w2_scale->data_ptr<float>(), b2 ? b2->data_ptr() : nullptr, tw.data_ptr<float>(),
                                ids.data_ptr(), tag(ids.scalar_type()), out.data_ptr(), (float)routed_scaling_factor,
                                (int)block_m, ws.data_ptr(), need, stream_of(hidden)));
+  if (inplace) written_in_place(hidden);
   return out;
 }
 
@@ -1213,6 +1220,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("any_observed", [](const std::vector<optional<Tensor>>& tensors) {
     return is_observed() || std::any_of(tensors.begin(), tensors.end(), [](const auto& t) { return is_observed(t); });
   });
+  m.def("written_in_place", &written_in_place);
   m.def("group_quant_2d", &group_quant_2d, Unlocked());
   m.def("per_token_quant", &per_token_quant, Unlocked());
   m.def("fused_rms_group_quant", &fused_rms_group_quant, Unlocked());

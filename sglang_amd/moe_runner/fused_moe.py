@@ -392,6 +392,8 @@ def fused_experts(
     filter_expert = c.num_experts is None or c.num_experts != c.num_local_experts
     if c.inplace:
         assert not c.no_combine, "no combine + inplace makes no sense"
+        if not operator:
+            _C.written_in_place(hidden_states)
         layer = _inplace_op if operator else inplace_fused_experts
         layer(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
               c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,

@@ -121,3 +121,29 @@ def test_moe_layer_says_that_it_has_no_backward(dev, name, activation):
         out.sum().backward()
     with torch.no_grad():
         assert not layer(h, t, inplace=False, activation=activation).requires_grad
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu"])
+def test_moe_layer_in_place_counts_as_a_write(dev, activation):
+    """A product that saved the hidden states for its backward must not use them after the layer overwrote them."""
+    h, t, layer = _moe(dev)
+    plain = layer(h, t, inplace=False, activation=activation)
+    before = h._version
+    scale = torch.ones(256, dtype=h.dtype, device=dev, requires_grad=True)
+    product = h * scale
+    assert h._version == before
+    assert layer(h, t, inplace=True, activation=activation) is h and torch.equal(h, plain)
+    assert h._version > before
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        product.sum().backward()
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu"])
+def test_moe_layer_in_place_on_inference_tensors(dev, activation):
+    h, t, layer = _moe(dev)
+    plain = layer(h, t, inplace=False, activation=activation)
+    with torch.inference_mode():
+        inner = h.clone()
+        assert torch.equal(layer(inner, t, inplace=True, activation=activation), plain)
+        other = h.clone()
+    assert torch.equal(layer(other, t, inplace=True, activation=activation), plain)  # outside the mode
