@@ -159,7 +159,9 @@ int sglamd_fp8_blockwise_scaled_mm_pow2(const void* a, int64_t lda, const void* 
 
 /* sglamd_fp8_blockwise_scaled_mm (scales_pow2 != 0: its _pow2 form) for a linear layer with a bias [N] of the output's
  * type: out = round(round(a b^T) + bias), what adding the bias to that operator's output gives
- * (fp8_utils.py:639-641), in one pass.  Any even bias address. */
+ * (fp8_utils.py:639-641), in one pass.  Any even bias address; but the persistent large-tile kernel takes a bias only at
+ * a multiple of 4 bytes and N >= 32.  A launch it would have run without the bias goes to one tile per workgroup
+ * otherwise: slower, and another order of the K sum, so equal to the sentence above only to the last place. */
 int sglamd_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
                                         int64_t sa_stride_m, int64_t sa_stride_k, const float* sb, int64_t sb_stride_n,
                                         int64_t sb_stride_k, int scales_pow2, const void* bias, void* out, int64_t ldc,

@@ -562,6 +562,13 @@ bool plain_bias(const optional<Tensor>& bias, const Tensor& out_like, int64_t n,
                    bias->device() == out_like.device());
 }
 
+// Whether a bias goes into the block-scaled GEMM.  The large-tile persistent kernel reads it in aligned words; with any
+// other bias that launch would run one tile per workgroup instead, which is slower and sums in another order, so there
+// the bias is added behind the GEMM and the result is the same wherever the bias lies.
+bool bias_in_gemm(const optional<Tensor>& bias, int64_t n) {
+  return bias && ((uintptr_t)bias->data_ptr() & 3) == 0 && n >= 32;
+}
+
 // The block-scaled linear layer (fp8_utils.py:612-642,645-696,814-834): quantise x [m, k] per 1x128 group, multiply by
 // weight [n, k] with 128x128 block scales, add the bias.
 optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws, const optional<Tensor>& bias) {
@@ -591,7 +598,7 @@ optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws
                                             SGLAMD_QUANT_FORM_RECIPROCAL, st));
     wsp = ws.data_ptr<float>(), ws_n = ws.stride(0), ws_k = ws.stride(1);
   }
-  if (bias) {
+  if (bias_in_gemm(bias, n)) {
     check(sglamd_fp8_blockwise_scaled_mm_bias(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, ue8m0,
                                               bias->data_ptr(), out.data_ptr(), n, tag(t), m, n, k,
                                               wb > 0 ? sc.at(wp) : nullptr, wb, st));
@@ -600,6 +607,7 @@ optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws
   auto fn = ue8m0 ? sglamd_fp8_blockwise_scaled_mm_pow2 : sglamd_fp8_blockwise_scaled_mm;
   check(fn(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, out.data_ptr(), n, tag(t), m, n, k,
            wb > 0 ? sc.at(wp) : nullptr, wb, st));
+  if (bias) out.add_(*bias);
   return out;
 }
 
@@ -618,7 +626,7 @@ optional<Tensor> block_matmul(const Tensor& a, const Tensor& b, const Tensor& sa
     return {};
   const c10::DeviceGuard guard(a.device());
   Tensor out = empty({m, n}, out_dtype, a);
-  if (bias && t == kFp8) {
+  if (t == kFp8 && bias_in_gemm(bias, n)) {
     void* wp;
     int64_t wb;
     const Tensor ws = gemm_workspace(m, n, k, false, a, &wp, &wb);
