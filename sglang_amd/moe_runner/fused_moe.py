@@ -171,6 +171,16 @@ def fused_experts_impl(
                            0 if config is None else config["BLOCK_SIZE_M"])
         if out is not None:
             return out
+    return _step_by_step(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, inplace, activation, is_gated,
+                         apply_router_weight_on_input, use_int8_w8a8, per_channel_quant, w1_scale, w2_scale, a1_scale,
+                         a2_scale, block_shape, no_combine, routed_scaling_factor, gemm1_alpha, gemm1_limit, swiglu_limit,
+                         config)
+
+
+def _step_by_step(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, inplace, activation, is_gated,
+                  apply_router_weight_on_input, use_int8_w8a8, per_channel_quant, w1_scale, w2_scale, a1_scale, a2_scale,
+                  block_shape, no_combine, routed_scaling_factor, gemm1_alpha, gemm1_limit, swiglu_limit, config):
+    """The kernel sequence of fused_moe.py:401-785 for any implemented configuration, operator by operator."""
     assert hidden_states.shape[1] == w1.shape[2], "Hidden size mismatch"
     assert topk_weights.shape == topk_ids.shape, "topk shape mismatch"
     assert hidden_states.is_contiguous(), "Hidden_states must be contiguous"
@@ -251,6 +261,8 @@ def fused_experts_impl(
     if routed_scaling_factor is None:
         routed_scaling_factor = 1.0
     moe_sum_reduce(intermediate_cache3, out_hidden_states, routed_scaling_factor)
+    if inplace:
+        _C.written_in_place(hidden_states)
     return out_hidden_states
 
 
@@ -377,23 +389,28 @@ def fused_experts(
     configuration picks the in-place or the out-of-place operator."""
     topk_weights, topk_ids, _ = topk_output
     c = moe_runner_config
-    if eager(hidden_states) and _plain_gated_silu(c.activation, c.is_gated, c.apply_router_weight_on_input, c.no_combine,
-                                                  c.gemm1_alpha, c.gemm1_clamp_limit, c.swiglu_limit, use_fp8_w8a8,
-                                                  use_int8_w8a8, use_int8_w8a16, use_int4_w4a16, per_channel_quant,
-                                                  a1_scale, a2_scale, block_shape):
+    plain = eager(hidden_states) and _plain_gated_silu(
+        c.activation, c.is_gated, c.apply_router_weight_on_input, c.no_combine, c.gemm1_alpha, c.gemm1_clamp_limit,
+        c.swiglu_limit, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16, per_channel_quant, a1_scale, a2_scale,
+        block_shape)
+    if plain:
         # (declines what _needs_operator is for)
         out = _C.moe_layer(hidden_states, w1, w2, w1_scale, w2_scale, b1, b2, topk_weights, topk_ids,
                            block_shape is not None, use_int8_w8a8, c.inplace,
                            1.0 if c.routed_scaling_factor is None else c.routed_scaling_factor, 0)
         if out is not None:
             return hidden_states if c.inplace else out
-    operator = _needs_operator(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, w1_scale, w2_scale, w1_zp, w2_zp,
-                               a1_scale, a2_scale)
-    filter_expert = c.num_experts is None or c.num_experts != c.num_local_experts
     if c.inplace:
         assert not c.no_combine, "no combine + inplace makes no sense"
-        if not operator:
-            _C.written_in_place(hidden_states)
+    operator = _needs_operator(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, w1_scale, w2_scale, w1_zp, w2_zp,
+                               a1_scale, a2_scale)
+    if plain and not operator:  # sizes, strides or types that the native layer does not take
+        return _step_by_step(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.inplace, c.activation, c.is_gated,
+                             c.apply_router_weight_on_input, use_int8_w8a8, per_channel_quant, w1_scale, w2_scale, a1_scale,
+                             a2_scale, block_shape, c.no_combine, c.routed_scaling_factor, c.gemm1_alpha,
+                             c.gemm1_clamp_limit, c.swiglu_limit, None)
+    filter_expert = c.num_experts is None or c.num_experts != c.num_local_experts
+    if c.inplace:
         layer = _inplace_op if operator else inplace_fused_experts
         layer(hidden_states, w1, w2, topk_weights, topk_ids, b1, b2, c.activation, c.is_gated,
               c.apply_router_weight_on_input, use_fp8_w8a8, use_int8_w8a8, use_int8_w8a16, use_int4_w4a16,
