@@ -244,7 +244,7 @@ def w8a8_block_fp8_matmul(A, B, As, Bs, block_size: List[int], output_dtype: tor
     (what the quantiser writes with scale_ue8m0=True; for the weights the same words on every row of a block)
     are expanded to the fp32 powers of two they stand for by one small launch each; when both operands came with
     such scales the GEMM is told so (the large-tile kernel then applies them inside the MFMA)."""
-    if block_size[0] == 128 and block_size[1] == 128 and A.dtype == fp8_dtype and eager(A):
+    if list(block_size) == [128, 128] and A.dtype == fp8_dtype and eager(A):
         out = _C.block_matmul(A, B, As, Bs, output_dtype, None)
         if out is not None:
             return out

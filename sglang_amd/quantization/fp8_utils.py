@@ -31,7 +31,7 @@ def _finish(out_2d: torch.Tensor, input: torch.Tensor, bias, dtype: torch.dtype)
 def _plain_block_linear(x, weight, block_size, weight_scale, bias):
     """The layer in one native call where its configuration is the plain one (128x128 scale blocks, whole groups of
     128 columns); None otherwise."""
-    if block_size[0] != 128 or block_size[1] != 128 or not eager(x):
+    if list(block_size) != [128, 128] or not eager(x):
         return None
     return _C.block_linear(x, weight, weight_scale, bias)
 

@@ -363,3 +363,17 @@ def test_topk_sigmoid_argument_checks(sa, dev):
     with pytest.raises(RuntimeError, match="topk must be less than or equal to num_experts"):
         sa.topk_sigmoid(torch.empty(4, 9, device=dev), torch.empty(4, 9, device=dev, dtype=torch.int32),
                         torch.zeros(4, 8, device=dev), False, None)
+
+
+def test_block_sizes_of_more_than_two_numbers_are_refused(sa, dev):
+    """fp8_kernel.py:1143 asserts two; the whole-layer call must not take the first two of three."""
+    from sglang_amd.quantization.fp8_kernel import w8a8_block_fp8_matmul
+    from sglang_amd.quantization.fp8_utils import dispatch_w8a8_block_fp8_linear
+
+    w = torch.ones(256, 256, device=dev).to(torch.float8_e4m3fn)
+    scale = torch.ones(2, 2, device=dev)
+    for block in ([128, 128, 128], (128, 128, 64)):
+        with pytest.raises(AssertionError):
+            dispatch_w8a8_block_fp8_linear()(torch.ones(4, 256, dtype=torch.bfloat16, device=dev), w, block, scale)
+        with pytest.raises(AssertionError):
+            w8a8_block_fp8_matmul(w[:4], w, torch.ones(4, 2, device=dev), scale, block, torch.bfloat16)
