@@ -172,7 +172,8 @@ __device__ __forceinline__ float wave_pick(float (&v)[EPL], int fallback, float 
 }
 
 // n / d for 0 <= n < 2^31 and a divisor known on the host: one 32 x 32 -> high 32 bit multiply, an add and a shift
-// (round-up method).  A 64-bit division by a kernel argument is over a hundred instructions.
+// (T. Granlund and P. Montgomery, Division by Invariant Integers using Multiplication, 1994: the round-up method).
+// A 64-bit division by a kernel argument is over a hundred instructions.
 struct FastDiv {
   uint32_t mul, shift;
   static FastDiv of(uint32_t d) {

@@ -52,8 +52,10 @@ constexpr int gemm8_big_smem() {
 // offset: 64 experts of [3072, 4096] at 28 rows stream at 4.2 TB/s, of [3072, 3968] at 5.2.  So every expert starts
 // elsewhere.  By the expert and nothing else: an expert's blocks share their weights through L2, and a gate column sums
 // in the order of its up column however the columns are tiled.  First GEMM of that layer 191 -> 154 us, [4096, 8192] 459
-// -> 399; layers of 8 to 32 experts with K = 4096 or 8192 gain 4-20 % in every scaling mode; pitches of 1024, 2048, 3072,
-// 5120, 6144, 7168 bytes do not change and keep their order of summation.
+// -> 399.  Whole layers of 8 to 256 experts with K = 4096 or 8192, 171 sizes in either scaling: 1.045x in the mean and up
+// to 1.18x; the losses are 64 experts of 1024 x 8192 (0.96x, two rounds of tiles).  Pitches of 1024, 2048, 3072, 5120,
+// 6144, 7168 bytes do not change and keep their order of summation.
+constexpr int MOE_ROTATE_MAX_TILES = 3 * 256;  // one-tile kernel: three rounds of the MI355X's 256 CUs
 __device__ __forceinline__ int moe_k_rotation(int64_t pitch, int expert, int nkb) {
   if (pitch & 4095) return 0;
   return __builtin_amdgcn_readfirstlane((int)((unsigned)(expert * 5) % (unsigned)nkb));
@@ -200,9 +202,10 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   const int kb_begin = (int)((int64_t)nkb_all * blockIdx.y / gridDim.y);
   const int kb_end = (int)((int64_t)nkb_all * (blockIdx.y + 1) / gridDim.y);
   const int nkb = kb_end - kb_begin;
-  // MoE: up to three rounds of one tile per CU; in a longer launch the workgroups have drifted apart by themselves and
-  // the rotation gives nothing (-6 to +3 % at 1024 to 1536 tiles)
-  const int rot = MOE && moe_tiles <= 768 ? moe_k_rotation(g.ldb, max(expert, 0), nkb) : 0;
+  // MoE: up to three rounds of one tile per CU (layers whose first GEMM has 513 to 768 tiles: 0.98 to 1.12x, 1.044x in
+  // the mean).  In the fourth round it gives nothing (0.98 to 1.04x, mean 1.002x); beyond, at 1536 tiles, the rotation
+  // would be ahead again (1.02 to 1.07x on two layers), which this rule leaves.
+  const int rot = MOE && moe_tiles <= MOE_ROTATE_MAX_TILES ? moe_k_rotation(g.ldb, max(expert, 0), nkb) : 0;
 
   // The loads are written as assembly so that the compiler's own wait-count bookkeeping does not know them:
   // it treats a direct-to-LDS load as a store every later LDS read might alias and would wait for all of them

@@ -959,9 +959,13 @@ bool moe_small_launch(int E, int64_t I) { return I > 0 && (int64_t)E * ceil_div(
 // A layer whose first GEMM would leave CUs idle in any height: how many tiles it has in 64-slot blocks (every expert's last
 // block half full) says how short its blocks may be.  While those fit one round, a tile's time is the launch's time and
 // the shortest tile wins; a little above, 128-slot blocks, up to the rows where two of them hold an expert.  0: no opinion.
-// Seventeen layers (4 to 64 experts of 256 to 1536, K from 1024 to 7168) at 54 to 500 rows, this rule against the bands below:
-// block-scaled 1.0 to 1.39x, row-scaled 1.0 to 1.37x; where the sweep was mixed (row-scaled at 73 to 112 rows, 128 slots above
-// 215 rows) the bands stay.
+// Twenty layers (4 to 256 experts of 256 to 2048, K from 1024 to 7168) at 12 to 500 rows, this rule against the bands below
+// where the two differ, mean and range:
+//   rows            52..72            73..104           105..169          170..215          above 215
+//   block, 64   1.05 (0.93-1.21)  1.16 (1.10-1.22)  1.17 (1.00-1.39)  1.10 (1.09-1.12)  1.14 (1.00-1.23)
+//   row, 64     1.09 (1.05-1.13)         -          1.11 (0.97-1.25)  1.10 (1.09-1.11)  1.11 (0.98-1.25)
+// 128 slots at 105..169 rows: 1.00 (0.94-1.10) block-scaled, 0.94 (two points) row-scaled.  Where an earlier sweep was mixed
+// (row-scaled at 73 to 112 rows, 128 slots above 215 rows) the bands stay.
 int moe_one_round_block(double rows, int E, int64_t I, bool row_scaled) {
   if (I <= 0 || rows <= 52) return 0;
   const double tiles = E * (rows / 64 + 0.5) * (double)ceil_div(2 * I, 256) * 256.0 / device_cus();
@@ -986,9 +990,11 @@ int moe_auto_block(int64_t M, int E, int topk, int64_t I) {
   // persistent walk, whose first GEMM also applies the activation), and 192-slot blocks once experts start to
   // overflow 128 slots (an expert's second block streams nothing new but still costs a tile).
   // Layers whose tiles do not fill the chip take one round whatever the height, so the shorter block wins where it holds
-  // an expert, and two full blocks of 128 beat 192 where half of the experts overflow those.  Seven layers of 8 to 64
-  // experts: 64 at 20..48 rows 4-14 % faster on each, 128 at 176..208 rows 15-29 %; in the bands between, the layers
-  // disagree by as much in both directions.
+  // an expert, and two full blocks of 128 beat 192 where half of the experts overflow those.  Sixteen such layers of 4 to 64
+  // experts: 64 at 14..52 rows 1.05x in the mean (0.94-1.11), 128 at 170..215 rows 1.17x (0.84-1.33, two of 48 points
+  // below 0.98); in the bands between, the layers disagree by as much in both directions.  (At 12 and 16 rows
+  // the streaming kernel would be ahead on layers of few experts, 1.35-1.55x at 4 and 0.99-1.40x at 8 of them, and behind
+  // from 64 on; this rule does not look.)
   const bool small = moe_small_launch(E, I);
   if (rows < 10) return 16;
   if (const int block = moe_one_round_block(rows, E, I, false)) return block;
@@ -998,9 +1004,9 @@ int moe_auto_block(int64_t M, int E, int topk, int64_t I) {
 }
 // The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue, so what counts is how
 // few rows a tile pads: the shortest block that still holds a whole expert (its weights are streamed once).  A layer that
-// fills the chip moves on sooner, since an expert that overflows adds a tile to a full round: measured on three layers
-// of 64 to 256 experts, 128 at 48 rows 1-9 % faster, 192 at 112 rows 2-10 %; on seven smaller ones 64 stays the faster one
-// at 48 rows by 4-15 %, and 128 at 176..208 rows is 12 % ahead of 192.
+// fills the chip moves on sooner, since an expert that overflows adds a tile to a full round.  Sixteen layers of 4 to 64
+// experts that do not fill it, these bands against the ones of a layer that does: 64 at 42..52 rows 1.06x in the mean
+// (0.96-1.11), at 53..56 1.01x (0.82-1.10); 128 at 105..112 rows 1.00x (0.80-1.09), at 170..215 1.10x (0.80-1.23).
 int moe_auto_block_rows(int64_t M, int E, int topk, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;

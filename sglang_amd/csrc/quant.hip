@@ -50,7 +50,7 @@ __device__ __forceinline__ void ue8m0_unpack_one(const Ue8m0Args& u, int64_t idx
 // Both operands' scales of a linear layer with packed UE8M0 weight scales, ready for the GEMM, in one launch: the first
 // `quant_blocks` workgroups quantise the activations (power-of-two scales as floats), the others expand the weights'.
 // In place of three launches (quantise to packed words, expand those, expand the weights'): 300 x 18432 rows against a
-// 7168 x 18432 weight 12.6 -> 6 us.
+// 7168 x 18432 weight 5.0 + 2.4 + 2.7 -> 5.6 us.
 template <typename T>
 __global__ __launch_bounds__(256) void group_quant_unpack_kernel(GroupQuantArgs a, unsigned quant_blocks, Ue8m0Args u) {
   if (blockIdx.x < quant_blocks) {
