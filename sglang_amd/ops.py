@@ -51,9 +51,11 @@ apply_shuffle_mul_sum = _K.apply_shuffle_mul_sum.default
 fp8_blockwise_scaled_grouped_mm = _K.fp8_blockwise_scaled_grouped_mm.default
 es_fp8_blockwise_scaled_grouped_mm = _K.es_fp8_blockwise_scaled_grouped_mm.default
 
+_is_dynamo_compiling, _Tensor = torch.compiler.is_dynamo_compiling, torch.Tensor
+
 
 def eager(x: torch.Tensor) -> bool:
     """Whether the whole-call functions of _C may be tried on `x` at all: a compiler that traces the caller cannot follow
-    them, and a tensor subclass would not get its own type back.  They look at the rest themselves (dispatch modes,
-    transforms, autograd) and answer None; the caller then goes through the operators."""
-    return not torch.compiler.is_compiling() and type(x) is torch.Tensor
+    them, and a tensor subclass would not get its own type back.  They look at the rest themselves (dispatch modes, which
+    the other tracers are, transforms, autograd) and answer None; the caller then goes through the operators."""
+    return not _is_dynamo_compiling() and type(x) is _Tensor
