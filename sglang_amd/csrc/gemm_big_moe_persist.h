@@ -33,11 +33,11 @@
 namespace sglamd {
 
 constexpr int GEMM8_MOE_PERSIST_MAX_KB = 256;  // 2 column blocks x K blocks: 512 table entries, one load per wave
-template <int MT>
+template <int MT, bool ACTQ, bool QUADS>
 constexpr int gemm8_moe_persist_smem() {
-  // two stages of A rows, B rows and A-row scales | 256 bytes for loads that must land nowhere |
-  // two weight-scale tables of 512 floats | eight staging patches of 32 rows x 144 bytes
-  return 2 * ((64 * MT + 256) * 128 + 64 * MT * 4) + 256 + 2 * 2048 + 8 * 4608;
+  // two stages of A rows and B rows, two of A-row scales (QUADS: of four K blocks each) | room for loads that must
+  // land nowhere | two weight-scale tables of 512 floats | eight staging patches of 32 rows x 128 bytes (ACTQ: 48)
+  return 2 * ((64 * MT + 256) * 128 + 64 * MT * (QUADS ? 16 : 4)) + (QUADS ? 1024 : 256) + 2 * 2048 + 8 * (ACTQ ? 32 * 48 : 32 * 128);
 }
 
 // ACTQ (first GEMM of a gated SiLU layer, FP8): the tile pairs 128 gate rows of the weight with their 128 up rows
@@ -45,8 +45,13 @@ constexpr int gemm8_moe_persist_smem() {
 // output sit in one lane -- and the epilogue writes what the unfused sequence's next launch would: silu(gate) * up
 // rounded as silu_and_mul rounds it, group-quantised to e4m3 (one 128-wide group per row and tile, its maximum
 // exchanged between the four waves that share the rows) into g.C ([pairs, N / 2] bytes, g.ldc bytes per row) and
-// the group scales into g.A16 ([pairs, N / 256] floats).  The 16-bit [gate | up] rows never exist.
-template <int MODE, typename OT, int MT, bool ACTQ = false>
+// the group scales into g.A16 ([pairs, N / 256] floats, g.lda16 of them from row to row).  The 16-bit [gate | up] rows never exist.
+//
+// QUADS: the activation-row scales come in aligned groups of four K blocks, one 16-byte load per row every fourth block
+// (a row's scales lie side by side, rows start at multiples of 16 bytes).  Each of a tile's rows is another token, so a
+// load of their scales is 64 cache lines for 64 words, as many requests as four 1 KB loads of its operands, and one load
+// per K block cost the layer 10 %: DeepSeek-V3, 4096 tokens, 2717 us with it, 2448 with the loads sent nowhere.
+template <int MODE, typename OT, int MT, bool ACTQ, bool QUADS>
 __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(gemm_is_block(MODE), "the persistent MoE kernel is built for the block-scaled modes");
@@ -55,9 +60,9 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   constexpr int BM = 64 * MT, BN = 256, WTM = 32 * MT;
   constexpr int A_LOADS = (BM / 8) / NW, APT = A_LOADS / MT;
   static_assert(A_LOADS == MT && APT == 1, "one A load per wave and row tile");
-  constexpr int A_STAGE = BM * 128, B_STAGE = BN * 128, S_STAGE = BM * 4;
+  constexpr int A_STAGE = BM * 128, B_STAGE = BN * 128, S_STAGE = BM * (QUADS ? 16 : 4);
   constexpr int B_BASE = NS * A_STAGE, S_BASE = B_BASE + NS * B_STAGE, NOWHERE = S_BASE + NS * S_STAGE;
-  constexpr int TBL_BASE = NOWHERE + 256, TBL_BYTES = 2048, STG_BASE = TBL_BASE + 2 * TBL_BYTES, STG_ROW = 144;
+  constexpr int TBL_BASE = NOWHERE + (QUADS ? 1024 : 256), TBL_BYTES = 2048, STG_BASE = TBL_BASE + 2 * TBL_BYTES, STG_ROW = ACTQ ? 48 : 128;
   typedef v16f acc16_t;
   typedef typename std::conditional<gemm_is_int8(MODE), v16i, v16f>::type prod16_t;
   typedef typename OT::storage OS;
@@ -97,7 +102,8 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   const int64_t a_rows = g.num_valid / g.top_k;
   const int a_bytes = (int)min(a_rows * g.lda, (int64_t)0x7fffffff);
   const int b_bytes = (int)min((int64_t)g.N * g.ldb, (int64_t)0x7fffffff);
-  const int s_bytes = (int)min(((a_rows - 1) * g.sa_sm + (int64_t)(nkb - 1) * g.sa_sk + 1) * 4, (int64_t)0x7fffffff);
+  const int s_bytes = QUADS ? (int)(((a_rows - 1) * g.sa_sm + ((nkb + 3) & ~3)) * 4)
+                            : (int)min(((a_rows - 1) * g.sa_sm + (int64_t)(nkb - 1) * g.sa_sk + 1) * 4, (int64_t)0x7fffffff);
   const int t_bytes =
       (int)min(((int64_t)((g.N - 1) >> 7) * g.sb_sn + (int64_t)(nkb - 1) * g.sb_sk + 1) * 4, (int64_t)0x7fffffff);
   const int c_bytes = (int)min((int64_t)g.num_valid * g.ldc * (ACTQ ? 1 : 2), (int64_t)0x7fffffff);
@@ -149,7 +155,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     {
       const int tok = s_rows[b][min(wave * 64 + lane, BM - 1)];
       const int srow = tok < g.num_valid ? tok / g.top_k : 0;
-      s_voff = (uint32_t)(srow * (int)g.sa_sm) << 2;
+      s_voff = QUADS && tok >= g.num_valid ? 0x7ffffff0u : (uint32_t)(srow * (int)g.sa_sm) << 2;
     }
     // weight-block scales: entry e = cb * nkb + kb, 64 entries per wave
     const int e = wave * 64 + lane;
@@ -171,6 +177,8 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     kq += nkb & (kq >> 31);
     return kq;
   };
+  // QUADS: byte offsets of the scales of the walk's blocks kb and kb + 1 in the scale stages, which take turns by quad
+  int quad = 0, s_now = 0, s_then = 0;
   auto issue_piece = [&](int kb, int kq, int stage, int t, int part) {
     const bool live = kb < nkb;
     const int koff = kq << 7;
@@ -184,7 +192,11 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
       dma16(Bmat, live ? b_bytes : 0, b_voff[l & 1] + (uint32_t)((l & 2) * 8 * (int)g.ldb), koff,
             B_BASE + stage * B_STAGE + (wave * 4 + l) * 1024);
     }
-    if (t == MT - 1) {
+    if (QUADS && t == MT - 1) {
+      // (no branch: it would split the step, and the compiler clones the K loop and spills)
+      const bool wanted = live && wave < BM / 64 && (kb == 0 || (kq & 3) == 0);
+      dma16(g.sa, wanted ? s_bytes : 0, s_voff, (kq >> 2) << 4, wanted ? S_BASE + quad * S_STAGE + wave * 1024 : NOWHERE);
+    } else if (t == MT - 1) {
       const bool mine = wave < BM / 64;
       dma4(g.sa, (live && mine) ? s_bytes : 0, s_voff, (kq * (int)g.sa_sk) << 2,
            mine ? S_BASE + stage * S_STAGE + wave * 256 : NOWHERE);
@@ -192,12 +204,18 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   };
   auto request_first_blocks = [&]() {
 #pragma unroll
-    for (int st = 0; st < NS; st++)
+    for (int st = 0; st < NS; st++) {
+      const int kq = block_at(st);
+      if (QUADS) {
+        quad = st == 0 ? 0 : ((kq & 3) == 0 ? 1 : 0);
+        (st == 0 ? s_now : s_then) = quad * S_STAGE + (kq & 3) * 4;
+      }
 #pragma unroll
       for (int t = 0; t < MT; t++) {
-        issue_piece(st, block_at(st), st, t, 0);
-        issue_piece(st, block_at(st), st, t, 1);
+        issue_piece(st, kq, st, t, 0);
+        issue_piece(st, kq, st, t, 1);
       }
+    }
   };
   // ids of sorted block pm for this thread's slot, or a padding id when there is no such block
   auto read_id = [&](int p) -> int {
@@ -219,7 +237,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
       xb[h][c] = smem + wm * WTM * 128 + off;
       wb[h][c] = smem + B_BASE + wn * 64 * 128 + off;
     }
-  const float* sa_lds = (const float*)(smem + S_BASE) + wm * WTM + frow;
+  const uint8_t* sa_lds = smem + S_BASE + (wm * WTM + frow) * (QUADS ? 16 : 4);
   auto xfrag = [&](int stage, int t, int h) -> v8i {
     const v4i lo = *(const v4i*)(xb[h][0] + stage * A_STAGE + t * 4096);
     const v4i hi = *(const v4i*)(xb[h][1] + stage * A_STAGE + t * 4096);
@@ -230,7 +248,10 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     const v4i hi = *(const v4i*)(wb[h][1] + stage * B_STAGE + j * 4096);
     return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   };
-  auto xscale = [&](int stage, int t) -> float { return sa_lds[stage * BM + t * 32]; };
+  // scale of row tile t in stage `stage` (QUADS: at offset `at`)
+  auto xscale = [&](int stage, int at, int t) -> float {
+    return QUADS ? *(const float*)(sa_lds + at + t * 512) : *(const float*)(sa_lds + stage * S_STAGE + t * 128);
+  };
 
   acc16_t acc[MT][2];
 #pragma unroll
@@ -326,12 +347,12 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     float sa_nxt, sb_nxt = sb_cur, sb1_nxt = sb1_cur;
     if (!last) {
       x0 = xfrag(cur, i + 1, 0);
-      sa_nxt = xscale(cur, i + 1);
+      sa_nxt = xscale(cur, s_now, i + 1);
       __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
     } else {
       x0 = xfrag(nxt, 0, 0);
       wf[1][0] = wfrag(nxt, 1, 0);
-      sa_nxt = xscale(nxt, 0);
+      sa_nxt = xscale(nxt, s_then, 0);
       sb_nxt = sb_mine[min(kb + 1, nkb - 1)];
       if constexpr (ACTQ) sb1_nxt = sb_mine[nkb + min(kb + 1, nkb - 1)];
       __builtin_amdgcn_sched_group_barrier(0x100, ACTQ ? 7 : 6, 0);
@@ -360,10 +381,15 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
   };
   auto k_block = [&](int kb, auto stage_c) {
     const int kq = block_at(kb + NS);
+    if (QUADS) quad ^= (kq & 3) == 0 ? 1 : 0;
     tile_step(kb, kq, stage_c, std::integral_constant<int, 0>{});
     if constexpr (MT > 1) tile_step(kb, kq, stage_c, std::integral_constant<int, 1>{});
     if constexpr (MT > 2) tile_step(kb, kq, stage_c, std::integral_constant<int, 2>{});
     if constexpr (MT > 3) tile_step(kb, kq, stage_c, std::integral_constant<int, 3>{});
+    if (QUADS) {
+      s_now = s_then;
+      s_then = quad * S_STAGE + (kq & 3) * 4;
+    }
   };
 
   uint8_t* stg = smem + STG_BASE + wave * (32 * STG_ROW);
@@ -388,7 +414,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
       for (int h = 0; h < 2; h++) wf[j][h] = wfrag(0, j, h);
     x0 = xfrag(0, 0, 0);
     x1 = xfrag(0, 0, 1);
-    sa_cur = xscale(0, 0);
+    sa_cur = xscale(0, s_now, 0);
     sb_cur = sb_mine[0];
     if constexpr (ACTQ) sb1_cur = sb_mine[nkb];
 
@@ -421,8 +447,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
     // staging rows (register r of tile (i, j) is C[.. + lane%32][.. + 32*j + 8*(r/4) + 4*(lane/32) + r%4]); 16-byte
     // stores, eight lanes per 128-byte row segment (a store instruction then touches 8 whole lines instead of 16
     // half lines: the vector memory pipe's cost per store follows the number of row segments), rows scattered to
-    // their (token, k) pair.  Staging rows are 144 bytes apart: 16-byte aligned pieces, two-way bank conflicts on
-    // the 8-byte writes at worst.
+    // their (token, k) pair.  The 16-byte pieces of a staging row are XOR-swizzled with its row, like the stages'.
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (ACTQ) {
       // acc[i][0][r] and acc[i][1][r] are gate and up of output column n0 + 32 wn + 8 (r/4) + 4 (lane/32) + r%4.
@@ -465,7 +490,7 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
         }
         const int mine = s_rows[buf_done][trow];
         if (wn == 0 && fk == 0 && mine < g.num_valid)
-          ((float*)g.A16)[(int64_t)mine * (half_n >> 7) + (n0_done >> 7)] = amax * (1.0f / 448.f);
+          ((float*)g.A16)[(int64_t)mine * g.lda16 + (n0_done >> 7)] = amax * (1.0f / 448.f);
         {
           // 32 rows x 32 bytes: two lanes per row, 16 bytes each
           const int row = lane >> 1, piece = lane & 1;
@@ -489,12 +514,12 @@ __global__ __launch_bounds__(512) void gemm8_moe_persist_kernel(GemmArgs g) {
         for (int rq = 0; rq < 4; rq++) {
           const v2i w = {(int)OT::pack2(acc[i][j][rq * 4] * wgt, acc[i][j][rq * 4 + 1] * wgt),
                          (int)OT::pack2(acc[i][j][rq * 4 + 2] * wgt, acc[i][j][rq * 4 + 3] * wgt)};
-          *(v2i*)(stg + frow * STG_ROW + (32 * j + 8 * rq + 4 * fk) * 2) = w;
+          *(v2i*)(stg + frow * STG_ROW + (((4 * j + rq) ^ (frow & 7)) << 4) + 8 * fk) = w;
         }
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const int row = (lane >> 3) + 8 * q, piece = lane & 7;
-        const v4i v = *(const v4i*)(stg + row * STG_ROW + piece * 16);
+        const v4i v = *(const v4i*)(stg + row * STG_ROW + ((piece ^ (row & 7)) << 4));
         const int m = s_rows[buf_done][wm * WTM + i * 32 + row];
         const int n = n0_done + wn * 64 + piece * 8;
         // padding slots and columns past N are sent outside the descriptor's range and dropped
@@ -534,10 +559,17 @@ static inline bool gemm8_moe_persist_ok(const GemmArgs& g) {
          (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll && (int64_t)g.N * g.ldb < 0x7fffffffll;
 }
 
-template <int MODE, typename OT, int MT, bool ACTQ = false>
-static int gemm8_moe_persist_launch(const GemmArgs& g, hipStream_t st) {
-  auto kern = gemm8_moe_persist_kernel<MODE, OT, MT, ACTQ>;
-  constexpr int smem = gemm8_moe_persist_smem<MT>();
+// Whether the activation scales can be fetched in groups of four K blocks: side by side, rows at multiples of 16 bytes
+// that hold whole groups.
+static inline bool gemm8_moe_quad_scales(const GemmArgs& g) {
+  return g.sa_sk == 1 && (g.sa_sm & 3) == 0 && (((g.K >> 7) & 3) == 0 || g.scale_rows_padded) &&
+         (((uintptr_t)g.sa) & 15) == 0 && (int64_t)(g.num_valid / g.top_k) * g.sa_sm * 4 < 0x7fffffffll;
+}
+
+template <int MODE, typename OT, int MT, bool ACTQ, bool QUADS>
+static int gemm8_moe_persist_launch_as(const GemmArgs& g, hipStream_t st) {
+  auto kern = gemm8_moe_persist_kernel<MODE, OT, MT, ACTQ, QUADS>;
+  constexpr int smem = gemm8_moe_persist_smem<MT, ACTQ, QUADS>();
   static SmemAttrOnce attr;
   hipError_t e = raise_dynamic_smem(attr, (const void*)kern, smem);
   if (e != hipSuccess) return fail(SGLAMD_EHIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
@@ -546,6 +578,12 @@ static int gemm8_moe_persist_launch(const GemmArgs& g, hipStream_t st) {
   const int64_t wgs = tiles < device_cus() ? tiles : device_cus();
   hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(512), smem, st, g);
   return check_launch("gemm8_moe_persist");
+}
+
+template <int MODE, typename OT, int MT, bool ACTQ = false>
+static int gemm8_moe_persist_launch(const GemmArgs& g, hipStream_t st) {
+  return gemm8_moe_quad_scales(g) ? gemm8_moe_persist_launch_as<MODE, OT, MT, ACTQ, true>(g, st)
+                                  : gemm8_moe_persist_launch_as<MODE, OT, MT, ACTQ, false>(g, st);
 }
 
 }  // namespace sglamd

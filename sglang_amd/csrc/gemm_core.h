@@ -77,7 +77,8 @@ struct GemmArgs {
   int rows_per_wg;  // skinny kernel: weight rows a workgroup owns (multiple of 4, <= 16*FN); 0 = 16*FN
   // skinny MoE kernel with in-kernel activation quantisation: the 16-bit rows that take A's place.
   // (The persistent MoE kernel with the activation in its epilogue has no such rows and finds the address of
-  // the group scales it writes, fp32 [pairs, N / 256], here: one more argument word would cost a scalar register.)
+  // the group scales it writes, fp32 [pairs, N / 256] at lda16 floats from row to row, here: one more argument word would
+  // cost a scalar register.)
   const void* A16;
   int64_t lda16;       // bytes between rows
   int act_mode;        // 1: quantise the rows of A16 in the kernel
@@ -94,6 +95,8 @@ struct GemmArgs {
   int sorted_stride;
   // block FP8: every scale is a power of two, so a kernel may apply them through the MFMA's scale operands
   int scales_pow2;
+  // MoE, block modes: the rows of `sa` hold whole groups of four floats, the last one padded (host only)
+  int scale_rows_padded;
 };
 
 // What only the generic kernel takes (kept out of GemmArgs: the specialised kernels sit at the edge of their

@@ -604,7 +604,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
                           int64_t ldc, int out_dtype, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                           const int32_t* num_tokens_post_padded, const float* topk_weights, int64_t num_valid_tokens,
                           int top_k, int mul_routed_weight, int block_m, int64_t max_m_blocks, int64_t N, int64_t K,
-                          void* stream) {
+                          void* stream, int scale_rows_padded = 0) {
   const DeviceScope scope;
   SGLAMD_REQUIRE(a && a_scale && w && w_scale && c && sorted_token_ids && expert_ids && num_tokens_post_padded,
                  SGLAMD_EINVAL, "fused_moe_gemm: null pointer");
@@ -644,6 +644,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
   g.top_k = top_k;
   g.num_valid = (int)num_valid_tokens;
   g.mul_weight = mul_routed_weight;
+  g.scale_rows_padded = scale_rows_padded;
   g.max_blocks_m = (int)max_m_blocks;
   hipStream_t st = (hipStream_t)stream;
   if (mode == GEMM_BLOCK_INT8) {
@@ -1196,11 +1197,54 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     if (rc) return rc;
     return sglamd_moe_sum_reduce(ws + w.c3, out, dtype, M, topk, H, routed_scaling_factor, stream);
   }
+  // Where the persistent walk takes the first GEMM, its epilogue applies SiLU * up and the group quantisation
+  // itself and writes the second GEMM's operand directly (same bits as the two launches it replaces).
+  const bool tall = !int8 && (block_m == 192 || (block_m == 128 && moe_persist128_enabled())) && moe_persist_enabled() &&
+                    moe_actq_enabled() && I % 128 == 0;
+  GemmArgs first = {};
+  first.A = ws + w.xq;
+  first.lda = H;
+  first.B = (const uint8_t*)w13;
+  first.ldb = H;
+  first.b_expert_stride = 2 * I * H;
+  first.sa = (const float*)(ws + w.xs);
+  first.sa_sm = KB1;
+  first.sa_sk = 1;
+  first.sb = w13_scale;
+  first.sb_se = (2 * I / 128) * KB1;
+  first.sb_sn = KB1;
+  first.sb_sk = 1;
+  first.C = ws + w.aq;                 // [T, I] e4m3
+  first.ldc = I;
+  first.A16 = ws + w.as;               // [T, I / 128] group scales, written by the kernel
+  first.lda16 = KB2;
+  first.M = (int)T;
+  first.N = (int)(2 * I);
+  first.K = (int)H;
+  first.sorted_ids = sorted;
+  first.expert_ids = expert;
+  first.num_post_pad = post;
+  first.top_k = topk;
+  first.num_valid = (int)T;
+  first.max_blocks_m = (int)w.max_blocks;
+  const bool act_fused = tall && gemm8_moe_persist_ok(first) && (int64_t)(2 * I / 256) * first.max_blocks_m > device_cus();
+  // The persistent walk fetches activation scales in groups of four K blocks: rows of another length are padded, in the
+  // place of the first GEMM's 16-bit output, which does not exist then.
+  const int64_t pitch1 = (KB1 + 3) & ~(int64_t)3, pitch2 = (KB2 + 3) & ~(int64_t)3;
+  const bool padded = act_fused && (pitch1 != KB1 || pitch2 != KB2) && up256(M * pitch1 * 4) + T * pitch2 * 4 <= T * 2 * I * 2;
+  if (padded) {
+    first.sa = (const float*)(ws + w.c1);
+    first.sa_sm = pitch1;
+    first.A16 = ws + w.c1 + up256(M * pitch1 * 4);
+    first.lda16 = pitch2;
+    first.scale_rows_padded = 1;
+  }
   if (!fuse_all) {
     GroupQuantArgs qa = {};
     qa.in = hidden;
     qa.q = ws + w.xq;
-    qa.s = ws + w.xs;
+    qa.s = (void*)first.sa;
+    qa.row_pitch = padded ? pitch1 : 0;
     qa.set_rows(M, H, 128);
     qa.layout = SGLAMD_SCALE_ROW_MAJOR;
     qa.scale_stride = 0;
@@ -1331,46 +1375,14 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     if (rc) return rc;
     return finish();
   }
-  // Where the persistent walk takes the first GEMM, its epilogue applies SiLU * up and the group quantisation
-  // itself and writes the second GEMM's operand directly (same bits as the two launches it replaces).
-  bool act_fused = false;
-  if (!int8 && (block_m == 192 || (block_m == 128 && moe_persist128_enabled())) && moe_persist_enabled() && moe_actq_enabled() &&
-      I % 128 == 0) {
-    GemmArgs g = {};
-    g.A = ws + w.xq;
-    g.lda = H;
-    g.B = (const uint8_t*)w13;
-    g.ldb = H;
-    g.b_expert_stride = 2 * I * H;
-    g.sa = (const float*)(ws + w.xs);
-    g.sa_sm = KB1;
-    g.sa_sk = 1;
-    g.sb = w13_scale;
-    g.sb_se = (2 * I / 128) * KB1;
-    g.sb_sn = KB1;
-    g.sb_sk = 1;
-    g.C = ws + w.aq;                 // [T, I] e4m3
-    g.ldc = I;
-    g.A16 = ws + w.as;               // [T, I / 128] group scales, written by the kernel
-    g.M = (int)T;
-    g.N = (int)(2 * I);
-    g.K = (int)H;
-    g.sorted_ids = sorted;
-    g.expert_ids = expert;
-    g.num_post_pad = post;
-    g.top_k = topk;
-    g.num_valid = (int)T;
-    g.max_blocks_m = (int)w.max_blocks;
-    if (gemm8_moe_persist_ok(g) && (int64_t)(2 * I / 256) * g.max_blocks_m > device_cus()) {
-      if (block_m == 192)
-        rc = dtype == SGLAMD_BF16 ? gemm8_moe_persist_launch<GEMM_BLOCK_FP8, BF16, 3, true>(g, (hipStream_t)stream)
-                                  : gemm8_moe_persist_launch<GEMM_BLOCK_FP8, F16, 3, true>(g, (hipStream_t)stream);
-      else
-        rc = dtype == SGLAMD_BF16 ? gemm8_moe_persist_launch<GEMM_BLOCK_FP8, BF16, 2, true>(g, (hipStream_t)stream)
-                                  : gemm8_moe_persist_launch<GEMM_BLOCK_FP8, F16, 2, true>(g, (hipStream_t)stream);
-      if (rc) return rc;
-      act_fused = true;
-    }
+  if (act_fused) {
+    if (block_m == 192)
+      rc = dtype == SGLAMD_BF16 ? gemm8_moe_persist_launch<GEMM_BLOCK_FP8, BF16, 3, true>(first, (hipStream_t)stream)
+                                : gemm8_moe_persist_launch<GEMM_BLOCK_FP8, F16, 3, true>(first, (hipStream_t)stream);
+    else
+      rc = dtype == SGLAMD_BF16 ? gemm8_moe_persist_launch<GEMM_BLOCK_FP8, BF16, 2, true>(first, (hipStream_t)stream)
+                                : gemm8_moe_persist_launch<GEMM_BLOCK_FP8, F16, 2, true>(first, (hipStream_t)stream);
+    if (rc) return rc;
   }
   if (!act_fused) {
     rc = moe_block_gemm(mode, ws + w.xq, H, (const float*)(ws + w.xs), KB1, 1, w13, 2 * I * H, H, w13_scale,
@@ -1382,9 +1394,9 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
                                           int8 ? 127.f : 448.f, SGLAMD_QUANT_FORM_RECIPROCAL, stream);
     if (rc) return rc;
   }
-  rc = moe_block_gemm(mode, ws + w.aq, I, (const float*)(ws + w.as), KB2, 1, w2, H * I, I, w2_scale, (H / 128) * KB2, KB2,
-                      1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1, grouped ? 0 : 1, block_m,
-                      w.max_blocks, H, I, stream);
+  rc = moe_block_gemm(mode, ws + w.aq, I, (const float*)first.A16, first.lda16, 1, w2, H * I, I, w2_scale,
+                      (H / 128) * KB2, KB2, 1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1,
+                      grouped ? 0 : 1, block_m, w.max_blocks, H, I, stream, first.scale_rows_padded);
   if (rc) return rc;
   return finish();
 }

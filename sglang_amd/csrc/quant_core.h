@@ -28,7 +28,8 @@ struct GroupQuantArgs {
   int groups_per_row;
   FastDiv per_row;         // division by groups_per_row; used while num_groups < 2^31
   int layout;
-  int64_t scale_stride;
+  int64_t scale_stride;    // column-major: between groups
+  int64_t row_pitch;       // row-major: floats from row to row, 0 when the rows are dense
   float eps, min8, max8;
   int form;
   int q_is_fp8;
@@ -87,7 +88,7 @@ __device__ __forceinline__ void group_quant_body(const GroupQuantArgs& a, const 
   // Lanes past the end keep running (they take part in the cross-lane max) on group 0's
   // address range but store nothing.
   const int64_t gg = active ? g : 0;
-  if (SILU || !row_major) locate(gg, row, col);
+  if (SILU || !row_major || a.row_pitch) locate(gg, row, col);
 
   float x[ELEMS];
   float amax = a.eps;
@@ -180,7 +181,7 @@ __device__ __forceinline__ void group_quant_body(const GroupQuantArgs& a, const 
 
   if (sub == 0) {
     if (row_major) {
-      ((float*)a.s)[gg] = s_store;
+      ((float*)a.s)[a.row_pitch ? row * a.row_pitch + col : gg] = s_store;
     } else if (!ue8m0) {
       ((float*)a.s)[(int64_t)col * a.scale_stride + row] = s_store;
     } else {
