@@ -61,6 +61,13 @@ __device__ __forceinline__ int moe_k_rotation(int64_t pitch, int expert, int nkb
   return __builtin_amdgcn_readfirstlane((int)((unsigned)(expert * 5) % (unsigned)nkb));
 }
 
+// Whether the activation scales can be fetched in groups of four K blocks: side by side, rows at multiples of 16 bytes
+// that hold whole groups.
+static inline bool moe_quad_scales(const GemmArgs& g) {
+  return g.sa_sk == 1 && (g.sa_sm & 3) == 0 && (((g.K >> 7) & 3) == 0 || g.scale_rows_padded) &&
+         (((uintptr_t)g.sa) & 15) == 0 && (int64_t)(g.num_valid / g.top_k) * g.sa_sm * 4 < 0x7fffffffll;
+}
+
 // MT = 32-row tiles per wave along M (4 -> 256-row workgroup tile, 2 -> 128-row tile).
 // Split-K: gridDim.y slices of the K blocks; with more than one slice every workgroup stores its fp32
 // partial tile (block mode: already scaled; row mode: raw accumulators) to slab blockIdx.y of g.C, which

@@ -559,13 +559,6 @@ static inline bool gemm8_moe_persist_ok(const GemmArgs& g) {
          (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll && (int64_t)g.N * g.ldb < 0x7fffffffll;
 }
 
-// Whether the activation scales can be fetched in groups of four K blocks: side by side, rows at multiples of 16 bytes
-// that hold whole groups.
-static inline bool gemm8_moe_quad_scales(const GemmArgs& g) {
-  return g.sa_sk == 1 && (g.sa_sm & 3) == 0 && (((g.K >> 7) & 3) == 0 || g.scale_rows_padded) &&
-         (((uintptr_t)g.sa) & 15) == 0 && (int64_t)(g.num_valid / g.top_k) * g.sa_sm * 4 < 0x7fffffffll;
-}
-
 template <int MODE, typename OT, int MT, bool ACTQ, bool QUADS>
 static int gemm8_moe_persist_launch_as(const GemmArgs& g, hipStream_t st) {
   auto kern = gemm8_moe_persist_kernel<MODE, OT, MT, ACTQ, QUADS>;
@@ -582,7 +575,7 @@ static int gemm8_moe_persist_launch_as(const GemmArgs& g, hipStream_t st) {
 
 template <int MODE, typename OT, int MT, bool ACTQ = false>
 static int gemm8_moe_persist_launch(const GemmArgs& g, hipStream_t st) {
-  return gemm8_moe_quad_scales(g) ? gemm8_moe_persist_launch_as<MODE, OT, MT, ACTQ, true>(g, st)
+  return moe_quad_scales(g) ? gemm8_moe_persist_launch_as<MODE, OT, MT, ACTQ, true>(g, st)
                                   : gemm8_moe_persist_launch_as<MODE, OT, MT, ACTQ, false>(g, st);
 }
 

@@ -97,6 +97,8 @@ struct GemmArgs {
   int scales_pow2;
   // MoE, block modes: the rows of `sa` hold whole groups of four floats, the last one padded (host only)
   int scale_rows_padded;
+  // MoE: sorted blocks that the launch is likely to run, 0 when the caller cannot say (host only)
+  int expected_blocks;
 };
 
 // What only the generic kernel takes (kept out of GemmArgs: the specialised kernels sit at the edge of their

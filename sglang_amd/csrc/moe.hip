@@ -252,7 +252,7 @@ __global__ __launch_bounds__(1024) void moe_prologue_kernel(const IdT* __restric
   else if (TABLES && wg == 0)
     moe_align_body<IdT, true>(topk_ids, nullptr, nullptr, nullptr, nullptr, nb, 1, numel, 0, 0, 0, 1, pa);
   else
-    group_quant_body<T, 128>(qa, (int64_t)(wg - (TABLES ? 1 : 0)) * 1024 + threadIdx.x);
+    group_quant_body<T, 128, false, true>(qa, (int64_t)(wg - (TABLES ? 1 : 0)) * 1024 + threadIdx.x);
 }
 
 // The same for the row-scaled layers: one row of hidden states per workgroup behind the sorting ones.
@@ -604,7 +604,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
                           int64_t ldc, int out_dtype, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                           const int32_t* num_tokens_post_padded, const float* topk_weights, int64_t num_valid_tokens,
                           int top_k, int mul_routed_weight, int block_m, int64_t max_m_blocks, int64_t N, int64_t K,
-                          void* stream, int scale_rows_padded = 0) {
+                          void* stream, int scale_rows_padded = 0, int expected_blocks = 0) {
   const DeviceScope scope;
   SGLAMD_REQUIRE(a && a_scale && w && w_scale && c && sorted_token_ids && expert_ids && num_tokens_post_padded,
                  SGLAMD_EINVAL, "fused_moe_gemm: null pointer");
@@ -645,6 +645,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
   g.num_valid = (int)num_valid_tokens;
   g.mul_weight = mul_routed_weight;
   g.scale_rows_padded = scale_rows_padded;
+  g.expected_blocks = expected_blocks;
   g.max_blocks_m = (int)max_m_blocks;
   hipStream_t st = (hipStream_t)stream;
   if (mode == GEMM_BLOCK_INT8) {
@@ -976,62 +977,115 @@ int moe_one_round_block(double rows, int E, int64_t I, bool row_scaled) {
   return tiles <= 200 ? 64 : 0;
 }
 
-int moe_auto_block(int64_t M, int E, int topk, int64_t I) {
+// Tiles of a layer's two GEMMs when every expert owns one block, 256 columns each.
+struct MoeTiles {
+  int64_t first, second;
+};
+MoeTiles moe_one_block_tiles(int E, int64_t H, int64_t I) { return {E * ceil_div(2 * I, 256), E * ceil_div(H, 256)}; }
+// Whether both GEMMs fill the chip, and so run the weight-streaming tile kernel (gemm_moe_stream.h) in its heights.
+bool moe_layer_streams(int E, int64_t H, int64_t I) {
+  const MoeTiles t = moe_one_block_tiles(E, H, I);
+  return moe_stream_enabled() && H > 0 && I > 0 && t.first >= device_cus() && t.second >= device_cus();
+}
+// Rows per expert from which 64-slot blocks take over from the 16-slot ones of the streaming kernel, on layers whose GEMMs
+// fill the chip.  That kernel reads the same bytes, but every 16 rows or 32 columns have a tile of their own and a drain at
+// its end.  Time in 16-slot blocks over time in 64-slot ones, block scales (row scales), at 1 / 2.5 / 6 / 10 rows:
+//   256 experts of 7168 x 2048 1.02 / 1.03 / 1.08 / 1.19 (1.01 / 1.03 / 1.06 / 1.12), 64 of 4096 x 1536 1.11 / 1.09 / 1.11 /
+//   1.18 (1.04 / 1.06 / 1.09 / 1.14), 256 of 2048 x 768 1.07 / 1.08 / 1.29 / 1.38 (1.07 / 1.09 / 1.24 / 1.30), 128 of
+//   2048 x 1024 0.95 / 0.99 / 1.05 / 1.16 (0.99 / 1.05 / 1.10 / 1.18): from 2.5 rows on, from 1 where the weights pass 1 GB;
+//   a second GEMM too short for the tile kernel's pipeline, 64 of 7168 x 512 1.02 / 1.04 / 1.09 / 1.19 (0.91 / 0.95 / 1.01 /
+//   1.05), 128 of 4096 x 256 0.92 / 0.99 / 1.03 / 1.17 (0.82 / 0.91 / 0.95 / 1.04): from 6 (10) on;
+//   a last round of tiles that leaves a sixth of the chip idle or more, 16 of 6144 x 2048 0.82 / 0.93 / 0.96 / 1.13 (0.85 /
+//   0.95 / 0.95 / 1.00), 32 of 5120 x 1536 0.96 / 0.95 / 0.92 / 0.96 (0.95 / 0.93 / 0.91 / 0.93): from 10 on.
+double moe_stream_from(int E, int64_t H, int64_t I, bool row_scaled) {
+  const MoeTiles t = moe_one_block_tiles(E, H, I);
+  auto full = [](int64_t tiles) { return (double)tiles / (ceil_div(tiles, device_cus()) * device_cus()) >= 0.9; };
+  if (!full(t.first) || !full(t.second)) return 10.;
+  if (I < 768 || H < 768) return row_scaled ? 10. : 6.;
+  return 3ll * E * H * I >= 1000000000ll ? 1. : 2.5;
+}
+// Whether a layer's largest expert is likely to fit one block of 64 slots: the mean, plus the spread that the largest of E
+// numbers of rows has.  One expert more than fits adds a tile to every column: 64 experts of 4096 x 1536 at 48 rows, three
+// rounds of tiles that become four, 227 -> 266 us.
+bool moe_fits_64(double rows, int E) { return rows + sqrt(2 * log((double)E) * rows) <= 64; }
+
+int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;  // tuning knob
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
-  // Measured on the DeepSeek-V3 layer (256 experts, top-8), layer time in us by block height:
-  //   rows/expert    8      10     12     16     24     32     48     56     64     96     112    128
-  //   16            1886   2030   2229   2896          5114
-  //   64            1946   1973   1946   1978   2038   2091   2276   2456   2747   3141   3389   4147
-  //   128                         1953   1970   2019   2075   2176   2220   2272   2458   2685   3236
-  //   192                         1976   1989   2024   2068   2184   2233   2287   2482   2577   2672
-  // The streaming kernel (16) wins while an expert's rows fit one MFMA row group.  Above that the tile kernels: 64-slot
-  // blocks for a few more rows, then 128-slot blocks (from there on a launch has more tiles than CUs and runs the
-  // persistent walk, whose first GEMM also applies the activation), and 192-slot blocks once experts start to
-  // overflow 128 slots (an expert's second block streams nothing new but still costs a tile).
+  // Layers that fill the chip, layer time in us by block height (64: the streaming tile kernel; 128 and 192: the persistent
+  // walk), 256 experts of 7168 x 2048, top-8:
+  //   rows/expert    1      3      6      10     16     24     32     48     56     64     96     112    128
+  //   16            1098   1670   1808   2040   2969   4115
+  //   64            1079   1618   1677   1714   1755   1802   1849   1994   2129   2415   3075   3279   3779
+  //   128           1243   1846   1907   1946   1987   2018   2069   2150   2189   2224   2364   2542   3017
+  //   192           1271   1890   1944   1978   2016   2044   2082   2177   2217   2270   2416   2494   2564
+  // Twelve layers of 8 to 256 experts: 64 slots are 1.05-1.2x ahead of 128 while they hold an expert; where there are at
+  // least four rounds of tiles an overflowing expert costs little and they stay ahead to 56 rows.  192 slots once experts
+  // start to overflow 128, and 128 again where half of them would overflow 192 (at 200 rows 1.02-1.2x on eight layers).
+  if (moe_layer_streams(E, H, I)) {
+    if (rows < moe_stream_from(E, H, I, false) || M <= 4) return 16;
+    if (moe_fits_64(rows, E) || (rows <= 56 && moe_one_block_tiles(E, H, I).first >= 4 * device_cus())) return 64;
+    if (rows <= 104 || (rows >= 180 && rows <= 215 && E < 256)) return 128;
+    return 192;
+  }
   // Layers whose tiles do not fill the chip take one round whatever the height, so the shorter block wins where it holds
   // an expert, and two full blocks of 128 beat 192 where half of the experts overflow those.  Sixteen such layers of 4 to 64
   // experts: 64 at 14..52 rows 1.05x in the mean (0.94-1.11), 128 at 170..215 rows 1.17x (0.84-1.33, two of 48 points
-  // below 0.98); in the bands between, the layers disagree by as much in both directions.  (At 12 and 16 rows
-  // the streaming kernel would be ahead on layers of few experts, 1.35-1.55x at 4 and 0.99-1.40x at 8 of them, and behind
-  // from 64 on; this rule does not look.)
+  // below 0.98); in the bands between, the layers disagree by as much in both directions.  Up to 8 experts the 16-slot
+  // blocks stay ahead to 14 rows (8 of 7168 x 2048 1.20x, of 2048 x 1024 1.24x, of 1024 x 2048 1.24x, of 4096 x 1536 0.95x
+  // at 12), from 16 experts on they are level from some 8 rows on.
   const bool small = moe_small_launch(E, I);
-  if (rows < 10) return 16;
+  if (rows < (small && E <= 8 ? 14 : 10)) return 16;
   if (const int block = moe_one_round_block(rows, E, I, false)) return block;
   if (rows < 14 || (small && rows <= 52)) return 64;
   if (rows <= 104 || (small && rows >= 170 && rows <= 215)) return 128;
   return 192;
 }
-// The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue, so what counts is how
-// few rows a tile pads: the shortest block that still holds a whole expert (its weights are streamed once).  A layer that
-// fills the chip moves on sooner, since an expert that overflows adds a tile to a full round.  Sixteen layers of 4 to 64
-// experts that do not fill it, these bands against the ones of a layer that does: 64 at 42..52 rows 1.06x in the mean
-// (0.96-1.11), at 53..56 1.01x (0.82-1.10); 128 at 105..112 rows 1.00x (0.80-1.09), at 170..215 1.10x (0.80-1.23).
-int moe_auto_block_rows(int64_t M, int E, int topk, int64_t I) {
+// The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue; the streaming tile kernel
+// takes 128 slots too.  Against one-tile launches of 128 slots it is 1.07-1.16x ahead on layers that fill the chip, and
+// ahead of 192 slots up to 118 rows (1.04-1.2x at 112 on eight layers) and again from 175 on (1.15-1.27x at 200, 1.0-1.1x at
+// 256, 1.04-1.07x at 400).
+int moe_auto_block_rows(int64_t M, int E, int topk, int64_t H, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
+  if (moe_layer_streams(E, H, I)) {
+    if (rows < moe_stream_from(E, H, I, true)) return 16;
+    if (moe_fits_64(rows, E)) return 64;
+    return rows <= 118 || rows >= 175 ? 128 : 192;
+  }
+  // What counts without it is how few rows a tile pads: the shortest block that still holds a whole expert (its weights are
+  // streamed once).  A layer that fills the chip moves on sooner, since an expert that overflows adds a tile to a full
+  // round.  Sixteen layers of 4 to 64 experts that do not fill it, these bands against the ones of a layer that does: 64 at
+  // 42..52 rows 1.06x in the mean (0.96-1.11), at 53..56 1.01x (0.82-1.10); 128 at 105..112 rows 1.00x (0.80-1.09), at
+  // 170..215 1.10x (0.80-1.23).
   const bool small = moe_small_launch(E, I);
-  if (rows <= 10) return 16;
+  if (rows < (small && E <= 8 ? 14 : 10.001)) return 16;
   if (const int block = moe_one_round_block(rows, E, I, true)) return block;
   if (rows <= (small ? 56 : 42)) return 64;
   if (rows <= (small ? 112 : 104) || (small && rows >= 170 && rows <= 215)) return 128;
   return 192;
 }
-int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1, 0); }
+// Sorted blocks that a layer with evenly spread routing has (GemmArgs::expected_blocks).
+int moe_expected_blocks(int64_t M, int E, int topk, int block_m) {
+  const double rows = (double)M * topk / E;
+  const double used = E * (1 - exp(-rows));
+  return (int)(rows <= 0.7 * block_m ? used + 0.5 : E * (rows / block_m + 0.5));
+}
+int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1, 0, 0); }
 }  // namespace
 
 extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, int64_t I, int E, int topk, int block_m) {
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
-  if (block_m == 0) block_m = moe_auto_block(M, E, topk, I);
+  if (block_m == 0) block_m = moe_auto_block(M, E, topk, H, I);
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
 extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk,
                                                     int block_m) {
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
-  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk, I) : moe_auto_block_rows(M, E, topk, I);
+  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk, H, I) : moe_auto_block_rows(M, E, topk, H, I);
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
@@ -1062,7 +1116,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   SGLAMD_REQUIRE(!row || I <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: intermediate size %lld is beyond %lld",
                  (long long)I, (long long)ROW_QUANT_MAX_HIDDEN);
   SGLAMD_REQUIRE(row || (!b13 && !b2), SGLAMD_ENOTSUP, "fused_moe: biases go with row-scaled weights");
-  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk, I) : moe_auto_block(M, E, topk, I);
+  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I);
   SGLAMD_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128 || block_m == 192, SGLAMD_EINVAL,
                  "fused_moe: block_m must be 16, 32, 64, 128 or 192");
   const MoeWs w = moe_ws_layout(M, H, I, E, topk, block_m);
@@ -1170,6 +1224,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     g.top_k = topk;
     g.num_valid = (int)T;
     g.max_blocks_m = (int)w.max_blocks;
+    g.expected_blocks = moe_expected_blocks(M, E, topk, block_m);
     GemmArgs h = g;
     h.A = ws + w.aq;
     h.lda = I;
@@ -1199,8 +1254,8 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   }
   // Where the persistent walk takes the first GEMM, its epilogue applies SiLU * up and the group quantisation
   // itself and writes the second GEMM's operand directly (same bits as the two launches it replaces).
-  const bool tall = !int8 && (block_m == 192 || (block_m == 128 && moe_persist128_enabled())) && moe_persist_enabled() &&
-                    moe_actq_enabled() && I % 128 == 0;
+  const bool fusable = mode == GEMM_BLOCK_FP8 && moe_actq_enabled();
+  const bool tall = fusable && (block_m == 192 || (block_m == 128 && moe_persist128_enabled())) && moe_persist_enabled();
   GemmArgs first = {};
   first.A = ws + w.xq;
   first.lda = H;
@@ -1227,27 +1282,30 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   first.top_k = topk;
   first.num_valid = (int)T;
   first.max_blocks_m = (int)w.max_blocks;
-  const bool act_fused = tall && gemm8_moe_persist_ok(first) && (int64_t)(2 * I / 256) * first.max_blocks_m > device_cus();
-  // The persistent walk fetches activation scales in groups of four K blocks: rows of another length are padded, in the
-  // place of the first GEMM's 16-bit output, which does not exist then.
+  first.expected_blocks = moe_expected_blocks(M, E, topk, block_m);
+  // These kernels fetch activation scales in groups of four K blocks: rows of another length are padded, in the place of
+  // the first GEMM's 16-bit output, which does not exist then.
   const int64_t pitch1 = (KB1 + 3) & ~(int64_t)3, pitch2 = (KB2 + 3) & ~(int64_t)3;
-  const bool padded = act_fused && (pitch1 != KB1 || pitch2 != KB2) && up256(M * pitch1 * 4) + T * pitch2 * 4 <= T * 2 * I * 2;
-  if (padded) {
-    first.sa = (const float*)(ws + w.c1);
-    first.sa_sm = pitch1;
-    first.A16 = ws + w.c1 + up256(M * pitch1 * 4);
-    first.lda16 = pitch2;
-    first.scale_rows_padded = 1;
-  }
+  const bool ragged = pitch1 != KB1 || pitch2 != KB2;
+  bool padded = fusable && ragged && up256(M * pitch1 * 4) + T * pitch2 * 4 <= T * 2 * I * 2;
+  GemmArgs as_padded = first;
+  as_padded.sa = (const float*)(ws + w.c1);
+  as_padded.sa_sm = pitch1;
+  as_padded.A16 = ws + w.c1 + up256(M * pitch1 * 4);
+  as_padded.lda16 = pitch2;
+  as_padded.scale_rows_padded = 1;
+  const bool streamed = fusable && block_m == 64 && moe_stream_takes<64>(padded ? as_padded : first, true);
+  const bool act_fused = streamed || (tall && gemm8_moe_persist_ok(first) && (int64_t)(2 * I / 256) * first.max_blocks_m > device_cus());
+  padded = padded && act_fused;
+  if (padded) first = as_padded;
   if (!fuse_all) {
     GroupQuantArgs qa = {};
     qa.in = hidden;
     qa.q = ws + w.xq;
     qa.s = (void*)first.sa;
-    qa.row_pitch = padded ? pitch1 : 0;
     qa.set_rows(M, H, 128);
     qa.layout = SGLAMD_SCALE_ROW_MAJOR;
-    qa.scale_stride = 0;
+    qa.scale_stride = first.sa_sm;
     qa.eps = 1e-10f;
     qa.min8 = int8 ? -128.f : -448.f;
     qa.max8 = int8 ? 127.f : 448.f;
@@ -1376,7 +1434,10 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     return finish();
   }
   if (act_fused) {
-    if (block_m == 192)
+    if (streamed)
+      rc = dtype == SGLAMD_BF16 ? gemm8_moe_stream_launch<GEMM_BLOCK_FP8, BF16, 64, true>(first, (hipStream_t)stream)
+                                : gemm8_moe_stream_launch<GEMM_BLOCK_FP8, F16, 64, true>(first, (hipStream_t)stream);
+    else if (block_m == 192)
       rc = dtype == SGLAMD_BF16 ? gemm8_moe_persist_launch<GEMM_BLOCK_FP8, BF16, 3, true>(first, (hipStream_t)stream)
                                 : gemm8_moe_persist_launch<GEMM_BLOCK_FP8, F16, 3, true>(first, (hipStream_t)stream);
     else
@@ -1387,7 +1448,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   if (!act_fused) {
     rc = moe_block_gemm(mode, ws + w.xq, H, (const float*)(ws + w.xs), KB1, 1, w13, 2 * I * H, H, w13_scale,
                         (2 * I / 128) * KB1, KB1, 1, ws + w.c1, 2 * I, dtype, sorted, expert, post, nullptr, T, topk, 0,
-                        block_m, w.max_blocks, 2 * I, H, stream);
+                        block_m, w.max_blocks, 2 * I, H, stream, 0, first.expected_blocks);
     if (rc) return rc;
     rc = sglamd_silu_mul_group_quant_8bit(ws + w.c1, dtype, ws + w.aq, int8 ? SGLAMD_I8 : SGLAMD_FP8_E4M3, ws + w.as, T,
                                           I, 128, SGLAMD_SCALE_ROW_MAJOR, 0, 1e-10f, int8 ? -128.f : -448.f,
@@ -1396,7 +1457,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   }
   rc = moe_block_gemm(mode, ws + w.aq, I, (const float*)first.A16, first.lda16, 1, w2, H * I, I, w2_scale,
                       (H / 128) * KB2, KB2, 1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1,
-                      grouped ? 0 : 1, block_m, w.max_blocks, H, I, stream, first.scale_rows_padded);
+                      grouped ? 0 : 1, block_m, w.max_blocks, H, I, stream, first.scale_rows_padded, first.expected_blocks);
   if (rc) return rc;
   return finish();
 }
@@ -1467,7 +1528,12 @@ extern "C" int sglamd_fused_moe_block_fp8_static(const void* hidden, int dtype, 
                                                  const void* topk_ids, int ids_dtype, void* out,
                                                  float routed_scaling_factor, int block_m, void* stream) {
   SGLAMD_REQUIRE(M > 0 && H > 0 && I > 0 && E > 0 && topk > 0, SGLAMD_EINVAL, "fused_moe_static: bad M/H/I/E/topk");
-  const int64_t need = sglamd_fused_moe_block_fp8_workspace(M, H, I, E, topk, block_m);
+  int64_t need = sglamd_fused_moe_block_fp8_workspace(M, H, I, E, topk, block_m);
+  if (block_m == 0 && need > SGLAMD_MOE_STATIC_SCRATCH_BYTES) {
+    // the shortest blocks pad the sorted list least
+    block_m = 16;
+    need = sglamd_fused_moe_block_fp8_workspace(M, H, I, E, topk, block_m);
+  }
   SGLAMD_REQUIRE(need > 0 && need <= SGLAMD_MOE_STATIC_SCRATCH_BYTES, SGLAMD_EINVAL,
                  "fused_moe_static: M=%lld tokens (H=%lld, I=%lld, E=%d, topk=%d) need %lld bytes of scratch, the "
                  "built-in array holds %lld; use sglamd_fused_moe_block_fp8 with a workspace",

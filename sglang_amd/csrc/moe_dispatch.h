@@ -3,6 +3,7 @@
 #pragma once
 #include "gemm_big.h"
 #include "gemm_big_moe_persist.h"
+#include "gemm_moe_stream.h"
 #include "gemm_skinny.h"
 
 namespace sglamd {
@@ -26,6 +27,20 @@ static inline bool moe_persist128_enabled() {
 // on the DeepSeek-V3 layer) and was only used where every expert owns the same number.  With an expert's blocks
 // meeting in one L2 it is level or ahead at every token count measured (3072 ... 12288: 0 ... -5.5 %), so it runs
 // wherever there are more tiles than CUs.
+static inline bool moe_stream_enabled() {
+  static const int v = getenv("SGLAMD_MOE_STREAM") ? atoi(getenv("SGLAMD_MOE_STREAM")) : 1;
+  return v != 0;
+}
+// Whether the weight-streaming tile kernel takes a launch.  It wants every CU busy: with fewer tiles a CU gets more of the
+// memory's bandwidth than this kernel's chain of K blocks takes (block scales, 12 rows per expert, one-tile kernel over
+// this one: 8 experts of 4096 x 1536 1.27x, 32 of 2048 x 768 1.04x, 16 of 3072 x 1024 1.16x; from one tile per CU on,
+// 16 of 6144 x 2048 0.90x, 32 of 5120 x 1536 0.91x).
+template <int BM>
+static inline bool moe_stream_takes(const GemmArgs& g, bool block) {
+  const int64_t blocks = g.expected_blocks > 0 ? g.expected_blocks : g.max_blocks_m;
+  return moe_stream_enabled() && gemm8_moe_stream_ok<BM>(g, block) && blocks * ((g.N + 255) / 256) * 16 >= (int64_t)device_cus() * 15;
+}
+
 template <int MODE, typename OT>
 static int dispatch_moe_gemm(const GemmArgs& g, int block_m, hipStream_t st) {
   // number of sorted blocks that will actually run is data dependent; every valid slot could own one
@@ -39,6 +54,8 @@ static int dispatch_moe_gemm(const GemmArgs& g, int block_m, hipStream_t st) {
       if (streaming_ok) return gemm8_skinny_launch<2, MODE, OT, true>(g, st, expect);
       return gemm8_launch<32, 128, 1, 2, MODE, OT, true>(g, st);
     case 64:
+      if (moe_stream_takes<64>(g, gemm_is_block(MODE)))
+        return gemm8_moe_stream_launch<MODE, OT, 64>(g, st);
       // the tile kernel with one 32-row tile per wave when its preconditions hold: the streaming kernel spends
       // four MFMA row groups per weight fragment and falls far behind it at this height
       if ((g.K % 128) == 0 && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll &&
@@ -48,6 +65,9 @@ static int dispatch_moe_gemm(const GemmArgs& g, int block_m, hipStream_t st) {
       if (streaming_ok) return gemm8_skinny_launch<4, MODE, OT, true>(g, st, expect);
       return gemm8_launch<64, 128, 2, 2, MODE, OT, true>(g, st);
     case 128:
+      if constexpr (!gemm_is_block(MODE)) {
+        if (moe_stream_takes<128>(g, false)) return gemm8_moe_stream_launch<MODE, OT, 128>(g, st);
+      }
       // 32x32x64-MFMA tile kernel when its preconditions hold (K % 128 == 0, operands below 2 GiB per matrix)
       if ((g.K % 128) == 0 && (g.K >> 7) <= GEMM8_BIG_MAX_KB && (int64_t)(g.num_valid / g.top_k) * g.lda < 0x7fffffffll &&
           (int64_t)g.N * g.ldb < 0x7fffffffll)

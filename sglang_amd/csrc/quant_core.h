@@ -28,8 +28,7 @@ struct GroupQuantArgs {
   int groups_per_row;
   FastDiv per_row;         // division by groups_per_row; used while num_groups < 2^31
   int layout;
-  int64_t scale_stride;    // column-major: between groups
-  int64_t row_pitch;       // row-major: floats from row to row, 0 when the rows are dense
+  int64_t scale_stride;    // column-major: between groups; PITCHED row-major: floats from row to row
   float eps, min8, max8;
   int form;
   int q_is_fp8;
@@ -51,13 +50,13 @@ struct GroupQuantArgs {
 
 // T: input storage tag; GROUP: elements per group.  ELEMS elements per lane (32 bytes),
 // LPG = GROUP / ELEMS lanes share a group.  SILU: input rows are [gate | up] of 2 * hidden and
-// x = T(silu(gate)) * up rounded to T.
+// x = T(silu(gate)) * up rounded to T.  PITCHED: rows of row-major scales lie scale_stride floats apart.
 //
 // HBM-bound as long as its instructions stay few: a wave64 VALU instruction takes a SIMD four cycles, so a lane's 16
 // elements may cost about 350 instructions before the arithmetic is the slower side.  Hence no 64-bit divisions, the
 // clamp as one v_med3_f32 (NaN in, lower bound out, like fmin(fmax())), and silu_rounded.  8192 bf16 rows of
 // 18432 gates and 18432 ups, UE8M0 scales: 170 -> 133 us (5.7 TB/s; a plain copy moves 5.1); of 7168 and 7168: 67 -> 51.
-template <typename T, int GROUP, bool SILU = false>
+template <typename T, int GROUP, bool SILU = false, bool PITCHED = false>
 __device__ __forceinline__ void group_quant_body(const GroupQuantArgs& a, const int64_t lane_global) {
   typedef typename T::storage S;
   constexpr int ELEMS = 32 / (int)sizeof(S);
@@ -88,7 +87,7 @@ __device__ __forceinline__ void group_quant_body(const GroupQuantArgs& a, const 
   // Lanes past the end keep running (they take part in the cross-lane max) on group 0's
   // address range but store nothing.
   const int64_t gg = active ? g : 0;
-  if (SILU || !row_major || a.row_pitch) locate(gg, row, col);
+  if (SILU || !row_major || PITCHED) locate(gg, row, col);
 
   float x[ELEMS];
   float amax = a.eps;
@@ -181,7 +180,7 @@ __device__ __forceinline__ void group_quant_body(const GroupQuantArgs& a, const 
 
   if (sub == 0) {
     if (row_major) {
-      ((float*)a.s)[a.row_pitch ? row * a.row_pitch + col : gg] = s_store;
+      ((float*)a.s)[PITCHED ? row * a.scale_stride + col : gg] = s_store;
     } else if (!ue8m0) {
       ((float*)a.s)[(int64_t)col * a.scale_stride + row] = s_store;
     } else {
