@@ -97,8 +97,8 @@ struct GemmArgs {
   int scales_pow2;
   // MoE, block modes: the rows of `sa` hold whole groups of four floats, the last one padded (host only)
   int scale_rows_padded;
-  // MoE: sorted blocks that the launch is likely to run, 0 when the caller cannot say (host only)
-  int expected_blocks;
+  // MoE: whether the weight-streaming tile kernel is wanted, 1 or -1; 0: the launch decides (host only)
+  int streams;
 };
 
 // What only the generic kernel takes (kept out of GemmArgs: the specialised kernels sit at the edge of their

@@ -604,7 +604,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
                           int64_t ldc, int out_dtype, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                           const int32_t* num_tokens_post_padded, const float* topk_weights, int64_t num_valid_tokens,
                           int top_k, int mul_routed_weight, int block_m, int64_t max_m_blocks, int64_t N, int64_t K,
-                          void* stream, int scale_rows_padded = 0, int expected_blocks = 0) {
+                          void* stream, int scale_rows_padded = 0, int streams = 0) {
   const DeviceScope scope;
   SGLAMD_REQUIRE(a && a_scale && w && w_scale && c && sorted_token_ids && expert_ids && num_tokens_post_padded,
                  SGLAMD_EINVAL, "fused_moe_gemm: null pointer");
@@ -645,7 +645,7 @@ static int moe_block_gemm(int mode, const void* a, int64_t lda, const float* a_s
   g.num_valid = (int)num_valid_tokens;
   g.mul_weight = mul_routed_weight;
   g.scale_rows_padded = scale_rows_padded;
-  g.expected_blocks = expected_blocks;
+  g.streams = streams;
   g.max_blocks_m = (int)max_m_blocks;
   hipStream_t st = (hipStream_t)stream;
   if (mode == GEMM_BLOCK_INT8) {
@@ -982,38 +982,55 @@ struct MoeTiles {
   int64_t first, second;
 };
 MoeTiles moe_one_block_tiles(int E, int64_t H, int64_t I) { return {E * ceil_div(2 * I, 256), E * ceil_div(H, 256)}; }
-// Whether both GEMMs fill the chip, and so run the weight-streaming tile kernel (gemm_moe_stream.h) in its heights.
-bool moe_layer_streams(int E, int64_t H, int64_t I) {
-  const MoeTiles t = moe_one_block_tiles(E, H, I);
-  return moe_stream_enabled() && H > 0 && I > 0 && t.first >= device_cus() && t.second >= device_cus();
-}
-// Rows per expert from which 64-slot blocks take over from the 16-slot ones of the streaming kernel, on layers whose GEMMs
-// fill the chip.  That kernel reads the same bytes, but every 16 rows or 32 columns have a tile of their own and a drain at
-// its end.  Time in 16-slot blocks over time in 64-slot ones, block scales (row scales), at 1 / 2.5 / 6 / 10 rows:
+// Whether a layer is one for the weight-streaming tile kernel (gemm_moe_stream.h; moe_stream_takes says why).
+bool moe_layer_streams(int E, int64_t H, int64_t I) { return moe_stream_enabled() && 3 * E * H * I >= MOE_STREAM_MIN_BYTES; }
+// Rows per expert from which 64-slot blocks take over from the 16-slot ones of the streaming kernel on such layers.  That
+// kernel reads the same bytes, but every 16 rows or 32 columns have a tile of their own and a drain at its end; a last round
+// of tiles that leaves part of the chip idle costs it less.  Time in 16-slot blocks over time in 64-slot ones, weights from
+// HBM, block scales (row scales), at 1 / 2.5 / 6 / 10 rows:
 //   256 experts of 7168 x 2048 1.02 / 1.03 / 1.08 / 1.19 (1.01 / 1.03 / 1.06 / 1.12), 64 of 4096 x 1536 1.11 / 1.09 / 1.11 /
 //   1.18 (1.04 / 1.06 / 1.09 / 1.14), 256 of 2048 x 768 1.07 / 1.08 / 1.29 / 1.38 (1.07 / 1.09 / 1.24 / 1.30), 128 of
-//   2048 x 1024 0.95 / 0.99 / 1.05 / 1.16 (0.99 / 1.05 / 1.10 / 1.18): from 2.5 rows on, from 1 where the weights pass 1 GB;
+//   2048 x 1024 0.95 / 0.99 / 1.05 / 1.16 (0.99 / 1.05 / 1.10 / 1.18): from 2.5 rows on, from 1.5 where the weights pass 1 GB;
 //   a second GEMM too short for the tile kernel's pipeline, 64 of 7168 x 512 1.02 / 1.04 / 1.09 / 1.19 (0.91 / 0.95 / 1.01 /
-//   1.05), 128 of 4096 x 256 0.92 / 0.99 / 1.03 / 1.17 (0.82 / 0.91 / 0.95 / 1.04): from 6 (10) on;
-//   a last round of tiles that leaves a sixth of the chip idle or more, 16 of 6144 x 2048 0.82 / 0.93 / 0.96 / 1.13 (0.85 /
-//   0.95 / 0.95 / 1.00), 32 of 5120 x 1536 0.96 / 0.95 / 0.92 / 0.96 (0.95 / 0.93 / 0.91 / 0.93): from 10 on.
+//   1.05), 64 of 1024 x 512 1.02 / 1.20 / 1.09 / 1.13 (0.93 / 1.08 / 1.02 / 1.03): from 2.5 (6) on;
+//   idle CUs in the first GEMM only, 32 of 2048 x 768 0.87 / 1.05 / 1.13 / 1.13 (0.81 / 0.96 / 1.08 / 1.07), 16 of
+//   4096 x 896 0.82 / 0.94 / 1.05 / 1.01 (0.79 / 0.94 / 1.03 / 0.95): from 3 (4) on;
+//   in the second, 16 of 6144 x 2048 0.82 / 0.93 / 0.96 / 1.13 (0.85 / 0.95 / 0.95 / 1.00), 32 of 5120 x 1536 0.96 / 0.95 /
+//   0.92 / 0.96 (0.95 / 0.93 / 0.91 / 0.93): from 10 (12) on; in both, 16 of 3072 x 1024 0.73 / 0.88 / 0.90 / 0.98 (0.79 /
+//   0.90 / 0.92 / 0.90), 8 of 7168 x 2048 0.67 / 0.92 / 0.85 / 0.98 (0.70 / 0.97 / 0.88 / 0.85): from 13 on.
 double moe_stream_from(int E, int64_t H, int64_t I, bool row_scaled) {
   const MoeTiles t = moe_one_block_tiles(E, H, I);
-  auto full = [](int64_t tiles) { return (double)tiles / (ceil_div(tiles, device_cus()) * device_cus()) >= 0.9; };
-  if (!full(t.first) || !full(t.second)) return 10.;
-  if (I < 768 || H < 768) return row_scaled ? 10. : 6.;
-  return 3ll * E * H * I >= 1000000000ll ? 1. : 2.5;
+  const int64_t cus = device_cus();
+  auto full = [&](int64_t tiles) { return (double)tiles / (ceil_div(tiles, cus) * cus) >= 0.9; };
+  if (!full(t.second)) return t.first < cus ? 13. : row_scaled ? 12. : 10.;
+  if (!full(t.first)) return row_scaled ? 4. : 3.;
+  if (I < 768 || H < 768) return row_scaled ? 6. : 2.5;
+  return 3 * E * H * I >= 1000000000ll ? 1.5 : 2.5;
 }
-// Whether a layer's largest expert is likely to fit one block of 64 slots: the mean, plus the spread that the largest of E
-// numbers of rows has.  One expert more than fits adds a tile to every column: 64 experts of 4096 x 1536 at 48 rows, three
-// rounds of tiles that become four, 227 -> 266 us.
-bool moe_fits_64(double rows, int E) { return rows + sqrt(2 * log((double)E) * rows) <= 64; }
+// Whether a layer's largest expert is likely to fit one block of 64 slots: the mean, plus most of the spread that the
+// largest of E numbers of rows has.  One expert that does not adds a tile to every column: 64 experts of 4096 x 1536 at 48
+// rows, three rounds of tiles that become four, 227 -> 266 us.
+bool moe_fits_64(double rows, int E) { return rows + 0.85 * std::sqrt(2 * std::log((double)E) * rows) <= 64; }
+// Blocks that an expert has in the mean when the numbers of rows are spread like independent draws.
+double moe_spread_blocks(double rows, int block) {
+  double blocks = 1;
+  for (int full = block; full < rows + 5 * std::sqrt(rows) && blocks < 1000; full += block)
+    blocks += 0.5 * std::erfc((full - rows) / std::sqrt(2 * rows));
+  return blocks;
+}
+// Or whether the first GEMM's tiles in 64-slot blocks (every expert's last one half full) take this share of one round: then
+// a tile's time is the launch's, and the shortest wins.  8 experts of 4096 x 1536 at 64..128 rows 1.06-1.16x over 128 slots,
+// 16 of 4096 x 896 at 80..112 1.06-1.14x, 16 of 3072 x 1024 at 64..96 1.01-1.06x; with row scales, where 128 slots stream too, up to
+// 1.1x for the first of them and 0.9-1.0x in between.
+bool moe_one_round_64(double rows, int E, int64_t I, double share) {
+  return E * (rows / 64 + 0.5) * (double)ceil_div(2 * I, 256) <= share * device_cus();
+}
 
-int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I) {
+int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I, bool int8 = false) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;  // tuning knob
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
-  // Layers that fill the chip, layer time in us by block height (64: the streaming tile kernel; 128 and 192: the persistent
+  // Layers whose weights come from HBM, layer time in us by block height (64: the streaming tile kernel; 128 and 192: the persistent
   // walk), 256 experts of 7168 x 2048, top-8:
   //   rows/expert    1      3      6      10     16     24     32     48     56     64     96     112    128
   //   16            1098   1670   1808   2040   2969   4115
@@ -1023,13 +1040,17 @@ int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I) {
   // Twelve layers of 8 to 256 experts: 64 slots are 1.05-1.2x ahead of 128 while they hold an expert; where there are at
   // least four rounds of tiles an overflowing expert costs little and they stay ahead to 56 rows.  192 slots once experts
   // start to overflow 128, and 128 again where half of them would overflow 192 (at 200 rows 1.02-1.2x on eight layers).
-  if (moe_layer_streams(E, H, I)) {
-    if (rows < moe_stream_from(E, H, I, false) || M <= 4) return 16;
-    if (moe_fits_64(rows, E) || (rows <= 56 && moe_one_block_tiles(E, H, I).first >= 4 * device_cus())) return 64;
+  // (INT8 layers have no activation in the first GEMM's epilogue and no place for padded rows of scales)
+  if (moe_layer_streams(E, H, I) && !(int8 && (H % 512 || I % 512))) {
+    const double from = moe_stream_from(E, H, I, false);
+    if (rows < (int8 && from < 4 ? 4 : from) || M <= 4) return 16;
+    if (moe_fits_64(rows, E) || (rows <= 56 && moe_one_block_tiles(E, H, I).first >= 4 * device_cus()) ||
+        moe_one_round_64(rows, E, I, 1.0))
+      return 64;
     if (rows <= 104 || (rows >= 180 && rows <= 215 && E < 256)) return 128;
     return 192;
   }
-  // Layers whose tiles do not fill the chip take one round whatever the height, so the shorter block wins where it holds
+  // The other layers.  Those whose tiles do not fill the chip take one round whatever the height, so the shorter block wins where it holds
   // an expert, and two full blocks of 128 beat 192 where half of the experts overflow those.  Sixteen such layers of 4 to 64
   // experts: 64 at 14..52 rows 1.05x in the mean (0.94-1.11), 128 at 170..215 rows 1.17x (0.84-1.33, two of 48 points
   // below 0.98); in the bands between, the layers disagree by as much in both directions.  Up to 8 experts the 16-slot
@@ -1043,17 +1064,17 @@ int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I) {
   return 192;
 }
 // The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue; the streaming tile kernel
-// takes 128 slots too.  Against one-tile launches of 128 slots it is 1.07-1.16x ahead on layers that fill the chip, and
-// ahead of 192 slots up to 118 rows (1.04-1.2x at 112 on eight layers) and again from 175 on (1.15-1.27x at 200, 1.0-1.1x at
-// 256, 1.04-1.07x at 400).
+// takes 128 slots too.  Against one-tile launches of 128 slots it is 1.07-1.16x ahead on layers that fill the chip; against
+// 192 slots it wins where it pads fewer rows: 1.04-1.2x at 112 rows on eight layers, 1.15-1.27x at 200, 1.0-1.1x at 256,
+// 1.04-1.07x at 400, while at 128 (0.92-1.08x), 160 (0.87-1.0x) and 312 (0.99x) it does not.
 int moe_auto_block_rows(int64_t M, int E, int topk, int64_t H, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
   if (moe_layer_streams(E, H, I)) {
     if (rows < moe_stream_from(E, H, I, true)) return 16;
-    if (moe_fits_64(rows, E)) return 64;
-    return rows <= 118 || rows >= 175 ? 128 : 192;
+    if (moe_fits_64(rows, E) || moe_one_round_64(rows, E, I, 0.7)) return 64;
+    return moe_spread_blocks(rows, 128) * 128 < 0.98 * moe_spread_blocks(rows, 192) * 192 ? 128 : 192;
   }
   // What counts without it is how few rows a tile pads: the shortest block that still holds a whole expert (its weights are
   // streamed once).  A layer that fills the chip moves on sooner, since an expert that overflows adds a tile to a full
@@ -1067,12 +1088,6 @@ int moe_auto_block_rows(int64_t M, int E, int topk, int64_t H, int64_t I) {
   if (rows <= (small ? 112 : 104) || (small && rows >= 170 && rows <= 215)) return 128;
   return 192;
 }
-// Sorted blocks that a layer with evenly spread routing has (GemmArgs::expected_blocks).
-int moe_expected_blocks(int64_t M, int E, int topk, int block_m) {
-  const double rows = (double)M * topk / E;
-  const double used = E * (1 - exp(-rows));
-  return (int)(rows <= 0.7 * block_m ? used + 0.5 : E * (rows / block_m + 0.5));
-}
 int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1, 0, 0); }
 }  // namespace
 
@@ -1085,7 +1100,7 @@ extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, in
 extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk,
                                                     int block_m) {
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
-  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk, H, I) : moe_auto_block_rows(M, E, topk, H, I);
+  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk, H, I, gemm_is_int8(mode)) : moe_auto_block_rows(M, E, topk, H, I);
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
 }
 
@@ -1116,7 +1131,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   SGLAMD_REQUIRE(!row || I <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: intermediate size %lld is beyond %lld",
                  (long long)I, (long long)ROW_QUANT_MAX_HIDDEN);
   SGLAMD_REQUIRE(row || (!b13 && !b2), SGLAMD_ENOTSUP, "fused_moe: biases go with row-scaled weights");
-  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I);
+  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I, int8);
   SGLAMD_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128 || block_m == 192, SGLAMD_EINVAL,
                  "fused_moe: block_m must be 16, 32, 64, 128 or 192");
   const MoeWs w = moe_ws_layout(M, H, I, E, topk, block_m);
@@ -1224,7 +1239,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
     g.top_k = topk;
     g.num_valid = (int)T;
     g.max_blocks_m = (int)w.max_blocks;
-    g.expected_blocks = moe_expected_blocks(M, E, topk, block_m);
+    g.streams = moe_layer_streams(E, H, I) ? 1 : -1;
     GemmArgs h = g;
     h.A = ws + w.aq;
     h.lda = I;
@@ -1282,7 +1297,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   first.top_k = topk;
   first.num_valid = (int)T;
   first.max_blocks_m = (int)w.max_blocks;
-  first.expected_blocks = moe_expected_blocks(M, E, topk, block_m);
+  first.streams = moe_layer_streams(E, H, I) ? 1 : -1;
   // These kernels fetch activation scales in groups of four K blocks: rows of another length are padded, in the place of
   // the first GEMM's 16-bit output, which does not exist then.
   const int64_t pitch1 = (KB1 + 3) & ~(int64_t)3, pitch2 = (KB2 + 3) & ~(int64_t)3;
@@ -1448,7 +1463,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   if (!act_fused) {
     rc = moe_block_gemm(mode, ws + w.xq, H, (const float*)(ws + w.xs), KB1, 1, w13, 2 * I * H, H, w13_scale,
                         (2 * I / 128) * KB1, KB1, 1, ws + w.c1, 2 * I, dtype, sorted, expert, post, nullptr, T, topk, 0,
-                        block_m, w.max_blocks, 2 * I, H, stream, 0, first.expected_blocks);
+                        block_m, w.max_blocks, 2 * I, H, stream, 0, first.streams);
     if (rc) return rc;
     rc = sglamd_silu_mul_group_quant_8bit(ws + w.c1, dtype, ws + w.aq, int8 ? SGLAMD_I8 : SGLAMD_FP8_E4M3, ws + w.as, T,
                                           I, 128, SGLAMD_SCALE_ROW_MAJOR, 0, 1e-10f, int8 ? -128.f : -448.f,
@@ -1457,7 +1472,7 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   }
   rc = moe_block_gemm(mode, ws + w.aq, I, (const float*)first.A16, first.lda16, 1, w2, H * I, I, w2_scale,
                       (H / 128) * KB2, KB2, 1, ws + w.c3, H, dtype, sorted, expert, post, topk_weights, T, 1,
-                      grouped ? 0 : 1, block_m, w.max_blocks, H, I, stream, first.scale_rows_padded, first.expected_blocks);
+                      grouped ? 0 : 1, block_m, w.max_blocks, H, I, stream, first.scale_rows_padded, first.streams);
   if (rc) return rc;
   return finish();
 }

@@ -31,14 +31,16 @@ static inline bool moe_stream_enabled() {
   static const int v = getenv("SGLAMD_MOE_STREAM") ? atoi(getenv("SGLAMD_MOE_STREAM")) : 1;
   return v != 0;
 }
-// Whether the weight-streaming tile kernel takes a launch.  It wants every CU busy: with fewer tiles a CU gets more of the
-// memory's bandwidth than this kernel's chain of K blocks takes (block scales, 12 rows per expert, one-tile kernel over
-// this one: 8 experts of 4096 x 1536 1.27x, 32 of 2048 x 768 1.04x, 16 of 3072 x 1024 1.16x; from one tile per CU on,
-// 16 of 6144 x 2048 0.90x, 32 of 5120 x 1536 0.91x).
+// Whether the weight-streaming tile kernel takes a launch: weights that come from HBM.  A layer of less than some 96 MB of
+// weights may find them in the 256 MB Infinity Cache from one call to the next; there the one-tile kernel, which starts a
+// tile sooner, is ahead (three layers used in turn, 12 rows per expert, one-tile kernel over this one: 8 experts of
+// 3072 x 1024 0.80, 16 of 1536 x 640 0.92; 64 of 1024 x 512, 101 MB, 1.13, 32 of 2048 x 768, 151 MB, 1.06).  With weights that have left the cache this one
+// is ahead on all of them (1.0-1.12x).
+constexpr int64_t MOE_STREAM_MIN_BYTES = 96000000;
 template <int BM>
 static inline bool moe_stream_takes(const GemmArgs& g, bool block) {
-  const int64_t blocks = g.expected_blocks > 0 ? g.expected_blocks : g.max_blocks_m;
-  return moe_stream_enabled() && gemm8_moe_stream_ok<BM>(g, block) && blocks * ((g.N + 255) / 256) * 16 >= (int64_t)device_cus() * 15;
+  if (g.streams < 0 || !moe_stream_enabled() || !gemm8_moe_stream_ok<BM>(g, block)) return false;
+  return g.streams > 0 || (int64_t)g.max_blocks_m * g.N * g.ldb >= MOE_STREAM_MIN_BYTES * 2 / 3;
 }
 
 template <int MODE, typename OT>
