@@ -148,8 +148,8 @@ int sglamd_fp8_blockwise_scaled_mm(const void* a, int64_t lda, const void* b, in
 /* The same GEMM for scales that are all powers of two -- UE8M0 scales, as DeepSeek-V3.1 checkpoints and the
  * reference's DeepGEMM path carry them (python/sglang/srt/layers/quantization/fp8_kernel.py:1149-1174 with
  * scale_ue8m0, python/sglang/srt/layers/quantization/fp8_utils.py:1348-1383), expanded to fp32 by
- * sglamd_ue8m0_unpack.  Same arguments and result up to fp32 summation order; where the launch runs the persistent
- * large-tile kernel, the scales' exponent bytes go into the MFMA's block-scale operands and the K blocks add up in
+ * sglamd_ue8m0_unpack.  Same arguments and result up to fp32 summation order; where the launch runs one of the
+ * large-tile kernels, the scales' exponent bytes go into the MFMA's block-scale operands and the K blocks add up in
  * the MFMA accumulators (no multiply-add per element and K block).  A scale that is not a power of two counts as
  * the power of two below it there; the other kernels use the scale as given. */
 int sglamd_fp8_blockwise_scaled_mm_pow2(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
@@ -167,6 +167,15 @@ int sglamd_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, const void* 
                                         int64_t sb_stride_k, int scales_pow2, const void* bias, void* out, int64_t ldc,
                                         int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
                                         int64_t workspace_bytes, void* stream);
+
+/* The block-scaled linear layer: x [M, K] (SGLAMD_F16 or SGLAMD_BF16, rows K elements apart) quantised per 1x128 group
+ * (sglamd_per_token_group_quant_8bit, reciprocal form, float scales), times w [N, K] with 128x128 block scales, plus an
+ * optional bias as sglamd_fp8_blockwise_scaled_mm_bias adds it.  One launch for a few rows, which the GEMM's workgroups
+ * quantise themselves; otherwise those two entry points in turn, through the scratch q (M * K bytes) and sa (M * K / 128
+ * floats).  The same bits either way. */
+int sglamd_fp8_block_linear(const void* x, int dtype, int64_t M, int64_t K, const void* w, int64_t ldb, const float* sb,
+                            int64_t sb_stride_n, int64_t sb_stride_k, const void* bias, void* out, int64_t ldc, int64_t N,
+                            void* q, float* sa, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The block-scaled GEMM on int8 operands: the int32 partial product of every 128-wide K block is exact and is
  * folded as float(p) * (sa[m, kb] * sb[n/128, kb]) into the fp32 accumulator.  Same arguments as above.

@@ -24,6 +24,9 @@
 // the kernel takes the 16-bit source rows,
 // quantises the tile's few rows per 128-wide group into LDS while the tile's first weight blocks are on their way,
 // with the very arithmetic of the stand-alone group-quant kernel, so a decode-sized layer saves that kernel's launch.
+// Dense launches of a few rows (DQ) do the same once per workgroup: the 16-bit rows come by direct-to-LDS loads in front of
+// the first weight blocks, so that quantising them does not wait for those, and lie quantised behind the rings for all of
+// the workgroup's tiles.
 #pragma once
 #include <stdlib.h>
 
@@ -54,14 +57,22 @@ constexpr int skinny_slot_bytes() {
 }
 // AQ rows of K bytes, each padded by 16 so that the rows' fragment reads spread over the banks, then their scales
 static inline int skinny_aq_bytes(int aq, int K) { return aq * (K + 16) + aq * ((K + 127) >> 7) * 4; }
+constexpr int SKINNY_DQ_PASSES = 8;  // DQ: passes of a workgroup over its rows, 64 bytes of registers a lane each
+// DQ: room for the 16-bit rows, in whole passes of a workgroup; the quantised rows and their scales take it over.
+static inline int skinny_dq_bytes(int M, int K, int kw) {
+  const int groups = M * (K >> 7), raw = (groups + 8 * kw - 1) / (8 * kw) * (kw * 2048), q = M * (K + 16) + groups * 4;
+  return raw > q ? raw : q;
+}
 // Waves that may split K, and K blocks in flight per wave: the rings of all waves fill the LDS of a CU (156 KB of
 // its 160), which is what keeps enough bytes in flight to stream from HBM at full rate.
+// (DQ: the waves and the blocks in flight of the plain launch, so that both sum in the same order.)
 template <int FM, int FN, int AQ = 0>
 constexpr int skinny_kw_max() {
   return AQ == 0 && skinny_slot_bytes<FM, FN, AQ>() <= 6656 ? 8 : 4;
 }
-template <int FM, int FN, int AQ = 0>
+template <int FM, int FN, int AQ = 0, bool DQ = false>
 constexpr int skinny_depth() {
+  if constexpr (DQ) return skinny_depth<FM, FN, 0, false>();
   constexpr int d = 159744 / (skinny_kw_max<FM, FN, AQ>() * skinny_slot_bytes<FM, FN, AQ>());
   // with AQ three slots: the quantised rows need their place too, and seven one-wave workgroups still share a CU,
   // which takes the 1792 tiles of the DeepSeek-V3 layer's second GEMM in one round
@@ -91,8 +102,9 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   constexpr int X_OFF = FN * 2048, SA_OFF = AQ > 0 ? 0 : (FN + FM) * 2048, SB_OFF = AQ > 0 ? FN * 2048 : SA_OFF + 256;
   // direct-to-LDS loads per K block and wave
   constexpr int LOADS = AQ > 0 ? 2 * FN + 1 : 2 * FN + 2 * FM + (BLK ? 2 : 0);
-  static_assert(AQ == 0 || (MOE && MODE == GEMM_BLOCK_FP8 && FM == 1 && AQ <= 16),
-                "in-kernel activation quantisation: MoE, block FP8, one row tile");
+  constexpr bool DQ = AQ > 0 && !MOE;
+  static_assert(AQ == 0 || (MODE == GEMM_BLOCK_FP8 && FM == 1 && AQ <= 16),
+                "in-kernel activation quantisation: block FP8, one row tile");
   static_assert(PD >= 1 && PD * LOADS < 64, "the vmcnt field counts up to 63 loads in flight");
   // a wave's partial tiles wait for the cross-wave sum in its last ring slot when they fit there; wide tiles put
   // them side by side over the whole ring area instead (behind a barrier: every wave's loads have landed by then)
@@ -235,7 +247,9 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       wv[j][0] = (paired || r0 < n_end) ? (uint32_t)(r0 * (int)g.ldb + chunk0 * 16) : SKINNY_NOWHERE;
       wv[j][1] = (paired || r1 < n_end) ? (uint32_t)(r1 * (int)g.ldb + chunk1 * 16) : SKINNY_NOWHERE;
     }
-    if constexpr (AQ > 0) {
+    if constexpr (DQ) {
+      aq_rows = g.M;
+    } else if constexpr (AQ > 0) {
       const int slot_id = lane < 16 ? s_rows[buf][lane] : 0x7fffffff;
       const int real = __popcll(__ballot(slot_id < g.num_valid));  // a block's real rows come first
       aq_rows = __builtin_amdgcn_readfirstlane(real < AQ ? real : AQ);
@@ -341,13 +355,13 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // AQ: the tile's rows, quantised, behind the rings: AQ rows of K bytes (stride K + 16) and their group scales.
   uint8_t* xq_rows = smem + KW * PD * SLOT;
   const int xq_stride = g.K + 16;
-  float* xq_scales = reinterpret_cast<float*>(xq_rows + AQ * xq_stride);
+  float* xq_scales = reinterpret_cast<float*>(xq_rows + (DQ ? g.M : AQ) * xq_stride);
   // Quantises the real rows of the tile whose slot ids are in s_rows[buf]: per pass 16 groups of 128 over all the
   // workgroup's lanes, LPG = 4 * KW lanes per group and 128 / LPG elements per lane.  The arithmetic is
   // group_quant_body's (reciprocal form, float scales), so bytes and scales are the ones the stand-alone kernels
   // write.  The caller makes the result visible to the other waves (a workgroup barrier) before anyone reads it.
   auto quantise_rows = [&](int buf) {
-   if constexpr (AQ > 0) {
+   if constexpr (AQ > 0 && MOE) {
     typedef typename OT::storage XS;
     constexpr int LPG = 4 * KW, EL = 128 / LPG, VEC = EL / 8;  // 16-byte loads per lane: EL 16-bit values
     static_assert(KW <= 4 && EL % 8 == 0, "a lane takes whole 16-byte pieces");
@@ -481,13 +495,79 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
     }
   };
 
+  // DQ: group gi of the M * nkb groups of 128 belongs to eight lanes, 16 values each; pass p holds the groups 8 * KW * p + tid / 8.
+  // The 16-bit values lie where the quantised rows go, pass by pass, 32 bytes a lane as two halves of 16.
+  constexpr int DQ_MAX_PASSES = SKINNY_DQ_PASSES;
+  const int dq_groups = DQ ? g.M * nkb : 0, dq_passes = (dq_groups + 8 * KW - 1) / (8 * KW);
+  auto fetch_dense = [&]() {
+    if constexpr (DQ) {
+      const v4i rs = descriptor(g.A16, ((int64_t)(g.M - 1) * g.lda16 + (int64_t)g.K * 2));
+      const uint32_t raw = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem + KW * PD * SLOT + wave * 2048;
+      for (int p = 0; p < dq_passes; p++) {
+        const int gi = p * 8 * KW + (tid >> 3), r = gi / nkb;
+        const uint32_t off = gi < dq_groups ? (uint32_t)(r * (int)g.lda16 + (gi - r * nkb) * 256 + (lane & 7) * 32) : SKINNY_NOWHERE;
+#pragma unroll
+        for (int h = 0; h < 2; h++) dma16(rs, off + (uint32_t)(h * 16), 0, raw + p * (KW * 2048) + h * 1024, false);
+      }
+    }
+  };
+  auto quantise_dense = [&]() {
+    if constexpr (DQ) {
+      typedef typename OT::storage XS;
+      v4i raw[DQ_MAX_PASSES][2];
+      const uint8_t* src = xq_rows + wave * 2048 + lane * 16;
+#pragma unroll
+      for (int p = 0; p < DQ_MAX_PASSES; p++)
+        if (p < dq_passes) {
+          raw[p][0] = *(const v4i*)(src + p * (KW * 2048));
+          raw[p][1] = *(const v4i*)(src + p * (KW * 2048) + 1024);
+        }
+      // the quantised rows replace the 16-bit ones
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+#pragma unroll
+      for (int p = 0; p < DQ_MAX_PASSES; p++)
+        if (p < dq_passes) {
+          // group_quant_body's arithmetic (reciprocal form, float scales)
+          const int gi = p * 8 * KW + (tid >> 3);
+          XS e[16];
+          float x[16];
+          __builtin_memcpy(e, raw[p], 32);
+          float amax = g.q_eps;
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            x[i] = OT::to_f32(e[i]);
+            amax = fmaxf(amax, fabsf(x[i]));
+          }
+          amax = lanes_max<8>(amax);
+          const float mul = g.q_max / amax;
+          uint32_t o[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            o[i] = pack4_e4m3(clampf(x[4 * i] * mul, g.q_min, g.q_max), clampf(x[4 * i + 1] * mul, g.q_min, g.q_max),
+                              clampf(x[4 * i + 2] * mul, g.q_min, g.q_max), clampf(x[4 * i + 3] * mul, g.q_min, g.q_max));
+          if (gi < dq_groups) {
+            const int r = gi / nkb, c = gi - r * nkb;
+            *(v4i*)(xq_rows + r * xq_stride + c * 128 + (lane & 7) * 16) = v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
+            if ((lane & 7) == 0) xq_scales[r * nkb + c] = amax * (1.0f / g.q_max);
+          }
+        }
+    }
+  };
+
   int tile = blockIdx.x;
   if (!tile_exists(tile)) return;
   setup(tile, 0);
+  if constexpr (DQ) fetch_dense();
 #pragma unroll
   for (int s = 0; s < PD; s++)
     if (s < n_my) issue(s, block_of(s));
-  if constexpr (AQ > 0) {
+  if constexpr (DQ) {
+    // the rows have landed when only the ring's loads are outstanding
+    if (n_my >= PD) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PD * LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    quantise_dense();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+  } else if constexpr (AQ > 0) {
     quantise_rows(0);
     if (KW > 1) __syncthreads();
   }
@@ -529,7 +609,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
         if (s < n_my) issue(s, block_of(s));
       // every wave is past its K loop (setup's barriers), so the rows can be replaced; with several waves the
       // barriers of the reduction below stand between these writes and the next tile's first reads
-      if constexpr (AQ > 0) quantise_rows(o_buf ^ 1);
+      if constexpr (AQ > 0 && MOE) quantise_rows(o_buf ^ 1);
     }
 
     // ---- reduce the KW partial tiles through LDS (every wave's own last ring slot) ------------------------------
@@ -671,19 +751,22 @@ static inline bool gemm8_skinny_ok(const GemmArgs& g, int64_t a_rows) {
 }
 
 // Workgroups of one launch that a CU holds at once: bounded by the LDS rings and by 32 wavefronts.
-template <int FM, int FN, int AQ = 0>
-static inline int skinny_resident_per_cu(int kw, int extra_bytes = 0) {
-  const int smem = skinny_smem_bytes<FM, FN, AQ>(kw, extra_bytes) + 1024;
-  int n = 163840 / smem;
+static inline int skinny_fit(int smem, int kw) {
+  int n = 163840 / (smem + 1024);
   if (n > 32 / kw) n = 32 / kw;
   return n < 1 ? 1 : n;
+}
+template <int FM, int FN, int AQ = 0>
+static inline int skinny_resident_per_cu(int kw, int extra_bytes = 0) {
+  return skinny_fit(skinny_smem_bytes<FM, FN, AQ>(kw, extra_bytes), kw);
 }
 
 template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int AQ = 0>
 static int gemm8_skinny_launch_kw(const GemmArgs& g, hipStream_t st) {
-  constexpr int PD = skinny_depth<FM, FN, AQ>();
-  const int aq_bytes = AQ > 0 ? skinny_aq_bytes(AQ, g.K) : 0;
-  const int smem = skinny_smem_bytes<FM, FN, AQ>(KW, aq_bytes);
+  constexpr bool DQ = AQ > 0 && !MOE;
+  constexpr int PD = skinny_depth<FM, FN, AQ, DQ>();
+  const int aq_bytes = DQ ? skinny_dq_bytes(g.M, g.K, KW) : AQ > 0 ? skinny_aq_bytes(AQ, g.K) : 0;
+  const int smem = DQ ? KW * PD * skinny_slot_bytes<FM, FN, AQ>() + aq_bytes : skinny_smem_bytes<FM, FN, AQ>(KW, aq_bytes);
   if (smem > 160 * 1024) return fail(SGLAMD_ENOTSUP, "gemm: K = %d is too long for in-kernel activation quantisation", g.K);
   const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
   const int tiles_n = (g.N + R - 1) / R;
@@ -692,7 +775,7 @@ static int gemm8_skinny_launch_kw(const GemmArgs& g, hipStream_t st) {
   if (tiles <= 0) return SGLAMD_OK;
   if (tiles > 0x7fffffff) return fail(SGLAMD_EINVAL, "gemm: grid too large");
   // as many workgroups as the chip holds at once; each walks tiles blockIdx.x, + gridDim.x, ...
-  const int64_t resident = (int64_t)device_cus() * skinny_resident_per_cu<FM, FN, AQ>(KW, aq_bytes);
+  const int64_t resident = (int64_t)device_cus() * (DQ ? skinny_fit(smem, KW) : skinny_resident_per_cu<FM, FN, AQ>(KW, aq_bytes));
   const unsigned blocks = (unsigned)(tiles < resident ? tiles : resident);
   auto kern = gemm8_skinny_kernel<FM, FN, MODE, OT, MOE, KW, PD, AQ>;
   if (smem > 64 * 1024) {
@@ -751,7 +834,7 @@ static int gemm8_skinny_launch_fn(const GemmArgs& g, hipStream_t st, int64_t exp
   // A launch that quantises its activations itself splits K the way the plain launch of the same shape would (up
   // to the four waves it supports): the same partial sums in the same order, so both give the same bits.
   int kw = skinny_pick_kw<FM, FN>(tiles, (g.K + 127) >> 7);
-  if (AQ > 0 && kw > 4) kw = 4;
+  if (AQ > 0 && MOE && kw > 4) kw = 4;
   skinny_last_shape = (FM << 16) | (FN << 8) | kw;
   switch (kw) {
     case 1:
@@ -761,7 +844,7 @@ static int gemm8_skinny_launch_fn(const GemmArgs& g, hipStream_t st, int64_t exp
     case 4:
       return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 4, AQ>(g, st);
     default:
-      if constexpr (skinny_kw_max<FM, FN, AQ>() >= 8) return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 8, AQ>(g, st);
+      if constexpr (skinny_kw_max<FM, FN, MOE ? AQ : 0>() >= 8) return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 8, AQ>(g, st);
       return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 4, AQ>(g, st);
   }
 }
@@ -794,51 +877,57 @@ static inline double skinny_cost(const GemmArgs& g, int rows) {
 // weight byte; the tile count should fill the resident workgroups a whole number of times (N = 7168 runs as 256
 // tiles of 28 rows instead of 224 of 32 with 32 CUs idle).  MoE launches keep the 32-row tile of the sorted-block
 // schedule's column split.
-template <int FM, int MODE, typename OT, bool MOE>
-static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expected_tiles_m) {
+template <int FM>
+static int skinny_plan(GemmArgs& g) {
   static const int force_fn = skinny_env("SGLAMD_SKINNY_FN");
   static const int force_rows = skinny_env("SGLAMD_SKINNY_ROWS");
+  int fn = (g.N % 32 == 0 && g.N >= 2048) ? 2 : 1;
+  // the search is a few microseconds of host time, as much as the launch itself: a thread remembers its last shapes
+  struct Plan {
+    int M, N, K, cus, fn, rows;
+  };
+  static thread_local Plan plans[32] = {};
+  const int cus = device_cus();
+  Plan& plan = plans[((uint32_t)g.M * 31u + (uint32_t)(g.N >> 3) * 7u + (uint32_t)(g.K >> 4)) & 31u];
+  if (plan.M == g.M && plan.N == g.N && plan.K == g.K && plan.cus == cus) {
+    g.rows_per_wg = plan.rows;
+    return plan.fn;
+  }
+  if (g.N >= 1024) {
+    double best = -1.0;
+    int best_rows = 16 * fn;
+    auto consider = [&](int f, double (*cost)(const GemmArgs&, int)) {
+      if (force_fn && force_fn != f) return;
+      for (int rows = 16 * f; rows > 16 * f - 16 && rows >= 12; rows -= 4) {
+        if (force_rows && force_rows != rows) continue;
+        const double c = cost(g, rows);
+        if (best < 0 || c < best - 1e-9) {
+          best = c;
+          best_rows = rows;
+          fn = f;
+        }
+      }
+    };
+    if constexpr (FM <= 2) {
+      consider(4, skinny_cost<FM, 4>);
+      consider(3, skinny_cost<FM, 3>);
+    }
+    consider(2, skinny_cost<FM, 2>);
+    consider(1, skinny_cost<FM, 1>);
+    g.rows_per_wg = best_rows == 16 * fn ? 0 : best_rows;
+  }
+  plan = Plan{g.M, g.N, g.K, cus, fn, g.rows_per_wg};
+  return fn;
+}
+template <int FM, int MODE, typename OT, bool MOE>
+static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expected_tiles_m) {
   GemmArgs g = g0;
   int fn = (g.N % 32 == 0 && g.N >= 2048) ? 2 : 1;
   if constexpr (!MOE) {
-    // the search is a few microseconds of host time, as much as the launch itself: a thread remembers its last shapes
-    struct Plan {
-      int M, N, K, cus, fn, rows;
-    };
-    static thread_local Plan plans[32] = {};
-    const int cus = device_cus();
-    Plan& plan = plans[((uint32_t)g.M * 31u + (uint32_t)(g.N >> 3) * 7u + (uint32_t)(g.K >> 4)) & 31u];
-    if (plan.M == g.M && plan.N == g.N && plan.K == g.K && plan.cus == cus) {
-      fn = plan.fn;
-      g.rows_per_wg = plan.rows;
-    } else {
-      if (g.N >= 1024) {
-        double best = -1.0;
-        int best_rows = 16 * fn;
-        auto consider = [&](int f, double (*cost)(const GemmArgs&, int)) {
-          if (force_fn && force_fn != f) return;
-          for (int rows = 16 * f; rows > 16 * f - 16 && rows >= 12; rows -= 4) {
-            if (force_rows && force_rows != rows) continue;
-            const double c = cost(g, rows);
-            if (best < 0 || c < best - 1e-9) {
-              best = c;
-              best_rows = rows;
-              fn = f;
-            }
-          }
-        };
-        if constexpr (FM <= 2) {
-          consider(4, skinny_cost<FM, 4>);
-          consider(3, skinny_cost<FM, 3>);
-        }
-        consider(2, skinny_cost<FM, 2>);
-        consider(1, skinny_cost<FM, 1>);
-        g.rows_per_wg = best_rows == 16 * fn ? 0 : best_rows;
-      }
-      plan = Plan{g.M, g.N, g.K, cus, fn, g.rows_per_wg};
-    }
-  } else if (force_fn == 1 || force_fn == 2) {
-    fn = force_fn;
+    fn = skinny_plan<FM>(g);
+  } else {
+    static const int force_fn = skinny_env("SGLAMD_SKINNY_FN");
+    if (force_fn == 1 || force_fn == 2) fn = force_fn;
   }
   if constexpr (FM <= 2 && !MOE) {
     if (fn == 4) return gemm8_skinny_launch_fn<FM, 4, MODE, OT, MOE>(g, st, expected_tiles_m);
@@ -846,6 +935,27 @@ static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expec
   }
   if (fn == 2) return gemm8_skinny_launch_fn<FM, 2, MODE, OT, MOE>(g, st, expected_tiles_m);
   return gemm8_skinny_launch_fn<FM, 1, MODE, OT, MOE>(g, st, expected_tiles_m);
+}
+
+// The dense launch that quantises its rows itself: `g` carries the 16-bit rows in A16 / lda16 and the quantisation
+// constants.  `launch` false: whether it takes the shape.
+template <int FN>
+static bool skinny_dq_fits(const GemmArgs& g) {
+  const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
+  const int kw = skinny_pick_kw<1, FN>((g.N + R - 1) / R, g.K >> 7);
+  const int groups = g.M * (g.K >> 7);
+  return (groups + 8 * kw - 1) / (8 * kw) <= SKINNY_DQ_PASSES &&
+         kw * skinny_depth<1, FN, 1, true>() * skinny_slot_bytes<1, FN, 1>() + skinny_dq_bytes(g.M, g.K, kw) <= 158 * 1024;
+}
+template <typename OT>
+static int gemm8_skinny_quantising(const GemmArgs& g0, hipStream_t st, bool launch) {
+  GemmArgs g = g0;
+  const int fn = skinny_plan<1>(g);
+  if (!launch) return fn == 4 ? skinny_dq_fits<4>(g) : fn == 3 ? skinny_dq_fits<3>(g) : fn == 2 ? skinny_dq_fits<2>(g) : skinny_dq_fits<1>(g);
+  if (fn == 4) return gemm8_skinny_launch_fn<1, 4, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
+  if (fn == 3) return gemm8_skinny_launch_fn<1, 3, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
+  if (fn == 2) return gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
+  return gemm8_skinny_launch_fn<1, 1, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
 }
 
 // Wide form for 33..64 activation rows on weights with many rows: four row tiles times FN = 6, 8 or 9 column tiles

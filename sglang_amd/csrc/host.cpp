@@ -586,26 +586,25 @@ optional<Tensor> block_linear(const Tensor& x, const Tensor& w, const Tensor& ws
   const int64_t wb = sglamd_gemm_workspace_bytes(m, n, k), wp = sc.take(wb > 0 ? wb : 0);
   sc.allocate(x);
   void* st = stream_of(x);
-  const float* wsp;
-  int64_t ws_n, ws_k;
-  if (ue8m0) {
-    check(sglamd_ue8m0_linear_operands(x.data_ptr(), tag(t), sc.at(q), (float*)sc.at(sa), m, k, ws.data_ptr(),
-                                       ws.stride(0), ws.stride(1), (float*)sc.at(sb), cdiv(n, 128), st));
-    wsp = (const float*)sc.at(sb), ws_n = kb, ws_k = 1;
-  } else {
-    check(sglamd_per_token_group_quant_8bit(x.data_ptr(), tag(t), sc.at(q), SGLAMD_FP8_E4M3, sc.at(sa), m, k, 128,
-                                            SGLAMD_SCALE_COL_MAJOR, m, 1e-10f, -448.f, 448.f,
-                                            SGLAMD_QUANT_FORM_RECIPROCAL, st));
-    wsp = ws.data_ptr<float>(), ws_n = ws.stride(0), ws_k = ws.stride(1);
+  if (!ue8m0) {
+    const bool inside = bias_in_gemm(bias, n);
+    check(sglamd_fp8_block_linear(x.data_ptr(), tag(t), m, k, w.data_ptr(), k, ws.data_ptr<float>(), ws.stride(0), ws.stride(1),
+                                  inside ? bias->data_ptr() : nullptr, out.data_ptr(), n, n, sc.at(q), (float*)sc.at(sa),
+                                  wb > 0 ? sc.at(wp) : nullptr, wb, st));
+    if (bias && !inside) out.add_(*bias);
+    return out;
   }
+  check(sglamd_ue8m0_linear_operands(x.data_ptr(), tag(t), sc.at(q), (float*)sc.at(sa), m, k, ws.data_ptr(), ws.stride(0),
+                                     ws.stride(1), (float*)sc.at(sb), cdiv(n, 128), st));
+  const float* wsp = (const float*)sc.at(sb);
+  const int64_t ws_n = kb, ws_k = 1;
   if (bias_in_gemm(bias, n)) {
     check(sglamd_fp8_blockwise_scaled_mm_bias(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, ue8m0,
                                               bias->data_ptr(), out.data_ptr(), n, tag(t), m, n, k,
                                               wb > 0 ? sc.at(wp) : nullptr, wb, st));
     return out;
   }
-  auto fn = ue8m0 ? sglamd_fp8_blockwise_scaled_mm_pow2 : sglamd_fp8_blockwise_scaled_mm;
-  check(fn(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, out.data_ptr(), n, tag(t), m, n, k,
+  check(sglamd_fp8_blockwise_scaled_mm_pow2(sc.at(q), k, w.data_ptr(), k, (float*)sc.at(sa), 1, m, wsp, ws_n, ws_k, out.data_ptr(), n, tag(t), m, n, k,
            wb > 0 ? sc.at(wp) : nullptr, wb, st));
   if (bias) out.add_(*bias);
   return out;
