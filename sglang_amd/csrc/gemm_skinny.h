@@ -92,6 +92,17 @@ constexpr int skinny_smem_bytes(int kw, int extra_bytes = 0) {
 // a lane with this offset fetches nothing and its LDS slot receives zeros.
 constexpr uint32_t SKINNY_NOWHERE = 0x7ffffff0u;
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// Waits until at most `blocks` (MAX where that is less) batches of LOADS loads are outstanding.
+template <int MAX, int LOADS>
+__device__ __forceinline__ void skinny_wait(int blocks) {
+  if constexpr (MAX > 0) {
+    if (blocks < MAX) return skinny_wait<MAX - 1, LOADS>(blocks);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(MAX * LOADS) : "memory");
+}
+#endif
+
 template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int PD, int AQ = 0>
 __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
@@ -586,16 +597,15 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
         consume(s, block_of(it + s), block_of(it + s + PD));
       }
     }
-    // the last PD .. 2*PD - 1 blocks (or all of them when the wave has fewer than 2*PD): the slots are drained
-    // together, refilled where a block is left, and drained once more
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    // the last PD .. 2*PD - 1 blocks (or all of them when the wave has fewer than 2*PD): as many are outstanding behind a
+    // slot as blocks are left, at most PD - 1
 #pragma unroll
-    for (int s = 0; s < PD; s++)
-      if (it + s < n_my) consume(s, block_of(it + s), it + s + PD < n_my ? block_of(it + s + PD) : -1);
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-#pragma unroll
-    for (int s = 0; s < PD; s++)
-      if (it + PD + s < n_my) consume(s, block_of(it + PD + s), -1);
+    for (int s = 0; s < 2 * PD - 1; s++)
+      if (it + s < n_my) {
+        const int behind = n_my - 1 - it - s;
+        skinny_wait<PD - 1, LOADS>(behind);
+        consume(s % PD, block_of(it + s), behind >= PD ? block_of(it + s + PD) : -1);
+      }
 
     // ---- what the finished tile's output needs, then the next tile's first blocks are requested ---------------
     const int o_n0 = n0, o_n_end = n_end, o_m0 = m0, o_expert = expert, o_buf = rows_buf;
