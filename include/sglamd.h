@@ -404,8 +404,8 @@ int sglamd_fused_rms_fp8_group_quant(const void* x1, int64_t x1_row_stride, cons
 /* The whole block-FP8 MoE layer from one host call (five launches on `stream`):
  *   quantise hidden (1x128 groups) + moe_align_block_size -> grouped GEMM with w13 -> silu*mul + quantise
  *   -> grouped GEMM with w2 (x routing weight) -> sum over top-k (x routed_scaling_factor).
- * Up to four tokens the activation step runs inside the two GEMMs, and a single token's sorting and quantising
- * too (four and three launches); where the sorted blocks are 128 or 192 slots tall and outnumber the compute
+ * Up to four tokens the activation step runs inside the two GEMMs (four launches), and a single token's sorting,
+ * quantising and sum too (two launches); where the sorted blocks are 128 or 192 slots tall and outnumber the compute
  * units, the first GEMM's epilogue applies silu*mul and the quantisation and writes the second GEMM's operand
  * (four launches, the same bits as the five).  The decode forms compute what the five-launch sequence computes; the bits are the
  * same when both split and walk K alike, which holds when 2I and H are at least 2048 and multiples of 32 (two

@@ -86,7 +86,13 @@ struct GemmArgs {
   float q_eps, q_min, q_max;
   // skinny MoE kernel, first GEMM of a gated layer: write silu(gate) * up (act_hidden wide) instead of [gate | up]
   int epi_silu;
-  // skinny MoE kernel sorting the routing itself (at most 32 pairs, 4 per expert): topk_ids as handed to the layer
+  // skinny MoE kernel of one token, second GEMM: the last of a column tile's workgroups to arrive writes sum_out, the pairs' rows
+  // summed and scaled.  sum_count: arrivals per column tile (sum_tiles of them), which the first GEMM clears (sum_out null).
+  void* sum_out;
+  float sum_scale;
+  int* sum_count;
+  int sum_tiles;
+  // skinny MoE kernel of one token: topk_ids as handed to the layer
   const void* route_ids;
   int route_ids_i64;
   int route_experts;

@@ -20,13 +20,16 @@
 //     block scale; the KW partial sums meet in LDS and leave as 8-byte stores.
 // The same kernel walks the fused-MoE sorted-block schedule (MOE = true): tile rows are gathered
 // through sorted_token_ids, the expert comes from expert_ids.
-// With AQ > 0 (MoE, block FP8, at most AQ real rows per sorted block) the activations are not read as FP8 at all:
-// the kernel takes the 16-bit source rows,
-// quantises the tile's few rows per 128-wide group into LDS while the tile's first weight blocks are on their way,
-// with the very arithmetic of the stand-alone group-quant kernel, so a decode-sized layer saves that kernel's launch.
-// Dense launches of a few rows (DQ) do the same once per workgroup: the 16-bit rows come by direct-to-LDS loads in front of
-// the first weight blocks, so that quantising them does not wait for those, and lie quantised behind the rings for all of
-// the workgroup's tiles.
+// With AQ > 0 (block FP8) the activations are not read as FP8 at all: the kernel takes the 16-bit source rows and quantises
+// the tile's few rows per 128-wide group into LDS while its first weight blocks are on their way, with the very arithmetic
+// of the stand-alone group-quant kernel, so a decode-sized layer saves that kernel's launch.
+//   MoE, AQ = 4: at most four real rows per sorted block, found through the sorted list and loaded into registers.
+//   Dense (DQ): once per workgroup, for all of its tiles; MoE of one token (SOLO, AQ = 1): pair p is row p, so nothing is
+//   sorted.  Both request the rows straight to LDS in front of the first weight blocks: quantising them waits for nothing
+//   else, where a load behind those drains the ring.  With the last arrivals' sum (sum_out) one token is two launches:
+//   GEMMs that sort for themselves, a sum behind them -> this, us, experts' weights from HBM, top-8 unless noted: 7168 x 2048
+//   73 -> 69, top-1 25.9 -> 22.1, 4096 x 1536 top-6 40.7 -> 32.1, 2048 x 768 26.1 -> 22.2 (of these the sum's launch 1.5, 0.6,
+//   1.5 and 0.7).  Four K blocks in flight instead of three change none of them.
 #pragma once
 #include <stdlib.h>
 
@@ -58,10 +61,10 @@ constexpr int skinny_slot_bytes() {
 // AQ rows of K bytes, each padded by 16 so that the rows' fragment reads spread over the banks, then their scales
 static inline int skinny_aq_bytes(int aq, int K) { return aq * (K + 16) + aq * ((K + 127) >> 7) * 4; }
 constexpr int SKINNY_DQ_PASSES = 8;  // DQ: passes of a workgroup over its rows, 64 bytes of registers a lane each
-// DQ: room for the 16-bit rows, in whole passes of a workgroup; the quantised rows and their scales take it over.
+// DQ, SOLO: room for the 16-bit rows, in whole passes of a workgroup, which the quantised rows take over, then their scales
 static inline int skinny_dq_bytes(int M, int K, int kw) {
-  const int groups = M * (K >> 7), raw = (groups + 8 * kw - 1) / (8 * kw) * (kw * 2048), q = M * (K + 16) + groups * 4;
-  return raw > q ? raw : q;
+  const int groups = M * (K >> 7);
+  return (groups + 8 * kw - 1) / (8 * kw) * (kw * 2048) + groups * 4;
 }
 // Waves that may split K, and K blocks in flight per wave: the rings of all waves fill the LDS of a CU (156 KB of
 // its 160), which is what keeps enough bytes in flight to stream from HBM at full rate.
@@ -93,6 +96,10 @@ constexpr int skinny_smem_bytes(int kw, int extra_bytes = 0) {
 constexpr uint32_t SKINNY_NOWHERE = 0x7ffffff0u;
 
 #if defined(__HIP_DEVICE_COMPILE__)
+template <typename T>
+__device__ __forceinline__ T scalar_load(const T* p) {
+  return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
 // Waits until at most `blocks` (MAX where that is less) batches of LOADS loads are outstanding.
 template <int MAX, int LOADS>
 __device__ __forceinline__ void skinny_wait(int blocks) {
@@ -114,6 +121,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // direct-to-LDS loads per K block and wave
   constexpr int LOADS = AQ > 0 ? 2 * FN + 1 : 2 * FN + 2 * FM + (BLK ? 2 : 0);
   constexpr bool DQ = AQ > 0 && !MOE;
+  constexpr bool SOLO = AQ == 1 && MOE;  // the routed pairs of one token: sorted block p is pair p
   static_assert(AQ == 0 || (MODE == GEMM_BLOCK_FP8 && FM == 1 && AQ <= 16),
                 "in-kernel activation quantisation: block FP8, one row tile");
   static_assert(PD >= 1 && PD * LOADS < 64, "the vmcnt field counts up to 63 loads in flight");
@@ -128,9 +136,6 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // for the cross-wave sum at the end of a tile.
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   __shared__ int s_rows[2][FM * 16];  // MoE: sorted slot ids of the tile's rows, for the current and the next tile
-  // MoE with the routing sorted in the kernel (at most 32 (token, expert) pairs, at most 4 per expert): expert and
-  // pair ids of each sorted block, and the number of blocks
-  __shared__ int s_blk_expert[MOE ? 32 : 1], s_blk_rows[MOE ? 32 : 1][4], s_nblk;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -145,48 +150,8 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   const int tiles_n = (g.N + R - 1) / R;
   const int tiles_m = MOE ? g.max_blocks_m : (g.M + 16 * FM - 1) / (16 * FM);
   const int total = tiles_n * tiles_m;
-  const bool self_sorted = MOE && g.route_ids != nullptr;
-  if (MOE && self_sorted) {
-    // What moe_align_block_size would hand over for these few pairs, in blocks of at most CAP rows (the rows a
-    // tile quantises itself, four otherwise): blocks in ascending order of expert (id -1, an expert that lives
-    // elsewhere, first: its rows are written as zeros), a block's pairs in ascending order of their index, ids
-    // outside [-1, route_experts) dropped.  An expert with more than CAP pairs (a token that names it several
-    // times) gets further blocks right behind its first.  One lane per pair; e is the id + 1, key orders the blocks.
-    constexpr int CAP = AQ > 0 ? AQ : 4;
-    static_assert(CAP == 1 || CAP == 2 || CAP == 4, "a block of the in-kernel sort holds 1, 2 or 4 rows");
-    if (wave == 0) {
-      const int numel = g.num_valid;
-      int e = -1;
-      if (lane < numel) {
-        e = (g.route_ids_i64 ? (int)((const int64_t*)g.route_ids)[lane] : ((const int32_t*)g.route_ids)[lane]) + 1;
-        if (e < 0 || e > g.route_experts) e = -1;
-      }
-      int slot = 0;
-      for (int j = 0; j < numel; j++) {
-        const int ej = __builtin_amdgcn_readlane(e, j);
-        slot += (j < lane && ej == e) ? 1 : 0;
-      }
-      const int key = e * 32 + slot / CAP;  // at most 32 pairs
-      const bool first = e >= 0 && slot % CAP == 0;
-      const unsigned long long firsts = __ballot(first);
-      int blk = 0;
-      for (int j = 0; j < numel; j++) {
-        const int kj = __builtin_amdgcn_readlane(key, j);
-        blk += (((firsts >> j) & 1ull) && kj < key) ? 1 : 0;
-      }
-      if (lane < 32) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) s_blk_rows[lane][q] = numel;
-      }
-      __builtin_amdgcn_wave_barrier();
-      if (e >= 0) s_blk_rows[blk][slot % CAP] = lane;
-      if (first) s_blk_expert[blk] = e - 1;
-      if (lane == 0) s_nblk = __popcll(firsts);
-    }
-    __syncthreads();
-  }
-  const int bstride = (MOE && !self_sorted && g.sorted_stride > 0) ? g.sorted_stride : 16 * FM;
-  const int post_pad = MOE ? __builtin_amdgcn_readfirstlane(self_sorted ? s_nblk * 16 * FM : *g.num_post_pad) : 0;
+  const int bstride = (MOE && g.sorted_stride > 0) ? g.sorted_stride : 16 * FM;
+  const int post_pad = MOE && !SOLO ? __builtin_amdgcn_readfirstlane(*g.num_post_pad) : 0;
   // MoE first GEMM of a gated layer with the activation in its output: a tile pairs 16 gate rows with the 16 up
   // rows of the same columns (weight rows n and act_hidden + n) and writes silu(gate) * up, act_hidden wide.
   const bool paired = MOE && FM == 1 && FN == 2 && g.epi_silu;
@@ -220,12 +185,23 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // ---- state of the tile being streamed (rewritten by setup() for the next one) ----------------------------
   int n0 = 0, n_end = 0, m0 = 0, expert = 0, rot = 0, rows_buf = 0;
   int aq_rows = 0;  // AQ: real rows of the tile's sorted block (<= AQ)
+  float solo_weight = 1.f;
   uint32_t wv[FN][2], xv[FM][2];
   uint32_t sav_off = SKINNY_NOWHERE, sbv_off = SKINNY_NOWHERE;
   v4i w_rs = descriptor(g.B, w_bytes), sb_rs = descriptor(g.sb, sb_bytes);
 
-  auto tile_exists = [&](int t) -> bool { return t < total && (!MOE || (t / tiles_n) * bstride < post_pad); };
-  // per-lane offsets and descriptors of tile t; MoE tiles read their rows' slot ids into s_rows[buf] first
+  auto tile_exists = [&](int t) -> bool { return t < total && (!MOE || SOLO || (t / tiles_n) * bstride < post_pad); };
+  // MoE: the expert and the rows' slot ids of the next tile, requested while the tile in front of it is streamed (8 to 37
+  // tokens of 256 experts of 7168 x 2048 0.2-1 % faster than two loads in turn between the tiles)
+  int ahead_expert = 0, ahead_row = 0;
+  auto look_ahead = [&](int t) {
+    if (MOE && !SOLO && tile_exists(t)) {
+      const int pid_m = t / tiles_n;
+      ahead_expert = g.expert_ids[pid_m];
+      ahead_row = tid < bstride && tid < FM * 16 ? g.sorted_ids[pid_m * bstride + tid] : g.num_valid;
+    }
+  };
+  // per-lane offsets and descriptors of tile t; MoE tiles put their rows' slot ids into s_rows[buf] first (look_ahead's)
   auto setup = [&](int t, int buf) {
     const int pid_n = t % tiles_n, pid_m = t / tiles_n;
     n0 = paired ? pid_n * 16 : pid_n * R;
@@ -242,13 +218,19 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
     // act_hidden + n.. (act_hidden % 256 == 0) sums in the same order as the two plain tiles that hold those rows.
     const uint32_t rot_key = MOE ? (uint32_t)((paired ? pid_n >> 1 : pid_n) & 7) : (uint32_t)pid_n;
     rot = __builtin_amdgcn_readfirstlane((int)((rot_key * 37u) % (uint32_t)nkb));
-    if (MOE) {
-      expert = __builtin_amdgcn_readfirstlane(self_sorted ? s_blk_expert[pid_m] : g.expert_ids[pid_m]);
+    if (SOLO) {
+      // ids outside [0, route_experts): an expert that lives elsewhere, whose row is zeros
+      // (scalar loads: a vector load would return behind the rows requested in front of it)
+      const int64_t id = g.route_ids_i64 ? scalar_load((const int64_t*)g.route_ids + pid_m) : scalar_load((const int32_t*)g.route_ids + pid_m);
+      expert = __builtin_amdgcn_readfirstlane(id >= 0 && id < g.route_experts ? (int)id : -1);
+      if (g.mul_weight) solo_weight = scalar_load(g.topk_w + pid_m);
+    } else if (MOE) {
+      expert = __builtin_amdgcn_readfirstlane(ahead_expert);
       __syncthreads();  // nobody still reads this buffer for the output of the tile before the last
-      if (tid < FM * 16)
-        s_rows[buf][tid] = self_sorted ? (tid < 4 ? s_blk_rows[pid_m][tid] : g.num_valid)
-                                       : (tid < bstride ? g.sorted_ids[m0 + tid] : g.num_valid);
+      if (tid < FM * 16) s_rows[buf][tid] = ahead_row;
       __syncthreads();
+    }
+    if (MOE) {
       w_rs = descriptor(g.B + (int64_t)max(expert, 0) * g.b_expert_stride, w_bytes);
       if (BLK) sb_rs = descriptor(g.sb + (int64_t)max(expert, 0) * g.sb_se, sb_bytes);
     }
@@ -260,6 +242,8 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
     }
     if constexpr (DQ) {
       aq_rows = g.M;
+    } else if constexpr (SOLO) {
+      aq_rows = 1;
     } else if constexpr (AQ > 0) {
       const int slot_id = lane < 16 ? s_rows[buf][lane] : 0x7fffffff;
       const int real = __popcll(__ballot(slot_id < g.num_valid));  // a block's real rows come first
@@ -366,13 +350,14 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // AQ: the tile's rows, quantised, behind the rings: AQ rows of K bytes (stride K + 16) and their group scales.
   uint8_t* xq_rows = smem + KW * PD * SLOT;
   const int xq_stride = g.K + 16;
-  float* xq_scales = reinterpret_cast<float*>(xq_rows + (DQ ? g.M : AQ) * xq_stride);
+  const int dq_groups = DQ ? g.M * nkb : nkb, dq_passes = (dq_groups + 8 * KW - 1) / (8 * KW);
+  float* xq_scales = reinterpret_cast<float*>(xq_rows + (DQ || SOLO ? dq_passes * (KW * 2048) : AQ * xq_stride));
   // Quantises the real rows of the tile whose slot ids are in s_rows[buf]: per pass 16 groups of 128 over all the
   // workgroup's lanes, LPG = 4 * KW lanes per group and 128 / LPG elements per lane.  The arithmetic is
   // group_quant_body's (reciprocal form, float scales), so bytes and scales are the ones the stand-alone kernels
   // write.  The caller makes the result visible to the other waves (a workgroup barrier) before anyone reads it.
   auto quantise_rows = [&](int buf) {
-   if constexpr (AQ > 0 && MOE) {
+   if constexpr (AQ > 1 && MOE) {
     typedef typename OT::storage XS;
     constexpr int LPG = 4 * KW, EL = 128 / LPG, VEC = EL / 8;  // 16-byte loads per lane: EL 16-bit values
     static_assert(KW <= 4 && EL % 8 == 0, "a lane takes whole 16-byte pieces");
@@ -506,84 +491,94 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
     }
   };
 
-  // DQ: group gi of the M * nkb groups of 128 belongs to eight lanes, 16 values each; pass p holds the groups 8 * KW * p + tid / 8.
-  // The 16-bit values lie where the quantised rows go, pass by pass, 32 bytes a lane as two halves of 16.
-  constexpr int DQ_MAX_PASSES = SKINNY_DQ_PASSES;
-  const int dq_groups = DQ ? g.M * nkb : 0, dq_passes = (dq_groups + 8 * KW - 1) / (8 * KW);
-  auto fetch_dense = [&]() {
-    if constexpr (DQ) {
-      const v4i rs = descriptor(g.A16, ((int64_t)(g.M - 1) * g.lda16 + (int64_t)g.K * 2));
+  // DQ, SOLO: group gi of the rows' groups of 128 belongs to eight lanes, 16 values each; pass p holds the groups
+  // 8 * KW * p + tid / 8.  The 16-bit values lie where the quantised rows go, pass by pass, 32 bytes a lane as two halves of 16.
+  // They are requested in front of the first weight blocks and waited for without these.
+  auto fetch_rows = [&](int pair) {
+    if constexpr (DQ || SOLO) {
+      const uint8_t* base = (const uint8_t*)g.A16 + (SOLO ? (int64_t)(pair / g.top_k) * g.lda16 : 0);
+      const v4i rs = descriptor(base, (SOLO ? 0 : (int64_t)(g.M - 1) * g.lda16) + (int64_t)g.K * 2);
       const uint32_t raw = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem + KW * PD * SLOT + wave * 2048;
       for (int p = 0; p < dq_passes; p++) {
-        const int gi = p * 8 * KW + (tid >> 3), r = gi / nkb;
+        const int gi = p * 8 * KW + (tid >> 3), r = SOLO ? 0 : gi / nkb;
         const uint32_t off = gi < dq_groups ? (uint32_t)(r * (int)g.lda16 + (gi - r * nkb) * 256 + (lane & 7) * 32) : SKINNY_NOWHERE;
 #pragma unroll
         for (int h = 0; h < 2; h++) dma16(rs, off + (uint32_t)(h * 16), 0, raw + p * (KW * 2048) + h * 1024, false);
       }
     }
   };
-  auto quantise_dense = [&]() {
-    if constexpr (DQ) {
+  // A chunk of passes at a time: its groups' quantised bytes end where, or before, the next chunk's 16-bit ones begin (one
+  // row; DQ has a single chunk).
+  auto quantise_fetched = [&]() {
+    if constexpr (DQ || SOLO) {
       typedef typename OT::storage XS;
-      v4i raw[DQ_MAX_PASSES][2];
       const uint8_t* src = xq_rows + wave * 2048 + lane * 16;
+      for (int p0 = 0; p0 < dq_passes; p0 += SKINNY_DQ_PASSES) {
+        v4i raw[SKINNY_DQ_PASSES][2];
 #pragma unroll
-      for (int p = 0; p < DQ_MAX_PASSES; p++)
-        if (p < dq_passes) {
-          raw[p][0] = *(const v4i*)(src + p * (KW * 2048));
-          raw[p][1] = *(const v4i*)(src + p * (KW * 2048) + 1024);
-        }
-      // the quantised rows replace the 16-bit ones
+        for (int p = 0; p < SKINNY_DQ_PASSES; p++)
+          if (p0 + p < dq_passes) {
+            raw[p][0] = *(const v4i*)(src + (p0 + p) * (KW * 2048));
+            raw[p][1] = *(const v4i*)(src + (p0 + p) * (KW * 2048) + 1024);
+          }
+        // the quantised rows replace the 16-bit ones
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+#pragma unroll
+        for (int p = 0; p < SKINNY_DQ_PASSES; p++)
+          if (p0 + p < dq_passes) {
+            // group_quant_body's arithmetic (reciprocal form, float scales)
+            const int gi = (p0 + p) * 8 * KW + (tid >> 3);
+            XS e[16];
+            float x[16];
+            __builtin_memcpy(e, raw[p], 32);
+            float amax = g.q_eps;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+              x[i] = OT::to_f32(e[i]);
+              amax = fmaxf(amax, fabsf(x[i]));
+            }
+            amax = lanes_max<8>(amax);
+            const float mul = g.q_max / amax;
+            uint32_t o[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+              o[i] = pack4_e4m3(clampf(x[4 * i] * mul, g.q_min, g.q_max), clampf(x[4 * i + 1] * mul, g.q_min, g.q_max),
+                                clampf(x[4 * i + 2] * mul, g.q_min, g.q_max), clampf(x[4 * i + 3] * mul, g.q_min, g.q_max));
+            if (gi < dq_groups) {
+              const int r = SOLO ? 0 : gi / nkb, c = gi - r * nkb;
+              *(v4i*)(xq_rows + r * xq_stride + c * 128 + (lane & 7) * 16) = v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
+              if ((lane & 7) == 0) xq_scales[r * nkb + c] = amax * (1.0f / g.q_max);
+            }
+          }
+      }
+      // visible to the other waves
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
-#pragma unroll
-      for (int p = 0; p < DQ_MAX_PASSES; p++)
-        if (p < dq_passes) {
-          // group_quant_body's arithmetic (reciprocal form, float scales)
-          const int gi = p * 8 * KW + (tid >> 3);
-          XS e[16];
-          float x[16];
-          __builtin_memcpy(e, raw[p], 32);
-          float amax = g.q_eps;
-#pragma unroll
-          for (int i = 0; i < 16; i++) {
-            x[i] = OT::to_f32(e[i]);
-            amax = fmaxf(amax, fabsf(x[i]));
-          }
-          amax = lanes_max<8>(amax);
-          const float mul = g.q_max / amax;
-          uint32_t o[4];
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-            o[i] = pack4_e4m3(clampf(x[4 * i] * mul, g.q_min, g.q_max), clampf(x[4 * i + 1] * mul, g.q_min, g.q_max),
-                              clampf(x[4 * i + 2] * mul, g.q_min, g.q_max), clampf(x[4 * i + 3] * mul, g.q_min, g.q_max));
-          if (gi < dq_groups) {
-            const int r = gi / nkb, c = gi - r * nkb;
-            *(v4i*)(xq_rows + r * xq_stride + c * 128 + (lane & 7) * 16) = v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
-            if ((lane & 7) == 0) xq_scales[r * nkb + c] = amax * (1.0f / g.q_max);
-          }
-        }
     }
   };
 
+  // pair of row r of the MoE tile at m0
+  auto row_id = [&](int buf, int at, int r) -> int { return SOLO ? (r == 0 ? at / (16 * FM) : g.num_valid) : s_rows[buf][r]; };
+
   int tile = blockIdx.x;
   if (!tile_exists(tile)) return;
+  fetch_rows(tile / tiles_n);
+  if (SOLO && g.sum_tiles > 0 && !g.sum_out)
+    for (int i = blockIdx.x * (64 * KW) + tid; i < g.sum_tiles; i += gridDim.x * (64 * KW)) g.sum_count[i] = 0;
+  look_ahead(tile);
   setup(tile, 0);
-  if constexpr (DQ) fetch_dense();
 #pragma unroll
   for (int s = 0; s < PD; s++)
     if (s < n_my) issue(s, block_of(s));
-  if constexpr (DQ) {
-    // the rows have landed when only the ring's loads are outstanding
-    if (n_my >= PD) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PD * LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-    quantise_dense();
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+  if constexpr (DQ || SOLO) {
+    skinny_wait<PD, LOADS>(n_my);
+    quantise_fetched();
   } else if constexpr (AQ > 0) {
     quantise_rows(0);
     if (KW > 1) __syncthreads();
   }
 
   for (;;) {
+    look_ahead(tile + (int)gridDim.x);
 #pragma unroll
     for (int i = 0; i < FM * FN; i++) acc[i] = acc_t{0, 0, 0, 0};
     // ---- the K loop: a ring of PD blocks in flight per wave -------------------------------------------------
@@ -611,7 +606,14 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
     const int o_n0 = n0, o_n_end = n_end, o_m0 = m0, o_expert = expert, o_buf = rows_buf;
     const int next = tile + (int)gridDim.x;
     const bool has_next = tile_exists(next);
+    const float o_weight = solo_weight;
     if (has_next) {
+      // (SOLO: the rows' place is free once every wave is past its K loop)
+      const bool other_row = SOLO && next / tiles_n / g.top_k != tile / tiles_n / g.top_k;
+      if (other_row) {
+        __syncthreads();
+        fetch_rows(next / tiles_n);
+      }
       setup(next, o_buf ^ 1);
       // with several waves the last slot of every ring carries the partial tiles first
 #pragma unroll
@@ -619,7 +621,11 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
         if (s < n_my) issue(s, block_of(s));
       // every wave is past its K loop (setup's barriers), so the rows can be replaced; with several waves the
       // barriers of the reduction below stand between these writes and the next tile's first reads
-      if constexpr (AQ > 0 && MOE) quantise_rows(o_buf ^ 1);
+      if constexpr (AQ > 1 && MOE) quantise_rows(o_buf ^ 1);
+      if (other_row) {
+        skinny_wait<PD - (KW > 1 ? 1 : 0), LOADS>(n_my);
+        quantise_fetched();
+      }
     }
 
     // ---- reduce the KW partial tiles through LDS (every wave's own last ring slot) ------------------------------
@@ -661,7 +667,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       if (paired) {
         // silu(gate) * up of the 16 x 16 patch, rounded as the stand-alone activation kernels round: the two GEMM
         // outputs to the 16-bit type first, then silu, then the product
-        const int tok = s_rows[o_buf][frow];
+        const int tok = row_id(o_buf, o_m0, frow);
         if (wave == 0 && tok < g.num_valid) {
           OS o[4];
 #pragma unroll
@@ -695,10 +701,11 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       bool row_ok;
       float wgt = 1.f;
       if (MOE) {
-        const int tok = s_rows[o_buf][i * 16 + frow];
+        const int tok = row_id(o_buf, o_m0, i * 16 + frow);
         row_ok = tok < g.num_valid;
         out_row = tok;
-        if (row_ok && g.mul_weight) wgt = g.topk_w[tok];
+        if (SOLO) wgt = o_weight;
+        else if (row_ok && g.mul_weight) wgt = g.topk_w[tok];
       } else {
         row_ok = (o_m0 + i * 16 + frow) < g.M;
         out_row = o_m0 + i * 16 + frow;
@@ -736,13 +743,57 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
         }
       }
       OS* crow = (OS*)g.C + out_row * g.ldc;
-      if (n + 3 < g.N && ((((uintptr_t)(crow + n)) & 7) == 0)) {
+      if (SOLO && g.sum_out) {  // (N % 32 == 0, and C is 256-byte aligned)
+        OS o[4] = {OT::from_f32(v[0]), OT::from_f32(v[1]), OT::from_f32(v[2]), OT::from_f32(v[3])};
+        uint64_t w2;
+        __builtin_memcpy(&w2, o, 8);
+        __hip_atomic_store((uint64_t*)(crow + n), w2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      } else if (n + 3 < g.N && ((((uintptr_t)(crow + n)) & 7) == 0)) {
         OS o[4] = {OT::from_f32(v[0]), OT::from_f32(v[1]), OT::from_f32(v[2]), OT::from_f32(v[3])};
         v2i w2;
         __builtin_memcpy(&w2, o, 8);
         *(v2i*)(crow + n) = w2;
       } else {
         for (int r = 0; r < 4 && n + r < g.N; r++) crow[n + r] = OT::from_f32(v[r]);
+      }
+    }
+    if constexpr (SOLO) {
+      // The pairs' patches went past this XCD's L2 (agent scope) and have arrived there before the tile is counted, so
+      // that whoever counts last reads all of them, in their order.
+      if (g.sum_out) {
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        if (KW > 1) __syncthreads();
+        if (wave == 0) {
+          int before = 0;
+          if (lane == 0) before = __hip_atomic_fetch_add(g.sum_count + o_n0 / (16 * FN), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          before = __builtin_amdgcn_readfirstlane(before);
+          asm volatile("" : : : "memory");
+          if (before == g.num_valid - 1 && lane < 4 * FN) {
+            const uint64_t* src = (const uint64_t*)((const OS*)g.C + o_n0 + 4 * lane);
+            const int64_t pitch = g.ldc / 4;
+            float sum[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int k0 = 0; k0 < g.num_valid; k0 += 8) {
+              uint64_t w[8];
+#pragma unroll
+              for (int k = 0; k < 8; k++)
+                w[k] = k0 + k < g.num_valid ? __hip_atomic_load(src + (k0 + k) * pitch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+#pragma unroll
+              for (int k = 0; k < 8; k++)
+                if (k0 + k < g.num_valid) {
+                  OS e[4];
+                  __builtin_memcpy(e, &w[k], 8);
+#pragma unroll
+                  for (int r = 0; r < 4; r++) sum[r] += OT::to_f32(e[r]);
+                }
+            }
+            OS o[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = OT::from_f32(sum[r] * g.sum_scale);
+            v2i w2;
+            __builtin_memcpy(&w2, o, 8);
+            *(v2i*)((OS*)g.sum_out + o_n0 + 4 * lane) = w2;
+          }
+        }
       }
     }
     if (!has_next) break;
@@ -761,8 +812,8 @@ static inline bool gemm8_skinny_ok(const GemmArgs& g, int64_t a_rows) {
 }
 
 // Workgroups of one launch that a CU holds at once: bounded by the LDS rings and by 32 wavefronts.
-static inline int skinny_fit(int smem, int kw) {
-  int n = 163840 / (smem + 1024);
+static inline int skinny_fit(int smem, int kw, int static_lds = 1024) {
+  int n = 163840 / (smem + static_lds);
   if (n > 32 / kw) n = 32 / kw;
   return n < 1 ? 1 : n;
 }
@@ -773,10 +824,10 @@ static inline int skinny_resident_per_cu(int kw, int extra_bytes = 0) {
 
 template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int AQ = 0>
 static int gemm8_skinny_launch_kw(const GemmArgs& g, hipStream_t st) {
-  constexpr bool DQ = AQ > 0 && !MOE;
+  constexpr bool DQ = AQ > 0 && !MOE, SOLO = AQ == 1 && MOE;
   constexpr int PD = skinny_depth<FM, FN, AQ, DQ>();
-  const int aq_bytes = DQ ? skinny_dq_bytes(g.M, g.K, KW) : AQ > 0 ? skinny_aq_bytes(AQ, g.K) : 0;
-  const int smem = DQ ? KW * PD * skinny_slot_bytes<FM, FN, AQ>() + aq_bytes : skinny_smem_bytes<FM, FN, AQ>(KW, aq_bytes);
+  const int aq_bytes = DQ || SOLO ? skinny_dq_bytes(SOLO ? 1 : g.M, g.K, KW) : AQ > 0 ? skinny_aq_bytes(AQ, g.K) : 0;
+  const int smem = DQ || SOLO ? KW * PD * skinny_slot_bytes<FM, FN, AQ>() + aq_bytes : skinny_smem_bytes<FM, FN, AQ>(KW, aq_bytes);
   if (smem > 160 * 1024) return fail(SGLAMD_ENOTSUP, "gemm: K = %d is too long for in-kernel activation quantisation", g.K);
   const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
   const int tiles_n = (g.N + R - 1) / R;
@@ -785,7 +836,7 @@ static int gemm8_skinny_launch_kw(const GemmArgs& g, hipStream_t st) {
   if (tiles <= 0) return SGLAMD_OK;
   if (tiles > 0x7fffffff) return fail(SGLAMD_EINVAL, "gemm: grid too large");
   // as many workgroups as the chip holds at once; each walks tiles blockIdx.x, + gridDim.x, ...
-  const int64_t resident = (int64_t)device_cus() * (DQ ? skinny_fit(smem, KW) : skinny_resident_per_cu<FM, FN, AQ>(KW, aq_bytes));
+  const int64_t resident = (int64_t)device_cus() * (SOLO ? skinny_fit(smem, KW, 128) : DQ ? skinny_fit(smem, KW) : skinny_resident_per_cu<FM, FN, AQ>(KW, aq_bytes));
   const unsigned blocks = (unsigned)(tiles < resident ? tiles : resident);
   auto kern = gemm8_skinny_kernel<FM, FN, MODE, OT, MOE, KW, PD, AQ>;
   if (smem > 64 * 1024) {
@@ -837,6 +888,8 @@ static inline int skinny_pick_kw(int64_t tiles, int nkb, int extra_bytes = 0) {
 // Shape of the last streaming launch of this thread and translation unit: (FM << 16) | (FN << 8) | KW.
 extern thread_local int skinny_last_shape;  // defined in gemm.hip
 
+// AQ: `g` carries the 16-bit source rows in A16 / lda16 (act_mode 1) and the quantisation constants.  MoE: every sorted block
+// holds at most AQ real rows; AQ = 1 has no sorted blocks but route_ids, the experts of one token's pairs.
 template <int FM, int FN, int MODE, typename OT, bool MOE, int AQ = 0>
 static int gemm8_skinny_launch_fn(const GemmArgs& g, hipStream_t st, int64_t expected_tiles_m) {
   const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
@@ -857,14 +910,6 @@ static int gemm8_skinny_launch_fn(const GemmArgs& g, hipStream_t st, int64_t exp
       if constexpr (skinny_kw_max<FM, FN, MOE ? AQ : 0>() >= 8) return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 8, AQ>(g, st);
       return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 4, AQ>(g, st);
   }
-}
-
-// MoE launch that quantises the activations in the kernel (see the head of this file): `g` carries the 16-bit
-// source rows in A16 / lda16 (act_mode 1) and the quantisation constants; every sorted block holds at
-// most four real rows (the caller launches it for at most four tokens).
-template <typename OT>
-static int gemm8_skinny_launch_actquant(const GemmArgs& g, hipStream_t st, int64_t expected_tiles_m) {
-  return gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, OT, true, 4>(g, st, expected_tiles_m);
 }
 
 // Cost of a dense launch with FN column tiles per workgroup trimmed to `rows` weight rows, in "weight rows streamed

@@ -1166,15 +1166,16 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   // tiles pair gate and up rows and write silu(gate) * up, the second GEMM quantises those 16-bit rows itself, at
   // most four per tile -- so these calls align the routing to blocks of 4 (a tile then holds one such block; an
   // expert named more than four times, which takes repeated ids within a token, gets several).  A single token
-  // also drops the sorting / quantising launch in front: both GEMMs sort the handful of routed pairs themselves and
-  // the first one quantises the hidden state itself (three launches; with more tokens the quantised rows of K = H
-  // bytes each would crowd the weight rings out of LDS: measured 150 against 120 us at two tokens).  Every variant produces the bits of the five-launch sequence.
+  // also drops the sorting / quantising launch in front, since its pairs are their own blocks and the first GEMM quantises
+  // the hidden state itself (with more tokens the quantised rows of K = H bytes each would crowd the weight rings out of
+  // LDS: measured 150 against 120 us at two tokens), and the sum behind: two launches.  Every variant produces the bits of
+  // the five-launch sequence.
   // SGLAMD_MOE_FUSE=1 keeps the launch in front, SGLAMD_MOE_FUSE=0 the whole sequence.
   static const int fuse_level = getenv("SGLAMD_MOE_FUSE") ? atoi(getenv("SGLAMD_MOE_FUSE")) : 2;
   const bool fuse_act = mode == GEMM_BLOCK_FP8 && fuse_level >= 1 && block_m == 16 && M <= 4 && T <= 32 && I % 256 == 0 &&
                         M * H * 2 < 0x7ffffff0ll && 2 * I * H < 0x7ffffff0ll && T * I * 2 < 0x7ffffff0ll;
-  // (T <= E: the in-kernel sort may open up to one block per pair, which is what the block bound then allows)
-  const bool fuse_all = fuse_act && fuse_level >= 2 && M == 1 && T <= E && !grouped;
+  // (T <= E: every pair has a block of its own; both GEMMs hold a 16-bit row in LDS beside the weight rings)
+  const bool fuse_all = fuse_act && fuse_level >= 2 && M == 1 && T <= E && H <= 32768 && I <= 32768 && !grouped;
   if (row) {
     const RowQuantArgs qa = {hidden, ws + w.xq, (float*)(ws + w.xs), H, M};
     const int nb = E + 1;
@@ -1374,6 +1375,8 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
       g.route_ids = topk_ids;
       g.route_ids_i64 = ids_dtype == SGLAMD_I64;
       g.route_experts = E;
+      g.sum_count = (int*)(ws + w.xq);  // (no quantised rows in this form)
+      g.sum_tiles = (int)(H / 32);
     } else {
       g.A = ws + w.xq;
       g.lda = H;
@@ -1442,10 +1445,18 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
       h.route_ids = topk_ids;
       h.route_ids_i64 = ids_dtype == SGLAMD_I64;
       h.route_experts = E;
+      h.sum_out = out;
+      h.sum_scale = routed_scaling_factor;
+      h.sum_count = (int*)(ws + w.xq);
+      h.sum_tiles = (int)(H / 32);
     }
-    rc = dtype == SGLAMD_BF16 ? gemm8_skinny_launch_actquant<BF16>(h, (hipStream_t)stream, expect)
-                              : gemm8_skinny_launch_actquant<F16>(h, (hipStream_t)stream, expect);
-    if (rc) return rc;
+    if (!fuse_all)
+      rc = dtype == SGLAMD_BF16 ? gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, BF16, true, 4>(h, st, expect)
+                                : gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, F16, true, 4>(h, st, expect);
+    else
+      rc = dtype == SGLAMD_BF16 ? gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, BF16, true, 1>(h, st, expect)
+                                : gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, F16, true, 1>(h, st, expect);
+    if (rc || fuse_all) return rc;
     return finish();
   }
   if (act_fused) {
