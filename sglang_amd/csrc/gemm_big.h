@@ -322,19 +322,33 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
 
   // Weight-block scales of this tile for the whole K range go to LDS once ([column block][K block]), so that
-  // the K loop has no memory instruction besides the direct-to-LDS loads and LDS reads.
+  // the K loop has no memory instruction besides the direct-to-LDS loads and LDS reads.  They are requested the same way, in
+  // front of the operands, which then do not wait for them to return (64 K blocks of a column block per load).
   float* sb_lds_all = (float*)(smem + SB_BASE);
   if (BLK) {
     const float* sb_tile = g.sb + (MOE ? (int64_t)max(expert, 0) * g.sb_se : 0);
-    for (int idx = tid; idx < (BN / 128) * nkb; idx += 128 * WGN) {
-      const int cb = idx / nkb, kb = idx - cb * nkb;
+    const int64_t span = ((int64_t)(nkb_all - 1) * g.sb_sk + 1) * 4;
+    auto kq_of = [&](int kb) -> int {
       int kq = kb_begin + kb;
       if constexpr (MOE) {
         kq += rot;
         if (kq >= nkb) kq -= nkb;
       }
-      sb_lds_all[cb * GEMM8_BIG_MAX_KB + kb] =
-          sb_tile[(int64_t)(min(n0 + cb * 128, g.N - 1) >> 7) * g.sb_sn + (int64_t)kq * g.sb_sk];
+      return kq;
+    };
+    auto row_of = [&](int cb) { return sb_tile + (int64_t)(min(n0 + cb * 128, g.N - 1) >> 7) * g.sb_sn; };
+    if (span < 0x7ffffff0ll) {
+      const int chunks = (nkb + 63) >> 6;
+      for (int c = wave; c < (BN / 128) * chunks; c += NW) {
+        const int cb = c / chunks, kb = (c - cb * chunks) * 64 + lane;
+        dma4(row_of(cb), (int)span, kb < nkb ? (uint32_t)(kq_of(kb) * (int)g.sb_sk) << 2 : 0x7ffffff0u, 0,
+             SB_BASE + (cb * GEMM8_BIG_MAX_KB + (c - cb * chunks) * 64) * 4);
+      }
+    } else {
+      for (int idx = tid; idx < (BN / 128) * nkb; idx += 128 * WGN) {
+        const int cb = idx / nkb, kb = idx - cb * nkb;
+        sb_lds_all[cb * GEMM8_BIG_MAX_KB + kb] = row_of(cb)[(int64_t)kq_of(kb) * g.sb_sk];
+      }
     }
   }
   const float* sb_mine = sb_lds_all + ((wn * 64) >> 7) * GEMM8_BIG_MAX_KB;
@@ -355,14 +369,18 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     }
   };
 
-  // Prologue: the first NS K blocks requested; block 0's weight fragments, the first row tile's activation
-  // fragments and the scales in registers.
+  // Prologue: the first NS K blocks requested; once the first has landed (the others are waited for where they are read),
+  // block 0's weight fragments, the first row tile's activation fragments and the scales in registers.
 #pragma unroll
   for (int st = 0; st < NS; st++)
 #pragma unroll
     for (int t = 0; t < MT; t++) issue_piece(st, block_at(st), st, t, 0), issue_piece(st, block_at(st), st, t, 1);
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-  __syncthreads();
+  constexpr int ahead = (NS - 1) * LPB;
+  static_assert(ahead < 64, "vmcnt field is 6 bits");
+  __builtin_amdgcn_s_waitcnt(0x0070 | (ahead & 15) | ((ahead >> 4) << 14));  // vmcnt(ahead) lgkmcnt(0)
+  asm volatile("" : : : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
   v8i wf[2][2];  // [column tile j][K half h]
 #pragma unroll
   for (int j = 0; j < 2; j++)
