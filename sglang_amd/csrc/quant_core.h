@@ -217,6 +217,20 @@ struct RowQuantArgs {
   int64_t rows;
 };
 
+// (int)roundf(x) for |x| below 2^22: with the largest float below one half, halves round away from zero and everything under
+// them stays (every float up to 200 compared).  Three instructions for roundf's eight: the INT8 rows were bound by their
+// arithmetic, 1000 x 28672 values 21.4 -> 18.9 us, 4000 x 18432 52 -> 46.
+__device__ __forceinline__ int round_away(float x) {
+#pragma clang fp contract(off)  // the scaled value is rounded before the sum
+  return (int)(x + copysignf(0x1.fffffep-2f, x));
+}
+// The low bytes of four integers.
+__device__ __forceinline__ uint32_t pack4_low(int a, int b, int c, int d) {
+  const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x0c0c0400u);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
 // TEAM: lanes that share a row, 32 or 64 (no barrier), a multiple of 64, or 0 for the whole workgroup; `row` is the lane's
 // own and may be past the end, since every lane takes part in the barrier.
 // A row of the experts' activations is 256 to 2048 values: a workgroup per row leaves most of its lanes without work, and
@@ -288,9 +302,7 @@ __device__ __forceinline__ void row_quant_body(const RowQuantArgs& a, int64_t ro
 #pragma unroll
       for (int j = 0; j < 4; j++) x[j] = T::to_f32(b[4 * h + j]) * mul;
       if constexpr (INT8) {
-        w[h] = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) w[h] |= ((uint32_t)(int)roundf(x[j]) & 0xff) << (8 * j);
+        w[h] = pack4_low(round_away(x[0]), round_away(x[1]), round_away(x[2]), round_away(x[3]));
       } else {
         w[h] = pack4_e4m3(clampf(x[0], -448.f, 448.f), clampf(x[1], -448.f, 448.f), clampf(x[2], -448.f, 448.f),
                           clampf(x[3], -448.f, 448.f));
