@@ -78,11 +78,7 @@ static inline bool moe_quad_scales(const GemmArgs& g) {
 // RAGGED: K is not a multiple of 128.  The last K block's 16-byte pieces past the end of a row are requested outside the
 // descriptor's range by both operands (zeros; a row's neighbour may hold NaN), which is a select per load: the row
 // modes only, which have no fold and so registers and issue slots to spare.
-// E8: every scale is a power of two; the MFMA applies them through its scale operands and the products of all K blocks add
-// up in its accumulators (see gemm8_big_persist_kernel).  Without the folds the loop is bound by what its loads move:
-// 7168 x 18432 at 300 rows (128-row tiles, K in three slices) 68.2 -> 66.2 us for the layer, at 700 rows 111 -> 104, level at
-// 100, where the weights are the time.
-template <int MODE, typename OT, int WGN, int MT, bool MOE = false, bool RAGGED = false, bool E8 = false>
+template <int MODE, typename OT, int WGN, int MT, bool MOE = false, bool RAGGED = false>
 __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub; buffer-resource builtins are device-only
   constexpr int BM = 64 * MT, BN = 64 * WGN, NW = 2 * WGN, WTM = 32 * MT;
@@ -156,8 +152,6 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   constexpr int APT = A_LOADS / MT;
   static_assert(A_LOADS % MT == 0 && B_LOADS == 4, "piece layout assumes 8 A row groups per tile and 4 B loads per wave");
   constexpr bool BLK = gemm_is_block(MODE);
-  constexpr bool FOLD = BLK && !E8;  // a K block's products are folded into the sums with their scales
-  static_assert(!E8 || MODE == GEMM_BLOCK_FP8, "scales through the MFMA's scale operands: FP8 only");
   // loads of piece t per wave, and of a whole block
   auto piece_loads = [](int t) constexpr { return APT + (4 / MT + ((4 % MT) > t ? 1 : 0)) + ((BLK && t == MT - 1) ? 1 : 0); };
   constexpr int LPB = A_LOADS + B_LOADS + (BLK ? 1 : 0);
@@ -353,9 +347,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   }
   const float* sb_mine = sb_lds_all + ((wn * 64) >> 7) * GEMM8_BIG_MAX_KB;
 
-  // MFMA of one 32x32 output tile over one 64-wide half of the K block; its scale operands are one except with E8
-  auto exponent = [](float v) -> int { return (int)((__builtin_bit_cast(uint32_t, v) >> 23) & 0xffu); };
-  int sx_cur = 0x7f7f7f7f, sw_cur = 0x7f7f7f7f;
+  // MFMA of one 32x32 output tile over one 64-wide half of the K block
   auto mm_half = [&](const v8i& w, const v8i& x, prod16_t c) -> prod16_t {
     if constexpr (gemm_is_int8(MODE)) {
       // v_mfma_i32_32x32x32_i8 takes 16 bytes per lane; the 32 bytes a lane holds per 64-byte half are two
@@ -365,7 +357,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       c = __builtin_amdgcn_mfma_i32_32x32x32_i8(wl, xl, c, 0, 0, 0);
       return __builtin_amdgcn_mfma_i32_32x32x32_i8(wh, xh, c, 0, 0, 0);
     } else {
-      return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, x, c, 0, 0, 0, sw_cur, 0, sx_cur);
+      return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, x, c, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
     }
   };
 
@@ -389,7 +381,6 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   v8i x0 = xfrag(0, 0, 0), x1 = xfrag(0, 0, 1);
   float sa_cur = BLK ? xscale(0, 0) : 1.f;
   float sb_cur = BLK ? sb_mine[0] : 1.f;
-  if constexpr (E8) sx_cur = exponent(sa_cur), sw_cur = exponent(sb_cur);
 
   // Schedule of one row tile (block mode), all of it issued by one wave in this order:
   //   M1: qa  = W[0][h0] x X[h0]      M2: qa += W[0][h1] x X[h1]
@@ -416,7 +407,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
   for (int r = 0; r < 16; r++) qa[r] = 0, qb[r] = 0, zero16[r] = 0;
   float scp = 0.f;
   auto fold = [&](acc16_t& dst, const prod16_t& q, float sc) {
-    if constexpr (FOLD) {
+    if constexpr (BLK) {
 #pragma unroll
       for (int r = 0; r < 16; r++) dst[r] = fmaf((float)q[r], sc, dst[r]);
     }
@@ -448,7 +439,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
     }();
     static_assert(keep < 64, "vmcnt field is 6 bits");
 
-    if constexpr (FOLD) {
+    if constexpr (BLK) {
       qa = mm_half(wf[0][0], x0, zero16);
       qa = mm_half(wf[0][1], x1, qa);
     } else {
@@ -468,7 +459,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       wf[0][1] = wfrag(nxt, 0, 1);
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
     }
-    if constexpr (FOLD) {
+    if constexpr (BLK) {
       fold(acc[prev][1], qb, scp);
       __builtin_amdgcn_sched_group_barrier(0x2, FOLDN, 0);
       qb = mm_half(wf[1][0], x0, zero16);
@@ -496,7 +487,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       }
       __builtin_amdgcn_sched_group_barrier(0x100, BLK ? 6 : 4, 0);
     }
-    if constexpr (FOLD) qb = mm_half(wf[1][1], x1, qb);
+    if constexpr (BLK) qb = mm_half(wf[1][1], x1, qb);
     else acc[i][1] = mm_half(wf[1][1], x1, acc[i][1]);
     __builtin_amdgcn_sched_group_barrier(0x8, MPH, 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -510,12 +501,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       wf[1][1] = wfrag(nxt, 1, 1);
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
     }
-    if constexpr (E8) {
-      sb_cur = sb_nxt;
-      sx_cur = exponent(sa_nxt);
-      sw_cur = exponent(sb_nxt);
-    }
-    if constexpr (FOLD) {
+    if constexpr (BLK) {
       scp = sa_cur * sb_cur;
       sa_cur = sa_nxt;
       sb_cur = sb_nxt;
@@ -540,7 +526,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm8_big_kernel(GemmArgs g) {
       }
     }
   }
-  if constexpr (FOLD) fold(acc[MT - 1][1], qb, scp);
+  if constexpr (BLK) fold(acc[MT - 1][1], qb, scp);
 
   // Epilogue.  Register r of tile (i, j) is C[m = .. + lane%32][n = .. + 8*(r/4) + 4*(lane/32) + r%4].
   typedef typename OT::storage OS;
@@ -821,15 +807,12 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool p
   return best;
 }
 
-template <int MODE, typename OT, int WGN, int MT, bool RAGGED = false, bool E8 = false>
+template <int MODE, typename OT, int WGN, int MT, bool RAGGED = false>
 static int gemm8_big_launch(const GemmArgs& g, hipStream_t st, int slices, void* workspace) {
   if constexpr (!gemm_is_block(MODE) && !RAGGED) {
     if (g.K & 127) return gemm8_big_launch<MODE, OT, WGN, MT, true>(g, st, slices, workspace);
   }
-  if constexpr (MODE == GEMM_BLOCK_FP8 && !E8) {
-    if (g.scales_pow2) return gemm8_big_launch<MODE, OT, WGN, MT, RAGGED, true>(g, st, slices, workspace);
-  }
-  auto kern = gemm8_big_kernel<MODE, OT, WGN, MT, false, RAGGED, E8>;
+  auto kern = gemm8_big_kernel<MODE, OT, WGN, MT, false, RAGGED>;
   constexpr int smem = gemm8_big_smem<WGN, MT>();
   static SmemAttrOnce attr;
   hipError_t e = raise_dynamic_smem(attr, (const void*)kern, smem);
