@@ -1089,6 +1089,12 @@ int moe_auto_block_rows(int64_t M, int E, int topk, int64_t H, int64_t I) {
   return 192;
 }
 int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1, 0, 0); }
+// The expert-major layer gives the bits of its separate operators, which know an expert's rows and nothing of the layer: it
+// leaves the 16-slot blocks, whose kernel sums K in another order than the tile kernels, where they do.
+int moe_grouped_layer_block(int64_t M, int E, int topk, int64_t H, int64_t I) {
+  const int separate = grouped_block_m(M * topk, E), block = moe_auto_block(M, E, topk, H, I);
+  return separate <= 32 || block <= 32 ? separate : block;
+}
 }  // namespace
 
 extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, int64_t I, int E, int topk, int block_m) {
@@ -1100,8 +1106,15 @@ extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, in
 extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk,
                                                     int block_m) {
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
-  if (block_m == 0) block_m = gemm_is_block(mode) ? moe_auto_block(M, E, topk, H, I, gemm_is_int8(mode)) : moe_auto_block_rows(M, E, topk, H, I);
-  return moe_ws_layout(M, H, I, E, topk, block_m).total;
+  const int picked = block_m                ? block_m
+                     : gemm_is_block(mode) ? moe_auto_block(M, E, topk, H, I, gemm_is_int8(mode))
+                                           : moe_auto_block_rows(M, E, topk, H, I);
+  int64_t total = moe_ws_layout(M, H, I, E, topk, picked).total;
+  if (block_m == 0 && mode == GEMM_BLOCK_FP8) {  // (the expert-major layer is sized here too)
+    const int64_t grouped = moe_ws_layout(M, H, I, E, topk, moe_grouped_layer_block(M, E, topk, H, I)).total;
+    if (grouped > total) total = grouped;
+  }
+  return total;
 }
 
 // What the expert-major form of the layer adds: the caller's tables, and routing weights that are rounded to the layer's
@@ -1131,7 +1144,9 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   SGLAMD_REQUIRE(!row || I <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: intermediate size %lld is beyond %lld",
                  (long long)I, (long long)ROW_QUANT_MAX_HIDDEN);
   SGLAMD_REQUIRE(row || (!b13 && !b2), SGLAMD_ENOTSUP, "fused_moe: biases go with row-scaled weights");
-  if (block_m == 0) block_m = row ? moe_auto_block_rows(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I, int8);
+  if (block_m == 0)
+    block_m = row ? moe_auto_block_rows(M, E, topk, H, I)
+              : grouped ? moe_grouped_layer_block(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I, int8);
   SGLAMD_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128 || block_m == 192, SGLAMD_EINVAL,
                  "fused_moe: block_m must be 16, 32, 64, 128 or 192");
   const MoeWs w = moe_ws_layout(M, H, I, E, topk, block_m);
