@@ -148,8 +148,8 @@ int sglamd_fp8_blockwise_scaled_mm(const void* a, int64_t lda, const void* b, in
 /* The same GEMM for scales that are all powers of two -- UE8M0 scales, as DeepSeek-V3.1 checkpoints and the
  * reference's DeepGEMM path carry them (python/sglang/srt/layers/quantization/fp8_kernel.py:1149-1174 with
  * scale_ue8m0, python/sglang/srt/layers/quantization/fp8_utils.py:1348-1383), expanded to fp32 by
- * sglamd_ue8m0_unpack.  Same arguments and result up to fp32 summation order; where the launch runs one of the
- * large-tile kernels, the scales' exponent bytes go into the MFMA's block-scale operands and the K blocks add up in
+ * sglamd_ue8m0_unpack.  Same arguments and result up to fp32 summation order; where the launch runs the persistent
+ * large-tile kernel, the scales' exponent bytes go into the MFMA's block-scale operands and the K blocks add up in
  * the MFMA accumulators (no multiply-add per element and K block).  A scale that is not a power of two counts as
  * the power of two below it there; the other kernels use the scale as given. */
 int sglamd_fp8_blockwise_scaled_mm_pow2(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
