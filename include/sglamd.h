@@ -177,6 +177,14 @@ int sglamd_fp8_block_linear(const void* x, int dtype, int64_t M, int64_t K, cons
                             int64_t sb_stride_n, int64_t sb_stride_k, const void* bias, void* out, int64_t ldc, int64_t N,
                             void* q, float* sa, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The per-channel FP8 linear layer: x [M, K] (SGLAMD_F16 or SGLAMD_BF16, rows K elements apart) quantised per row
+ * (sglamd_per_token_quant_fp8), times w [N, K] with one scale per weight row, plus an optional bias (sglamd_fp8_scaled_mm).
+ * One launch for a few rows, otherwise those two entry points in turn, through the scratch q (M * K bytes) and sa (M floats).
+ * The same bits either way. */
+int sglamd_fp8_row_linear(const void* x, int dtype, int64_t M, int64_t K, const void* w, int64_t ldb, const float* sb,
+                          const void* bias, void* out, int64_t ldc, int64_t N, void* q, float* sa, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
 /* The block-scaled GEMM on int8 operands: the int32 partial product of every 128-wide K block is exact and is
  * folded as float(p) * (sa[m, kb] * sb[n/128, kb]) into the fp32 accumulator.  Same arguments as above.
  * Stands in for w8a8_block_int8_matmul (python/sglang/srt/layers/quantization/int8_kernel.py:228-441, a Triton

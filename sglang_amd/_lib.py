@@ -31,6 +31,7 @@ SIGNATURES = {
     "sglamd_fp8_blockwise_scaled_mm_bias": [_p, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _i64, _i, _p, _p, _i64, _i,
                                             _i64, _i64, _i64, _p, _i64, _p],
     "sglamd_fp8_block_linear": [_p, _i, _i64, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _p, _i64, _p],
+    "sglamd_fp8_row_linear": [_p, _i, _i64, _i64, _p, _i64, _p, _p, _p, _i64, _i64, _p, _p, _p, _i64, _p],
     "sglamd_int8_blockwise_scaled_mm": [_p, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i, _i64, _i64,
                                        _i64, _p, _i64, _p],
     "sglamd_fp8_scaled_mm": [_p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _i, _i64, _i64, _i64, _p, _i64, _p],

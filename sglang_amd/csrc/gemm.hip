@@ -9,8 +9,9 @@ thread_local int skinny_last_shape = 0;
 
 extern template int dispatch_out<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out_biased<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
-extern template int dispatch_quantising<false>(const GemmArgs&, int, hipStream_t, bool);
-extern template int dispatch_quantising<true>(const GemmArgs&, int, hipStream_t, bool);
+extern template int dispatch_quantising<GEMM_BLOCK_FP8, false>(const GemmArgs&, int, hipStream_t, bool);
+extern template int dispatch_quantising<GEMM_BLOCK_FP8, true>(const GemmArgs&, int, hipStream_t, bool);
+extern template int dispatch_quantising<GEMM_ROW_FP8, false>(const GemmArgs&, int, hipStream_t, bool);
 extern template int dispatch_out<GEMM_ROW_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out<GEMM_ROW_INT8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out<GEMM_BLOCK_INT8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
@@ -103,13 +104,15 @@ static int quantising_max_rows() {
   static const int v = getenv("SGLAMD_LINEAR_FUSE_ROWS") ? atoi(getenv("SGLAMD_LINEAR_FUSE_ROWS")) : 4;  // tuning knob
   return v;
 }
-// Which of them do.  A launch less saves 2-3 us; every workgroup quantising every row costs it time that grows with M * K
-// and delays its weight stream.  Two launches -> one, us, weights read from HBM (N x K): one row 7168 x 18432 25.2 -> 24.2,
-// 7168 x 16384 23.2 -> 22.2, 36864 x 7168 44.0 -> 42.2, 4096 x 4096 11.8 -> 9.5; two rows 23.2 -> 23.4 at 16384, 24.8 -> 25.2
-// at 18432, but 44.2 -> 43.2 at 7168; four rows 24576 x 1536 12.5 -> 10.3, 4096 x 4096 11.5 -> 9.0, 1024 x 7168 11.6 -> 9.5,
-// 36864 x 7168 44.2 -> 44.3.  At eight rows it turns: 36864 x 1024 12.6 -> 16.1, 24576 x 1536 12.4 -> 12.1.
+// Which of them do.  A launch less saves 1-2 us; every workgroup quantising every row costs it time that grows with M * K
+// and delays its weight stream.  Two launches -> one, us, weights from HBM, queue kept full, block scales (row scales):
+//   one row    36864 x 7168 42.6 -> 41.2, 7168 x 16384 21.9 -> 21.4, 24576 x 1536 10.9 -> 8.9 (11.2 -> 9.5), 4096 x 4096 7.5 -> 6.3
+//              (8.1 -> 6.7), 1024 x 7168 8.3 -> 6.6 (8.7 -> 6.9), (10240 x 8192 17.8 -> 16.7)
+//   two rows   36864 x 7168 42.6 -> 42.1, 4096 x 4096 7.7 -> 6.5 (8.1 -> 7.0), 1024 x 7168 8.3 -> 7.2 (8.8 -> 7.8)
+//   three      36864 x 7168 42.7 -> 42.9, 1024 x 7168 8.4 -> 7.9 (8.8 -> 8.6), (10240 x 8192 17.9 -> 18.9)
+//   four       36864 x 7168 42.7 -> 43.4, 4096 x 4096 7.9 -> 7.2 (8.2 -> 8.0), 1024 x 7168 8.4 -> 8.2 (8.8 -> 9.1)
 static bool linear_quantises(int64_t M, int64_t K) {
-  return M >= 1 && M <= quantising_max_rows() && (M == 1 || M * K <= 28672);
+  return M >= 1 && M <= quantising_max_rows() && (M == 1 || M * K <= 16384);
 }
 
 extern "C" int sglamd_fp8_block_linear(const void* x, int dtype, int64_t M, int64_t K, const void* w, int64_t ldb,
@@ -144,8 +147,8 @@ extern "C" int sglamd_fp8_block_linear(const void* x, int dtype, int64_t M, int6
     g.N = (int)N;
     g.K = (int)K;
     g.bias = bias;
-    if (gemm8_skinny_ok(g, M) && (bias ? dispatch_quantising<true> : dispatch_quantising<false>)(g, dtype, (hipStream_t)stream, false))
-      return (bias ? dispatch_quantising<true> : dispatch_quantising<false>)(g, dtype, (hipStream_t)stream, true);
+    if (gemm8_skinny_ok(g, M) && (bias ? dispatch_quantising<GEMM_BLOCK_FP8, true> : dispatch_quantising<GEMM_BLOCK_FP8, false>)(g, dtype, (hipStream_t)stream, false))
+      return (bias ? dispatch_quantising<GEMM_BLOCK_FP8, true> : dispatch_quantising<GEMM_BLOCK_FP8, false>)(g, dtype, (hipStream_t)stream, true);
   }
   const int rc = sglamd_per_token_group_quant_8bit(x, dtype, q, SGLAMD_FP8_E4M3, sa, M, K, 128, SGLAMD_SCALE_COL_MAJOR, M, 1e-10f,
                                                    -448.f, 448.f, SGLAMD_QUANT_FORM_RECIPROCAL, stream);
@@ -194,6 +197,40 @@ extern "C" int sglamd_fp8_scaled_mm(const void* a, int64_t lda, const void* b, i
                                     void* stream) {
   return rowwise(GEMM_ROW_FP8, "fp8_scaled_mm", a, lda, b, ldb, sa, sb, bias, out, ldc, out_dtype, M, N, K, workspace,
                  workspace_bytes, stream);
+}
+
+extern "C" int sglamd_fp8_row_linear(const void* x, int dtype, int64_t M, int64_t K, const void* w, int64_t ldb, const float* sb,
+                                     const void* bias, void* out, int64_t ldc, int64_t N, void* q, float* sa, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  const char* op = "fp8_row_linear";
+  SGLAMD_REQUIRE(x && w && sb && out && q && sa, SGLAMD_EINVAL, "%s: null pointer", op);
+  SGLAMD_REQUIRE(dtype == SGLAMD_BF16 || dtype == SGLAMD_F16, SGLAMD_EINVAL, "%s: dtype must be Half or BFloat16", op);
+  const DeviceScope scope;
+  if (linear_quantises(M, K) && K % 128 == 0 && ((uintptr_t)x % 16) == 0) {
+    int rc = check_common(op, x, w, out, M, N, K, K, ldb, ldc);
+    if (rc) return rc;
+    GemmArgs g = {};
+    g.A16 = x;
+    g.lda16 = K * 2;
+    g.act_mode = 1;
+    g.q_min = -448.f;
+    g.q_max = 448.f;
+    g.lda = K;
+    g.B = (const uint8_t*)w;
+    g.ldb = ldb;
+    g.sb = sb;
+    g.bias = bias;
+    g.C = out;
+    g.ldc = ldc;
+    g.M = (int)M;
+    g.N = (int)N;
+    g.K = (int)K;
+    if (gemm8_skinny_ok(g, M) && dispatch_quantising<GEMM_ROW_FP8, false>(g, dtype, (hipStream_t)stream, false))
+      return dispatch_quantising<GEMM_ROW_FP8, false>(g, dtype, (hipStream_t)stream, true);
+  }
+  const int rc = sglamd_per_token_quant_fp8(x, dtype, q, sa, M, K, stream);
+  if (rc) return rc;
+  return rowwise(GEMM_ROW_FP8, op, q, K, w, ldb, sa, sb, bias, out, ldc, dtype, M, N, K, workspace, workspace_bytes, stream);
 }
 
 extern "C" int sglamd_int8_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,

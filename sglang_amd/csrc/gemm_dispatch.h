@@ -146,14 +146,14 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
   return gemm8_launch<128, 128, 2, 2, MODE, OT, false>(g, st);
 }
 
-// A block-scaled FP8 linear layer of a few rows in one launch (gemm8_skinny_quantising).
-template <bool BIASED>
+// An FP8 linear layer of a few rows in one launch (gemm8_skinny_quantising).
+template <int MODE, bool BIASED>
 int dispatch_quantising(const GemmArgs& g, int out_dtype, hipStream_t st, bool launch) {
   if (launch) RAN(SGLAMD_KERNEL_STREAMING);
   if constexpr (BIASED)
-    return out_dtype == SGLAMD_BF16 ? gemm8_skinny_quantising<Biased<BF16>>(g, st, launch)
-                                    : gemm8_skinny_quantising<Biased<F16>>(g, st, launch);
-  return out_dtype == SGLAMD_BF16 ? gemm8_skinny_quantising<BF16>(g, st, launch) : gemm8_skinny_quantising<F16>(g, st, launch);
+    return out_dtype == SGLAMD_BF16 ? gemm8_skinny_quantising<MODE, Biased<BF16>>(g, st, launch)
+                                    : gemm8_skinny_quantising<MODE, Biased<F16>>(g, st, launch);
+  return out_dtype == SGLAMD_BF16 ? gemm8_skinny_quantising<MODE, BF16>(g, st, launch) : gemm8_skinny_quantising<MODE, F16>(g, st, launch);
 }
 
 template <int MODE>

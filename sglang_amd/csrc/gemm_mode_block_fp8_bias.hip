@@ -3,5 +3,5 @@
 
 namespace sglamd {
 template int dispatch_out_biased<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
-template int dispatch_quantising<true>(const GemmArgs&, int, hipStream_t, bool);
+template int dispatch_quantising<GEMM_BLOCK_FP8, true>(const GemmArgs&, int, hipStream_t, bool);
 }  // namespace sglamd

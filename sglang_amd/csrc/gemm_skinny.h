@@ -119,11 +119,11 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   constexpr int SLOT = skinny_slot_bytes<FM, FN, AQ>();
   constexpr int X_OFF = FN * 2048, SA_OFF = AQ > 0 ? 0 : (FN + FM) * 2048, SB_OFF = AQ > 0 ? FN * 2048 : SA_OFF + 256;
   // direct-to-LDS loads per K block and wave
-  constexpr int LOADS = AQ > 0 ? 2 * FN + 1 : 2 * FN + 2 * FM + (BLK ? 2 : 0);
+  constexpr int LOADS = AQ > 0 ? 2 * FN + (BLK ? 1 : 0) : 2 * FN + 2 * FM + (BLK ? 2 : 0);
   constexpr bool DQ = AQ > 0 && !MOE;
   constexpr bool SOLO = AQ == 1 && MOE;  // the routed pairs of one token: sorted block p is pair p
-  static_assert(AQ == 0 || (MODE == GEMM_BLOCK_FP8 && FM == 1 && AQ <= 16),
-                "in-kernel activation quantisation: block FP8, one row tile");
+  static_assert(AQ == 0 || ((MODE == GEMM_BLOCK_FP8 || (MODE == GEMM_ROW_FP8 && !MOE)) && FM == 1 && AQ <= 16),
+                "in-kernel activation quantisation: FP8, one row tile");
   static_assert(PD >= 1 && PD * LOADS < 64, "the vmcnt field counts up to 63 loads in flight");
   // a wave's partial tiles wait for the cross-wave sum in its last ring slot when they fit there; wide tiles put
   // them side by side over the whole ring area instead (behind a barrier: every wave's loads have landed by then)
@@ -135,6 +135,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // Per wave a ring of PD slots.  The last slot of every wave doubles as the place where its partial tiles wait
   // for the cross-wave sum at the end of a tile.
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  __shared__ uint32_t s_amax[DQ && !BLK ? 16 : 1];  // DQ, row scales: the rows' maxima (bits of floats that are not negative)
   __shared__ int s_rows[2][FM * 16];  // MoE: sorted slot ids of the tile's rows, for the current and the next tile
 
   const int tid = threadIdx.x;
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       dma16(w_rs, wv[j][1] | kill1, koff, base + j * 2048 + 1024, true);
     }
     if constexpr (AQ > 0) {
-      dma4(sb_rs, sbv_off, (kb * (int)g.sb_sk) << 2, base + SB_OFF);
+      if (BLK) dma4(sb_rs, sbv_off, (kb * (int)g.sb_sk) << 2, base + SB_OFF);
     } else {
 #pragma unroll
       for (int i = 0; i < FM; i++) {
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
         const uint8_t* xr = xq_rows + frow * xq_stride + (kb_now << 7) + fk * 32;
         lo = *(const v4i*)xr;
         hi = *(const v4i*)(xr + 16);
-        sav[0] = xq_scales[frow * nkb + kb_now];
+        if (BLK) sav[0] = xq_scales[frow * nkb + kb_now];
       }
       xf[0] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     } else {
@@ -523,10 +524,26 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
           }
         // the quantised rows replace the 16-bit ones
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        if constexpr (!BLK) {
+          // (one chunk: the rows' maxima over all of their groups)
+#pragma unroll
+          for (int p = 0; p < SKINNY_DQ_PASSES; p++)
+            if (p0 + p < dq_passes) {
+              const int gi = (p0 + p) * 8 * KW + (tid >> 3);
+              XS e[16];
+              __builtin_memcpy(e, raw[p], 32);
+              float m = 0.f;
+#pragma unroll
+              for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(OT::to_f32(e[i])));
+              m = lanes_max<8>(m);
+              if ((lane & 7) == 0 && gi < dq_groups) atomicMax(&s_amax[gi / nkb], __float_as_uint(m));
+            }
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        }
 #pragma unroll
         for (int p = 0; p < SKINNY_DQ_PASSES; p++)
           if (p0 + p < dq_passes) {
-            // group_quant_body's arithmetic (reciprocal form, float scales)
+            // group_quant_body's arithmetic (reciprocal form, float scales); row scales: row_quant_body's
             const int gi = (p0 + p) * 8 * KW + (tid >> 3);
             XS e[16];
             float x[16];
@@ -535,10 +552,17 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
 #pragma unroll
             for (int i = 0; i < 16; i++) {
               x[i] = OT::to_f32(e[i]);
-              amax = fmaxf(amax, fabsf(x[i]));
+              if (BLK) amax = fmaxf(amax, fabsf(x[i]));
             }
-            amax = lanes_max<8>(amax);
-            const float mul = g.q_max / amax;
+            float mul;
+            if constexpr (BLK) {
+              amax = lanes_max<8>(amax);
+              mul = g.q_max / amax;
+            } else {
+              const float scale = __uint_as_float(s_amax[gi < dq_groups ? gi / nkb : 0]) / 448.0f;
+              mul = (scale == 0.f) ? 0.f : 1.0f / scale;
+              amax = scale;
+            }
             uint32_t o[4];
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -547,7 +571,11 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
             if (gi < dq_groups) {
               const int r = SOLO ? 0 : gi / nkb, c = gi - r * nkb;
               *(v4i*)(xq_rows + r * xq_stride + c * 128 + (lane & 7) * 16) = v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
-              if ((lane & 7) == 0) xq_scales[r * nkb + c] = amax * (1.0f / g.q_max);
+              if constexpr (BLK) {
+                if ((lane & 7) == 0) xq_scales[r * nkb + c] = amax * (1.0f / g.q_max);
+              } else {
+                if ((lane & 7) == 0 && c == 0) xq_scales[r] = amax;
+              }
             }
           }
       }
@@ -562,6 +590,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   int tile = blockIdx.x;
   if (!tile_exists(tile)) return;
   fetch_rows(tile / tiles_n);
+  if (DQ && !BLK && tid < 16) s_amax[tid] = 0;  // (visible behind the barrier in front of the first maxima)
   if (SOLO && g.sum_tiles > 0 && !g.sum_out)
     for (int i = blockIdx.x * (64 * KW) + tid; i < g.sum_tiles; i += gridDim.x * (64 * KW)) g.sum_count[i] = 0;
   look_ahead(tile);
@@ -717,7 +746,8 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       const float* sb_row = g.sb;
       const OS* bias = (const OS*)g.bias;
       if constexpr (!gemm_is_block(MODE)) {
-        sam = g.sa[MOE ? (out_row / g.top_k) * g.sa_sm : out_row];
+        if constexpr (DQ) sam = xq_scales[out_row];
+        else sam = g.sa[MOE ? (out_row / g.top_k) * g.sa_sm : out_row];
         if (MOE) {
           sb_row += (int64_t)max(o_expert, 0) * g.sb_se;
           if (bias) bias += (int64_t)max(o_expert, 0) * g.sb_sk;
@@ -996,21 +1026,24 @@ static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expec
 // constants.  `launch` false: whether it takes the shape.
 template <int FN>
 static bool skinny_dq_fits(const GemmArgs& g) {
-  const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
-  const int kw = skinny_pick_kw<1, FN>((g.N + R - 1) / R, g.K >> 7);
+  const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN, tiles = (g.N + R - 1) / R;
+  const int kw = skinny_pick_kw<1, FN>(tiles, g.K >> 7);
   const int groups = g.M * (g.K >> 7);
-  return (groups + 8 * kw - 1) / (8 * kw) <= SKINNY_DQ_PASSES &&
-         kw * skinny_depth<1, FN, 1, true>() * skinny_slot_bytes<1, FN, 1>() + skinny_dq_bytes(g.M, g.K, kw) <= 158 * 1024;
+  const int smem = kw * skinny_depth<1, FN, 1, true>() * skinny_slot_bytes<1, FN, 1>() + skinny_dq_bytes(g.M, g.K, kw);
+  // the rows must not take a workgroup's place on a CU: one row of 57344 x 8192 75.1 -> 81.4 us with three instead of four
+  const int plain = skinny_resident_per_cu<1, FN>(kw), wanted = (tiles + device_cus() - 1) / device_cus();
+  return (groups + 8 * kw - 1) / (8 * kw) <= SKINNY_DQ_PASSES && smem <= 158 * 1024 &&
+         skinny_fit(smem, kw) >= (wanted < plain ? wanted : plain);
 }
-template <typename OT>
+template <int MODE, typename OT>
 static int gemm8_skinny_quantising(const GemmArgs& g0, hipStream_t st, bool launch) {
   GemmArgs g = g0;
   const int fn = skinny_plan<1>(g);
   if (!launch) return fn == 4 ? skinny_dq_fits<4>(g) : fn == 3 ? skinny_dq_fits<3>(g) : fn == 2 ? skinny_dq_fits<2>(g) : skinny_dq_fits<1>(g);
-  if (fn == 4) return gemm8_skinny_launch_fn<1, 4, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
-  if (fn == 3) return gemm8_skinny_launch_fn<1, 3, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
-  if (fn == 2) return gemm8_skinny_launch_fn<1, 2, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
-  return gemm8_skinny_launch_fn<1, 1, GEMM_BLOCK_FP8, OT, false, 1>(g, st, 1);
+  if (fn == 4) return gemm8_skinny_launch_fn<1, 4, MODE, OT, false, 1>(g, st, 1);
+  if (fn == 3) return gemm8_skinny_launch_fn<1, 3, MODE, OT, false, 1>(g, st, 1);
+  if (fn == 2) return gemm8_skinny_launch_fn<1, 2, MODE, OT, false, 1>(g, st, 1);
+  return gemm8_skinny_launch_fn<1, 1, MODE, OT, false, 1>(g, st, 1);
 }
 
 // Wide form for 33..64 activation rows on weights with many rows: four row tiles times FN = 6, 8 or 9 column tiles

@@ -659,10 +659,9 @@ optional<Tensor> row_linear(const Tensor& x, const Tensor& weight, const Tensor&
   const int64_t wb = sglamd_gemm_workspace_bytes(m, n, k), wp = sc.take(wb > 0 ? wb : 0);
   sc.allocate(x);
   void* st = stream_of(x);
-  check(sglamd_per_token_quant_fp8(x.data_ptr(), tag(t), sc.at(q), (float*)sc.at(sa), m, k, st));
-  check(sglamd_fp8_scaled_mm(sc.at(q), k, weight.data_ptr(), ld(weight, 1), (float*)sc.at(sa), ws.data_ptr<float>(),
-                             bias ? bias->data_ptr() : nullptr, out.data_ptr(), n, tag(t), m, n, k,
-                             wb > 0 ? sc.at(wp) : nullptr, wb, st));
+  check(sglamd_fp8_row_linear(x.data_ptr(), tag(t), m, k, weight.data_ptr(), ld(weight, 1), ws.data_ptr<float>(),
+                              bias ? bias->data_ptr() : nullptr, out.data_ptr(), n, n, sc.at(q), (float*)sc.at(sa),
+                              wb > 0 ? sc.at(wp) : nullptr, wb, st));
   return out;
 }
 
