@@ -4,6 +4,8 @@
 // top-k sum reduce.
 #include "moe_dispatch.h"
 #include "quant_core.h"
+#include <algorithm>
+#include <cmath>
 
 namespace sglamd {
 
@@ -986,44 +988,89 @@ MoeTiles moe_one_block_tiles(int E, int64_t H, int64_t I) { return {E * ceil_div
 bool moe_layer_streams(int E, int64_t H, int64_t I) { return moe_stream_enabled() && 3 * E * H * I >= MOE_STREAM_MIN_BYTES; }
 // Rows per expert from which 64-slot blocks take over from the 16-slot ones of the streaming kernel on such layers.  That
 // kernel reads the same bytes, but every 16 rows or 32 columns have a tile of their own and a drain at its end; a last round
-// of tiles that leaves part of the chip idle costs it less.  Time in 16-slot blocks over time in 64-slot ones, weights from
-// HBM, block scales (row scales), at 1 / 2.5 / 6 / 10 rows:
-//   256 experts of 7168 x 2048 1.02 / 1.03 / 1.08 / 1.19 (1.01 / 1.03 / 1.06 / 1.12), 64 of 4096 x 1536 1.11 / 1.09 / 1.11 /
-//   1.18 (1.04 / 1.06 / 1.09 / 1.14), 256 of 2048 x 768 1.07 / 1.08 / 1.29 / 1.38 (1.07 / 1.09 / 1.24 / 1.30), 128 of
-//   2048 x 1024 0.95 / 0.99 / 1.05 / 1.16 (0.99 / 1.05 / 1.10 / 1.18): from 2.5 rows on, from 1.5 where the weights pass 1 GB;
-//   a second GEMM too short for the tile kernel's pipeline, 64 of 7168 x 512 1.02 / 1.04 / 1.09 / 1.19 (0.91 / 0.95 / 1.01 /
-//   1.05), 64 of 1024 x 512 1.02 / 1.20 / 1.09 / 1.13 (0.93 / 1.08 / 1.02 / 1.03): from 2.5 (6) on;
-//   idle CUs in the first GEMM only, 32 of 2048 x 768 0.87 / 1.05 / 1.13 / 1.13 (0.81 / 0.96 / 1.08 / 1.07), 16 of
-//   4096 x 896 0.82 / 0.94 / 1.05 / 1.01 (0.79 / 0.94 / 1.03 / 0.95): from 3 (4) on;
-//   in the second, 16 of 6144 x 2048 0.82 / 0.93 / 0.96 / 1.13 (0.85 / 0.95 / 0.95 / 1.00), 32 of 5120 x 1536 0.96 / 0.95 /
-//   0.92 / 0.96 (0.95 / 0.93 / 0.91 / 0.93): from 10 (12) on; in both, 16 of 3072 x 1024 0.73 / 0.88 / 0.90 / 0.98 (0.79 /
-//   0.90 / 0.92 / 0.90), 8 of 7168 x 2048 0.67 / 0.92 / 0.85 / 0.98 (0.70 / 0.97 / 0.88 / 0.85): from 13 on.
-double moe_stream_from(int E, int64_t H, int64_t I, bool row_scaled) {
+// of tiles that leaves part of the chip idle costs it less.  Where the lines lie: layer time in 16-slot blocks over 64-slot
+// ones, weights from HBM, 38 layers of 8 to 256 experts (hidden x intermediate), all four quantisations:
+//   both GEMMs fill whole rounds.  Block FP8 at 1 / 2.5 / 5 / 10 rows: 256 of 7168 x 2048 1.01 / 1.02 / 1.06 / 1.19, 128 of 5120
+//   x 768 1.04 / 1.06 / 1.16 / 1.36, 32 of 4096 x 1024 0.90 / 1.10 / 1.10 / 1.22; per-channel INT8 1.01 / 1.03 / 1.05 / 1.12,
+//   1.03 / 1.02 / 1.11 / 1.24, 0.92 / 1.09 / 1.06 / 1.08, block INT8 of the first and the last 1.00 / 1.01 / 1.03 / 1.15, 0.88 /
+//   1.07 / 1.05 / 1.11: from 2.5, from 2 where the weights pass 1 GB (128 of 7168 x 1536 at 1.5 / 2 / 3.5 1.02 / 0.98 / 1.04);
+//   a second GEMM too short for the tile kernel's pipeline (2.5 / 5 / 8 / 10 rows): block FP8 64 of 1024 x 512 1.13 / 1.01 /
+//   1.07 / 1.10, with two rounds and more in the first 256 of 4096 x 256 0.94 / 0.99 / 1.07 / 1.14; block INT8 64 of 4096 x 512
+//   0.93 / 0.93 / 0.97 / 1.05; row scales the same 0.93 / 0.91 / 0.92 / 0.99: from 2.5, 5.5, 8 and 11;
+//   idle CUs in the first GEMM only (2.5 / 5 / 9 / 11): rounds and a part of one, 64 of 2048 x 768 0.96 / 0.96 / 1.01 / 1.10
+//   (row scales 0.94 / 0.94 / 0.95 / 1.02), 64 of 6144 x 1792 0.95 / 1.01 / 1.06 / 1.13 (0.94 / 0.99 / 1.03 / 1.08): from 5 (9);
+//   part of one round, 32 of 2048 x 768 1.08 / 1.08 / 1.14 / 1.10 (1.01 / 1.01 / 1.04 / 1.02): from 3 (4), but with at most 60 % of
+//   it 16 of 4096 x 896 1.05 / 1.05 / 0.98 / 1.00 (1.02 / 1.01 / 0.91 / 0.93): from 3 (11), and with a short second GEMM as well
+//   32 of 6144 x 384 0.85 / 0.82 / 0.85 / 0.90 (0.77 / 0.75 / 0.79 / 0.81): from 13;
+//   in the second, 16 of 6144 x 2048 at 2.5 / 5 / 8 / 10 / 12 0.92 / 0.93 / 0.95 / 1.12 / 1.19 (0.93 / 0.93 / 0.94 / 0.99 /
+//   1.01): from 10 (12); in both, 32 of 5120 x 1536 0.91 / 0.90 / 0.92 / 0.94 / 1.05 (0.91 / 0.89 / 0.91 / 0.92 / 0.96): from
+//   12, less than a round of the first at 10 / 12 / 14 / 16, 16 of 2048 x 1024 0.95 / 0.95 / 0.97 / 1.03, 8 of 7168 x 2048 0.98 /
+//   0.94 / 1.13 / 1.12: from 13, at most 40 % of it 8 of 4096 x 1536 0.87 / 0.85 / 0.94 / 0.99: from 15.
+double moe_stream_from(int E, int64_t H, int64_t I, int mode) {
   const MoeTiles t = moe_one_block_tiles(E, H, I);
   const int64_t cus = device_cus();
+  const bool fp8 = mode == GEMM_BLOCK_FP8;
   auto full = [&](int64_t tiles) { return (double)tiles / (ceil_div(tiles, cus) * cus) >= 0.9; };
-  if (!full(t.second)) return t.first < cus ? 13. : row_scaled ? 12. : 10.;
-  if (!full(t.first)) return row_scaled ? 4. : 3.;
-  if (I < 768 || H < 768) return row_scaled ? 6. : 2.5;
-  return 3 * E * H * I >= 1000000000ll ? 1.5 : 2.5;
+  if (!full(t.second)) {
+    if (t.first < cus) return t.first <= 0.4 * cus ? 15. : 13.;
+    return fp8 && full(t.first) ? 10. : 12.;
+  }
+  if (!full(t.first)) {
+    if (t.first > cus) return fp8 ? 5. : 9.;
+    if (I < 512) return 13.;
+    return fp8 ? 3. : t.first <= 0.6 * cus ? 11. : 4.;
+  }
+  if (I < 768 || H < 768) return fp8 ? (t.first >= 2 * cus ? 5.5 : 2.5) : gemm_is_block(mode) ? 8. : 11.;
+  return 3 * E * H * I >= 1000000000ll ? 2. : 2.5;
 }
-// Whether a layer's largest expert is likely to fit one block of 64 slots: the mean, plus most of the spread that the
-// largest of E numbers of rows has.  One expert that does not adds a tile to every column: 64 experts of 4096 x 1536 at 48
-// rows, three rounds of tiles that become four, 227 -> 266 us.
-bool moe_fits_64(double rows, int E) { return rows + 0.85 * std::sqrt(2 * std::log((double)E) * rows) <= 64; }
-// Blocks that an expert has in the mean when the numbers of rows are spread like independent draws.
-double moe_spread_blocks(double rows, int block) {
-  double blocks = 1;
-  for (int full = block; full < rows + 5 * std::sqrt(rows) && blocks < 1000; full += block)
-    blocks += 0.5 * std::erfc((full - rows) / std::sqrt(2 * rows));
-  return blocks;
+// Rounds of tiles, one per CU, that a grouped GEMM of `cols` column tiles is expected to take in blocks of `block` slots, when
+// `experts` experts hold rows of this mean and variance, drawn independently: an expert's blocks are one and one for each
+// multiple of the block that its rows pass, their sum is taken as normally distributed.
+double moe_rounds(int experts, double rows, double var, int block, int64_t cols) {
+  // P(a count of this mean and deviation > x)
+  auto beyond = [](double x, double mean, double dev) { return 0.5 * std::erfc((x + 0.5 - mean) / (dev * M_SQRT2)); };
+  const double dev = std::sqrt(var);
+  int64_t sure = std::max<int64_t>(0, (int64_t)std::floor((rows - 5 * dev) / block));
+  double blocks = experts * (1. + sure), spread = 0;
+  for (int64_t j = sure + 1; j * block < rows + 5 * dev; j++) {
+    const double p = beyond((double)(j * block), rows, dev);
+    blocks += experts * p;
+    spread += experts * p * (1 - p);
+  }
+  spread = std::sqrt(spread) + 1e-3;
+  const int64_t cus = device_cus();
+  sure = std::max<int64_t>(0, (int64_t)std::floor((blocks - 5 * spread) * cols / cus));
+  double rounds = 1. + sure;
+  for (int64_t k = sure + 1; (double)(k * cus) / cols < blocks + 5 * spread + 1; k++)
+    rounds += beyond((double)(k * cus / cols), blocks, spread);
+  return rounds;
 }
-// Or whether the first GEMM's tiles in 64-slot blocks (every expert's last one half full) take this share of one round: then
-// a tile's time is the launch's, and the shortest wins.  8 experts of 4096 x 1536 at 64..128 rows 1.06-1.16x over 128 slots,
-// 16 of 4096 x 896 at 80..112 1.06-1.14x, 16 of 3072 x 1024 at 64..96 1.01-1.06x; with row scales, where 128 slots stream too, up to
-// 1.1x for the first of them and 0.9-1.0x in between.
-bool moe_one_round_64(double rows, int E, int64_t I, double share) {
-  return E * (rows / 64 + 0.5) * (double)ceil_div(2 * I, 256) <= share * device_cus();
+// The height of such a layer's blocks, 64 slots or more: the one whose rounds of tiles take the least time.  What a round
+// takes hardly depends on how many of its slots hold a row (the weights are its time, or the products of whole tiles), so
+// it is K times a constant of the height, relative to 192 slots: block scales 0.66 (64 slots, the streaming tile kernel), 0.82
+// (128, the persistent walk), row scales 0.67 and 0.74 (both the streaming tile kernel).  What that decides: one round of
+// short tiles against one of tall ones, a second block for an expert that overflows while the round has room for it, tall
+// ones when it has not.  Whole layers, weights from HBM, 38 layers of 8 to 256 experts, 28 to 4096 rows per expert; the rule's
+// height over the best of the three, mean (points above 1.03), in brackets the bands by rows that it replaces:
+//   block FP8 1.004 (62 of 1180) [1.018 (201)], block INT8 1.004 (45 of 873) [1.022 (179)], per-channel FP8 and INT8 1.007 (213
+//   of 2360) [1.025 (515)].
+// 8 experts of 4096 x 1536, 150 rows: 64 / 128 / 192 slots 112 / 79 / 93 us (t = 96, 128 tiles of one block: two blocks of 128
+// are still one round); 16 of 6144 x 2048, 150 rows 269 / 217 / 184 (256, 384), 190 rows 333 / 228 / 262; 64 of 4096 x 1536
+// (768, 1024), 150 rows 516 / 422 / 335, 208 rows 685 / 460 / 511.
+int moe_height_by_rounds(int E, int topk, int64_t H, int64_t I, double rows, bool row_scaled) {
+  // every token names topk different experts of E
+  const double var = std::max(1e-3, rows * (1 - (double)topk / E));
+  if (rows + 5 * std::sqrt(var) <= 64) return 64;
+  const int heights[3] = {64, 128, 192};
+  const double round[3] = {row_scaled ? 0.67 : 0.66, row_scaled ? 0.74 : 0.82, 1.};
+  int best = 0;
+  double least = 0;
+  for (int i = 0; i < 3; i++) {
+    const double t = round[i] * (H * moe_rounds(E, rows, var, heights[i], ceil_div(2 * I, 256)) +
+                                 I * moe_rounds(E, rows, var, heights[i], ceil_div(H, 256)));
+    if (i == 0 || t < least) best = heights[i], least = t;
+  }
+  return best;
 }
 
 int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I, bool int8 = false) {
@@ -1037,18 +1084,10 @@ int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I, bool int8 =
   //   64            1079   1618   1677   1714   1755   1802   1849   1994   2129   2415   3075   3279   3779
   //   128           1243   1846   1907   1946   1987   2018   2069   2150   2189   2224   2364   2542   3017
   //   192           1271   1890   1944   1978   2016   2044   2082   2177   2217   2270   2416   2494   2564
-  // Twelve layers of 8 to 256 experts: 64 slots are 1.05-1.2x ahead of 128 while they hold an expert; where there are at
-  // least four rounds of tiles an overflowing expert costs little and they stay ahead to 56 rows.  192 slots once experts
-  // start to overflow 128, and 128 again where half of them would overflow 192 (at 200 rows 1.02-1.2x on eight layers).
   // (INT8 layers have no activation in the first GEMM's epilogue and no place for padded rows of scales)
   if (moe_layer_streams(E, H, I) && !(int8 && (H % 512 || I % 512))) {
-    const double from = moe_stream_from(E, H, I, false);
-    if (rows < (int8 && from < 4 ? 4 : from) || M <= 4) return 16;
-    if (moe_fits_64(rows, E) || (rows <= 56 && moe_one_block_tiles(E, H, I).first >= 4 * device_cus()) ||
-        moe_one_round_64(rows, E, I, 1.0))
-      return 64;
-    if (rows <= 104 || (rows >= 180 && rows <= 215 && E < 256)) return 128;
-    return 192;
+    if (M <= 4 || rows < moe_stream_from(E, H, I, int8 ? GEMM_BLOCK_INT8 : GEMM_BLOCK_FP8)) return 16;
+    return moe_height_by_rounds(E, topk, H, I, rows, false);
   }
   // The other layers.  Those whose tiles do not fill the chip take one round whatever the height, so the shorter block wins where it holds
   // an expert, and two full blocks of 128 beat 192 where half of the experts overflow those.  Sixteen such layers of 4 to 64
@@ -1064,18 +1103,13 @@ int moe_auto_block(int64_t M, int E, int topk, int64_t H, int64_t I, bool int8 =
   return 192;
 }
 // The row-scaled modes have no persistent walk and no activation in the first GEMM's epilogue; the streaming tile kernel
-// takes 128 slots too.  Against one-tile launches of 128 slots it is 1.07-1.16x ahead on layers that fill the chip; against
-// 192 slots it wins where it pads fewer rows: 1.04-1.2x at 112 rows on eight layers, 1.15-1.27x at 200, 1.0-1.1x at 256,
-// 1.04-1.07x at 400, while at 128 (0.92-1.08x), 160 (0.87-1.0x) and 312 (0.99x) it does not.
+// takes 128 slots too (1.07-1.16x over one-tile launches of that height on layers that fill the chip).
 int moe_auto_block_rows(int64_t M, int E, int topk, int64_t H, int64_t I) {
   static const int forced = getenv("SGLAMD_MOE_BLOCK_M") ? atoi(getenv("SGLAMD_MOE_BLOCK_M")) : 0;
   if (forced == 16 || forced == 32 || forced == 64 || forced == 128 || forced == 192) return forced;
   const double rows = (double)M * topk / (E > 0 ? E : 1);
-  if (moe_layer_streams(E, H, I)) {
-    if (rows < moe_stream_from(E, H, I, true)) return 16;
-    if (moe_fits_64(rows, E) || moe_one_round_64(rows, E, I, 0.7)) return 64;
-    return moe_spread_blocks(rows, 128) * 128 < 0.98 * moe_spread_blocks(rows, 192) * 192 ? 128 : 192;
-  }
+  if (moe_layer_streams(E, H, I))
+    return rows < moe_stream_from(E, H, I, GEMM_ROW_INT8) ? 16 : moe_height_by_rounds(E, topk, H, I, rows, true);
   // What counts without it is how few rows a tile pads: the shortest block that still holds a whole expert (its weights are
   // streamed once).  A layer that fills the chip moves on sooner, since an expert that overflows adds a tile to a full
   // round.  Sixteen layers of 4 to 64 experts that do not fill it, these bands against the ones of a layer that does: 64 at
