@@ -9,7 +9,7 @@
 //     K block certifies both what has landed and what may be overwritten (gemm8_big_kernel has one per row tile);
 //   * the request stream does not stop at a tile's end: it moves on to the next tile D blocks before the products do,
 //     the next tile's slot ids, tables, routing weights and scales arriving by direct-to-LDS loads like everything else;
-//   * only the 32-row tiles that hold a real row are multiplied;
+//   * the 32-row tiles behind the last real row are not multiplied;
 //   * the weights of an expert with a single block are read once by one workgroup, so they are loaded with the streaming
 //     hint and leave the caches to the rows: 512 tokens of the DeepSeek-V3 layer 1934 -> 1763 us.  An expert's several
 //     blocks meet in L2, and with the hint they would not (8 experts, 4096 tokens, persistent walk 1615 -> 1882).
@@ -263,11 +263,17 @@ __global__ __launch_bounds__(512) void gemm8_moe_stream_kernel(GemmArgs g) {
   }
   int round = 0, list = 0, buf = 0, rot_now = rot;
   int a_cur = 0, w_cur = 0, s_cur = 0;
-  // 32-row tiles with a real row of the sorted block in list `l`: a block's real rows come first
+  // 32-row tiles up to the last one that holds a real row of the sorted block in list `l`: the sort puts them first, a caller's
+  // own lists need not
   auto live_tiles = [&](int l) -> int {
     const int* rows = (const int*)(smem + IDS_BASE) + l * BM;
-    const int head = lane < RT ? rows[lane * 32] : 0x7fffffff;
-    return max(1, __builtin_amdgcn_readfirstlane((int)__popcll(__ballot(head < g.num_valid))));
+    int live = 1;
+#pragma unroll
+    for (int u = 0; u < BM / 64; u++) {
+      const uint64_t real = __ballot(rows[u * 64 + lane] < g.num_valid);
+      if (real) live = u * 2 + (real >> 32 ? 2 : 1);
+    }
+    return __builtin_amdgcn_readfirstlane(live);
   };
   int live_now = live_tiles(0);
   // What a block needs first is fetched under the last products of the block before: its weights, the fragments and scales

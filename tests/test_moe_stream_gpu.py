@@ -86,3 +86,43 @@ def test_ids_that_live_elsewhere(dev):
                     w2_scale=torch.from_numpy(w2s).to(dev), block_shape=[128, 128], config={"BLOCK_SIZE_M": 64}, use_fp8_w8a8=True)
     assert_gemm_close(out, ref.float(), "moe stream, ids of -1")
     assert not out[7::50].any()
+
+
+@pytest.mark.parametrize("mode,block_m", [("block_fp8", 64), ("row_int8", 64), ("row_int8", 128), ("row_fp8", 128)])
+def test_slots_anywhere_in_a_block(dev, mode, block_m):
+    """The grouped GEMMs take every slot below num_valid_tokens, wherever a caller's list has it: blocks whose tiles begin with
+    padding, or hold nothing else in front of their rows, give the bits of the sorted list."""
+    from sglang_amd.moe_runner.moe_align_block_size import moe_align_block_size
+    from sglang_amd.ops import fused_moe_block_fp8_gemm_, fused_moe_gemm_any_
+
+    E, N, K = 70, 1024, 1024
+    g = torch.Generator().manual_seed(block_m)
+    ti = _ids(E, g).to(dev)
+    M = ti.numel()
+    print(f"moe stream, slots anywhere mode={mode} block_m={block_m} M={M}", flush=True)
+    int8 = mode.endswith("int8")
+    q13, s13, _, _ = _moe_weights(E, N // 2, K, g, "int8" if int8 else "fp8")
+    w = _dev_w(q13, dev, int8)
+    a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).to(dev) if int8 else (
+        torch.randn(M, K, generator=g).mul_(50).clamp_(-448, 448).to(dev).to(torch.float8_e4m3fn))
+    tw = torch.rand(M, 1, generator=g).add_(0.25).to(dev)
+    if mode == "block_fp8":
+        sa, sb = torch.rand(M, K // 128, generator=g).to(dev), torch.rand(E, N // 128, K // 128, generator=g).to(dev)
+    else:
+        sa, sb = torch.rand(M, 1, generator=g).to(dev), torch.from_numpy(s13).to(dev)
+
+    def gemm(slots, experts, post):
+        c = torch.full((M, N), float("nan"), device=dev, dtype=torch.bfloat16)
+        if mode == "block_fp8":
+            fused_moe_block_fp8_gemm_(a, sa, w, sb, c, tw, slots, experts, post, True, 1, block_m)
+        else:
+            fused_moe_gemm_any_(a, sa, w, sb, c, tw, slots, experts, post, True, 1, block_m, block_shape=None, bias=None)
+        return c
+
+    slots, experts, post = moe_align_block_size(ti, block_m, E)
+    want = gemm(slots, experts, post)
+    assert torch.isfinite(want.float()).all()
+    whole = slots[: slots.numel() // block_m * block_m].view(-1, block_m)
+    shuffled = torch.stack([block[torch.randperm(block_m, generator=g).to(dev)] for block in whole])
+    for other in (whole.flip(1), whole.roll(7, 1), whole.roll(-1, 1), shuffled):
+        assert torch.equal(gemm(torch.cat([other.reshape(-1), slots[whole.numel():]]), experts, post), want)
