@@ -289,6 +289,11 @@ int sglamd_fused_moe_block_fp8_gemm(const void* a, int64_t lda, const float* a_s
                                     int64_t num_valid_tokens, int top_k, int mul_routed_weight, int block_m,
                                     int64_t max_m_blocks, int64_t N, int64_t K, void* stream);
 
+/* Diagnostic with no counterpart in the reference: whether the grouped GEMMs above and below take their weights for ones that
+ * come from HBM (1) or may lie in the caches (0), by the experts that a sorted list of max_m_blocks blocks has room for beside
+ * its pairs.  Host code; they run other kernels in 64- and 128-slot blocks. */
+int sglamd_moe_list_streams(int64_t num_valid_tokens, int64_t max_m_blocks, int block_m, int64_t N, int64_t w_stride_n);
+
 /* The same sorted-block grouped GEMM with int8 operands: the use_int8_w8a8 / block_shape [128,128]
  * configuration of fused_moe_kernel (fused_moe_triton_kernels.py:323-638; activation quantisation
  * branch :764-777; native model torch_w8a8_block_int8_moe, test/registered/quant/test_block_int8.py:101-131).

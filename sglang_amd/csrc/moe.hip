@@ -690,6 +690,10 @@ extern "C" int sglamd_fused_moe_block_int8_gemm(const void* a, int64_t lda, cons
                         max_m_blocks, N, K, stream);
 }
 
+extern "C" int sglamd_moe_list_streams(int64_t num_valid_tokens, int64_t max_m_blocks, int block_m, int64_t N, int64_t w_stride_n) {
+  return block_m > 1 && moe_list_streams(num_valid_tokens, max_m_blocks, block_m, N, w_stride_n);
+}
+
 extern "C" int sglamd_topk_softmax(float* topk_weights, int32_t* topk_indices, const void* gating_output, int g_dtype,
                                   int64_t num_tokens, int64_t num_experts, int64_t topk, int renormalize,
                                   float moe_softcapping, const float* correction_bias, void* stream) {

@@ -1,6 +1,7 @@
 // Which kernel a fused-MoE grouped GEMM over sorted blocks runs, by block height: shared by the block-scaled modes
 // (moe.hip) and the row-scaled ones (moe_rows.hip).
 #pragma once
+#include <algorithm>
 #include "gemm_big.h"
 #include "gemm_big_moe_persist.h"
 #include "gemm_moe_stream.h"
@@ -37,10 +38,17 @@ static inline bool moe_stream_enabled() {
 // 3072 x 1024 0.80, 16 of 1536 x 640 0.92; 64 of 1024 x 512, 101 MB, 1.13, 32 of 2048 x 768, 151 MB, 1.06).  With weights that have left the cache this one
 // is ahead on all of them (1.0-1.12x).
 constexpr int64_t MOE_STREAM_MIN_BYTES = 96000000;
+// The same for a grouped GEMM called on its own, which knows its list of sorted blocks but not how many experts there are.  A
+// list has room for the pairs and for block_m - 1 slots of padding per expert, so what is left beside the pairs says how
+// many experts it was made for; the blocks themselves do not (8192 pairs of 8 experts are 136 blocks of 64).
+static inline bool moe_list_streams(int64_t num_valid, int64_t max_blocks, int block_m, int64_t N, int64_t ldb) {
+  const int64_t experts = std::min(num_valid, (max_blocks * block_m - num_valid) / (block_m - 1));
+  return experts * N * ldb >= MOE_STREAM_MIN_BYTES * 2 / 3;
+}
 template <int BM>
 static inline bool moe_stream_takes(const GemmArgs& g, bool block) {
   if (g.streams < 0 || !moe_stream_enabled() || !gemm8_moe_stream_ok<BM>(g, block)) return false;
-  return g.streams > 0 || (int64_t)g.max_blocks_m * g.N * g.ldb >= MOE_STREAM_MIN_BYTES * 2 / 3;
+  return g.streams > 0 || moe_list_streams(g.num_valid, g.max_blocks_m, BM, g.N, g.ldb);
 }
 
 template <int MODE, typename OT>

@@ -56,3 +56,15 @@ def test_heights_of_extreme_layers():
         for m, h, i, e, topk in ((64, 7168, 2048, 8, 8), (192, 7168, 2048, 8, 8), (200, 8192, 8192, 1, 1),
                                  (1 << 20, 7168, 2048, 8, 8), (1, 7168, 2048, 256, 8), (4096, 4096, 1536, 2047, 8)):
             assert _picked(mode, m, h, i, e, topk) in (16, 64, 128, 192)
+
+
+@pytest.mark.parametrize("block_m", [64, 128])
+@pytest.mark.parametrize("experts", [1, 4, 8, 64, 256])
+def test_separate_grouped_gemms_count_experts_not_blocks(experts, block_m):
+    """A list made for `experts` experts (and the ids of -1), or for fewer pairs than that, of any number of pairs."""
+    n, k = 1024, 1024
+    for pairs in (1, 5, 60, 64, 1000, 8192, 100000):
+        for buckets in (experts, experts + 1):
+            blocks = -(-(pairs + min(pairs, buckets) * (block_m - 1)) // block_m)
+            got = _lib.lib.sglamd_moe_list_streams(pairs, blocks, block_m, n, k)
+            assert got == (min(pairs, buckets) * n * k >= 64000000)
