@@ -983,49 +983,37 @@ int moe_one_round_block(double rows, int E, int64_t I, bool row_scaled) {
   return tiles <= 200 ? 64 : 0;
 }
 
-// Tiles of a layer's two GEMMs when every expert owns one block, 256 columns each.
-struct MoeTiles {
-  int64_t first, second;
-};
-MoeTiles moe_one_block_tiles(int E, int64_t H, int64_t I) { return {E * ceil_div(2 * I, 256), E * ceil_div(H, 256)}; }
 // Whether a layer is one for the weight-streaming tile kernel (gemm_moe_stream.h; moe_stream_takes says why).
 bool moe_layer_streams(int E, int64_t H, int64_t I) { return moe_stream_enabled() && 3 * E * H * I >= MOE_STREAM_MIN_BYTES; }
 // Rows per expert from which 64-slot blocks take over from the 16-slot ones of the streaming kernel on such layers.  That
-// kernel reads the same bytes, but every 16 rows or 32 columns have a tile of their own and a drain at its end; a last round
-// of tiles that leaves part of the chip idle costs it less.  Where the lines lie: layer time in 16-slot blocks over 64-slot
-// ones, weights from HBM, 38 layers of 8 to 256 experts (hidden x intermediate), all four quantisations:
-//   both GEMMs fill whole rounds.  Block FP8 at 1 / 2.5 / 5 / 10 rows: 256 of 7168 x 2048 1.01 / 1.02 / 1.06 / 1.19, 128 of 5120
-//   x 768 1.04 / 1.06 / 1.16 / 1.36, 32 of 4096 x 1024 0.90 / 1.10 / 1.10 / 1.22; per-channel INT8 1.01 / 1.03 / 1.05 / 1.12,
-//   1.03 / 1.02 / 1.11 / 1.24, 0.92 / 1.09 / 1.06 / 1.08, block INT8 of the first and the last 1.00 / 1.01 / 1.03 / 1.15, 0.88 /
-//   1.07 / 1.05 / 1.11: from 2.5, from 2 where the weights pass 1 GB (128 of 7168 x 1536 at 1.5 / 2 / 3.5 1.02 / 0.98 / 1.04);
-//   a second GEMM too short for the tile kernel's pipeline (2.5 / 5 / 8 / 10 rows): block FP8 64 of 1024 x 512 1.13 / 1.01 /
-//   1.07 / 1.10, with two rounds and more in the first 256 of 4096 x 256 0.94 / 0.99 / 1.07 / 1.14; block INT8 64 of 4096 x 512
-//   0.93 / 0.93 / 0.97 / 1.05; row scales the same 0.93 / 0.91 / 0.92 / 0.99: from 2.5, 5.5, 8 and 11;
-//   idle CUs in the first GEMM only (2.5 / 5 / 9 / 11): rounds and a part of one, 64 of 2048 x 768 0.96 / 0.96 / 1.01 / 1.10
-//   (row scales 0.94 / 0.94 / 0.95 / 1.02), 64 of 6144 x 1792 0.95 / 1.01 / 1.06 / 1.13 (0.94 / 0.99 / 1.03 / 1.08): from 5 (9);
-//   part of one round, 32 of 2048 x 768 1.08 / 1.08 / 1.14 / 1.10 (1.01 / 1.01 / 1.04 / 1.02): from 3 (4), but with at most 60 % of
-//   it 16 of 4096 x 896 1.05 / 1.05 / 0.98 / 1.00 (1.02 / 1.01 / 0.91 / 0.93): from 3 (11), and with a short second GEMM as well
-//   32 of 6144 x 384 0.85 / 0.82 / 0.85 / 0.90 (0.77 / 0.75 / 0.79 / 0.81): from 13;
-//   in the second, 16 of 6144 x 2048 at 2.5 / 5 / 8 / 10 / 12 0.92 / 0.93 / 0.95 / 1.12 / 1.19 (0.93 / 0.93 / 0.94 / 0.99 /
-//   1.01): from 10 (12); in both, 32 of 5120 x 1536 0.91 / 0.90 / 0.92 / 0.94 / 1.05 (0.91 / 0.89 / 0.91 / 0.92 / 0.96): from
-//   12, less than a round of the first at 10 / 12 / 14 / 16, 16 of 2048 x 1024 0.95 / 0.95 / 0.97 / 1.03, 8 of 7168 x 2048 0.98 /
-//   0.94 / 1.13 / 1.12: from 13, at most 40 % of it 8 of 4096 x 1536 0.87 / 0.85 / 0.94 / 0.99: from 15.
+// kernel reads the same bytes, but every 16 rows or 32 columns have a tile of their own and a drain at its end; rounds of tiles
+// that leave part of the chip idle cost it less.  So the line follows how much of its rounds a layer fills with one block per
+// expert (both GEMMs, by time).  Best lines of 98 (block FP8) and 158 (row scales) layers of 8 to 256 experts, weights from HBM:
+//   filled below 0.46     11 to 18 / 13 to 20      (8 experts of 4096 x 1536, hidden x intermediate: 16 / 16)
+//          0.46 to 0.59   9 to 14 / 8 to 14        (16 of 2048 x 1024: 14 / 14; 16 of 4096 x 896: level from 2 to 13 / 12)
+//          0.59 to 0.75   9 to 13 / 11 to 14       (32 of 3072 x 1152: 13 / 13)
+//          0.75 to 0.80   10 / 9 to 12             (32 of 5120 x 1536: 10 / 12)
+//          0.80 to 0.84   2 to 7 / 2 to 11         (64 of 2048 x 768: 7 / 10)
+//          0.84 to 0.94   2 to 8 / 2 to 10         (64 of 6144 x 1792: 3.5 / 6; 16 of 6144 x 2048: 8 / 10)
+//          above          0.5 to 4, from 1 GB of weights on 0.5 to 3.5, either (256 of 7168 x 2048: 1 / 1; 128 of 2048 x 1024: 4 / 3)
+// A second GEMM too short for the tile kernel's pipeline: block FP8 0.59 to 0.84 filled 1.3 to 5, with more than a round in the
+// first 8 and more; above 0.94 0.5 to 3, with two rounds and more in the first 2.7 to 5.6; block INT8 6 to 8; row scales, whose
+// 128-slot blocks have a pipeline from 512 columns on, below that 8 to 10, from three rounds in the first on 5 to 6.
+// Time in 16-slot blocks over time in 64-slot ones, block FP8, at 1 / 2.5 / 5 / 10 rows: 256 of 7168 x 2048 1.01 / 1.02 / 1.06 /
+// 1.19, 32 of 4096 x 1024 0.90 / 1.10 / 1.10 / 1.22, 16 of 6144 x 2048 0.85 / 0.92 / 0.93 / 1.12, 32 of 5120 x 1536 0.88 / 0.91 /
+// 0.90 / 0.94, 8 of 4096 x 1536 0.71 / 0.77 / 0.92 / 0.87.
 double moe_stream_from(int E, int64_t H, int64_t I, int mode) {
-  const MoeTiles t = moe_one_block_tiles(E, H, I);
-  const int64_t cus = device_cus();
-  const bool fp8 = mode == GEMM_BLOCK_FP8;
-  auto full = [&](int64_t tiles) { return (double)tiles / (ceil_div(tiles, cus) * cus) >= 0.9; };
-  if (!full(t.second)) {
-    if (t.first < cus) return t.first <= 0.4 * cus ? 15. : 13.;
-    return fp8 && full(t.first) ? 10. : 12.;
-  }
-  if (!full(t.first)) {
-    if (t.first > cus) return fp8 ? 5. : 9.;
-    if (I < 512) return 13.;
-    return fp8 ? 3. : t.first <= 0.6 * cus ? 11. : 4.;
-  }
-  if (I < 768 || H < 768) return fp8 ? (t.first >= 2 * cus ? 5.5 : 2.5) : gemm_is_block(mode) ? 8. : 11.;
-  return 3 * E * H * I >= 1000000000ll ? 2. : 2.5;
+  const int64_t cus = device_cus(), first = E * ceil_div(2 * I, 256), second = E * ceil_div(H, 256);
+  const double filled = (double)(H * first + I * second) / (cus * (H * ceil_div(first, cus) + I * ceil_div(second, cus)));
+  const bool fp8 = mode == GEMM_BLOCK_FP8, block = gemm_is_block(mode);
+  const bool short_second = I < (block ? 768 : 512);
+  if (filled < 0.46) return 16;
+  if (filled < 0.59) return 13;
+  if (fp8 && short_second && filled < 0.84) return first > cus ? 8 : 4;
+  if (filled < 0.80) return filled < 0.75 ? 12 : 10;
+  if (filled < 0.94) return fp8 ? (filled < 0.84 ? 5 : 6) : short_second || filled < 0.84 ? 9 : 8;
+  if (short_second) return fp8 ? (first >= 2 * cus ? 4.5 : 2) : block ? 7 : first >= 3 * cus ? 6 : 9;
+  return 3 * E * H * I >= 1000000000ll ? 2 : 2.5;
 }
 // Rounds of tiles, one per CU, that a grouped GEMM of `cols` column tiles is expected to take in blocks of `block` slots, when
 // `experts` experts hold rows of this mean and variance, drawn independently: an expert's blocks are one and one for each
@@ -1050,29 +1038,35 @@ double moe_rounds(int experts, double rows, double var, int block, int64_t cols)
   return rounds;
 }
 // The height of such a layer's blocks, 64 slots or more: the one whose rounds of tiles take the least time.  What a round
-// takes hardly depends on how many of its slots hold a row (the weights are its time, or the products of whole tiles), so
-// it is K times a constant of the height, relative to 192 slots: block scales 0.66 (64 slots, the streaming tile kernel), 0.82
-// (128, the persistent walk), row scales 0.67 and 0.74 (both the streaming tile kernel).  What that decides: one round of
-// short tiles against one of tall ones, a second block for an expert that overflows while the round has room for it, tall
-// ones when it has not.  Whole layers, weights from HBM, 38 layers of 8 to 256 experts, 28 to 4096 rows per expert; the rule's
-// height over the best of the three, mean (points above 1.03), in brackets the bands by rows that it replaces:
-//   block FP8 1.004 (62 of 1180) [1.018 (201)], block INT8 1.004 (45 of 873) [1.022 (179)], per-channel FP8 and INT8 1.007 (213
-//   of 2360) [1.025 (515)].
-// 8 experts of 4096 x 1536, 150 rows: 64 / 128 / 192 slots 112 / 79 / 93 us (t = 96, 128 tiles of one block: two blocks of 128
-// are still one round); 16 of 6144 x 2048, 150 rows 269 / 217 / 184 (256, 384), 190 rows 333 / 228 / 262; 64 of 4096 x 1536
-// (768, 1024), 150 rows 516 / 422 / 335, 208 rows 685 / 460 / 511.
+// takes hardly depends on how many of its slots hold a row (the weights are its time, or the products of whole tiles): it is
+// linear in K, with a share of the height, relative to 192 slots.  Block scales 0.66 (64 slots, the streaming tile kernel) and 0.82
+// (128, the persistent walk); row scales 0.76 and 0.86 on the streaming tile kernel, while a tile of the one-tile kernel (192
+// slots, and K too short for the other's pipeline) costs 340 bytes of K more for its drain and ramp.  What that decides: one
+// round of short tiles against one of tall ones, a second block for an expert that overflows while the round has room for it,
+// tall blocks when it has not.
+// Whole layers, weights from HBM, 98 layers of every quantisation, 8 to 256 experts, 1 to 4096 rows per expert: time of the
+// picked height (16 slots among them) over the fastest one, mean, and in brackets with the bands by rows that stood here:
+//   block FP8 1.004 (1.012), block INT8 1.008 (1.015), per-channel FP8 1.004 (1.017), per-channel INT8 1.004 (1.019).
+// 8 experts of 4096 x 1536, 150 rows 113 / 79 / 94 (two blocks of 128 are still one round); 16 of 6144 x 2048, 150 rows 269 / 217
+// / 184, 190 rows 333 / 228 / 262; 64 of 4096 x 1536, 150 rows 516 / 422 / 335, 208 rows 688 / 460 / 512.
 int moe_height_by_rounds(int E, int topk, int64_t H, int64_t I, double rows, bool row_scaled) {
   // every token names topk different experts of E
   const double var = std::max(1e-3, rows * (1 - (double)topk / E));
-  if (rows + 5 * std::sqrt(var) <= 64) return 64;
-  const int heights[3] = {64, 128, 192};
-  const double round[3] = {row_scaled ? 0.67 : 0.66, row_scaled ? 0.74 : 0.82, 1.};
+  struct Round {
+    int slots, pipeline;         // K from which the height's kernel is not the one-tile kernel
+    double share, one_tile, ramp;  // time per K in either, and what the one-tile kernel adds
+  };
+  static const Round block_scaled[3] = {{64, 0, 0.66, 0, 0}, {128, 0, 0.82, 0, 0}, {192, 0, 1, 0, 0}};
+  static const Round row_scales[3] = {{64, 768, 0.76, 0.65, 340}, {128, 512, 0.86, 0.85, 340}, {192, 1 << 30, 0, 1, 340}};
   int best = 0;
   double least = 0;
-  for (int i = 0; i < 3; i++) {
-    const double t = round[i] * (H * moe_rounds(E, rows, var, heights[i], ceil_div(2 * I, 256)) +
-                                 I * moe_rounds(E, rows, var, heights[i], ceil_div(H, 256)));
-    if (i == 0 || t < least) best = heights[i], least = t;
+  for (const Round& r : row_scaled ? row_scales : block_scaled) {
+    auto time = [&](int64_t K, int64_t N) {
+      const double round = K >= r.pipeline ? r.share * K : r.one_tile * K + r.ramp;
+      return round * moe_rounds(E, rows, var, r.slots, ceil_div(N, 256));
+    };
+    const double t = time(H, 2 * I) + time(I, H);
+    if (!best || t < least) best = r.slots, least = t;
   }
   return best;
 }
