@@ -1013,7 +1013,7 @@ double moe_stream_from(int E, int64_t H, int64_t I, int mode) {
   if (filled < 0.80) return filled < 0.75 ? 12 : 10;
   if (filled < 0.94) return fp8 ? (filled < 0.84 ? 5 : 6) : short_second || filled < 0.84 ? 9 : 8;
   if (short_second) return fp8 ? (first >= 2 * cus ? 4.5 : 2) : block ? 7 : first >= 3 * cus ? 6 : 9;
-  return 3 * E * H * I >= 1000000000ll ? 2 : 2.5;
+  return 3 * E * H * I >= 1000000000ll ? 1.5 : 2.5;
 }
 // Rounds of tiles, one per CU, that a grouped GEMM of `cols` column tiles is expected to take in blocks of `block` slots, when
 // `experts` experts hold rows of this mean and variance, drawn independently: an expert's blocks are one and one for each
@@ -1040,30 +1040,31 @@ double moe_rounds(int experts, double rows, double var, int block, int64_t cols)
 // The height of such a layer's blocks, 64 slots or more: the one whose rounds of tiles take the least time.  What a round
 // takes hardly depends on how many of its slots hold a row (the weights are its time, or the products of whole tiles): it is
 // linear in K, with a share of the height, relative to 192 slots.  Block scales 0.66 (64 slots, the streaming tile kernel) and 0.82
-// (128, the persistent walk); row scales 0.76 and 0.86 on the streaming tile kernel, while a tile of the one-tile kernel (192
-// slots, and K too short for the other's pipeline) costs 340 bytes of K more for its drain and ramp.  What that decides: one
-// round of short tiles against one of tall ones, a second block for an expert that overflows while the round has room for it,
-// tall blocks when it has not.
+// (128, the persistent walk); row scales 0.83 and 0.90 on the streaming tile kernel, which starts and drains once a launch (460
+// bytes of K), while the one-tile kernel (192 slots, and K too short for the other's pipeline) does so at every tile (630).
+// What that decides: one round of short tiles against one of tall ones, a second block for an expert that overflows while
+// the round has room for it, tall blocks when it has not.
 // Whole layers, weights from HBM, 98 layers of every quantisation, 8 to 256 experts, 1 to 4096 rows per expert: time of the
 // picked height (16 slots among them) over the fastest one, mean, and in brackets with the bands by rows that stood here:
-//   block FP8 1.004 (1.012), block INT8 1.008 (1.015), per-channel FP8 1.004 (1.017), per-channel INT8 1.004 (1.019).
+//   block FP8 1.004 (1.012), block INT8 1.008 (1.015), per-channel FP8 1.004 (1.017), per-channel INT8 1.003 (1.019).
 // 8 experts of 4096 x 1536, 150 rows 113 / 79 / 94 (two blocks of 128 are still one round); 16 of 6144 x 2048, 150 rows 269 / 217
 // / 184, 190 rows 333 / 228 / 262; 64 of 4096 x 1536, 150 rows 516 / 422 / 335, 208 rows 688 / 460 / 512.
 int moe_height_by_rounds(int E, int topk, int64_t H, int64_t I, double rows, bool row_scaled) {
   // every token names topk different experts of E
   const double var = std::max(1e-3, rows * (1 - (double)topk / E));
   struct Round {
-    int slots, pipeline;         // K from which the height's kernel is not the one-tile kernel
-    double share, one_tile, ramp;  // time per K in either, and what the one-tile kernel adds
+    int slots, pipeline;        // K from which the height's kernel is not the one-tile kernel
+    double share, launch;       // what a round of it takes per K, and a launch
+    double one_tile, ramp;      // what a round of the one-tile kernel takes per K, and on top
   };
-  static const Round block_scaled[3] = {{64, 0, 0.66, 0, 0}, {128, 0, 0.82, 0, 0}, {192, 0, 1, 0, 0}};
-  static const Round row_scales[3] = {{64, 768, 0.76, 0.65, 340}, {128, 512, 0.86, 0.85, 340}, {192, 1 << 30, 0, 1, 340}};
+  static const Round block_scaled[3] = {{64, 0, 0.66, 0, 0, 0}, {128, 0, 0.82, 0, 0, 0}, {192, 0, 1, 0, 0, 0}};
+  static const Round row_scales[3] = {{64, 768, 0.83, 460, 0.47, 630}, {128, 512, 0.90, 460, 0.85, 630}, {192, 1 << 30, 0, 0, 1, 630}};
   int best = 0;
   double least = 0;
   for (const Round& r : row_scaled ? row_scales : block_scaled) {
     auto time = [&](int64_t K, int64_t N) {
-      const double round = K >= r.pipeline ? r.share * K : r.one_tile * K + r.ramp;
-      return round * moe_rounds(E, rows, var, r.slots, ceil_div(N, 256));
+      const double rounds = moe_rounds(E, rows, var, r.slots, ceil_div(N, 256));
+      return K >= r.pipeline ? r.share * K * rounds + r.launch : (r.one_tile * K + r.ramp) * rounds;
     };
     const double t = time(H, 2 * I) + time(I, H);
     if (!best || t < least) best = r.slots, least = t;
