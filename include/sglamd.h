@@ -418,9 +418,9 @@ int sglamd_fused_rms_fp8_group_quant(const void* x1, int64_t x1_row_stride, cons
  *   quantise hidden (1x128 groups) + moe_align_block_size -> grouped GEMM with w13 -> silu*mul + quantise
  *   -> grouped GEMM with w2 (x routing weight) -> sum over top-k (x routed_scaling_factor).
  * Up to four tokens the activation step runs inside the two GEMMs (four launches), and a single token's sorting,
- * quantising and sum too (two launches); where the sorted blocks are 128 or 192 slots tall and outnumber the compute
- * units, the first GEMM's epilogue applies silu*mul and the quantisation and writes the second GEMM's operand
- * (four launches, the same bits as the five).  The decode forms compute what the five-launch sequence computes; the bits are the
+ * quantising and sum too (two launches); where the sorted blocks are 64 slots tall on layers of 96 MB of weights and more, or
+ * 128 or 192 slots tall and outnumber the compute units, the first GEMM's epilogue applies silu*mul and the quantisation and
+ * writes the second GEMM's operand (four launches, the same bits as the five).  The decode forms compute what the five-launch sequence computes; the bits are the
  * same when both split and walk K alike, which holds when 2I and H are at least 2048 and multiples of 32 (two
  * column tiles per workgroup in either form) and the plain launch shares K among at most four waves, as at the
  * DeepSeek-V3 dimensions; otherwise the fp32 partial sums meet in another order and the results agree to fp32

@@ -11,13 +11,15 @@
 //     the next tile's slot ids, tables, routing weights and scales arriving by direct-to-LDS loads like everything else;
 //   * the 32-row tiles behind the last real row are not multiplied;
 //   * the weights of an expert with a single block are read once by one workgroup, so they are loaded with the streaming
-//     hint and leave the caches to the rows: 512 tokens of the DeepSeek-V3 layer 1934 -> 1763 us.  An expert's several
+//     hint and leave the caches to the rows: 512 tokens of the DeepSeek-V3 layer, GEMM 1225 -> 1096 and 683 -> 637 us, with
+//     the same 7.5 and 3.8 GB fetched.  An expert's several
 //     blocks meet in L2, and with the hint they would not (8 experts, 4096 tokens, persistent walk 1615 -> 1882).
 //   * activation scales come in aligned groups of four K blocks (see gemm8_moe_persist_kernel).
 // A wave multiplies every row tile with one column tile, so LDS is read for one MFMA pair where gemm8_big_kernel's waves
-// read it for two: from some 56 rows on (block scales), or 118 (row scales), that kernel and its persistent walk win.
+// read it for two: once the weights are no longer the time, that kernel and its persistent walk win (moe_height_by_rounds).
 // Whole layers, us, before -> this kernel: 256 experts of 7168 x 2048, top-8, 128 / 256 / 512 / 1024 / 1536 tokens 1807 ->
-// 1644, 2018 -> 1702, 1980 -> 1758, 2160 -> 1849, 2270 -> 1994 (5.9 to 6.6 TB/s of weights); 64 INT8 experts of 4096 x 1536,
+// 1644, 2018 -> 1702, 1980 -> 1758, 2160 -> 1849, 2270 -> 1994 (512 tokens by trace: 6.9 and 5.9 TB/s of weights in the two
+// GEMMs, matrix pipe 9 and 8 % busy); 64 INT8 experts of 4096 x 1536,
 // row scales, top-6, 100 / 250 / 500 / 1000 tokens 249 -> 218, 266 -> 232, 295 -> 251, 334 -> 288.
 #pragma once
 #include "gemm_big.h"

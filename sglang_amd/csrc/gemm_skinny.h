@@ -28,7 +28,7 @@
 //   sorted.  Both request the rows straight to LDS in front of the first weight blocks: quantising them waits for nothing
 //   else, where a load behind those drains the ring.  With the last arrivals' sum (sum_out) one token is two launches:
 //   GEMMs that sort for themselves, a sum behind them -> this, us, experts' weights from HBM, top-8 unless noted: 7168 x 2048
-//   73 -> 69, top-1 25.9 -> 22.1, 4096 x 1536 top-6 40.7 -> 32.1, 2048 x 768 26.1 -> 22.2 (of these the sum's launch 1.5, 0.6,
+//   71.3 -> 66.9 (the router's launch included), top-1 25.9 -> 22.1, 4096 x 1536 top-6 40.7 -> 32.1, 2048 x 768 26.1 -> 22.2 (of these the sum's launch 1.5, 0.6,
 //   1.5 and 0.7).  Four K blocks in flight instead of three change none of them.
 #pragma once
 #include <stdlib.h>

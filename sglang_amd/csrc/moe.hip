@@ -927,7 +927,7 @@ extern "C" int sglamd_fp8_blockwise_scaled_grouped_mm(void* output, int out_dtyp
 // ---------------------------------------------------------------------------------------
 // Whole block-FP8 MoE layer from one host call: quantise + align (one kernel) -> grouped GEMM 1 ->
 // silu*mul + quantise (one kernel) -> grouped GEMM 2 (x routing weight) -> top-k sum.
-// Five launches on one stream (four for up to four tokens, three for one); all intermediates live in the
+// Five launches on one stream (four for up to four tokens, two for one); all intermediates live in the
 // caller's workspace.
 // ---------------------------------------------------------------------------------------
 static_assert(GEMM_BLOCK_FP8 == (int)SGLAMD_MOE_BLOCK_FP8 && GEMM_ROW_FP8 == (int)SGLAMD_MOE_ROW_FP8 &&

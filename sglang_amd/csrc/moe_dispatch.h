@@ -21,13 +21,7 @@ static inline bool moe_persist128_enabled() {
   return v != 0 && moe_persist_enabled();
 }
 
-// The persistent walk hands out tiles by position, not by arrival.  A sorted block that is an expert's second one
-// finds the weights its first block has just streamed in L2 and finishes in half the time, and a fixed walk cannot
-// balance that the way the dispatch order of a one-tile-per-workgroup launch does; until the tiles went to XCDs in
-// contiguous ranges the walk therefore lost 5 % where half of the experts own one block and half two (6144 tokens
-// on the DeepSeek-V3 layer) and was only used where every expert owns the same number.  With an expert's blocks
-// meeting in one L2 it is level or ahead at every token count measured (3072 ... 12288: 0 ... -5.5 %), so it runs
-// wherever there are more tiles than CUs.
+// tuning knob: SGLAMD_MOE_STREAM=0 keeps the weight-streaming tile kernel out
 static inline bool moe_stream_enabled() {
   static const int v = getenv("SGLAMD_MOE_STREAM") ? atoi(getenv("SGLAMD_MOE_STREAM")) : 1;
   return v != 0;
@@ -51,6 +45,13 @@ static inline bool moe_stream_takes(const GemmArgs& g, bool block) {
   return g.streams > 0 || moe_list_streams(g.num_valid, g.max_blocks_m, BM, g.N, g.ldb);
 }
 
+// The persistent walk hands out tiles by position, not by arrival.  A sorted block that is an expert's second one
+// finds the weights its first block has just streamed in L2 and finishes in half the time, and a fixed walk cannot
+// balance that the way the dispatch order of a one-tile-per-workgroup launch does; until the tiles went to XCDs in
+// contiguous ranges the walk therefore lost 5 % where half of the experts own one block and half two (6144 tokens
+// on the DeepSeek-V3 layer) and was only used where every expert owns the same number.  With an expert's blocks
+// meeting in one L2 it is level or ahead at every token count measured (3072 ... 12288: 0 ... -5.5 %), so it runs
+// wherever there are more tiles than CUs.
 template <int MODE, typename OT>
 static int dispatch_moe_gemm(const GemmArgs& g, int block_m, hipStream_t st) {
   // number of sorted blocks that will actually run is data dependent; every valid slot could own one
