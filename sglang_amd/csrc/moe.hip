@@ -1018,7 +1018,7 @@ double moe_stream_from(int E, int64_t H, int64_t I, int mode) {
 // Rounds of tiles, one per CU, that a grouped GEMM of `cols` column tiles is expected to take in blocks of `block` slots, when
 // `experts` experts hold rows of this mean and variance, drawn independently: an expert's blocks are one and one for each
 // multiple of the block that its rows pass, their sum is taken as normally distributed.
-double moe_rounds(int experts, double rows, double var, int block, int64_t cols) {
+double moe_rounds(int experts, double rows, double var, int block, int64_t cols, int64_t cus) {
   // P(a count of this mean and deviation > x)
   auto beyond = [](double x, double mean, double dev) { return 0.5 * std::erfc((x + 0.5 - mean) / (dev * M_SQRT2)); };
   const double dev = std::sqrt(var);
@@ -1030,7 +1030,6 @@ double moe_rounds(int experts, double rows, double var, int block, int64_t cols)
     spread += experts * p * (1 - p);
   }
   spread = std::sqrt(spread) + 1e-3;
-  const int64_t cus = device_cus();
   sure = std::max<int64_t>(0, (int64_t)std::floor((blocks - 5 * spread) * cols / cus));
   double rounds = 1. + sure;
   for (int64_t k = sure + 1; (double)(k * cus) / cols < blocks + 5 * spread + 1; k++)
@@ -1052,6 +1051,7 @@ double moe_rounds(int experts, double rows, double var, int block, int64_t cols)
 int moe_height_by_rounds(int E, int topk, int64_t H, int64_t I, double rows, bool row_scaled) {
   // every token names topk different experts of E
   const double var = std::max(1e-3, rows * (1 - (double)topk / E));
+  const int64_t cus = device_cus();
   struct Round {
     int slots, pipeline;        // K from which the height's kernel is not the one-tile kernel
     double share, launch;       // what a round of it takes per K, and a launch
@@ -1063,7 +1063,7 @@ int moe_height_by_rounds(int E, int topk, int64_t H, int64_t I, double rows, boo
   double least = 0;
   for (const Round& r : row_scaled ? row_scales : block_scaled) {
     auto time = [&](int64_t K, int64_t N) {
-      const double rounds = moe_rounds(E, rows, var, r.slots, ceil_div(N, 256));
+      const double rounds = moe_rounds(E, rows, var, r.slots, ceil_div(N, 256), cus);
       return K >= r.pipeline ? r.share * K * rounds + r.launch : (r.one_tile * K + r.ramp) * rounds;
     };
     const double t = time(H, 2 * I) + time(I, H);
@@ -1124,13 +1124,14 @@ int moe_auto_block_rows(int64_t M, int E, int topk, int64_t H, int64_t I) {
 int grouped_block_m(int64_t rows, int E) { return moe_auto_block(rows, E, 1, 0, 0); }
 // The expert-major layer gives the bits of its separate operators, which know an expert's rows and nothing of the layer: it
 // leaves the 16-slot blocks, whose kernel sums K in another order than the tile kernels, where they do.
-int moe_grouped_layer_block(int64_t M, int E, int topk, int64_t H, int64_t I) {
-  const int separate = grouped_block_m(M * topk, E), block = moe_auto_block(M, E, topk, H, I);
+int moe_grouped_layer_block(int64_t M, int E, int topk, int block) {  // block: the layer's own choice
+  const int separate = grouped_block_m(M * topk, E);
   return separate <= 32 || block <= 32 ? separate : block;
 }
 }  // namespace
 
 extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, int64_t I, int E, int topk, int block_m) {
+  const DeviceScope scope;
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
   if (block_m == 0) block_m = moe_auto_block(M, E, topk, H, I);
   return moe_ws_layout(M, H, I, E, topk, block_m).total;
@@ -1138,13 +1139,14 @@ extern "C" int64_t sglamd_fused_moe_block_fp8_workspace(int64_t M, int64_t H, in
 
 extern "C" int64_t sglamd_fused_moe_layer_workspace(int mode, int64_t M, int64_t H, int64_t I, int E, int topk,
                                                     int block_m) {
+  const DeviceScope scope;
   if (M <= 0 || H <= 0 || I <= 0 || E <= 0 || topk <= 0) return 0;
   const int picked = block_m                ? block_m
                      : gemm_is_block(mode) ? moe_auto_block(M, E, topk, H, I, gemm_is_int8(mode))
                                            : moe_auto_block_rows(M, E, topk, H, I);
   int64_t total = moe_ws_layout(M, H, I, E, topk, picked).total;
   if (block_m == 0 && mode == GEMM_BLOCK_FP8) {  // (the expert-major layer is sized here too)
-    const int64_t grouped = moe_ws_layout(M, H, I, E, topk, moe_grouped_layer_block(M, E, topk, H, I)).total;
+    const int64_t grouped = moe_ws_layout(M, H, I, E, topk, moe_grouped_layer_block(M, E, topk, picked)).total;
     if (grouped > total) total = grouped;
   }
   return total;
@@ -1177,9 +1179,10 @@ static int moe_layer(int mode, const void* hidden, int dtype, int64_t M, int64_t
   SGLAMD_REQUIRE(!row || I <= ROW_QUANT_MAX_HIDDEN, SGLAMD_ENOTSUP, "fused_moe: intermediate size %lld is beyond %lld",
                  (long long)I, (long long)ROW_QUANT_MAX_HIDDEN);
   SGLAMD_REQUIRE(row || (!b13 && !b2), SGLAMD_ENOTSUP, "fused_moe: biases go with row-scaled weights");
-  if (block_m == 0)
-    block_m = row ? moe_auto_block_rows(M, E, topk, H, I)
-              : grouped ? moe_grouped_layer_block(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I, int8);
+  if (block_m == 0) {
+    block_m = row ? moe_auto_block_rows(M, E, topk, H, I) : moe_auto_block(M, E, topk, H, I, int8);
+    if (grouped) block_m = moe_grouped_layer_block(M, E, topk, block_m);
+  }
   SGLAMD_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128 || block_m == 192, SGLAMD_EINVAL,
                  "fused_moe: block_m must be 16, 32, 64, 128 or 192");
   const MoeWs w = moe_ws_layout(M, H, I, E, topk, block_m);
