@@ -6,6 +6,7 @@ namespace sglamd {
 
 thread_local int last_kernel = 0;
 thread_local int skinny_last_shape = 0;
+thread_local int strip_last_shape = 0;
 
 extern template int dispatch_out<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
 extern template int dispatch_out_biased<GEMM_BLOCK_FP8>(const GemmArgs&, int, hipStream_t, void*, int64_t);
@@ -243,6 +244,7 @@ extern "C" int sglamd_int8_scaled_mm(const void* a, int64_t lda, const void* b, 
 
 extern "C" int sglamd_last_gemm_kernel(void) { return last_kernel; }
 extern "C" int sglamd_last_streaming_shape(void) { return skinny_last_shape; }
+extern "C" int sglamd_last_strip_shape(void) { return strip_last_shape; }
 
 extern "C" int sglamd_streaming_piece_offset(int kb, int lchunk, int64_t K, int64_t* offset) {
   const SkinnyPiece pc = skinny_piece(kb, lchunk, (int)K);
@@ -254,9 +256,12 @@ extern "C" int sglamd_streaming_piece_offset(int kb, int lchunk, int64_t K, int6
 extern "C" int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M >= (1ll << 31) || N <= 0 || K <= 0) return 0;
   const DeviceScope scope;
-  if (M <= 64 && !small_m_uses_tile(M, N, K)) return 0;
+  const StripPlan strip = dense_choice(M, N, K).strip;
+  const int64_t strip_need = strip.rows && strip.slices > 1 ? (int64_t)strip.slices * M * N * 4 : 0;
+  if (M <= 64 && !small_m_uses_tile(M, N, K)) return strip_need;
   const BigConfig cfg = gemm8_big_config(M, N, K);
   int64_t need = cfg.slices > 1 ? (int64_t)cfg.slices * M * N * 4 : 0;
+  if (strip_need > need) need = strip_need;
   // a launch of 256-row tiles cut in two along N (column_split) splits K on its second part; whether the launch
   // uses 256-row tiles depends on the operand mode, so the larger of the two needs is reported
   const int64_t n1 = M > 64 ? column_split(M, N, K) : 0;

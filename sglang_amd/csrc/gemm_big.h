@@ -746,6 +746,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
+template <int MODE, typename OT>
+static int splitk_reduce(const GemmArgs& g, int slices, const void* workspace, hipStream_t st) {
+  const int64_t total4 = ((int64_t)g.M * g.N) >> 2;
+  const unsigned rblocks = (unsigned)(total4 / 256 + 1 < 4096 ? total4 / 256 + 1 : 4096);
+  hipLaunchKernelGGL((splitk_reduce_kernel<MODE, OT>), dim3(rblocks), dim3(256), 0, st, (const float*)workspace, slices, g);
+  return check_launch("splitk_reduce");
+}
+
 // Tile height (64, 128 or 256 rows) and number of K slices for the large-M kernel.  One workgroup occupies a
 // CU, so the cost of a launch is (rounds of one workgroup per CU) x (work per workgroup); the 128-row tile does
 // half the work per workgroup at a somewhat lower MFMA efficiency and is preferred when it removes a mostly
@@ -828,12 +836,7 @@ static int gemm8_big_launch(const GemmArgs& g, hipStream_t st, int slices, void*
   part.C = workspace;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)slices), dim3(128 * WGN), smem, st, part);
   int rc = check_launch("gemm8_big(split-K)");
-  if (rc) return rc;
-  const int64_t total4 = ((int64_t)g.M * g.N) >> 2;
-  const unsigned rblocks = (unsigned)(total4 / 256 + 1 < 4096 ? total4 / 256 + 1 : 4096);
-  hipLaunchKernelGGL((splitk_reduce_kernel<MODE, OT>), dim3(rblocks), dim3(256), 0, st, (const float*)workspace, slices,
-                     g);
-  return check_launch("splitk_reduce");
+  return rc ? rc : splitk_reduce<MODE, OT>(g, slices, workspace, st);
 }
 
 // Fused-MoE launch of the same kernel: sorted blocks of 64*MT slots (128 or 192), no split-K.

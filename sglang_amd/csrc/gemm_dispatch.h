@@ -6,6 +6,7 @@
 #include "gemm_big.h"
 #include "gemm_big_persist.h"
 #include "gemm_skinny.h"
+#include "gemm_strip.h"
 
 namespace sglamd {
 
@@ -55,6 +56,7 @@ static int persist_workgroups() {
 // Which kernel the last dense GEMM call of this thread launched (SGLAMD_KERNEL_* of the header): lets a test
 // assert that it exercises the kernel it was written for, whatever the launch heuristics choose.
 extern thread_local int last_kernel;  // defined in gemm.hip
+extern thread_local int strip_last_shape;
 #define RAN(code) (last_kernel = (code))
 
 // A launch of 256x256 tiles whose last round of one tile per CU is mostly empty is cut in two along N: the
@@ -75,6 +77,64 @@ static int64_t column_split(int64_t M, int64_t N, int64_t K) {
   return first * 256;
 }
 
+// 33 to 1024 rows: the tile kernels (or, up to 64 rows, what small_m_uses_tile says), the strip kernel, or the streaming kernel walking
+// several row tiles?  Small weights are not worth a tile launch: it leaves most of the chip idle, or splits K and needs a second
+// launch, where the streaming kernel's small tiles fill it (2048 x 2048 at 128 rows, quantiser included, 15.2 -> 8.7 us, 1024 x 7168
+// 17.6 -> 12.3, 512 x 512 at 320 rows 8.7 -> 6.5), until reading the weights once per row tile costs more (4096 x 4096 at 150 rows
+// 20 -> 23).  The strip kernel takes over from weights of about 25 MB (28672 x 4096 at 64 / 128 rows 35 / 40 -> 27 / 33 us, 7168 x 16384
+// 38 / 48 -> 33 / 41).  The line between them is drawn by each form's time from a fitted model.  Over 2335 points (186 weights from
+// HBM, three scaling modes) and 949 (three weights in turn, up to 85 MB, so from the Infinity Cache): 1.13x in the mean of
+// either, 0.98 of the fastest form's, the worst point 0.93x, eight below 0.97.
+struct DenseChoice {
+  int row_tile = 0;  // streaming kernel in row tiles of this many rows
+  StripPlan strip;   // strip.rows > 0: strip kernel
+};
+static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
+  DenseChoice best;
+  if (M <= 32 || M > 1024 || (K & 127)) return best;
+  // the models are a few microseconds of host time: a thread remembers its last shapes (see skinny_plan)
+  struct Known {
+    int64_t M, N, K, cus;
+    DenseChoice choice;
+  };
+  static thread_local Known known[32] = {};
+  const int64_t cus = device_cus();
+  Known& slot = known[((uint32_t)M * 31u + (uint32_t)(N >> 3) * 7u + (uint32_t)(K >> 7)) & 31u];
+  if (slot.M == M && slot.N == N && slot.K == K && slot.cus == cus) return slot.choice;
+
+  const double common = 5.0 + 0.7e-6 * M * K;  // launch and quantiser
+  bool fills[2];
+  const double small[2] = {skinny_row_tiles_us<2>(M, N, K, &fills[0]), skinny_row_tiles_us<4>(M, N, K, &fills[1])};
+  const bool streamed = M <= 64 && !small_m_uses_tile(M, N, K);  // today's form is the streaming kernel's 64-row tile
+  double least;
+  bool row_tiles = true;
+  if (streamed) {
+    least = common + small[1];
+  } else {
+    const int nkb = (int)(K >> 7);
+    const bool persistent = !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
+    const BigConfig cfg = gemm8_big_config(M, N, K, persistent);
+    const int64_t cols = ceil_div(N, 256) * cfg.slices, rounds = ceil_div(ceil_div(M, cfg.bm) * cols, cus);
+    // a K block of a tile, or of the weights that the column tiles in flight read (6.7 TB/s from the Infinity Cache, 5.2 else)
+    const double block = std::max(cfg.bm == 64 ? 0.52 : cfg.bm == 128 ? 1.04 : 1.85, (N * K > 85000000 ? 0.0063 : 0.0049) * std::min(cols, cus));
+    least = common + rounds * ((double)nkb / cfg.slices * block + 2.2);
+    row_tiles = M > 64 || cfg.slices > 1;  // up to 64 rows the model is not fine enough to tell them from one launch of 64-row tiles
+    if (cfg.slices > 1) least += 3.2 + 1.86e-6 * cfg.slices * M * N;
+  }
+  for (int f = 0; f < 2 && row_tiles; f++) {
+    if (!fills[f]) continue;
+    const double us = (common + small[f]) * (streamed && f == 1 ? 1.0 : 1.12);
+    if (us < least) least = us, best.row_tile = f ? 64 : 32;
+  }
+  if (M <= STRIP_MAX_ROWS) {
+    const StripPlan plan = strip_plan(M, N, K);
+    // (on large weights with a K of some length the tile kernel is slower than its model: not one of them lost)
+    if ((common + plan.us) * (N * K >= 30000000 && K >= 2560 ? 0.93 : 1.1) < least) best.row_tile = 0, best.strip = plan;
+  }
+  slot = Known{M, N, K, cus, best};
+  return best;
+}
+
 // The row modes' tile kernel also takes a K that is not a multiple of 128, from 512 up: 8192 x 4112 at 100 / 300 / 1000 rows
 // 43 / 45 / 60 -> 21 / 32 / 46 us (4096: 20 / 23 / 39), 28672 x 4112 at 2048 rows 407 -> 281.  Shorter sums are a launch of
 // 12 to 17 us either way and stay with the generic kernel.
@@ -86,6 +146,23 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
   const int wgs = gemm_is_block(MODE) ? persist_workgroups() : 0;
   const int nkb = g.K >> 7;
   const bool persistent = wgs > 0 && (wgs & 7) == 0 && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
+  strip_last_shape = 0;
+  if (big && may_split && g.M > 32) {
+    const DenseChoice choice = dense_choice(g.M, g.N, g.K);
+    const StripPlan& plan = choice.strip;
+    if (choice.row_tile && gemm8_skinny_ok(g, g.M)) {
+      if (choice.row_tile == 64) return gemm8_skinny_launch<4, MODE, OT, false>(g, st, ceil_div(g.M, 64));
+      return gemm8_skinny_launch<2, MODE, OT, false>(g, st, ceil_div(g.M, 32));
+    }
+    if (plan.rows && strip_ok<MODE>(g) &&
+        (plan.slices == 1 || (workspace && ((uintptr_t)workspace & 15) == 0 && (int64_t)plan.slices * g.M * g.N * 4 <= workspace_bytes))) {
+      // (the class of the shape: the kernels that this one stands in for)
+      const bool wide = gemm8_skinny_wide<MODE, OT>(g, st, false) > 0;
+      RAN(g.M > 64 ? SGLAMD_KERNEL_TILE128 : wide ? SGLAMD_KERNEL_STREAMING_WIDE : SGLAMD_KERNEL_TILE64);
+      strip_last_shape = ((g.M + 31) / 32 << 24) | (plan.slices << 16) | plan.rows;
+      return gemm8_strip_launch<MODE, OT>(g, plan, st, workspace);
+    }
+  }
   if (big && may_split && g.M > 64) {
     const BigConfig whole = gemm8_big_config(g.M, g.N, g.K, persistent);
     const int64_t n1 = whole.bm == 256 && whole.slices == 1 ? column_split(g.M, g.N, g.K) : 0;

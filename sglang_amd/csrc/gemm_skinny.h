@@ -31,6 +31,8 @@
 //   71.3 -> 66.9 (the router's launch included), top-1 25.9 -> 22.1, 4096 x 1536 top-6 40.7 -> 32.1, 2048 x 768 26.1 -> 22.2 (of these the sum's launch 1.5, 0.6,
 //   1.5 and 0.7).  Four K blocks in flight instead of three change none of them.
 #pragma once
+#include <algorithm>
+
 #include <stdlib.h>
 
 #include "gemm_core.h"
@@ -1004,6 +1006,35 @@ static int skinny_plan(GemmArgs& g) {
   plan = Plan{g.M, g.N, g.K, cus, fn, g.rows_per_wg};
   return fn;
 }
+// Time in us, without what all forms have in common (launch, quantiser), of a dense launch that walks M rows in row tiles of 16 * FM,
+// the weights read once for each of them (past the first from L2 or the Infinity Cache).  A round of workgroups takes
+// the longer of a wave's chain of K blocks and the CU's bytes, and all of the other.  Fitted to 6354 launches of 160 weights of up
+// to 85 MB at 33 to 1000 rows, FM = 2 and 4, three weights in turn and enough to come from HBM: 10 % rms.  *fills: more than a quarter of the CUs have a tile.
+template <int FM>
+static double skinny_row_tiles_us(int64_t M, int64_t N, int64_t K, bool* fills) {
+  GemmArgs g = {};
+  g.M = (int)M, g.N = (int)N, g.K = (int)K;
+  const int fn = skinny_plan<FM>(g);
+  const int rows = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * fn, nkb = (int)((K + 127) >> 7);
+  const int64_t tiles = ceil_div(N, rows) * ceil_div(M, 16 * FM), cus = device_cus();
+  int kw = 1, per_cu = 1;
+  auto residency = [&](auto fn_c) {
+    kw = skinny_pick_kw<FM, decltype(fn_c)::value>(tiles, nkb);
+    per_cu = skinny_resident_per_cu<FM, decltype(fn_c)::value>(kw);
+  };
+  if (fn == 1) residency(std::integral_constant<int, 1>{});
+  else if (fn == 2) residency(std::integral_constant<int, 2>{});
+  else if constexpr (FM <= 2) {
+    if (fn == 3) residency(std::integral_constant<int, 3>{});
+    else residency(std::integral_constant<int, 4>{});
+  }
+  *fills = tiles * 4 > cus;
+  const int64_t rounds = ceil_div(tiles, cus * per_cu), active = std::min<int64_t>(per_cu, ceil_div(tiles, cus));
+  const double chain = 1.26 + 0.07 * FM * fn * (double)ceil_div(nkb, kw);
+  const double bytes = active * (rows + 0.27 * 16 * FM) * (double)K / 46400.;
+  return (double)rounds * (chain + bytes);
+}
+
 template <int FM, int MODE, typename OT, bool MOE>
 static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expected_tiles_m) {
   GemmArgs g = g0;
@@ -1046,7 +1077,8 @@ static int gemm8_skinny_quantising(const GemmArgs& g0, hipStream_t st, bool laun
   return gemm8_skinny_launch_fn<1, 1, MODE, OT, false, 1>(g, st, 1);
 }
 
-// Wide form for 33..64 activation rows on weights with many rows: four row tiles times FN = 6, 8 or 9 column tiles
+// Wide form for 33..64 activation rows on weights with many rows and a K that is no multiple of 128 (the others run the strip
+// kernel, 51 -> 44 us on DeepSeek-V3 gate_up at 64 rows): four row tiles times FN = 6, 8 or 9 column tiles
 // (96..144 weight rows) per workgroup, four waves that share K block by block, one ring slot per wave (the four
 // slots and what is in flight to them fill most of LDS).  Per K block a workgroup then fetches 8 KB of activation
 // rows for 12..18 KB of weight rows, where the two-column-tile form fetches 8 KB for 4 KB; the tile count is made a
