@@ -783,7 +783,7 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool p
   // weighted by what a row costs in that tile (the smaller tiles re-read more of the weights per row and fill
   // the matrix pipe less well; a 256-row launch with more tiles than CUs runs the persistent kernel when the
   // caller says so, which hides its tile boundaries), plus for split K the fp32 slabs' trip through HBM
-  // (8 bytes per element and slice at ~4 TB/s against ~7.7 ns per tile row and K block).  Fitted to a sweep
+  // (8 bytes per element and slice at 4 to 5 TB/s against ~7.7 ns per tile row and K block).  Fitted to a sweep
   // of M = 65..2048 on the DeepSeek-V3 gate_up, down and q_b weights: within 5 % of the best height there.
   BigConfig best = {256, 1};
   double best_cost = 1e30;
@@ -794,19 +794,23 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool p
     const int64_t tiles = ((M + bm - 1) / bm) * ((N + 255) / 256);
     const int slices = gemm8_big_slices(tiles, N, K);
     const int64_t rounds = (tiles * slices + cus - 1) / cus;
-    const double weight = bm == 64 ? 1.6 : bm == 128 ? 1.2 : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
+    // (64-row tiles in several rounds read each weight byte once per row tile from further away: gate_up at M = 400, four rounds of
+    // them, 176 us, 158 in 128-row tiles, 138 in 256-row tiles)
+    const double weight = bm == 64 ? (rounds > 1 ? 2.0 : 1.6) : bm == 128 ? 1.2 : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
     // a single row of tiles only loads the rows that exist: M = 192 in 256-row tiles costs what 192 rows cost
     // (gate_up at M = 192: 89.6 us in 256-row tiles against 102.5 in 64-row tiles, which need two rounds)
     const double rows = M <= bm ? (double)((M + 63) / 64 * 64) : (double)bm;
     double cost = (double)rounds * rows / slices * weight;
     // one partly filled round without split K: the workgroups that do run share the fabric among fewer, so a
     // tile takes less than in a full round (fitted with the rest: cost ~ sqrt of the fill, at most a quarter off;
-    // Llama-3-70B qkv at M = 512: 160 tiles of 128 rows take 47.8 us, 80 tiles of 256 rows split 3 ways 62.5)
-    if (slices == 1 && rounds == 1 && tiles < cus) {
-      const double fill = std::sqrt((double)tiles / cus);
-      cost *= fill > 0.75 ? fill : 0.75;
+    // Llama-3-70B qkv at M = 512: 160 tiles of 128 rows take 47.8 us, 80 tiles of 256 rows split 3 ways 62.5).  With K split too, a
+    // tenth off at most (o_proj at M = 400: 224 workgroups of 128 rows, two slices, 74 us, one round of 196 64-row tiles 95; Llama down
+    // at M = 700: 192 of 256 rows, two slices, 177 us, 192 of 128 rows 202; qkv at M = 256: 240 of 128 rows, three, 46 us, 160 of 64 rows 53)
+    if (rounds == 1 && tiles * slices < cus && (slices == 1 || M > bm)) {
+      const double fill = std::sqrt((double)(tiles * slices) / cus), most = slices == 1 ? 0.75 : 0.9;
+      cost *= fill > most ? fill : most;
     }
-    if (slices > 1) cost += 4.0 + (double)slices * M * N * 8.0 / 4000.0 / (nkb * 7.7);
+    if (slices > 1) cost += 4.0 + (double)slices * M * N * 8.0 / (M > bm ? 5000.0 : 4000.0) / (nkb * 7.7);
     if (cost < best_cost) {
       best_cost = cost;
       best = {bm, slices};
