@@ -77,7 +77,7 @@ static int64_t column_split(int64_t M, int64_t N, int64_t K) {
   return first * 256;
 }
 
-// 33 to 1024 rows: the tile kernels (or, up to 64 rows, what small_m_uses_tile says), the strip kernel, or the streaming kernel walking
+// 17 to 1024 rows: the tile kernels (or, up to 64 rows, what small_m_uses_tile says), the strip kernel, or the streaming kernel walking
 // several row tiles?  Small weights are not worth a tile launch: it leaves most of the chip idle, or splits K and needs a second
 // launch, where the streaming kernel's small tiles fill it (2048 x 2048 at 128 rows, quantiser included, 15.2 -> 8.7 us, 1024 x 7168
 // 17.6 -> 12.3, 512 x 512 at 320 rows 8.7 -> 6.5), until reading the weights once per row tile costs more (4096 x 4096 at 150 rows
@@ -85,13 +85,19 @@ static int64_t column_split(int64_t M, int64_t N, int64_t K) {
 // 38 / 48 -> 33 / 41).  The line between them is drawn by each form's time from a fitted model.  Over 2335 points (186 weights from
 // HBM, three scaling modes) and 949 (three weights in turn, up to 85 MB, so from the Infinity Cache): 1.13x in the mean of
 // either, 0.98 of the fastest form's, the worst point 0.93x, eight below 0.97.
+// Row tiles of 16 rows instead of 32, at 17 to 64 rows: a shorter chain per wave, at twice the reads, so only while the weights are
+// a few MB (704 x 4736 at 24 rows 10.6 -> 9.9 us, 1152 x 7040 16.0 -> 14.2; 4096 x 4096 11.6 -> 12.4).
+// A ragged K: rows start anywhere in a 128-byte line, and every form pays for it, by the factors below (the mean over 720 points to
+// their models).  512 x 1424 at 96 rows 13.6 -> 7.3 us, 23800 x 5984 at 80 rows 62 -> 45; beyond 128 rows only weights up to 2 MB
+// (512 x 1424 at 200 rows 13.7 -> 7.4, 848 x 1904 15.4 -> 10.1; 680 x 4768 at 320 rows 19.7 against 18.9).
 struct DenseChoice {
   int row_tile = 0;  // streaming kernel in row tiles of this many rows
   StripPlan strip;   // strip.rows > 0: strip kernel
 };
 static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
   DenseChoice best;
-  if (M <= 32 || M > 1024 || (K & 127)) return best;
+  const bool ragged = (K & 127) != 0;
+  if (M <= 16 || M > 1024 || (ragged && M > 128 && N * K > 2000000)) return best;
   // the models are a few microseconds of host time: a thread remembers its last shapes (see skinny_plan)
   struct Known {
     int64_t M, N, K, cus;
@@ -103,33 +109,47 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
   if (slot.M == M && slot.N == N && slot.K == K && slot.cus == cus) return slot.choice;
 
   const double common = 5.0 + 0.7e-6 * M * K;  // launch and quantiser
-  bool fills[2];
-  const double small[2] = {skinny_row_tiles_us<2>(M, N, K, &fills[0]), skinny_row_tiles_us<4>(M, N, K, &fills[1])};
-  const bool streamed = M <= 64 && !small_m_uses_tile(M, N, K);  // today's form is the streaming kernel's 64-row tile
+  bool fills[3];
+  double small[3] = {M <= 64 ? skinny_row_tiles_us<1>(M, N, K, &fills[0]) * (ragged ? 1.25 : 1.0) : 1e30,
+                     skinny_row_tiles_us<2>(M, N, K, &fills[1]) * (ragged ? 1.25 : 1.0),
+                     M > 32 ? skinny_row_tiles_us<4>(M, N, K, &fills[2]) * (ragged ? 1.15 : 1.0) : 1e30};
+  if (M <= 64 && small[0] * 1.02 + 0.02 * common < small[1] && N * K <= 10000000) {
+    small[1] = small[0], fills[1] = fills[0];  // 16-row tiles in place of the 32-row ones
+  } else {
+    small[0] = 1e30;
+  }
+  const int small_rows = small[0] < 1e30 ? 16 : 32;
+  if (M <= 32) {  // the streaming kernel in either case: one tile of 32 rows or two of 16
+    if (small_rows == 16) best.row_tile = 16;
+    slot = Known{M, N, K, cus, best};
+    return best;
+  }
+  const bool streamed = M <= 64 && !small_m_uses_tile(M, N, K);  // without this choice: the streaming kernel's 64-row tile
   double least;
   bool row_tiles = true;
   if (streamed) {
-    least = common + small[1];
+    least = common + small[2];
   } else {
-    const int nkb = (int)(K >> 7);
-    const bool persistent = !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
+    const int nkb = (int)((K + 127) >> 7);
+    const bool persistent = !ragged && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
     const BigConfig cfg = gemm8_big_config(M, N, K, persistent);
     const int64_t cols = ceil_div(N, 256) * cfg.slices, rounds = ceil_div(ceil_div(M, cfg.bm) * cols, cus);
     // a K block of a tile, or of the weights that the column tiles in flight read (6.7 TB/s from the Infinity Cache, 5.2 else)
     const double block = std::max(cfg.bm == 64 ? 0.52 : cfg.bm == 128 ? 1.04 : 1.85, (N * K > 85000000 ? 0.0063 : 0.0049) * std::min(cols, cus));
-    least = common + rounds * ((double)nkb / cfg.slices * block + 2.2);
+    double us = rounds * ((double)nkb / cfg.slices * block + 2.2);
     row_tiles = M > 64 || cfg.slices > 1;  // up to 64 rows the model is not fine enough to tell them from one launch of 64-row tiles
-    if (cfg.slices > 1) least += 3.2 + 1.86e-6 * cfg.slices * M * N;
+    if (cfg.slices > 1) us += 3.2 + 1.86e-6 * cfg.slices * M * N;
+    least = common + us * (ragged ? 1.15 : 1.0);
   }
-  for (int f = 0; f < 2 && row_tiles; f++) {
+  for (int f = 1; f < 3 && row_tiles; f++) {
     if (!fills[f]) continue;
-    const double us = (common + small[f]) * (streamed && f == 1 ? 1.0 : 1.12);
-    if (us < least) least = us, best.row_tile = f ? 64 : 32;
+    const double us = (common + small[f]) * (streamed && f == 2 ? 1.0 : 1.12);
+    if (us < least) least = us, best.row_tile = f == 2 ? 64 : small_rows;
   }
   if (M <= STRIP_MAX_ROWS) {
     const StripPlan plan = strip_plan(M, N, K);
     // (on large weights with a K of some length the tile kernel is slower than its model: not one of them lost)
-    if ((common + plan.us) * (N * K >= 30000000 && K >= 2560 ? 0.93 : 1.1) < least) best.row_tile = 0, best.strip = plan;
+    if ((common + plan.us * (ragged ? 1.12 : 1.0)) * (N * K >= 30000000 && K >= 2560 ? 0.93 : 1.1) < least) best.row_tile = 0, best.strip = plan;
   }
   slot = Known{M, N, K, cus, best};
   return best;
@@ -147,11 +167,12 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
   const int nkb = g.K >> 7;
   const bool persistent = wgs > 0 && (wgs & 7) == 0 && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
   strip_last_shape = 0;
-  if (big && may_split && g.M > 32) {
+  if (big && may_split && g.M > 16) {
     const DenseChoice choice = dense_choice(g.M, g.N, g.K);
     const StripPlan& plan = choice.strip;
     if (choice.row_tile && gemm8_skinny_ok(g, g.M)) {
       if (choice.row_tile == 64) return gemm8_skinny_launch<4, MODE, OT, false>(g, st, ceil_div(g.M, 64));
+      if (choice.row_tile == 16) return gemm8_skinny_launch<1, MODE, OT, false>(g, st, ceil_div(g.M, 16));
       return gemm8_skinny_launch<2, MODE, OT, false>(g, st, ceil_div(g.M, 32));
     }
     if (plan.rows && strip_ok<MODE>(g) &&

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
 
   const int R = g.rows_per_wg, slices = g.max_blocks_m;
   const int tiles_n = (g.N + R - 1) / R, items = tiles_n * slices, G = (int)gridDim.x;
-  const int nkb_all = g.K >> 7;
+  const int nkb_all = (g.K + 127) >> 7;
   // item: slice by slice, the column tiles of each
   auto k_first = [&](int slice) -> int { return __builtin_amdgcn_readfirstlane(nkb_all * slice / slices); };
   // Column tiles start their walk at different K blocks where the weight rows' pitch would put the same block of all rows on a
@@ -94,6 +94,15 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
     const v4i a_rs = descriptor(g.A, (int64_t)g.M * g.lda), b_rs = descriptor(g.B, (int64_t)g.N * g.ldb);
     const v4i s_rs = descriptor(g.sa, BLK ? ((int64_t)(g.M - 1) * g.sa_sm + (int64_t)(nkb_all - 1) * g.sa_sk + 1) * 4 : 0);
     const bool nt = g.streams > 0;
+    // row modes: K need not fill its last block, whose pieces past the end of a row are requested out of range (zeros; a row's
+    // neighbour may hold NaN).  Whether the lane's piece is one of them, by the parity of the group of rows.
+    bool dead[2] = {};
+    if constexpr (!BLK) {
+      if (g.K & 127) {
+#pragma unroll
+        for (int l = 0; l < 2; l++) dead[l] = ((lane & 7) ^ ((l * 4 + (lane >> 4)) & 7)) >= (g.K & 127) >> 4;
+      }
+    }
 
     // the request stream: block `rk` of item `at`
     uint32_t voff[LPB];
@@ -139,15 +148,16 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
       if (kq >= r_nkb) kq -= r_nkb;
       kq = __builtin_amdgcn_readfirstlane(kq + r_begin);
       const int stage = __builtin_amdgcn_readfirstlane(r_stage * STAGE);
+      const bool tail = !BLK && kq == nkb_all - 1;
 #pragma unroll
       for (int u = 0; u < LPB; u++) {
         const int e = u * NL + loader;
-        const uint32_t to = (uint32_t)(stage + e * 1024);
+        const uint32_t to = (uint32_t)(stage + e * 1024), vo = tail && dead[e & 1] ? OUTSIDE : voff[u];
         if (u * NL + NL <= WG || e < WG) {
-          if (nt) dma16_nt(b_rs, voff[u], kq << 7, to);
-          else dma16(b_rs, voff[u], kq << 7, to);
+          if (nt) dma16_nt(b_rs, vo, kq << 7, to);
+          else dma16(b_rs, vo, kq << 7, to);
         } else if (u * NL + NL <= WG + AG || e < WG + AG) {
-          dma16(a_rs, voff[u], kq << 7, to);
+          dma16(a_rs, vo, kq << 7, to);
         } else if (u * NL + NL <= UNITS || e < UNITS) {
           dma4(s_rs, voff[u], (kq * (int)g.sa_sk) << 2, (uint32_t)(stage + S_OFF + (e - WG - AG) * 256));
         }
@@ -418,10 +428,10 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
 #endif
 }
 
-// What the kernel takes: whole K blocks, 32-bit offsets.
+// What the kernel takes: 32-bit offsets, whole K blocks in the block modes.
 template <int MODE>
 static inline bool strip_ok(const GemmArgs& g) {
-  if (g.M < 33 || g.M > STRIP_MAX_ROWS || !gemm8_big_ok(g)) return false;
+  if (g.M < 33 || g.M > STRIP_MAX_ROWS || !gemm8_big_ok(g, !gemm_is_block(MODE))) return false;
   if (!gemm_is_block(MODE)) return true;
   const int64_t nkb = g.K >> 7;
   return ((int64_t)(g.M - 1) * g.sa_sm + (nkb - 1) * g.sa_sk + 1) * 4 < 0x7ffffff0ll && ((nkb - 1) * g.sb_sk + 1) * 4 < 0x7ffffff0ll;
@@ -437,7 +447,7 @@ struct StripPlan {
 // of 92 weights of 0.3 to 470 MB, three scaling modes, weights from HBM and from the Infinity Cache: 7 % rms.
 static inline StripPlan strip_plan(int64_t M, int64_t N, int64_t K) {
   StripPlan best;
-  const int64_t nkb = K >> 7, cus = device_cus();
+  const int64_t nkb = (K + 127) >> 7, cus = device_cus();
   const int rt = M <= 64 ? 2 : M <= 96 ? 3 : 4;
   const double chain = rt == 2 ? 0.247 : rt == 3 ? 0.366 : 0.470;
   for (int rows = 32; rows <= 160; rows += 16) {

@@ -142,6 +142,42 @@ def test_streaming_kernel_over_row_tiles(dev, mode, M, N, K):
     _check(out, ref, f"row tiles {mode} M={M} N={N} K={K}")
 
 
+# a K that does not fill its last block: one piece, seven, K split; rows that are views
+@pytest.mark.parametrize("mode", ["row_fp8", "row_int8"])
+@pytest.mark.parametrize("M,N,K,pitch,kernel", [
+    (33, 30016, 4112, 0, "strip"),
+    (80, 23800, 5984, 16, "strip"),
+    (128, 28673, 3184, 128, "strip"),
+    (48, 9000, 6416, 0, "strip"),       # K split
+    (100, 9000, 6512, 16, "strip"),
+    (96, 512, 1424, 0, 2),              # row tiles of 32 rows, 64, 16
+    (110, 2160, 2672, 16, 4),
+    (200, 584, 1264, 0, 4),
+    (50, 968, 4928, 0, 1),
+    (20, 600, 1936, 16, 1),
+])
+def test_ragged_k(dev, mode, M, N, K, pitch, kernel):
+    from sglang_amd._lib import lib
+
+    print(f"ragged {mode} M={M} N={N} K={K} pitch +{pitch}", flush=True)
+    out, ref = _run(dev, mode, M, N, K, torch.bfloat16, True, pitch, col_scales=False)
+    if kernel == "strip":
+        assert lib.sglamd_last_strip_shape(), "not the strip kernel"
+    else:
+        assert lib.sglamd_last_gemm_kernel() == 1 and lib.sglamd_last_streaming_shape() >> 16 == kernel
+    _check(out, ref, f"ragged {mode} M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("M,N,K", [(17, 704, 4736), (31, 1152, 896), (32, 768, 7936), (33, 512, 1408), (64, 640, 4736)])
+def test_row_tiles_of_16(dev, mode, M, N, K):
+    from sglang_amd._lib import lib
+
+    out, ref = _run(dev, mode, M, N, K, torch.bfloat16, False, 0, col_scales=False)
+    assert lib.sglamd_last_gemm_kernel() == 1 and lib.sglamd_last_streaming_shape() >> 16 == 1
+    _check(out, ref, f"row tiles of 16 {mode} M={M} N={N} K={K}")
+
+
 def test_without_workspace_the_strip_kernel_does_not_split(dev):
     """A call that has no room for the slabs runs what it ran before."""
     from sglang_amd._lib import lib
