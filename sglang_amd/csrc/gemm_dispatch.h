@@ -87,6 +87,10 @@ static int64_t column_split(int64_t M, int64_t N, int64_t K) {
 // either, 0.98 of the fastest form's, the worst point 0.93x, eight below 0.97.
 // Row tiles of 16 rows instead of 32, at 17 to 64 rows: a shorter chain per wave, at twice the reads, so only while the weights are
 // a few MB (704 x 4736 at 24 rows 10.6 -> 9.9 us, 1152 x 7040 16.0 -> 14.2; 4096 x 4096 11.6 -> 12.4).
+// Strips at 17 to 32 rows: weights of 100 MB and more in tiles of 96 to 160 rows that fill 0.85 of their rounds (36864 x 7168 at 24 / 32
+// rows 49 / 51 -> 45 / 46 us, 40000 x 4096 36 / 37 -> 31, 57344 x 8192 79 / 81 -> 76 / 77; 42 points 1.05x in the mean, the worst 0.95x).
+// Narrower tiles (20000 x 8192 in tiles of 80: 33.5 -> 39), K slices (10240 x 16384 33 -> 37) and smaller weights (24576 x 1536 from HBM 13
+// -> 14) stay with the streaming kernel.
 // A ragged K: rows start anywhere in a 128-byte line, and every form pays for it, by the factors below (the mean over 720 points to
 // their models).  512 x 1424 at 96 rows 13.6 -> 7.3 us, 23800 x 5984 at 80 rows 62 -> 45; beyond 128 rows only weights up to 2 MB
 // (512 x 1424 at 200 rows 13.7 -> 7.4, 848 x 1904 15.4 -> 10.1; 680 x 4768 at 320 rows 19.7 against 18.9).
@@ -119,8 +123,11 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
     small[0] = 1e30;
   }
   const int small_rows = small[0] < 1e30 ? 16 : 32;
-  if (M <= 32) {  // the streaming kernel in either case: one tile of 32 rows or two of 16
+  if (M <= 32) {  // the streaming kernel, one tile of 32 rows or two of 16, or strips of weights too large for the caches
     if (small_rows == 16) best.row_tile = 16;
+    const StripPlan plan = N * K >= 100000000 ? strip_plan(M, N, K) : StripPlan();
+    const int64_t tiles = plan.rows ? ceil_div(N, plan.rows) : 0;
+    if (plan.rows >= 96 && plan.slices == 1 && tiles * 20 >= ceil_div(tiles, cus) * cus * 17) best.strip = plan;
     slot = Known{M, N, K, cus, best};
     return best;
   }
@@ -179,7 +186,7 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
         (plan.slices == 1 || (workspace && ((uintptr_t)workspace & 15) == 0 && (int64_t)plan.slices * g.M * g.N * 4 <= workspace_bytes))) {
       // (the class of the shape: the kernels that this one stands in for)
       const bool wide = gemm8_skinny_wide<MODE, OT>(g, st, false) > 0;
-      RAN(g.M > 64 ? SGLAMD_KERNEL_TILE128 : wide ? SGLAMD_KERNEL_STREAMING_WIDE : SGLAMD_KERNEL_TILE64);
+      RAN(g.M <= 32 ? SGLAMD_KERNEL_STREAMING : g.M > 64 ? SGLAMD_KERNEL_TILE128 : wide ? SGLAMD_KERNEL_STREAMING_WIDE : SGLAMD_KERNEL_TILE64);
       strip_last_shape = ((g.M + 31) / 32 << 24) | (plan.slices << 16) | plan.rows;
       return gemm8_strip_launch<MODE, OT>(g, plan, st, workspace);
     }

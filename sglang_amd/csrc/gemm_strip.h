@@ -1,4 +1,4 @@
-// Weight-streaming GEMM for 33 to 128 activation rows: every workgroup owns all rows and up to 128 or 160 weight rows, and
+// Weight-streaming GEMM for 17 to 128 activation rows (up to 32 of them for weights past 100 MB): every workgroup owns all rows and up to 128 or 160 weight rows, and
 // walks (K slice, column tile) items one after the other.
 //
 // What bounds these calls is how many bytes a CU takes in, weights from HBM and activation rows from L2 alike (about 34 KB a
@@ -11,7 +11,7 @@
 //   * one barrier a K block: by then every fragment of the block is in registers and the next block has landed;
 //   * tiles of any multiple of 16 weight rows, so that the items fill the chip: 36864 weight rows are 256 tiles of 144 where
 //     the tile kernel has 144 tiles of 256 for 256 CUs.
-// Kernel alone, us, tile kernel (17..64 rows: wide streaming form) -> this, cold weights: 36864 x 7168 at 64 / 96 / 128 rows 51 / 66 /
+// Kernel alone, us, tile kernel (64 rows: wide streaming form) -> this, cold weights: 36864 x 7168 at 64 / 96 / 128 rows 51 / 66 /
 // 69 -> 44 / 49 / 54; 57344 x 8192 at 128 rows 113 -> 100.  At 128 rows the loaders alone, without a product, need 46: the rest is
 // the clock (1.75 to 1.9 GHz under load) and the fragment reads.  Not faster, and not kept: the loads spread over the
 // multiplying waves (61 at 128 rows), two waves to a strip with half of the rows each (69), four stages instead of three, a
@@ -22,7 +22,12 @@
 namespace sglamd {
 
 constexpr int STRIP_MAX_ROWS = 128;  // activation rows
-constexpr int STRIP_STAGES = 3;
+// Stages: what LDS holds.  Up to 32 rows, where a block takes the multiplying waves little, the blocks in flight are what keeps HBM
+// busy (36864 x 7168 at 32 rows: streaming kernel 51, three stages 48, five 45 us); else three are as good as four.
+template <int RT, int NS>
+constexpr int strip_stages() {
+  return RT > 1 ? 3 : NS == 3 ? 8 : NS == 4 ? 6 : 5;
+}
 constexpr int STRIP_MAX_KB = 256;  // K blocks of a slice: what a row of the scale table holds
 
 // One K block in LDS: weights, rows, row scales
@@ -33,7 +38,7 @@ constexpr int strip_stage() {
 // the stages, a patch of 32 rows x 64 bytes per multiplying wave, two tables of three rows of weight scales
 template <int MODE, int RT, int NS>
 constexpr int strip_smem() {
-  return STRIP_STAGES * strip_stage<MODE, RT, NS>() + NS * 2048 + (gemm_is_block(MODE) ? 2 * 3 * STRIP_MAX_KB * 4 : 0);
+  return strip_stages<RT, NS>() * strip_stage<MODE, RT, NS>() + NS * 2048 + (gemm_is_block(MODE) ? 2 * 3 * STRIP_MAX_KB * 4 : 0);
 }
 
 // RT row tiles of 32, NS strips of 32 weight rows.  g.rows_per_wg: weight rows of a tile (a multiple of 16); g.max_blocks_m: K slices
@@ -42,13 +47,13 @@ template <int MODE, typename OT, int RT, int NS>
 __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr bool BLK = gemm_is_block(MODE);
-  constexpr int BM = 32 * RT, D = STRIP_STAGES, NL = 8 - NS;
+  constexpr int D = strip_stages<RT, NS>(), NL = 8 - NS;
   // wave-wide loads of a K block: groups of eight weight rows, of eight rows, of 64 row scales; loading wave l issues l, l + NL, ...
   constexpr int WG = 4 * NS, AG = 4 * RT, SG = BLK ? (RT + 1) / 2 : 0, UNITS = WG + AG + SG;
   constexpr int LPB = (UNITS + NL - 1) / NL;
   constexpr int STAGE = strip_stage<MODE, RT, NS>(), A_OFF = WG * 1024, S_OFF = A_OFF + AG * 1024;
   constexpr int PATCH_BASE = D * STAGE, TBL_BASE = PATCH_BASE + NS * 2048, TBL_BYTES = 3 * STRIP_MAX_KB * 4;
-  static_assert(RT >= 2 && (RT & 1) == 0 || RT == 3, "fragments of two row tiles, by the parity of the tile");
+  static_assert(RT >= 1 && RT <= 4, "fragments of two row tiles, by the parity of the tile");
   static_assert((D - 1) * LPB < 64, "vmcnt field is 6 bits");
   typedef typename std::conditional<MODE == GEMM_ROW_INT8, v16i, v16f>::type acc16_t;
   typedef typename std::conditional<gemm_is_int8(MODE), v16i, v16f>::type prod16_t;
@@ -166,10 +171,15 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
       r_stage = r_stage == D - 1 ? 0 : r_stage + 1;
     };
     const bool full = UNITS % NL == 0 || (LPB - 1) * NL + loader < UNITS;  // issues LPB loads a block, not one less
-    // all but the last `blocks` blocks requested have landed
-#define STRIP_LANDED(blocks)                                                          \
-  if (full) asm volatile("s_waitcnt vmcnt(%0)" : : "n"((blocks)*LPB) : "memory");     \
-  else asm volatile("s_waitcnt vmcnt(%0)" : : "n"((blocks) * (LPB - 1)) : "memory")
+    // all but the last `blocks` blocks requested (at most `most`, a constant) have landed
+    auto landed = [&](int blocks, auto most) {
+#pragma unroll
+      for (int d = decltype(most)::value; d >= 0; d--)
+        if (blocks == d) {
+          if (full) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(d * LPB) : "memory");
+          else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(d * (LPB - 1)) : "memory");
+        }
+    };
     int left = 0;  // blocks of this workgroup's items
     for (int it = first; it < items; it += G) {
       const int slice = __builtin_amdgcn_readfirstlane(it / tiles_n);
@@ -177,23 +187,15 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
     }
     enter();
     for (int d = 0; d < D; d++) request();
-    if (left >= D) {
-      STRIP_LANDED(D - 1);
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-    }
+    left = __builtin_amdgcn_readfirstlane(left);
+    landed(min(left, D) - 1, std::integral_constant<int, D - 1>{});
     __builtin_amdgcn_s_barrier();
     for (; left > 0; left--) {
       // the next block has landed; behind the barrier this one is in the multiplying waves' registers, and its stage is free
-      if (left >= D) {
-        STRIP_LANDED(D - 2);
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-      }
+      landed(max(min(left, D) - 2, 0), std::integral_constant<int, D - 2>{});
       __builtin_amdgcn_s_barrier();
       request();
     }
-#undef STRIP_LANDED
     return;
   }
 
@@ -257,7 +259,7 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
   // fragments of two row tiles, by the parity of the tile; tiles go from the last one down
   v8i wf[2], x[2][2];
   float sa[2];
-  constexpr int T1 = RT - 1, T2 = RT - 2;
+  constexpr int T1 = RT - 1, T2 = RT > 1 ? RT - 2 : 0;
 #pragma unroll
   for (int h = 0; h < 2; h++) {
     wf[h] = frag(wave * 4096, h);
@@ -275,6 +277,33 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
     for (int kb = 0; kb < nkb; kb++) {
       const int now = st * STAGE, st_next = st == D - 1 ? 0 : st + 1, then = st_next * STAGE;
       float sbv_n = 1.f, sbv1_n = 1.f;
+      if constexpr (RT == 1) {
+        // one tile: the next block's fragments are read while the products are on their way, and these are folded behind that
+        if constexpr (BLK) q[0] = mm_half(wf[1], x[0][1], mm_half(wf[0], x[0][0], zero16));
+        else acc[0] = mm_half(wf[1], x[0][1], mm_half(wf[0], x[0][0], acc[0]));
+        sc = sa[0] * sbv;
+        sc1 = sa[0] * sbv1;
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : : : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" : : : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          wf[h] = frag(then + wave * 4096, h);
+          x[0][h] = frag(then + A_OFF, h);
+        }
+        if constexpr (BLK) {
+          const bool last = kb + 1 == nkb;
+          sa[0] = row_scale(then, 0);
+          sbv = *(last ? sb0_next : sb0 + kb + 1);
+          sbv1 = *(last ? sb1_next : sb1 + kb + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fold(acc[0], q[0]);
+        st = st_next;
+        continue;
+      }
       auto tile = [&](auto tile_c) {
         constexpr int i = decltype(tile_c)::value, p = i & 1, prev = i == RT - 1 ? 0 : i + 1;
         // the fragments that take this tile's registers: two tiles on in this block, or of the next one's first two
@@ -319,17 +348,17 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
         }
         __builtin_amdgcn_sched_barrier(0);
       };
-      if constexpr (RT > 5) tile(std::integral_constant<int, 5>{});
-      if constexpr (RT > 4) tile(std::integral_constant<int, 4>{});
       if constexpr (RT > 3) tile(std::integral_constant<int, 3>{});
       if constexpr (RT > 2) tile(std::integral_constant<int, 2>{});
-      tile(std::integral_constant<int, 1>{});
-      tile(std::integral_constant<int, 0>{});
+      if constexpr (RT > 1) {
+        tile(std::integral_constant<int, 1>{});
+        tile(std::integral_constant<int, 0>{});
+      }
       sbv = sbv_n;
       sbv1 = sbv1_n;
       st = st_next;
     }
-    fold(acc[0], q[0]);
+    if constexpr (RT > 1) fold(acc[0], q[0]);
 
     // ---- the finished tile leaves; the next one's first blocks are on their way -----------------------------------
     const int n0 = pn * R, n_end = min(n0 + R, (int)g.N), nw = n0 + wave * 32;
@@ -431,7 +460,7 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
 // What the kernel takes: 32-bit offsets, whole K blocks in the block modes.
 template <int MODE>
 static inline bool strip_ok(const GemmArgs& g) {
-  if (g.M < 33 || g.M > STRIP_MAX_ROWS || !gemm8_big_ok(g, !gemm_is_block(MODE))) return false;
+  if (g.M < 17 || g.M > STRIP_MAX_ROWS || !gemm8_big_ok(g, !gemm_is_block(MODE))) return false;
   if (!gemm_is_block(MODE)) return true;
   const int64_t nkb = g.K >> 7;
   return ((int64_t)(g.M - 1) * g.sa_sm + (nkb - 1) * g.sa_sk + 1) * 4 < 0x7ffffff0ll && ((nkb - 1) * g.sb_sk + 1) * 4 < 0x7ffffff0ll;
@@ -448,8 +477,8 @@ struct StripPlan {
 static inline StripPlan strip_plan(int64_t M, int64_t N, int64_t K) {
   StripPlan best;
   const int64_t nkb = (K + 127) >> 7, cus = device_cus();
-  const int rt = M <= 64 ? 2 : M <= 96 ? 3 : 4;
-  const double chain = rt == 2 ? 0.247 : rt == 3 ? 0.366 : 0.470;
+  const int rt = M <= 32 ? 1 : M <= 64 ? 2 : M <= 96 ? 3 : 4;
+  const double chain = rt == 1 ? 0.13 : rt == 2 ? 0.247 : rt == 3 ? 0.366 : 0.470;
   for (int rows = 32; rows <= 160; rows += 16) {
     const int64_t tiles = (N + rows - 1) / rows;
     for (int slices = 1; slices <= 12; slices++) {
@@ -457,7 +486,7 @@ static inline StripPlan strip_plan(int64_t M, int64_t N, int64_t K) {
       if (nkb > (int64_t)slices * STRIP_MAX_KB) continue;
       const int64_t items = tiles * slices, rounds = (items + cus - 1) / cus;
       const double fill = items < cus ? (double)items / cus : 1.0;
-      const double own = chain * (rows > 128 ? 1.36 : 1.0), in = (0.0032 * rows + 0.016 * rt) * fill * (1.2 - 0.2 * fill);
+      const double own = chain * (rows > 128 ? 1.36 : 1.0), in = ((rt == 1 ? 0.0040 : 0.0032) * rows + 0.016 * rt) * fill * (1.2 - 0.2 * fill);
       double us = rounds * ((double)nkb / slices * (own > in ? own + 0.47 * in : in + 0.47 * own) + 2.85);
       // (as many items as CUs and short ones: all of them write their slabs at once, 10 to 18 % on top at 96 rows and more)
       if (slices > 1) us = us * (items == cus && nkb < 32 * slices && M > 64 ? 1.1 : 1.0) + 3.2 + (double)slices * M * N * 1.48e-6;
@@ -490,10 +519,15 @@ static int gemm8_strip_launch(const GemmArgs& whole, const StripPlan& plan, hipS
   g.streams = (int64_t)g.N * g.K >= (96ll << 20);
   if (plan.slices > 1) g.C = workspace;
   int rc;
-  if (plan.rows <= 128)
-    rc = g.M <= 64 ? gemm8_strip_start<MODE, OT, 2, 4>(g, st) : g.M <= 96 ? gemm8_strip_start<MODE, OT, 3, 4>(g, st) : gemm8_strip_start<MODE, OT, 4, 4>(g, st);
-  else
-    rc = g.M <= 64 ? gemm8_strip_start<MODE, OT, 2, 5>(g, st) : g.M <= 96 ? gemm8_strip_start<MODE, OT, 3, 5>(g, st) : gemm8_strip_start<MODE, OT, 4, 5>(g, st);
+  auto start = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    if (g.M <= 32) return gemm8_strip_start<MODE, OT, 1, NS>(g, st);
+    if constexpr (NS == 3) return gemm8_strip_start<MODE, OT, 2, 4>(g, st);
+    else return g.M <= 64 ? gemm8_strip_start<MODE, OT, 2, NS>(g, st) : g.M <= 96 ? gemm8_strip_start<MODE, OT, 3, NS>(g, st) : gemm8_strip_start<MODE, OT, 4, NS>(g, st);
+  };
+  if (plan.rows <= 96 && g.M <= 32) rc = start(std::integral_constant<int, 3>{});
+  else if (plan.rows <= 128) rc = start(std::integral_constant<int, 4>{});
+  else rc = start(std::integral_constant<int, 5>{});
   if (rc || plan.slices == 1) return rc;
   return splitk_reduce<MODE, OT>(whole, plan.slices, workspace, st);
 }

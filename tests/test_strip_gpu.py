@@ -1,4 +1,4 @@
-"""Dense GEMMs of 33 to 1024 rows off the tile kernels: the strip kernel (weights in tiles of 16 to 160 rows, loading and multiplying
+"""Dense GEMMs of 17 to 1024 rows off the tile kernels: the strip kernel (weights in tiles of 16 to 160 rows, loading and multiplying
 waves) and the streaming kernel walking several row tiles, at the edges of their tiles, against the oracle."""
 import numpy as np
 import pytest
@@ -71,6 +71,10 @@ def _check(out, ref, what):
 # scale blocks; several items per workgroup; K split, and K blocks that do not divide by the slices
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("M,N,K,pitch", [
+    (17, 40009, 2560, 0),       # one row tile: five strips
+    (31, 65540, 2048, 128),     # ... four, two tiles a workgroup
+    (24, 24570, 4224, 0),       # ... three
+    (32, 28672, 3584, 0),
     (33, 30016, 4096, 0),
     (64, 30024, 4096, 128),     # five strips, the last tile ragged
     (65, 28681, 4096, 0),       # N odd: single stores
@@ -145,6 +149,7 @@ def test_streaming_kernel_over_row_tiles(dev, mode, M, N, K):
 # a K that does not fill its last block: one piece, seven, K split; rows that are views
 @pytest.mark.parametrize("mode", ["row_fp8", "row_int8"])
 @pytest.mark.parametrize("M,N,K,pitch,kernel", [
+    (18, 24580, 4112, 16, "strip"),
     (33, 30016, 4112, 0, "strip"),
     (80, 23800, 5984, 16, "strip"),
     (128, 28673, 3184, 128, "strip"),
