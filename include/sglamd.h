@@ -240,6 +240,7 @@ int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 #define SGLAMD_KERNEL_PERSISTENT256_POW2 7 /* the persistent kernel applying power-of-two scales inside the MFMA */
 #define SGLAMD_KERNEL_STREAMING_WIDE 8  /* 33..64 rows, wide weights, long K: strip kernel, or (K % 128 != 0) the weight-streaming
                                            kernel with 96..144 weight rows per workgroup */
+#define SGLAMD_KERNEL_TILE192 9       /* 192-row tiles of the tile kernel */
 int sglamd_last_gemm_kernel(void);
 /* The same for the streaming kernel's shape: (FM << 16) | (FN << 8) | KW of the last dense launch of it on this thread
  * -- FM 16-row activation tiles, FN 16-row weight tiles per workgroup, KW waves sharing a tile's K range. */

@@ -754,7 +754,7 @@ static int splitk_reduce(const GemmArgs& g, int slices, const void* workspace, h
   return check_launch("splitk_reduce");
 }
 
-// Tile height (64, 128 or 256 rows) and number of K slices for the large-M kernel.  One workgroup occupies a
+// Tile height (64, 128, 192 or 256 rows) and number of K slices for the large-M kernel.  One workgroup occupies a
 // CU, so the cost of a launch is (rounds of one workgroup per CU) x (work per workgroup); the 128-row tile does
 // half the work per workgroup at a somewhat lower MFMA efficiency and is preferred when it removes a mostly
 // empty last round.  K is split when the tile grid alone cannot fill the chip (every slice keeps >= 8 blocks).
@@ -770,10 +770,11 @@ static inline int gemm8_big_slices(int64_t tiles, int64_t N, int64_t K) {
   if (s > 16) s = 16;
   return s < 1 ? 1 : (int)s;
 }
-static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool persistent_256 = false) {
-  // tuning knob: force the tile height (64, 128 or 256)
+// persistent_256: 1 when launches of 256-row tiles may run the persistent kernel, 2 when it applies the scales inside the MFMA
+static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, int persistent_256 = 0) {
+  // tuning knob: force the tile height (64, 128, 192 or 256)
   static const int forced = getenv("SGLAMD_BIG_BM") ? atoi(getenv("SGLAMD_BIG_BM")) : 0;
-  if (forced == 64 || forced == 128 || forced == 256)
+  if (forced == 64 || forced == 128 || forced == 192 || forced == 256)
     return {forced, gemm8_big_slices(((M + forced - 1) / forced) * ((N + 255) / 256), N, K)};
   if (M <= 64) {
     // one row of 64-row tiles: K is split until the grid fills the chip
@@ -789,14 +790,31 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool p
   double best_cost = 1e30;
   const int cus = device_cus();
   const double nkb = (double)(K >> 7);
-  for (int bm = 64; bm <= 256; bm *= 2) {
-    if (bm == 256 && M <= 128) break;
+  for (int bm = 64; bm <= 256; bm += 64) {
+    if (bm > 128 && M <= 128) break;
+    // up to 192 rows one of the two: gate_up at 150 rows 79 us in 192-row tiles, 86 in 256-row tiles, 7168 x 18432 52.7 and 53.4, but 8192 x
+    // 28672 79.4 and 76.5
+    if (M <= 192 && bm == (K < 20480 ? 256 : 192)) continue;
     const int64_t tiles = ((M + bm - 1) / bm) * ((N + 255) / 256);
+    // 192 rows, between the heights that leave many rows or CUs idle: 8192 x 28672 at 560 / 640 rows 198 / 219 -> 159 / 158 us, 7168 x
+    // 18432 at 560 rows 122 -> 99, gate_up at 560 rows 196 -> 165, 57344 x 8192 at 380 rows 208 -> 180, 7168 x 18432 at 3100 / 3400 rows,
+    // where the persistent kernel's second round is half full, 451 / 466 -> 394 / 411.  Of 415 points of 27 weights and 129 to 4000 rows
+    // it is chosen at 143, 1.12x in the mean.  Not for
+    //   * a few K blocks, where the drains decide (8000 x 768 at 1500 rows 23.2 us in 256-row tiles, 22.9; with scales inside the MFMA,
+    //     which the persistent kernel alone has, 24576 x 1536 at 900 / 1300 rows 42 / 61 us and 46 / 66, x 2560 at 950 rows 63 and 67);
+    //   * what the persistent kernel and the launch behind it (column_split) take between one round and one and three eighths of (7168 x
+    //     18432 at 2400 / 2765 / 3023 rows 334 / 347 / 376 us, 363 / 367 / 380 in 192-row tiles);
+    //   * weights past the 470 MB that were measured.
+    if (bm == 192) {
+      const int64_t whole = (M + 255) / 256 * ((N + 255) / 256);
+      if (K < (persistent_256 > 1 && whole > cus ? 4096 : 1152)) continue;
+      if (persistent_256 && whole > cus && (N * K > 500000000 || ((N & 255) == 0 && K >= 4096 && whole < 2 * cus && (whole - cus) * 8 <= cus * 3))) continue;
+    }
     const int slices = gemm8_big_slices(tiles, N, K);
     const int64_t rounds = (tiles * slices + cus - 1) / cus;
     // (64-row tiles in several rounds read each weight byte once per row tile from further away: gate_up at M = 400, four rounds of
     // them, 176 us, 158 in 128-row tiles, 138 in 256-row tiles)
-    const double weight = bm == 64 ? (rounds > 1 ? 2.0 : 1.6) : bm == 128 ? 1.2 : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
+    const double weight = bm == 64 ? (rounds > 1 ? 2.0 : 1.6) : bm == 128 ? 1.2 : bm == 192 ? (M <= bm ? 1.0 : slices > 3 ? 1.12 : 1.06) : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
     // a single row of tiles only loads the rows that exist: M = 192 in 256-row tiles costs what 192 rows cost
     // (gate_up at M = 192: 89.6 us in 256-row tiles against 102.5 in 64-row tiles, which need two rounds)
     const double rows = M <= bm ? (double)((M + 63) / 64 * 64) : (double)bm;
@@ -810,7 +828,7 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, bool p
       const double fill = std::sqrt((double)(tiles * slices) / cus), most = slices == 1 ? 0.75 : 0.9;
       cost *= fill > most ? fill : most;
     }
-    if (slices > 1) cost += 4.0 + (double)slices * M * N * 8.0 / (M > bm ? 5000.0 : 4000.0) / (nkb * 7.7);
+    if (slices > 1) cost += 4.0 + (double)slices * M * N * 8.0 / (M > bm ? 5000.0 : 4500.0) / (nkb * 7.7);
     if (cost < best_cost) {
       best_cost = cost;
       best = {bm, slices};

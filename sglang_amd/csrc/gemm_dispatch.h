@@ -117,12 +117,10 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
   double small[3] = {M <= 64 ? skinny_row_tiles_us<1>(M, N, K, &fills[0]) * (ragged ? 1.25 : 1.0) : 1e30,
                      skinny_row_tiles_us<2>(M, N, K, &fills[1]) * (ragged ? 1.25 : 1.0),
                      M > 32 ? skinny_row_tiles_us<4>(M, N, K, &fills[2]) * (ragged ? 1.15 : 1.0) : 1e30};
-  if (M <= 64 && small[0] * 1.02 + 0.02 * common < small[1] && N * K <= 10000000) {
-    small[1] = small[0], fills[1] = fills[0];  // 16-row tiles in place of the 32-row ones
-  } else {
-    small[0] = 1e30;
-  }
-  const int small_rows = small[0] < 1e30 ? 16 : 32;
+  const bool streamed = M <= 64 && !small_m_uses_tile(M, N, K);  // without this choice: the streaming kernel's 32- or 64-row tile
+  int small_rows = 32;
+  if (M <= 64 && (streamed || fills[0]) && small[0] * 1.02 + 0.02 * common < small[1] && N * K <= 10000000)
+    small_rows = 16, small[1] = small[0], fills[1] = true;
   if (M <= 32) {  // the streaming kernel, one tile of 32 rows or two of 16, or strips of weights too large for the caches
     if (small_rows == 16) best.row_tile = 16;
     const StripPlan plan = N * K >= 100000000 ? strip_plan(M, N, K) : StripPlan();
@@ -131,7 +129,6 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
     slot = Known{M, N, K, cus, best};
     return best;
   }
-  const bool streamed = M <= 64 && !small_m_uses_tile(M, N, K);  // without this choice: the streaming kernel's 64-row tile
   double least;
   bool row_tiles = true;
   if (streamed) {
@@ -142,7 +139,7 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
     const BigConfig cfg = gemm8_big_config(M, N, K, persistent);
     const int64_t cols = ceil_div(N, 256) * cfg.slices, rounds = ceil_div(ceil_div(M, cfg.bm) * cols, cus);
     // a K block of a tile, or of the weights that the column tiles in flight read (6.7 TB/s from the Infinity Cache, 5.2 else)
-    const double block = std::max(cfg.bm == 64 ? 0.52 : cfg.bm == 128 ? 1.04 : 1.85, (N * K > 85000000 ? 0.0063 : 0.0049) * std::min(cols, cus));
+    const double block = std::max(cfg.bm == 64 ? 0.52 : cfg.bm == 128 ? 1.04 : cfg.bm == 192 ? 1.45 : 1.85, (N * K > 85000000 ? 0.0063 : 0.0049) * std::min(cols, cus));
     double us = rounds * ((double)nkb / cfg.slices * block + 2.2);
     row_tiles = M > 64 || cfg.slices > 1;  // up to 64 rows the model is not fine enough to tell them from one launch of 64-row tiles
     if (cfg.slices > 1) us += 3.2 + 1.86e-6 * cfg.slices * M * N;
@@ -150,7 +147,7 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
   }
   for (int f = 1; f < 3 && row_tiles; f++) {
     if (!fills[f]) continue;
-    const double us = (common + small[f]) * (streamed && f == 2 ? 1.0 : 1.12);
+    const double us = (common + small[f]) * (streamed && f == 2 ? 1.0 : ragged && M > 128 ? 1.25 : 1.12);
     if (us < least) least = us, best.row_tile = f == 2 ? 64 : small_rows;
   }
   if (M <= STRIP_MAX_ROWS) {
@@ -173,6 +170,7 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
   const int wgs = gemm_is_block(MODE) ? persist_workgroups() : 0;
   const int nkb = g.K >> 7;
   const bool persistent = wgs > 0 && (wgs & 7) == 0 && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
+  const int tiles_256 = persistent ? (MODE == GEMM_BLOCK_FP8 && g.scales_pow2 ? 2 : 1) : 0;
   strip_last_shape = 0;
   if (big && may_split && g.M > 16) {
     const DenseChoice choice = dense_choice(g.M, g.N, g.K);
@@ -192,7 +190,7 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
     }
   }
   if (big && may_split && g.M > 64) {
-    const BigConfig whole = gemm8_big_config(g.M, g.N, g.K, persistent);
+    const BigConfig whole = gemm8_big_config(g.M, g.N, g.K, tiles_256);
     const int64_t n1 = whole.bm == 256 && whole.slices == 1 ? column_split(g.M, g.N, g.K) : 0;
     if (n1 > 0) {
       typedef typename OT::storage OS;
@@ -222,14 +220,15 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
   }
   {
     if (big) {
-      const BigConfig cfg = gemm8_big_config(g.M, g.N, g.K, persistent);
+      const BigConfig cfg = gemm8_big_config(g.M, g.N, g.K, tiles_256);
       const int bm = cfg.bm;
       int slices = cfg.slices;
       while (slices > 1 && (int64_t)slices * g.M * g.N * 4 > workspace_bytes) slices--;
       if (!workspace || ((uintptr_t)workspace & 15)) slices = 1;
-      RAN(bm == 64 ? SGLAMD_KERNEL_TILE64 : bm == 128 ? SGLAMD_KERNEL_TILE128 : SGLAMD_KERNEL_TILE256);
+      RAN(bm == 64 ? SGLAMD_KERNEL_TILE64 : bm == 128 ? SGLAMD_KERNEL_TILE128 : bm == 192 ? SGLAMD_KERNEL_TILE192 : SGLAMD_KERNEL_TILE256);
       if (bm == 64) return gemm8_big_launch<MODE, OT, 4, 1>(g, st, slices, workspace);
       if (bm == 128) return gemm8_big_launch<MODE, OT, 4, 2>(g, st, slices, workspace);
+      if (bm == 192) return gemm8_big_launch<MODE, OT, 4, 3>(g, st, slices, workspace);
       if (big_wgn() == 2) return gemm8_big_launch<MODE, OT, 2, 4>(g, st, slices, workspace);
       if constexpr (gemm_is_block(MODE)) {
         const bool bias_ok = !out_biased<OT> || (g.N >= 32 && ((uintptr_t)g.bias & 3) == 0);

@@ -1009,7 +1009,8 @@ static int skinny_plan(GemmArgs& g) {
 // Time in us, without what all forms have in common (launch, quantiser), of a dense launch that walks M rows in row tiles of 16 * FM,
 // the weights read once for each of them (past the first from L2 or the Infinity Cache).  A round of workgroups takes
 // the longer of a wave's chain of K blocks and the CU's bytes, and all of the other.  Fitted to 6354 launches of 160 weights of up
-// to 85 MB at 33 to 1000 rows, FM = 2 and 4, three weights in turn and enough to come from HBM: 10 % rms.  *fills: more than a quarter of the CUs have a tile.
+// to 85 MB at 33 to 1000 rows, FM = 2 and 4, three weights in turn and enough to come from HBM: 10 % rms.  *fills: more than a quarter (FM = 1:
+// half) of the CUs have a tile.
 template <int FM>
 static double skinny_row_tiles_us(int64_t M, int64_t N, int64_t K, bool* fills) {
   GemmArgs g = {};
@@ -1028,7 +1029,7 @@ static double skinny_row_tiles_us(int64_t M, int64_t N, int64_t K, bool* fills) 
     if (fn == 3) residency(std::integral_constant<int, 3>{});
     else residency(std::integral_constant<int, 4>{});
   }
-  *fills = tiles * 4 > cus;
+  *fills = tiles * (FM == 1 ? 2 : 4) > cus;
   const int64_t rounds = ceil_div(tiles, cus * per_cu), active = std::min<int64_t>(per_cu, ceil_div(tiles, cus));
   const double chain = 1.26 + 0.07 * FM * fn * (double)ceil_div(nkb, kw);
   const double bytes = active * (rows + 0.27 * 16 * FM) * (double)K / 46400.;
