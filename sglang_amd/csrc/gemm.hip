@@ -102,18 +102,22 @@ extern "C" int sglamd_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, c
 
 // Linear layers of up to this many rows may quantise them in the GEMM's own workgroups (0: none).
 static int quantising_max_rows() {
-  static const int v = getenv("SGLAMD_LINEAR_FUSE_ROWS") ? atoi(getenv("SGLAMD_LINEAR_FUSE_ROWS")) : 4;  // tuning knob
+  static const int v = getenv("SGLAMD_LINEAR_FUSE_ROWS") ? atoi(getenv("SGLAMD_LINEAR_FUSE_ROWS")) : 16;  // tuning knob
   return v;
 }
 // Which of them do.  A launch less saves 1-2 us; every workgroup quantising every row costs it time that grows with M * K
 // and delays its weight stream.  Two launches -> one, us, weights from HBM, queue kept full, block scales (row scales):
 //   one row    36864 x 7168 42.6 -> 41.2, 7168 x 16384 21.9 -> 21.4, 24576 x 1536 10.9 -> 8.9 (11.2 -> 9.5), 4096 x 4096 7.5 -> 6.3
 //              (8.1 -> 6.7), 1024 x 7168 8.3 -> 6.6 (8.7 -> 6.9), (10240 x 8192 17.8 -> 16.7)
-//   two rows   36864 x 7168 42.6 -> 42.1, 4096 x 4096 7.7 -> 6.5 (8.1 -> 7.0), 1024 x 7168 8.3 -> 7.2 (8.8 -> 7.8)
+//   two rows   36864 x 7168 42.6 -> 42.1, 24576 x 1536 10.6 -> 8.6 (11.0 -> 9.1), 4096 x 4096 7.6 -> 6.4 (7.9 -> 6.9), 1024 x 7168 8.3 -> 7.2
 //   three      36864 x 7168 42.7 -> 42.9, 1024 x 7168 8.4 -> 7.9 (8.8 -> 8.6), (10240 x 8192 17.9 -> 18.9)
-//   four       36864 x 7168 42.7 -> 43.4, 4096 x 4096 7.9 -> 7.2 (8.2 -> 8.0), 1024 x 7168 8.4 -> 8.2 (8.8 -> 9.1)
-static bool linear_quantises(int64_t M, int64_t K) {
-  return M >= 1 && M <= quantising_max_rows() && (M == 1 || M * K <= 16384);
+//   four       36864 x 7168 42.7 -> 43.4, 24576 x 1536 10.8 -> 9.0 (11.0 -> 9.8), 4096 x 4096 7.6 -> 7.0 (7.9 -> 7.7), 1024 x 1024 7.2 -> 5.5
+//   eight      24576 x 1536 10.8 -> 9.6 (11.3 -> 10.7), 4096 x 4096 7.8 -> 8.4, 1024 x 1024 7.1 -> 6.0 (7.6 -> 6.8), 4096 x 2048 7.6 -> 7.2
+//              (7.5 -> 7.7)
+//   sixteen    4096 x 512 6.9 -> 6.0 (7.8 -> 7.3), 1024 x 1024 7.3 -> 6.9 (7.6 -> 8.1)
+// and of a call that the host launches in 9.5 us (10) with an empty queue, 2.5 us: 1024 x 1024 at four to twelve rows 9.5 -> 6.5 (10 -> 7).
+static bool linear_quantises(int64_t M, int64_t K, bool row_scales) {
+  return M >= 1 && M <= quantising_max_rows() && (M == 1 || M * K <= (M > 4 && row_scales ? 12288 : 16384));
 }
 
 extern "C" int sglamd_fp8_block_linear(const void* x, int dtype, int64_t M, int64_t K, const void* w, int64_t ldb,
@@ -126,7 +130,7 @@ extern "C" int sglamd_fp8_block_linear(const void* x, int dtype, int64_t M, int6
   SGLAMD_REQUIRE(K > 0 && K % 128 == 0, SGLAMD_EINVAL, "%s: K (%lld) must be a positive multiple of 128", op, (long long)K);
   SGLAMD_REQUIRE(!bias || ((uintptr_t)bias & 1) == 0, SGLAMD_EINVAL, "%s: odd bias pointer", op);
   const DeviceScope scope;
-  if (linear_quantises(M, K) && ((uintptr_t)x % 16) == 0) {
+  if (linear_quantises(M, K, false) && ((uintptr_t)x % 16) == 0) {
     int rc = check_common(op, x, w, out, M, N, K, K, ldb, ldc);
     if (rc) return rc;
     GemmArgs g = {};
@@ -207,7 +211,7 @@ extern "C" int sglamd_fp8_row_linear(const void* x, int dtype, int64_t M, int64_
   SGLAMD_REQUIRE(x && w && sb && out && q && sa, SGLAMD_EINVAL, "%s: null pointer", op);
   SGLAMD_REQUIRE(dtype == SGLAMD_BF16 || dtype == SGLAMD_F16, SGLAMD_EINVAL, "%s: dtype must be Half or BFloat16", op);
   const DeviceScope scope;
-  if (linear_quantises(M, K) && K % 128 == 0 && ((uintptr_t)x % 16) == 0) {
+  if (linear_quantises(M, K, true) && K % 128 == 0 && ((uintptr_t)x % 16) == 0) {
     int rc = check_common(op, x, w, out, M, N, K, K, ldb, ldc);
     if (rc) return rc;
     GemmArgs g = {};

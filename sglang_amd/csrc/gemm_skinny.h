@@ -63,10 +63,18 @@ constexpr int skinny_slot_bytes() {
 // AQ rows of K bytes, each padded by 16 so that the rows' fragment reads spread over the banks, then their scales
 static inline int skinny_aq_bytes(int aq, int K) { return aq * (K + 16) + aq * ((K + 127) >> 7) * 4; }
 constexpr int SKINNY_DQ_PASSES = 8;  // DQ: passes of a workgroup over its rows, 64 bytes of registers a lane each
-// DQ, SOLO: room for the 16-bit rows, in whole passes of a workgroup, which the quantised rows take over, then their scales
-static inline int skinny_dq_bytes(int M, int K, int kw) {
+// DQ, SOLO: room for the 16-bit rows, in whole passes of the waves that quantise, which the quantised rows take over, then their scales
+static inline int skinny_dq_bytes(int M, int K, int qw) {
   const int groups = M * (K >> 7);
-  return (groups + 8 * kw - 1) / (8 * kw) * (kw * 2048) + groups * 4;
+  return (groups + 8 * qw - 1) / (8 * qw) * (qw * 2048) + groups * 4;
+}
+// DQ: the waves that quantise where the KW that share a tile's K blocks take several passes for it (each 0.4 us with one wave: a
+// launch of 512 x 512 took 4.4 us at two rows, 5.5 at eight and 7.1 at sixteen; with four waves 4.7, 4.8 and 5.0).  The others end behind it.
+constexpr int skinny_dq_helped(int kw) { return kw < 4 ? 4 : 8; }
+static inline int skinny_dq_waves(int groups, int kw, int64_t tiles) {
+  const int qw = skinny_dq_helped(kw);
+  const int64_t per_cu = (tiles + device_cus() - 1) / device_cus();
+  return groups > 8 * kw && per_cu * qw <= 12 ? qw : kw;  // (three waves to a SIMD)
 }
 // Waves that may split K, and K blocks in flight per wave: the rings of all waves fill the LDS of a CU (156 KB of
 // its 160), which is what keeps enough bytes in flight to stream from HBM at full rate.
@@ -112,8 +120,8 @@ __device__ __forceinline__ void skinny_wait(int blocks) {
 }
 #endif
 
-template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int PD, int AQ = 0>
-__global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
+template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int PD, int AQ = 0, int QW = KW>
+__global__ __launch_bounds__(64 * QW) void gemm8_skinny_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
   typedef typename AccT<MODE>::type acc_t;
   typedef typename OT::storage OS;
@@ -353,8 +361,8 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   // AQ: the tile's rows, quantised, behind the rings: AQ rows of K bytes (stride K + 16) and their group scales.
   uint8_t* xq_rows = smem + KW * PD * SLOT;
   const int xq_stride = g.K + 16;
-  const int dq_groups = DQ ? g.M * nkb : nkb, dq_passes = (dq_groups + 8 * KW - 1) / (8 * KW);
-  float* xq_scales = reinterpret_cast<float*>(xq_rows + (DQ || SOLO ? dq_passes * (KW * 2048) : AQ * xq_stride));
+  const int dq_groups = DQ ? g.M * nkb : nkb, dq_passes = (dq_groups + 8 * QW - 1) / (8 * QW);
+  float* xq_scales = reinterpret_cast<float*>(xq_rows + (DQ || SOLO ? dq_passes * (QW * 2048) : AQ * xq_stride));
   // Quantises the real rows of the tile whose slot ids are in s_rows[buf]: per pass 16 groups of 128 over all the
   // workgroup's lanes, LPG = 4 * KW lanes per group and 128 / LPG elements per lane.  The arithmetic is
   // group_quant_body's (reciprocal form, float scales), so bytes and scales are the ones the stand-alone kernels
@@ -495,7 +503,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   };
 
   // DQ, SOLO: group gi of the rows' groups of 128 belongs to eight lanes, 16 values each; pass p holds the groups
-  // 8 * KW * p + tid / 8.  The 16-bit values lie where the quantised rows go, pass by pass, 32 bytes a lane as two halves of 16.
+  // 8 * QW * p + tid / 8.  The 16-bit values lie where the quantised rows go, pass by pass, 32 bytes a lane as two halves of 16.
   // They are requested in front of the first weight blocks and waited for without these.
   auto fetch_rows = [&](int pair) {
     if constexpr (DQ || SOLO) {
@@ -503,10 +511,10 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
       const v4i rs = descriptor(base, (SOLO ? 0 : (int64_t)(g.M - 1) * g.lda16) + (int64_t)g.K * 2);
       const uint32_t raw = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem + KW * PD * SLOT + wave * 2048;
       for (int p = 0; p < dq_passes; p++) {
-        const int gi = p * 8 * KW + (tid >> 3), r = SOLO ? 0 : gi / nkb;
+        const int gi = p * 8 * QW + (tid >> 3), r = SOLO ? 0 : gi / nkb;
         const uint32_t off = gi < dq_groups ? (uint32_t)(r * (int)g.lda16 + (gi - r * nkb) * 256 + (lane & 7) * 32) : SKINNY_NOWHERE;
 #pragma unroll
-        for (int h = 0; h < 2; h++) dma16(rs, off + (uint32_t)(h * 16), 0, raw + p * (KW * 2048) + h * 1024, false);
+        for (int h = 0; h < 2; h++) dma16(rs, off + (uint32_t)(h * 16), 0, raw + p * (QW * 2048) + h * 1024, false);
       }
     }
   };
@@ -521,8 +529,8 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
 #pragma unroll
         for (int p = 0; p < SKINNY_DQ_PASSES; p++)
           if (p0 + p < dq_passes) {
-            raw[p][0] = *(const v4i*)(src + (p0 + p) * (KW * 2048));
-            raw[p][1] = *(const v4i*)(src + (p0 + p) * (KW * 2048) + 1024);
+            raw[p][0] = *(const v4i*)(src + (p0 + p) * (QW * 2048));
+            raw[p][1] = *(const v4i*)(src + (p0 + p) * (QW * 2048) + 1024);
           }
         // the quantised rows replace the 16-bit ones
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
@@ -531,7 +539,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
 #pragma unroll
           for (int p = 0; p < SKINNY_DQ_PASSES; p++)
             if (p0 + p < dq_passes) {
-              const int gi = (p0 + p) * 8 * KW + (tid >> 3);
+              const int gi = (p0 + p) * 8 * QW + (tid >> 3);
               XS e[16];
               __builtin_memcpy(e, raw[p], 32);
               float m = 0.f;
@@ -546,7 +554,7 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
         for (int p = 0; p < SKINNY_DQ_PASSES; p++)
           if (p0 + p < dq_passes) {
             // group_quant_body's arithmetic (reciprocal form, float scales); row scales: row_quant_body's
-            const int gi = (p0 + p) * 8 * KW + (tid >> 3);
+            const int gi = (p0 + p) * 8 * QW + (tid >> 3);
             XS e[16];
             float x[16];
             __builtin_memcpy(e, raw[p], 32);
@@ -599,10 +607,11 @@ __global__ __launch_bounds__(64 * KW) void gemm8_skinny_kernel(GemmArgs g) {
   setup(tile, 0);
 #pragma unroll
   for (int s = 0; s < PD; s++)
-    if (s < n_my) issue(s, block_of(s));
+    if (s < n_my && (QW == KW || wave < KW)) issue(s, block_of(s));
   if constexpr (DQ || SOLO) {
-    skinny_wait<PD, LOADS>(n_my);
+    skinny_wait<PD, LOADS>(QW == KW || wave < KW ? n_my : 0);
     quantise_fetched();
+    if (QW > KW && wave >= KW) return;  // (barriers count the waves that are left)
   } else if constexpr (AQ > 0) {
     quantise_rows(0);
     if (KW > 1) __syncthreads();
@@ -854,11 +863,16 @@ static inline int skinny_resident_per_cu(int kw, int extra_bytes = 0) {
   return skinny_fit(skinny_smem_bytes<FM, FN, AQ>(kw, extra_bytes), kw);
 }
 
-template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int AQ = 0>
+template <int FM, int FN, int MODE, typename OT, bool MOE, int KW, int AQ = 0, int QW = KW>
 static int gemm8_skinny_launch_kw(const GemmArgs& g, hipStream_t st) {
   constexpr bool DQ = AQ > 0 && !MOE, SOLO = AQ == 1 && MOE;
+  if constexpr (DQ && QW == KW && skinny_dq_helped(KW) > KW) {
+    const int rows = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
+    constexpr int HELPED = skinny_dq_helped(KW);
+    if (skinny_dq_waves(g.M * (g.K >> 7), KW, (g.N + rows - 1) / rows) > KW) return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, KW, AQ, HELPED>(g, st);
+  }
   constexpr int PD = skinny_depth<FM, FN, AQ, DQ>();
-  const int aq_bytes = DQ || SOLO ? skinny_dq_bytes(SOLO ? 1 : g.M, g.K, KW) : AQ > 0 ? skinny_aq_bytes(AQ, g.K) : 0;
+  const int aq_bytes = DQ || SOLO ? skinny_dq_bytes(SOLO ? 1 : g.M, g.K, QW) : AQ > 0 ? skinny_aq_bytes(AQ, g.K) : 0;
   const int smem = DQ || SOLO ? KW * PD * skinny_slot_bytes<FM, FN, AQ>() + aq_bytes : skinny_smem_bytes<FM, FN, AQ>(KW, aq_bytes);
   if (smem > 160 * 1024) return fail(SGLAMD_ENOTSUP, "gemm: K = %d is too long for in-kernel activation quantisation", g.K);
   const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN;
@@ -868,15 +882,15 @@ static int gemm8_skinny_launch_kw(const GemmArgs& g, hipStream_t st) {
   if (tiles <= 0) return SGLAMD_OK;
   if (tiles > 0x7fffffff) return fail(SGLAMD_EINVAL, "gemm: grid too large");
   // as many workgroups as the chip holds at once; each walks tiles blockIdx.x, + gridDim.x, ...
-  const int64_t resident = (int64_t)device_cus() * (SOLO ? skinny_fit(smem, KW, 128) : DQ ? skinny_fit(smem, KW) : skinny_resident_per_cu<FM, FN, AQ>(KW, aq_bytes));
+  const int64_t resident = (int64_t)device_cus() * (SOLO ? skinny_fit(smem, KW, 128) : DQ ? skinny_fit(smem, QW) : skinny_resident_per_cu<FM, FN, AQ>(KW, aq_bytes));
   const unsigned blocks = (unsigned)(tiles < resident ? tiles : resident);
-  auto kern = gemm8_skinny_kernel<FM, FN, MODE, OT, MOE, KW, PD, AQ>;
+  auto kern = gemm8_skinny_kernel<FM, FN, MODE, OT, MOE, KW, PD, AQ, QW>;
   if (smem > 64 * 1024) {
     static SmemAttrOnce attr;
     hipError_t e = raise_dynamic_smem(attr, (const void*)kern, smem);
     if (e != hipSuccess) return fail(SGLAMD_EHIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * KW), smem, st, g);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * QW), smem, st, g);
   return check_launch("gemm8_skinny");
 }
 
@@ -1056,22 +1070,26 @@ static int gemm8_skinny_launch(const GemmArgs& g0, hipStream_t st, int64_t expec
 
 // The dense launch that quantises its rows itself: `g` carries the 16-bit rows in A16 / lda16 and the quantisation
 // constants.  `launch` false: whether it takes the shape.
-template <int FN>
+// Past four rows a launch less is worth four passes of 0.25 us over them (block scales: 32768 x 512 at eight / twelve rows, four and
+// six passes, 8.1 / 8.0 -> 7.9 / 8.8 us) or two (row scales, which meet twice: 1024 x 1024 at twelve / sixteen rows, three and four,
+// 7.5 / 7.6 -> 7.5 / 8.1; 32768 x 512 at eight, four, 9.0 -> 9.5).
+template <int MODE, int FN>
 static bool skinny_dq_fits(const GemmArgs& g) {
   const int R = g.rows_per_wg > 0 ? g.rows_per_wg : 16 * FN, tiles = (g.N + R - 1) / R;
   const int kw = skinny_pick_kw<1, FN>(tiles, g.K >> 7);
-  const int groups = g.M * (g.K >> 7);
-  const int smem = kw * skinny_depth<1, FN, 1, true>() * skinny_slot_bytes<1, FN, 1>() + skinny_dq_bytes(g.M, g.K, kw);
+  const int groups = g.M * (g.K >> 7), qw = skinny_dq_waves(groups, kw, tiles);
+  const int smem = kw * skinny_depth<1, FN, 1, true>() * skinny_slot_bytes<1, FN, 1>() + skinny_dq_bytes(g.M, g.K, qw);
   // the rows must not take a workgroup's place on a CU: one row of 57344 x 8192 75.1 -> 81.4 us with three instead of four
   const int plain = skinny_resident_per_cu<1, FN>(kw), wanted = (tiles + device_cus() - 1) / device_cus();
-  return (groups + 8 * kw - 1) / (8 * kw) <= SKINNY_DQ_PASSES && smem <= 158 * 1024 &&
-         skinny_fit(smem, kw) >= (wanted < plain ? wanted : plain);
+  const int most = g.M <= 4 ? SKINNY_DQ_PASSES : gemm_is_block(MODE) ? 4 : 2;
+  return (groups + 8 * qw - 1) / (8 * qw) <= most && smem <= 158 * 1024 &&
+         skinny_fit(smem, qw) >= (wanted < plain ? wanted : plain);
 }
 template <int MODE, typename OT>
 static int gemm8_skinny_quantising(const GemmArgs& g0, hipStream_t st, bool launch) {
   GemmArgs g = g0;
   const int fn = skinny_plan<1>(g);
-  if (!launch) return fn == 4 ? skinny_dq_fits<4>(g) : fn == 3 ? skinny_dq_fits<3>(g) : fn == 2 ? skinny_dq_fits<2>(g) : skinny_dq_fits<1>(g);
+  if (!launch) return fn == 4 ? skinny_dq_fits<MODE, 4>(g) : fn == 3 ? skinny_dq_fits<MODE, 3>(g) : fn == 2 ? skinny_dq_fits<MODE, 2>(g) : skinny_dq_fits<MODE, 1>(g);
   if (fn == 4) return gemm8_skinny_launch_fn<1, 4, MODE, OT, false, 1>(g, st, 1);
   if (fn == 3) return gemm8_skinny_launch_fn<1, 3, MODE, OT, false, 1>(g, st, 1);
   if (fn == 2) return gemm8_skinny_launch_fn<1, 2, MODE, OT, false, 1>(g, st, 1);
