@@ -152,8 +152,11 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
   }
   if (M <= STRIP_MAX_ROWS) {
     const StripPlan plan = strip_plan(M, N, K);
-    // (on large weights with a K of some length the tile kernel is slower than its model: not one of them lost)
-    if ((common + plan.us * (ragged ? 1.12 : 1.0)) * (N * K >= 30000000 && K >= 2560 ? 0.93 : 1.1) < least) best.row_tile = 0, best.strip = plan;
+    // (on large weights with a K of some length the tile kernel is slower than its model; not with K split, or half of the CUs, at more than 96 rows on
+    // weights that come from the Infinity Cache: 8192 x 8192 at 114 / 128 rows 25.4 / 26.0 us, 26.6 / 27.6 in strips,
+    // 12288 x 4096 at 128 rows 22.4 and 24.0)
+    const double margin = N * K < 30000000 || K < 2560 ? 1.1 : M > 96 && N * K < 75000000 && (plan.slices > 1 || ceil_div(N, plan.rows) * 2 < cus) ? 1.0 : 0.93;
+    if ((common + plan.us * (ragged ? 1.12 : 1.0)) * margin < least) best.row_tile = 0, best.strip = plan;
   }
   slot = Known{M, N, K, cus, best};
   return best;
