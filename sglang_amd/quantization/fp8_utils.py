@@ -24,7 +24,8 @@ def _finish(out_2d: torch.Tensor, input: torch.Tensor, bias, dtype: torch.dtype)
     """Add the bias in place and restore the activation's leading dimensions."""
     if bias is not None:
         out_2d += bias
-    out_2d = out_2d.to(dtype)
+    if out_2d.dtype != dtype:
+        out_2d = out_2d.to(dtype)
     return out_2d if input.dim() == 2 else out_2d.view(*input.shape[:-1], out_2d.shape[-1])
 
 
@@ -41,8 +42,9 @@ def _dynamic_block_quant_only(input_scale, block_size) -> None:
     before any work, with the exception a caller's fall-through catches."""
     if input_scale is not None:
         raise NotImplementedError("a static activation scale is not implemented for the block-FP8 linear")
-    if not all(b in (64, 128) for b in block_size):
-        raise NotImplementedError("scale blocks of 64 or 128 in each direction are implemented")
+    for b in block_size:
+        if b != 128 and b != 64:
+            raise NotImplementedError("scale blocks of 64 or 128 in each direction are implemented")
 
 
 def triton_w8a8_block_fp8_linear(input, weight, block_size: List[int], weight_scale, input_scale=None, bias=None):
@@ -108,7 +110,8 @@ def aiter_w8a8_block_fp8_linear(input, weight, block_size: List[int], weight_sca
     x_q = _rows(input)
     if input_scale.numel() != x_q.shape[0] * (-(-x_q.shape[1] // 128)):
         raise NotImplementedError("the input scale must hold one value per row and 128 columns")
-    input_scale = input_scale.view(x_q.shape[0], -1)
+    if input_scale.dim() != 2 or input_scale.shape[0] != x_q.shape[0]:  # (a view of the same shape is 0.7 us)
+        input_scale = input_scale.view(x_q.shape[0], -1)
     if eager(x_q):
         out = _C.block_matmul(x_q, weight, input_scale, weight_scale, torch.bfloat16, bias)
         if out is not None:
