@@ -20,7 +20,8 @@ def _codes(shape, int8, g):
 
 
 def _run(dev, mode, M, N, K, dtype, bias, pitch, col_scales):
-    """(output, reference); operands are views into rows of K + pitch bytes, the bytes past K NaN codes."""
+    """(output, reference); operands are views into rows of K + pitch bytes, the bytes past K NaN codes, and with a pitch the output
+    one into longer rows too."""
     from sglang_amd._lib import lib
 
     int8 = mode.endswith("int8")
@@ -37,7 +38,9 @@ def _run(dev, mode, M, N, K, dtype, bias, pitch, col_scales):
     bi = torch.randn(N, generator=g).to(dtype) if bias else None
     # through the C ABI, which takes any pitch and any N
     need = lib.sglamd_gemm_workspace_bytes(M, N, K)
-    scratch, out = torch.empty(max(need, 16), dtype=torch.uint8, device=dev), torch.empty(M, N, dtype=dtype, device=dev)
+    scratch, ldc = torch.empty(max(need, 16), dtype=torch.uint8, device=dev), N + (13 if pitch else 0)
+    rows = torch.full((M, ldc), 7.0, dtype=dtype, device=dev)
+    out = rows[:, :N]
     tag, stream = 2 if dtype == torch.bfloat16 else 1, torch.cuda.current_stream().cuda_stream
     if mode.startswith("block"):
         xs = (torch.rand(M, K // 128, generator=g) * 1e-2 + 1e-3)
@@ -47,15 +50,15 @@ def _run(dev, mode, M, N, K, dtype, bias, pitch, col_scales):
                       else (lib.sglamd_fp8_blockwise_scaled_mm, og.block_fp8_matmul))
         ws_d = ws.to(dev)
         rc = fn(ad.data_ptr(), ad.stride(0), bd.data_ptr(), bd.stride(0), xs_d.data_ptr(), xs_d.stride(0), xs_d.stride(1),
-                ws_d.data_ptr(), ws_d.stride(0), ws_d.stride(1), out.data_ptr(), N, tag, M, N, K, scratch.data_ptr(), need, stream)
-        assert rc == 0
+                ws_d.data_ptr(), ws_d.stride(0), ws_d.stride(1), out.data_ptr(), ldc, tag, M, N, K, scratch.data_ptr(), need, stream)
+        assert rc == 0 and bool((rows[:, N:] == 7.0).all())
         return out, ref_mm(an, bn, xs.numpy(), ws.numpy(), return_fp32=True)
     s_a, s_b = torch.rand(M, generator=g) * 1e-2 + 1e-3, torch.rand(N, generator=g) * 1e-2 + 1e-3
     fn, ref_mm = ((lib.sglamd_int8_scaled_mm, og.int8_scaled_mm) if int8 else (lib.sglamd_fp8_scaled_mm, og.fp8_scaled_mm))
     sa_d, sb_d, bi_d = s_a.to(dev), s_b.to(dev), None if bi is None else bi.to(dev)
     rc = fn(ad.data_ptr(), ad.stride(0), bd.data_ptr(), bd.stride(0), sa_d.data_ptr(), sb_d.data_ptr(), 0 if bi is None else bi_d.data_ptr(),
-            out.data_ptr(), N, tag, M, N, K, scratch.data_ptr(), need, stream)
-    assert rc == 0
+            out.data_ptr(), ldc, tag, M, N, K, scratch.data_ptr(), need, stream)
+    assert rc == 0 and bool((rows[:, N:] == 7.0).all())
     return out, ref_mm(an, bn, s_a.numpy(), s_b.numpy(), out_dtype=dtype, bias=bi).float()
 
 
