@@ -249,6 +249,15 @@ int sglamd_last_streaming_shape(void);
  * << 16) | weight rows per tile. */
 int sglamd_last_strip_shape(void);
 
+/* Diagnostic with no counterpart in the reference, host code: which form the launch heuristics give a dense GEMM whose
+ * operands have no gaps and that has the scratch it asks for.  plan[0..3]: activation rows per tile, weight rows per tile, K
+ * slices, K blocks in LDS (0 where the form has no such choice). */
+#define SGLAMD_PLAN_STREAMING 1 /* streaming kernel, all rows in one tile */
+#define SGLAMD_PLAN_ROW_TILES 2 /* ... in row tiles of plan[0] rows */
+#define SGLAMD_PLAN_STRIPS 3    /* strip kernel */
+#define SGLAMD_PLAN_TILES 4     /* tile kernel, or the generic one where that does not take the call */
+int sglamd_dense_plan(int block_scales, int64_t M, int64_t N, int64_t K, int32_t* plan);
+
 /* Diagnostic with no counterpart in the reference: the byte offset inside a row at which the streaming kernel's
  * lane chunk `lchunk` (0..7) fetches its 16 bytes of K block `kb`, written to *offset; returns 1 when that piece
  * lies past the end of K (it is then not used, and the offset names a piece inside the row).  Host code; lets a

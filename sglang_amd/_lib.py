@@ -40,6 +40,7 @@ SIGNATURES = {
     "sglamd_last_gemm_kernel": [],
     "sglamd_last_streaming_shape": [],
     "sglamd_last_strip_shape": [],
+    "sglamd_dense_plan": [_i, _i64, _i64, _i64, _p],
     "sglamd_moe_list_streams": [_i64, _i64, _i, _i64, _i64],
     "sglamd_streaming_piece_offset": [_i, _i, _i64, _p],
     "sglamd_ue8m0_unpack": [_p, _i64, _i64, _i64, _p, _i64, _i64, _p],

@@ -250,6 +250,14 @@ extern "C" int sglamd_last_gemm_kernel(void) { return last_kernel; }
 extern "C" int sglamd_last_streaming_shape(void) { return skinny_last_shape; }
 extern "C" int sglamd_last_strip_shape(void) { return strip_last_shape; }
 
+extern "C" int sglamd_dense_plan(int block_scales, int64_t M, int64_t N, int64_t K, int32_t* plan) {
+  const char* op = "dense_plan";
+  SGLAMD_REQUIRE(plan, SGLAMD_EINVAL, "%s: null pointer", op);
+  SGLAMD_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), SGLAMD_EINVAL, "%s: sizes out of range", op);
+  const DeviceScope scope;
+  return dense_plan(block_scales != 0, M, N, K, plan);
+}
+
 extern "C" int sglamd_streaming_piece_offset(int kb, int lchunk, int64_t K, int64_t* offset) {
   const SkinnyPiece pc = skinny_piece(kb, lchunk, (int)K);
   if (offset) *offset = pc.offset;

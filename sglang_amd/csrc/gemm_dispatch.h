@@ -162,6 +162,26 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+// The same for a test (sglamd_dense_plan): operands without gaps, 16-byte aligned scratch of the size that
+// sglamd_gemm_workspace_bytes reports.
+static inline int dense_plan(bool block, int64_t M, int64_t N, int64_t K, int32_t* plan) {
+  const DenseChoice choice = dense_choice(M, N, K);
+  plan[0] = plan[1] = plan[2] = plan[3] = 0;
+  if (choice.row_tile) {
+    plan[0] = choice.row_tile;
+    return SGLAMD_PLAN_ROW_TILES;
+  }
+  if (choice.strip.rows && (!block || strip_tables_hold(M, N, K, choice.strip))) {
+    plan[0] = (int32_t)((M + 31) / 32 * 32), plan[1] = choice.strip.rows, plan[2] = choice.strip.slices, plan[3] = strip_depth(M, choice.strip.rows);
+    return SGLAMD_PLAN_STRIPS;
+  }
+  if (M <= 64 && !small_m_uses_tile(M, N, K)) return SGLAMD_PLAN_STREAMING;
+  const int64_t nkb = K >> 7;
+  const BigConfig cfg = gemm8_big_config(M, N, K, block && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB);
+  plan[0] = cfg.bm, plan[1] = 256, plan[2] = cfg.slices;
+  return SGLAMD_PLAN_TILES;
+}
+
 // The row modes' tile kernel also takes a K that is not a multiple of 128, from 512 up: 8192 x 4112 at 100 / 300 / 1000 rows
 // 43 / 45 / 60 -> 21 / 32 / 46 us (4096: 20 / 23 / 39), 28672 x 4112 at 2048 rows 407 -> 281.  Shorter sums are a launch of
 // 12 to 17 us either way and stay with the generic kernel.
@@ -183,7 +203,7 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
       if (choice.row_tile == 16) return gemm8_skinny_launch<1, MODE, OT, false>(g, st, ceil_div(g.M, 16));
       return gemm8_skinny_launch<2, MODE, OT, false>(g, st, ceil_div(g.M, 32));
     }
-    if (plan.rows && strip_ok<MODE>(g) &&
+    if (plan.rows && strip_ok<MODE>(g, plan) &&
         (plan.slices == 1 || (workspace && ((uintptr_t)workspace & 15) == 0 && (int64_t)plan.slices * g.M * g.N * 4 <= workspace_bytes))) {
       // (the class of the shape: the kernels that this one stands in for)
       const bool wide = gemm8_skinny_wide<MODE, OT>(g, st, false) > 0;

@@ -35,7 +35,7 @@ template <int MODE, int RT, int NS>
 constexpr int strip_stage() {
   return NS * 4096 + RT * 4096 + (gemm_is_block(MODE) ? (RT + 1) / 2 * 256 : 0);
 }
-// the stages, a patch of 32 rows x 64 bytes per multiplying wave, two tables of three rows of weight scales
+// the stages, a patch of 32 rows x 64 bytes per multiplying wave, two tables of three rows of weight scales (see strip_tables_hold)
 template <int MODE, int RT, int NS>
 constexpr int strip_smem() {
   return strip_stages<RT, NS>() * strip_stage<MODE, RT, NS>() + NS * 2048 + (gemm_is_block(MODE) ? 2 * 3 * STRIP_MAX_KB * 4 : 0);
@@ -457,19 +457,34 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
 #endif
 }
 
-// What the kernel takes: 32-bit offsets, whole K blocks in the block modes.
-template <int MODE>
-static inline bool strip_ok(const GemmArgs& g) {
-  if (g.M < 17 || g.M > STRIP_MAX_ROWS || !gemm8_big_ok(g, !gemm_is_block(MODE))) return false;
-  if (!gemm_is_block(MODE)) return true;
-  const int64_t nkb = g.K >> 7;
-  return ((int64_t)(g.M - 1) * g.sa_sm + (nkb - 1) * g.sa_sk + 1) * 4 < 0x7ffffff0ll && ((nkb - 1) * g.sb_sk + 1) * 4 < 0x7ffffff0ll;
-}
-
 struct StripPlan {
   int rows = 0, slices = 1;  // weight rows of a tile, K slices
   double us = 1e30;
 };
+// Strips of 32 weight rows, and stages in LDS, of the kernel that runs tiles of `rows` weight rows.
+static inline int strip_strips(int64_t M, int rows) { return rows <= 96 && M <= 32 ? 3 : rows <= 128 ? 4 : 5; }
+static inline int strip_depth(int64_t M, int rows) {
+  const int ns = strip_strips(M, rows);
+  return M > 32 ? strip_stages<2, 4>() : ns == 3 ? strip_stages<1, 3>() : ns == 4 ? strip_stages<1, 4>() : strip_stages<1, 5>();
+}
+// The weight scales of the block modes lie in two tables, those of an item and of the one behind it.  The loading waves
+// write the table of item j + 2 over that of item j as soon as the request stream, as many blocks ahead of the products as
+// there are stages, enters it: item j's last block has passed its barrier by then if item j + 1 has at least stages - 1 blocks.
+// With fewer (17 x 790016 x 128: one block an item, five stages) a workgroup may only have two items.
+static inline bool strip_tables_hold(int64_t M, int64_t N, int64_t K, const StripPlan& plan) {
+  const int64_t items = ceil_div(N, plan.rows) * plan.slices;
+  return items <= 2 * (int64_t)device_cus() || (K >> 7) / plan.slices >= strip_depth(M, plan.rows) - 1;
+}
+// What the kernel takes: 32-bit offsets, whole K blocks in the block modes and enough of them for the scale tables.
+template <int MODE>
+static inline bool strip_ok(const GemmArgs& g, const StripPlan& plan) {
+  if (g.M < 17 || g.M > STRIP_MAX_ROWS || !gemm8_big_ok(g, !gemm_is_block(MODE))) return false;
+  if (!gemm_is_block(MODE)) return true;
+  const int64_t nkb = g.K >> 7;
+  return strip_tables_hold(g.M, g.N, g.K, plan) && ((int64_t)(g.M - 1) * g.sa_sm + (nkb - 1) * g.sa_sk + 1) * 4 < 0x7ffffff0ll &&
+         ((nkb - 1) * g.sb_sk + 1) * 4 < 0x7ffffff0ll;
+}
+
 // The tile and the number of K slices of a launch, and its time in us without what all forms have in common (launch, quantiser):
 // rounds of items x (K blocks of an item x the time of a block + its drain), and a second launch where K is split.  A
 // block takes the longer of the multiplying wave's chain and the bytes' way in, and half of the other.  Fitted to 4752 launches
@@ -525,8 +540,9 @@ static int gemm8_strip_launch(const GemmArgs& whole, const StripPlan& plan, hipS
     if constexpr (NS == 3) return gemm8_strip_start<MODE, OT, 2, 4>(g, st);
     else return g.M <= 64 ? gemm8_strip_start<MODE, OT, 2, NS>(g, st) : g.M <= 96 ? gemm8_strip_start<MODE, OT, 3, NS>(g, st) : gemm8_strip_start<MODE, OT, 4, NS>(g, st);
   };
-  if (plan.rows <= 96 && g.M <= 32) rc = start(std::integral_constant<int, 3>{});
-  else if (plan.rows <= 128) rc = start(std::integral_constant<int, 4>{});
+  const int ns = strip_strips(g.M, plan.rows);
+  if (ns == 3) rc = start(std::integral_constant<int, 3>{});
+  else if (ns == 4) rc = start(std::integral_constant<int, 4>{});
   else rc = start(std::integral_constant<int, 5>{});
   if (rc || plan.slices == 1) return rc;
   return splitk_reduce<MODE, OT>(whole, plan.slices, workspace, st);

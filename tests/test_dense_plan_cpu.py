@@ -1,0 +1,78 @@
+"""What the launch heuristics of the dense GEMMs choose, as far as it decides whether a launch is right: host code, no GPU."""
+import ctypes
+
+import pytest
+
+from sglang_amd import _lib
+
+STREAMING, ROW_TILES, STRIPS, TILES = 1, 2, 3, 4  # SGLAMD_PLAN_* of include/sglamd.h
+CUS = 256  # what the library takes without a GPU
+
+
+def _plan(M, N, K, block=True):
+    plan = (ctypes.c_int32 * 4)()
+    form = _lib.lib.sglamd_dense_plan(int(block), M, N, K, plan)
+    assert form in (STREAMING, ROW_TILES, STRIPS, TILES)
+    return form, list(plan)
+
+
+def _wrong_scales(blocks, depth):
+    """The strip kernel's order of requests, barriers and reads of one workgroup: how many blocks of its items (of blocks[j] K
+    blocks each) read a weight-scale table that another item's request has been written over or may be."""
+    stream = [(j, k) for j, n in enumerate(blocks) for k in range(n)]
+    table, wrong, at = [None, None], 0, 0
+
+    def request():
+        nonlocal at
+        if at < len(stream):
+            item, k = stream[at]
+            if k == 0:
+                table[item & 1] = item
+            at += 1
+
+    for _ in range(depth):
+        request()
+    # block 0's scales are read behind the first barrier, before anything else is requested
+    wrong += table[0] != 0
+    for b in range(len(stream)):
+        # behind block b's barrier the loading waves request one block, the others read block b + 1's scales, in either order
+        item = stream[b + 1][0] if b + 1 < len(stream) else None
+        before = item is not None and table[item & 1] != item
+        request()
+        wrong += item is not None and (before or table[item & 1] != item)
+    return wrong
+
+
+def test_model_of_the_scale_tables():
+    assert _wrong_scales([1] * 12, 5) == 10 and _wrong_scales([2] * 12, 5) > 0 and _wrong_scales([3] * 12, 5) > 0
+    for depth in (3, 5, 6, 8):
+        assert _wrong_scales([depth - 1] * 12, depth) == 0 and _wrong_scales([depth - 2] * 12, depth) > 0
+        assert _wrong_scales([1, 1], depth) == 0
+
+
+@pytest.mark.parametrize("K", [128, 256, 384, 512, 640, 768, 896, 1024, 2048])
+def test_strips_keep_the_scales_of_every_item(K):
+    """Few K blocks and many weight rows: no workgroup of a strip launch asks for an item's scales while the item two before
+    still needs the place."""
+    strips = 0
+    for M in (17, 24, 32, 33, 64, 65, 96, 97, 128):
+        for N in [1 << p for p in range(12, 22)] + [3 << p for p in range(11, 20)] + [261376, 398592, 790016, 791808, 200008]:
+            if N * K >= 2**31:
+                continue
+            form, (_, cols, slices, depth) = _plan(M, N, K)
+            if form != STRIPS:
+                continue
+            strips += 1
+            items, nkb = -(-N // cols) * slices, K // 128
+            mine = range(0, items, CUS)  # of the workgroup with the most of them
+            blocks = [nkb * (i * slices // items + 1) // slices - nkb * (i * slices // items) // slices for i in mine]
+            if len(blocks) > 12:
+                blocks = blocks[:12]
+            assert _wrong_scales(blocks, depth) == 0, f"M={M} N={N} K={K}: {blocks} K blocks, {depth} stages"
+    assert strips or K < 512
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 791808, 128), (24, 398592, 256), (32, 261376, 384)])
+def test_too_few_k_blocks_for_strips(M, N, K):
+    assert _plan(M, N, K)[0] == STREAMING
+    assert _plan(M, N, K, block=False)[0] == STRIPS  # the row modes have no such tables

@@ -100,6 +100,30 @@ def test_strip_kernel(dev, mode, M, N, K, pitch):
     _check(out, ref, f"strip {mode} M={M} N={N} K={K}")
 
 
+# the shortest K of each depth with three and more tiles a workgroup, where the weight scales of a tile are requested while the
+# one before is multiplied; a block less, and block scales stay with the streaming kernel
+@pytest.mark.parametrize("mode", ["block_fp8", "block_int8"])
+@pytest.mark.parametrize("M,N,K,strips", [
+    (17, 195416, 512, True),    # five stages
+    (23, 209576, 512, True),
+    (31, 127568, 896, True),    # six
+    (33, 200008, 512, True),    # three
+    (80, 200008, 512, True),
+    (100, 200008, 768, True),
+    (32, 261376, 384, False),
+    (17, 398592, 256, False),
+    (24, 790016, 128, False),
+])
+def test_few_k_blocks_and_many_tiles(dev, mode, M, N, K, strips):
+    from sglang_amd._lib import lib
+
+    print(f"short K {mode} M={M} N={N} K={K}", flush=True)
+    out, ref = _run(dev, mode, M, N, K, torch.bfloat16, False, 0, col_scales=True)
+    shape = lib.sglamd_last_strip_shape()
+    assert (shape != 0) == strips and (not strips or -(-N // (shape & 0xFFFF)) > 512), f"{shape:#x}"
+    _check(out, ref, f"short K {mode} M={M} N={N} K={K}")
+
+
 @pytest.mark.parametrize("mode", ["row_fp8", "row_int8"])
 @pytest.mark.parametrize("M,N,K", [(65, 28681, 4096), (100, 9000, 9600)])
 def test_strip_kernel_half_and_bias(dev, mode, M, N, K):
