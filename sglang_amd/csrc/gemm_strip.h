@@ -284,7 +284,8 @@ __global__ __launch_bounds__(512) void gemm8_strip_kernel(GemmArgs g) {
         sc = sa[0] * sbv;
         sc1 = sa[0] * sbv1;
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("" : : : "memory");
+        // (as below: the products, which the compiler may put behind the barrier, do not wait for the fragments in front of it)
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" : : : "memory");
         __builtin_amdgcn_sched_barrier(0);

@@ -72,3 +72,45 @@ def test_last_build_left_no_gemm_kernel_in_scratch():
         for line in lines:
             name, vgprs, agprs, sgprs, scratch, waves = line.split()
             assert int(scratch) == 0, f"{name} uses {scratch} bytes of scratch per lane"
+
+
+def test_strip_kernels_hold_their_fragments_before_they_free_the_stage(tmp_path):
+    """The barrier of a K block hands its place in LDS to the loading waves: every LDS read in front of it must have returned,
+    which is an s_waitcnt lgkmcnt(0) between the last of them and the barrier, in the order of the code."""
+    import re
+    import shutil
+    import subprocess
+
+    import pytest
+
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    built = os.path.join(ROOT, "sglang_amd", "libsglamd.so")
+    if not (os.path.exists(objdump) and os.path.exists(built)):
+        pytest.skip("no built library, or no disassembler")
+    lib = tmp_path / "libsglamd.so"
+    shutil.copy(built, lib)
+
+    def run(*args):
+        return subprocess.run([objdump, *args], capture_output=True, text=True, check=True, cwd=tmp_path).stdout
+
+    run("--offloading", str(lib))
+    kernels = 0
+    for code in sorted(tmp_path.glob("*gfx950*")):
+        names = sorted(set(re.findall(r"\b(\S*gemm8_strip_kernel\S*E)$", run("-t", str(code)), flags=re.M)))
+        if not names:
+            continue
+        kernel, reading, barriers = None, False, 0
+        for line in run("-d", "--no-show-raw-insn", "--disassemble-symbols=" + ",".join(names), str(code)).splitlines():
+            start = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+            if start:
+                kernel, reading, kernels = start.group(1), False, kernels + 1
+            op = line.split("//")[0].strip()
+            if op.startswith("ds_read"):
+                reading = True
+            elif op.startswith("s_waitcnt") and "lgkmcnt(0)" in op or op.startswith("s_endpgm"):
+                reading = False
+            elif op == "s_barrier":
+                barriers += 1
+                assert not reading, f"{kernel}: LDS reads in flight at a barrier"
+        assert barriers >= 2 * len(names)
+    assert kernels > 0
