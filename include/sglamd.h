@@ -231,18 +231,18 @@ int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /* Which kernel the last dense GEMM call (the four entry points above) of the calling thread launched; 0 before
  * the first call.  Diagnostic with no counterpart in the reference: the kernel is chosen from the shape by launch
  * heuristics, and a parity test uses this to assert that it covers the kernel it was written for. */
-#define SGLAMD_KERNEL_STREAMING 1     /* weight-streaming kernel (M <= 32, on small weights up to 1024 rows in row tiles), or strip kernel at 17..32 rows */
-#define SGLAMD_KERNEL_TILE64 2        /* 64-row tiles: tile kernel, or strip kernel (sglamd_last_strip_shape) */
-#define SGLAMD_KERNEL_TILE128 3       /* 128-row tiles: tile kernel, or strip kernel */
+#define SGLAMD_KERNEL_STREAMING 1     /* weight-streaming kernel (M <= 32, on small weights up to 1024 rows in row tiles) */
+#define SGLAMD_KERNEL_TILE64 2        /* tile kernel, 64-row tiles */
+#define SGLAMD_KERNEL_TILE128 3       /* tile kernel, 128-row tiles */
 #define SGLAMD_KERNEL_TILE256 4       /* tile kernel, 256-row tiles, one tile per workgroup */
 #define SGLAMD_KERNEL_PERSISTENT256 5 /* 256x256 tiles, one workgroup per CU walking several tiles */
 #define SGLAMD_KERNEL_GENERIC 6       /* register-staged fallback (operands of 2 GiB and more; K % 128 != 0 in block modes or below 512) */
 #define SGLAMD_KERNEL_PERSISTENT256_POW2 7 /* the persistent kernel applying power-of-two scales inside the MFMA */
-#define SGLAMD_KERNEL_STREAMING_WIDE 8  /* 33..64 rows, wide weights, long K: strip kernel, or (K split wanted and no workspace) the
-                                           weight-streaming kernel with 96..144 weight rows per workgroup */
-#define SGLAMD_KERNEL_TILE192 9       /* 192-row tiles of the tile kernel */
+#define SGLAMD_KERNEL_STREAMING_WIDE 8  /* weight-streaming kernel, 33..64 rows x 96..144 weight rows per workgroup */
+#define SGLAMD_KERNEL_TILE192 9       /* tile kernel, 192-row tiles */
+#define SGLAMD_KERNEL_STRIP 10        /* strip kernel (sglamd_last_strip_shape) */
 int sglamd_last_gemm_kernel(void);
-/* The same for the streaming kernel's shape: (FM << 16) | (FN << 8) | KW of the last dense launch of it on this thread
+/* The streaming kernel's shape, 0 when the last dense GEMM call of this thread did not run it: (FM << 16) | (FN << 8) | KW
  * -- FM 16-row activation tiles, FN 16-row weight tiles per workgroup, KW waves sharing a tile's K range. */
 int sglamd_last_streaming_shape(void);
 /* The strip kernel's shape, 0 when the last dense GEMM call of this thread did not run it: (32-row tiles << 24) | (K slices

@@ -55,8 +55,7 @@ static int persist_workgroups() {
 
 // Which kernel the last dense GEMM call of this thread launched (SGLAMD_KERNEL_* of the header): lets a test
 // assert that it exercises the kernel it was written for, whatever the launch heuristics choose.
-extern thread_local int last_kernel;  // defined in gemm.hip
-extern thread_local int strip_last_shape;
+extern thread_local int last_kernel, strip_last_shape;  // defined in gemm.hip
 #define RAN(code) (last_kernel = (code))
 
 // A launch of 256x256 tiles whose last round of one tile per CU is mostly empty is cut in two along N: the
@@ -165,7 +164,7 @@ static DenseChoice dense_choice(int64_t M, int64_t N, int64_t K) {
 // The same for a test (sglamd_dense_plan): operands without gaps, 16-byte aligned scratch of the size that
 // sglamd_gemm_workspace_bytes reports.
 static inline int dense_plan(bool block, int64_t M, int64_t N, int64_t K, int32_t* plan) {
-  const DenseChoice choice = dense_choice(M, N, K);
+  const DenseChoice choice = block && (K & 127) ? DenseChoice() : dense_choice(M, N, K);
   plan[0] = plan[1] = plan[2] = plan[3] = 0;
   if (choice.row_tile) {
     plan[0] = choice.row_tile;
@@ -194,7 +193,7 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
   const int nkb = g.K >> 7;
   const bool persistent = wgs > 0 && (wgs & 7) == 0 && !(nkb & 1) && nkb >= 4 && nkb <= GEMM8_PERSIST_USE_MAX_KB;
   const int tiles_256 = persistent ? (MODE == GEMM_BLOCK_FP8 && g.scales_pow2 ? 2 : 1) : 0;
-  strip_last_shape = 0;
+  strip_last_shape = skinny_last_shape = 0;
   if (big && may_split && g.M > 16) {
     const DenseChoice choice = dense_choice(g.M, g.N, g.K);
     const StripPlan& plan = choice.strip;
@@ -205,9 +204,7 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
     }
     if (plan.rows && strip_ok<MODE>(g, plan) &&
         (plan.slices == 1 || (workspace && ((uintptr_t)workspace & 15) == 0 && (int64_t)plan.slices * g.M * g.N * 4 <= workspace_bytes))) {
-      // (the class of the shape: the kernels that this one stands in for)
-      const bool wide = gemm8_skinny_wide<MODE, OT>(g, st, false) > 0;
-      RAN(g.M <= 32 ? SGLAMD_KERNEL_STREAMING : g.M > 64 ? SGLAMD_KERNEL_TILE128 : wide ? SGLAMD_KERNEL_STREAMING_WIDE : SGLAMD_KERNEL_TILE64);
+      RAN(SGLAMD_KERNEL_STRIP);
       strip_last_shape = ((g.M + 31) / 32 << 24) | (plan.slices << 16) | plan.rows;
       return gemm8_strip_launch<MODE, OT>(g, plan, st, workspace);
     }
@@ -276,7 +273,10 @@ static int dispatch_dense(const GemmArgs& g, hipStream_t st, void* workspace, in
 // An FP8 linear layer of a few rows in one launch (gemm8_skinny_quantising).
 template <int MODE, bool BIASED>
 int dispatch_quantising(const GemmArgs& g, int out_dtype, hipStream_t st, bool launch) {
-  if (launch) RAN(SGLAMD_KERNEL_STREAMING);
+  if (launch) {
+    RAN(SGLAMD_KERNEL_STREAMING);
+    strip_last_shape = 0;
+  }
   if constexpr (BIASED)
     return out_dtype == SGLAMD_BF16 ? gemm8_skinny_quantising<MODE, Biased<BF16>>(g, st, launch)
                                     : gemm8_skinny_quantising<MODE, Biased<F16>>(g, st, launch);

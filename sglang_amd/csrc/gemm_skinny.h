@@ -931,7 +931,7 @@ static inline int skinny_pick_kw(int64_t tiles, int nkb, int extra_bytes = 0) {
   return best;
 }
 
-// Shape of the last streaming launch of this thread and translation unit: (FM << 16) | (FN << 8) | KW.
+// Shape of this thread's last dense GEMM call, if that is a streaming launch: (FM << 16) | (FN << 8) | KW.
 extern thread_local int skinny_last_shape;  // defined in gemm.hip
 
 // AQ: `g` carries the 16-bit source rows in A16 / lda16 (act_mode 1) and the quantisation constants.  MoE: every sorted block
@@ -944,7 +944,7 @@ static int gemm8_skinny_launch_fn(const GemmArgs& g, hipStream_t st, int64_t exp
   // to the four waves it supports): the same partial sums in the same order, so both give the same bits.
   int kw = skinny_pick_kw<FM, FN>(tiles, (g.K + 127) >> 7);
   if (AQ > 0 && MOE && kw > 4) kw = 4;
-  skinny_last_shape = (FM << 16) | (FN << 8) | kw;
+  if (!MOE) skinny_last_shape = (FM << 16) | (FN << 8) | kw;
   switch (kw) {
     case 1:
       return gemm8_skinny_launch_kw<FM, FN, MODE, OT, MOE, 1, AQ>(g, st);

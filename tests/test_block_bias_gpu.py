@@ -5,17 +5,20 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-STREAMING, TILE64, TILE128, TILE256, PERSISTENT256, POW2, WIDE = 1, 2, 3, 4, 5, 7, 8  # SGLAMD_KERNEL_* of include/sglamd.h
+STREAMING, TILE64, TILE128, TILE256, PERSISTENT256, POW2, TILE192, STRIP = 1, 2, 3, 4, 5, 7, 9, 10  # SGLAMD_KERNEL_* of include/sglamd.h
 
 
 @pytest.mark.parametrize("M,N,K,kernel", [
     (1, 1000, 1024, STREAMING),
     (24, 776, 2048, STREAMING),
     (40, 512, 1024, STREAMING),
-    (40, 512, 7168, TILE64),            # K split: the bias in the reduction
+    (40, 512, 12288, TILE64),           # K split: the bias in the reduction
+    (40, 512, 7168, STRIP),             # ... of strips
     (48, 24640, 512, TILE64),           # ragged last column tile
-    (40, 36864, 5120, WIDE),
+    (40, 36864, 5120, STRIP),
+    (24, 40000, 2560, STRIP),           # one row tile
     (128, 33026, 512, TILE128),         # N not a multiple of 4
+    (300, 24577, 1280, TILE192),        # N odd
     (1000, 14340, 512, TILE256),
     (512, 36864, 512, TILE256),         # cut in two along N
     (2500, 8392, 512, PERSISTENT256),   # last column tile of 200: a patch that starts inside the last 32 columns

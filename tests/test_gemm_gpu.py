@@ -76,14 +76,15 @@ def _pack_ue8m0(exps: torch.Tensor) -> torch.Tensor:
 
 
 @pytest.mark.parametrize("M,N,K,kernel", [(768, 33280, 1024, 7), (520, 33024, 512, 7), (2304, 10240, 768, 7),
-                                          (1024, 33280, 16640, 7), (64, 36864, 512, 2), (40, 512, 7168, 2),
-                                          (128, 33024, 512, 3), (128, 7168, 18432, 3), (1000, 14336, 512, 4),
+                                          (1024, 33280, 16640, 7), (64, 36864, 512, 2), (40, 512, 12288, 2),
+                                          (128, 33024, 512, 3), (130, 7424, 5632, 3), (1000, 14336, 512, 4),
+                                          (40, 512, 7168, 10), (128, 7168, 18432, 10), (300, 24577, 1280, 9),
                                           (1024, 36864, 512, 7)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
 def test_block_gemm_with_packed_power_of_two_scales(sa, dev, M, N, K, kernel, out_dtype):
     """Packed UE8M0 scales on both operands: the persistent kernel (code 7; the last shape is cut in two along N)
     hands their exponent bytes to the MFMA instead of multiplying every partial product; launches that take the
-    one-tile-per-workgroup kernels (codes 2-4, with and without split K) use the expanded scales as floats.  Exponents differ per row and K block (activations, 2^-14..2^-5) and per
+    one-tile-per-workgroup kernels (codes 2-4 and 9, with and without split K) or strips (10) use the expanded scales as floats.  Exponents differ per row and K block (activations, 2^-14..2^-5) and per
     128x128 block (weights), so a scale applied to the wrong row, block or operand shows; the oracle gets the
     powers of two as fp32.  The result must also agree with the same launch through the fp32-scale entry, which
     runs the multiply-add form of the kernel."""
@@ -489,23 +490,32 @@ def test_streaming_kernel_with_two_row_tiles_and_three_or_four_column_tiles(sa, 
 
 
 # kernel codes of include/sglamd.h
-_STREAMING, _TILE64, _TILE128, _TILE256, _PERSISTENT256, _GENERIC, _WIDE = 1, 2, 3, 4, 5, 6, 8
+_STREAMING, _TILE64, _TILE128, _TILE256, _PERSISTENT256, _GENERIC, _WIDE, _TILE192, _STRIP = 1, 2, 3, 4, 5, 6, 8, 9, 10
 
 
 @pytest.mark.parametrize("M,N,K,kernel", [
     (9, 512, 1024, _STREAMING),
     (40, 512, 1024, _STREAMING),       # up to 64 rows and a small weight: the streaming kernel's 64-row form
     (24, 768, 2048, _STREAMING),       # ... and its 32-row form
-    (40, 8192, 1024, _TILE64),         # one row of 64-row tiles, K not split (8 K blocks)
-    (40, 512, 7168, _TILE64),          # the same with K split over the workgroups
+    (40, 9216, 1024, _TILE64),         # one row of 64-row tiles, K not split (8 K blocks)
+    (40, 512, 12288, _TILE64),         # the same with K split over the workgroups
     (24, 24576, 512, _STREAMING),      # up to 32 rows: the streaming kernel whatever the weight
     (48, 24576, 512, _TILE64),         # 33..64 rows go to the tile kernel once about a hundred workgroups come together
-    (40, 36864, 5120, _WIDE),          # 33..64 rows, many weight rows, long K: 256 workgroups of 144 weight rows (nine column tiles)
-    (64, 24576, 5248, _WIDE),          # ... of 96 weight rows (six column tiles)
-    (50, 32768, 5632, _WIDE),          # ... of 128 weight rows (eight column tiles)
-    (33, 30016, 5184, _WIDE),          # ... trimmed rows per workgroup, ragged last workgroup, ragged last K block
+    (40, 8192, 1024, _STRIP),          # 33..128 rows on weights from a few MB: strips, too few for the chip
+    (40, 512, 7168, _STRIP),           # ... with K split 12 ways
+    (40, 36864, 5120, _STRIP),         # ... many weight rows: 256 workgroups of 144
+    (64, 24576, 5248, _STRIP),         # ... of 96
+    (50, 32768, 5632, _STRIP),         # ... of 128
+    # a K that does not fill its last block, which the strips take in the row modes alone: with block scales the streaming
+    # kernel's wide form, four row tiles and
+    (33, 30016, 5184, _WIDE),          # ... trimmed rows per workgroup, ragged last workgroup
+    (40, 36864, 5200, _WIDE),          # ... 256 workgroups of 144 weight rows (nine column tiles)
+    (64, 24576, 5328, _WIDE),          # ... of 96 (six)
+    (50, 32768, 5712, _WIDE),          # ... of 128 (eight)
     (128, 33024, 512, _TILE128),       # 129 column tiles: 64-row tiles would need a second round
-    (128, 7168, 18432, _TILE128),      # few column tiles, long K: 128-row tiles with K split 9 ways
+    (130, 7424, 5632, _TILE128),       # few column tiles, long K: 128-row tiles with K split 4 ways
+    (128, 7168, 18432, _STRIP),        # ... up to 128 rows strips, K split
+    (300, 24584, 1280, _TILE192),      # 192-row tiles, last column tile of eight columns
     (1000, 14336, 512, _TILE256),      # 224 tiles of 256 rows in one round, last row tile ragged
     (100, 520, 400, _GENERIC),         # K not a multiple of 128
 ])
@@ -546,6 +556,8 @@ def test_every_dense_kernel_in_every_mode(sa, dev, M, N, K, kernel, mode):
             ref = og.int8_scaled_mm(aq, bq, xs, ws, out_dtype=torch.bfloat16).float()
             out = sa.int8_scaled_mm(a_d, b_d.t(), torch.from_numpy(xs).to(dev).view(M, 1),
                                     torch.from_numpy(ws).to(dev).view(N, 1), torch.bfloat16, None)
+    if kernel == _WIDE and mode.startswith("row"):
+        kernel = _STRIP
     assert lib.sglamd_last_gemm_kernel() == kernel, f"ran kernel {lib.sglamd_last_gemm_kernel()}, meant for {kernel}"
     assert_gemm_close(out, ref, f"{mode} M={M} N={N} K={K}")
     o, r = out.float().cpu(), torch.as_tensor(ref).float()

@@ -14,12 +14,12 @@ GENERIC, TILES = 6, (2, 3, 4)  # SGLAMD_KERNEL_* of include/sglamd.h
 @pytest.mark.parametrize("int8", [False, True])
 @pytest.mark.parametrize("M,N,K", [
     (65, 264, 528),       # one piece in the last block, ragged column tile
-    (100, 8192, 4208),    # seven pieces, 64- or 128-row tiles in one slice
+    (100, 33024, 752),    # seven pieces, 128-row tiles in one slice
     (130, 520, 4112),     # K split over workgroups, the last slice ends in one piece
     (300, 1000, 2096),    # split, ragged rows
     (1000, 14336, 592),   # 256-row tiles
     (40, 20480, 1040),    # 33..64 rows
-    (64, 12288, 4208),    # ... K split
+    (200, 520, 4208),     # K split, seven pieces in the last slice
     (100, 520, 400),      # short K stays with the generic kernel
 ])
 def test_ragged_k(dev, int8, M, N, K):

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("int8", [False, True])
-@pytest.mark.parametrize("M,N,K", [(65, 264, 4096), (130, 512, 8192), (300, 1000, 4096)])
+@pytest.mark.parametrize("M,N,K", [(65, 264, 4096), (130, 512, 16384), (300, 1000, 4096)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_alignment_of_scales_and_bias(dev, int8, M, N, K, bias):
     import sglang_amd as sa

@@ -95,7 +95,8 @@ def test_strip_kernel(dev, mode, M, N, K, pitch):
     print(f"strip {mode} M={M} N={N} K={K} pitch +{pitch}", flush=True)
     out, ref = _run(dev, mode, M, N, K, torch.bfloat16, False, pitch, col_scales=M % 2 == 0)
     shape = lib.sglamd_last_strip_shape()
-    assert shape >> 24 == -(-M // 32), f"not the strip kernel: {shape:#x}"
+    assert shape >> 24 == -(-M // 32) and lib.sglamd_last_gemm_kernel() == 10, f"not the strip kernel: {shape:#x}"
+    assert lib.sglamd_last_streaming_shape() == 0
     assert (shape >> 16 & 0xFF) > 1 or N > 10000, "meant to split K"
     _check(out, ref, f"strip {mode} M={M} N={N} K={K}")
 
