@@ -790,11 +790,17 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, int pe
   double best_cost = 1e30;
   const int cus = device_cus();
   const double nkb = (double)(K >> 7);
+  const int64_t whole = (M + 255) / 256 * ((N + 255) / 256);
+  // 192 rows?  (see below)
+  const bool tall = K >= (persistent_256 > 1 && whole > cus ? 4096 : 1152) &&
+                    !(persistent_256 && whole > cus && (N * K > 500000000 || ((N & 255) == 0 && K >= 4096 && whole < 2 * cus && (whole - cus) * 8 <= cus * 3)));
   for (int bm = 64; bm <= 256; bm += 64) {
     if (bm > 128 && M <= 128) break;
+    if (bm == 192 && !tall) continue;
     // up to 192 rows one of the two: gate_up at 150 rows 79 us in 192-row tiles, 86 in 256-row tiles, 7168 x 18432 52.7 and 53.4, but 8192 x
-    // 28672 79.4 and 76.5
-    if (M <= 192 && bm == (K < 20480 ? 256 : 192)) continue;
+    // 28672 79.4 and 76.5.  A K too short for 192 rows: 256-row tiles unless 128-row tiles fit one round (192 x 65536 x 1024 in 256-, 128-row
+    // tiles 24.7, 32.0 us, 160 x 57344 x 896 21.0, 24.8, 150 x 33792 x 640 15.3, in 64-row tiles 16.0; 140 x 30720 x 640 15.1, 13.2)
+    if (M <= 192 && (tall ? bm == (K < 20480 ? 256 : 192) : bm == 256 && 2 * whole <= cus)) continue;
     const int64_t tiles = ((M + bm - 1) / bm) * ((N + 255) / 256);
     // 192 rows, between the heights that leave many rows or CUs idle: 8192 x 28672 at 560 / 640 rows 198 / 219 -> 159 / 158 us, 7168 x
     // 18432 at 560 rows 122 -> 99, gate_up at 560 rows 196 -> 165, 57344 x 8192 at 380 rows 208 -> 180, 7168 x 18432 at 3100 / 3400 rows,
@@ -805,11 +811,6 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, int pe
     //   * what the persistent kernel and the launch behind it (column_split) take between one round and one and three eighths of (7168 x
     //     18432 at 2400 / 2765 / 3023 rows 334 / 347 / 376 us, 363 / 367 / 380 in 192-row tiles);
     //   * weights past the 470 MB that were measured.
-    if (bm == 192) {
-      const int64_t whole = (M + 255) / 256 * ((N + 255) / 256);
-      if (K < (persistent_256 > 1 && whole > cus ? 4096 : 1152)) continue;
-      if (persistent_256 && whole > cus && (N * K > 500000000 || ((N & 255) == 0 && K >= 4096 && whole < 2 * cus && (whole - cus) * 8 <= cus * 3))) continue;
-    }
     const int slices = gemm8_big_slices(tiles, N, K);
     const int64_t rounds = (tiles * slices + cus - 1) / cus;
     // (64-row tiles in several rounds read each weight byte once per row tile from further away: gate_up at M = 400, four rounds of

@@ -76,3 +76,22 @@ def test_strips_keep_the_scales_of_every_item(K):
 def test_too_few_k_blocks_for_strips(M, N, K):
     assert _plan(M, N, K)[0] == STREAMING
     assert _plan(M, N, K, block=False)[0] == STRIPS  # the row modes have no such tables
+
+
+@pytest.mark.parametrize("M,N,K,rows", [
+    # K too short for 192-row tiles: the fastest height measured (us in 64-, 128-, 256-row tiles)
+    (150, 33792, 640, 256),    # 16.0, -, 15.3
+    (150, 33792, 1024, 256),   # 19.2, -, 18.4
+    (192, 36864, 1024, 256),   # 20.1, -, 19.3
+    (131, 49152, 512, 256),    # -, 18.5, 15.1
+    (160, 57344, 896, 256),    # -, 24.8, 21.0
+    (192, 65536, 1024, 256),   # -, 32.0, 24.7
+    (140, 30720, 640, 128),    # -, 13.2, 15.1
+    (192, 31744, 1024, 128),   # -, 16.6, 18.9
+    (150, 36864, 7168, 192),
+    (150, 8192, 28672, 256),
+])
+@pytest.mark.parametrize("block", [False, True])
+def test_tile_heights_at_129_to_192_rows(M, N, K, rows, block):
+    form, plan = _plan(M, N, K, block)
+    assert form == TILES and plan[0] == rows
