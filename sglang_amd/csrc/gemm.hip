@@ -268,12 +268,12 @@ extern "C" int sglamd_streaming_piece_offset(int kb, int lchunk, int64_t K, int6
 extern "C" int64_t sglamd_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M >= (1ll << 31) || N <= 0 || K <= 0) return 0;
   const DeviceScope scope;
-  const StripPlan strip = dense_choice(M, N, K).strip;
-  const int64_t strip_need = strip.rows && strip.slices > 1 ? (int64_t)strip.slices * M * N * 4 : 0;
-  if (M <= 64 && !small_m_uses_tile(M, N, K)) return strip_need;
+  const DenseChoice choice = dense_choice(M, N, K);
+  if (choice.row_tile) return 0;
+  if (choice.strip.rows) return choice.strip.slices > 1 ? (int64_t)choice.strip.slices * M * N * 4 : 0;
+  if (M <= 64 && !small_m_uses_tile(M, N, K)) return 0;
   const BigConfig cfg = gemm8_big_config(M, N, K);
   int64_t need = cfg.slices > 1 ? (int64_t)cfg.slices * M * N * 4 : 0;
-  if (strip_need > need) need = strip_need;
   // a launch of 256-row tiles cut in two along N (column_split) splits K on its second part; whether the launch
   // uses 256-row tiles depends on the operand mode, so the larger of the two needs is reported
   const int64_t n1 = M > 64 ? column_split(M, N, K) : 0;

@@ -78,6 +78,23 @@ def test_too_few_k_blocks_for_strips(M, N, K):
     assert _plan(M, N, K, block=False)[0] == STRIPS  # the row modes have no such tables
 
 
+def test_scratch_is_asked_for_where_it_is_used():
+    """Slabs for the K slices that the launch has, and none for one that does not split K.  (Row modes; a tile launch that is cut in
+    two along N splits K on its second part alone.)"""
+    seen = set()
+    for M in (1, 16, 17, 32, 40, 64, 65, 96, 128, 129, 200, 320, 700, 1024, 1500):
+        for N in (256, 512, 1000, 1152, 2048, 2050, 4096, 7168, 9000, 14336, 24576, 36864):
+            for K in (512, 1024, 1664, 2048, 4096, 7168, 8192, 16384):
+                form, (_, _, slices, _) = _plan(M, N, K, block=False)
+                need = _lib.lib.sglamd_gemm_workspace_bytes(M, N, K)
+                split = form in (STRIPS, TILES) and slices > 1
+                seen.add((form, split))
+                if form == TILES and not split and N > 256 * CUS // -(-M // 256):
+                    continue  # (may be cut in two)
+                assert need == (slices * M * N * 4 if split else 0), f"M={M} N={N} K={K}: form {form}, {slices} slices, {need} bytes"
+    assert seen == {(STREAMING, False), (ROW_TILES, False), (STRIPS, False), (STRIPS, True), (TILES, False), (TILES, True)}
+
+
 @pytest.mark.parametrize("M,N,K,rows", [
     # K too short for 192-row tiles: the fastest height measured (us in 64-, 128-, 256-row tiles)
     (150, 33792, 640, 256),    # 16.0, -, 15.3
