@@ -110,7 +110,8 @@ def aiter_w8a8_block_fp8_linear(input, weight, block_size: List[int], weight_sca
     x_q = _rows(input)
     if input_scale.numel() != x_q.shape[0] * (-(-x_q.shape[1] // 128)):
         raise NotImplementedError("the input scale must hold one value per row and 128 columns")
-    if input_scale.dim() != 2 or input_scale.shape[0] != x_q.shape[0]:  # (a view of the same shape is 0.7 us)
+    # (a view of the same shape is 0.7 us; one of no rows has no second extent, and is refused)
+    if input_scale.dim() != 2 or input_scale.shape[0] != x_q.shape[0] or input_scale.numel() == 0:
         input_scale = input_scale.view(x_q.shape[0], -1)
     if eager(x_q):
         out = _C.block_matmul(x_q, weight, input_scale, weight_scale, torch.bfloat16, bias)

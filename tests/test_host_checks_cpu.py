@@ -67,3 +67,12 @@ def test_moe_kernel_configuration_without_a_block_height(monkeypatch):
     with pytest.raises(RuntimeError, match="block_m must be positive"):
         module.invoke_fused_moe_kernel(torch.zeros(4, 128, dtype=torch.bfloat16), b, c, b_scale, None, ids, expert, post,
                                        False, 1, {"BLOCK_SIZE_M": 0}, [128, 128])
+
+
+@pytest.mark.parametrize("shape", [(0, 2), (0,), (0, 0), (0, 5)])
+def test_prequantised_linear_refuses_scales_of_no_rows(shape):
+    from sglang_amd.quantization.fp8_utils import aiter_w8a8_block_fp8_linear
+
+    q, w = (torch.zeros(rows, 256).to(torch.float8_e4m3fn) for rows in (0, 256))
+    with pytest.raises(RuntimeError, match="reshape tensor of 0 elements"):
+        aiter_w8a8_block_fp8_linear(q, w, [128, 128], torch.ones(2, 2), input_scale=torch.empty(shape))
