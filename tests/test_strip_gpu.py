@@ -1,4 +1,4 @@
-"""Dense GEMMs of 17 to 1024 rows off the tile kernels: the strip kernel (weights in tiles of 16 to 160 rows, loading and multiplying
+"""Dense GEMMs of 17 to 1024 rows off the tile kernels: the strip kernel (weights in tiles of 32 to 160 rows, loading and multiplying
 waves) and the streaming kernel walking several row tiles, at the edges of their tiles, against the oracle."""
 import numpy as np
 import pytest
@@ -125,8 +125,8 @@ def test_few_k_blocks_and_many_tiles(dev, mode, M, N, K, strips):
     _check(out, ref, f"short K {mode} M={M} N={N} K={K}")
 
 
-@pytest.mark.parametrize("mode", ["row_fp8", "row_int8"])
-@pytest.mark.parametrize("M,N,K", [(65, 28681, 4096), (100, 9000, 9600)])
+@pytest.mark.parametrize("mode", MODES)  # (the block modes without a bias: tests/test_block_bias_gpu.py)
+@pytest.mark.parametrize("M,N,K", [(65, 28681, 4096), (100, 9000, 9600), (30, 40009, 2560)])
 def test_strip_kernel_half_and_bias(dev, mode, M, N, K):
     from sglang_amd._lib import lib
 
@@ -207,7 +207,7 @@ def test_row_tiles_of_16(dev, mode, M, N, K):
     from sglang_amd._lib import lib
 
     out, ref = _run(dev, mode, M, N, K, torch.bfloat16, False, 0, col_scales=False)
-    assert lib.sglamd_last_gemm_kernel() == 1 and lib.sglamd_last_streaming_shape() >> 16 == 1
+    assert lib.sglamd_last_gemm_kernel() == 1 and lib.sglamd_last_streaming_shape() >> 16 == 1 and not lib.sglamd_last_strip_shape()
     _check(out, ref, f"row tiles of 16 {mode} M={M} N={N} K={K}")
 
 

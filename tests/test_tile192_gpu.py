@@ -28,3 +28,14 @@ def test_tiles_of_192_rows(dev, mode, M, N, K, pitch):
     out, ref = _run(dev, mode, M, N, K, torch.bfloat16, False, pitch, col_scales=M % 2 == 0)
     assert lib.sglamd_last_gemm_kernel() == TILE192, f"kernel {lib.sglamd_last_gemm_kernel()}"
     _check(out, ref, f"192-row tiles {mode} M={M} N={N} K={K}")
+
+
+@pytest.mark.parametrize("mode", MODES)  # (a bias with block scales: tests/test_block_bias_gpu.py)
+@pytest.mark.parametrize("M,N,K", [(300, 24577, 1280), (383, 7172, 12288)])
+def test_tiles_of_192_rows_half_and_bias(dev, mode, M, N, K):
+    from sglang_amd._lib import lib
+
+    print(f"192-row tiles, half, {mode} M={M} N={N} K={K}", flush=True)
+    out, ref = _run(dev, mode, M, N, K, torch.float16, True, 0, False)
+    assert lib.sglamd_last_gemm_kernel() == TILE192, f"kernel {lib.sglamd_last_gemm_kernel()}"
+    _check(out, ref, f"192-row tiles {mode} M={M} N={N} K={K} half, bias")
