@@ -814,8 +814,13 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, int pe
     const int slices = gemm8_big_slices(tiles, N, K);
     const int64_t rounds = (tiles * slices + cus - 1) / cus;
     // (64-row tiles in several rounds read each weight byte once per row tile from further away: gate_up at M = 400, four rounds of
-    // them, 176 us, 158 in 128-row tiles, 138 in 256-row tiles)
-    const double weight = bm == 64 ? (rounds > 1 ? 2.0 : 1.6) : bm == 128 ? 1.2 : bm == 192 ? (M <= bm ? 1.0 : slices > 3 ? 1.12 : 1.06) : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
+    // them, 176 us, 158 in 128-row tiles, 138 in 256-row tiles).  Less so where a tile has four to eight K blocks, and neither 192-row tiles nor the
+    // persistent kernel are there: four rounds of them against three of 128-row tiles take 0.86 to 0.98 of the time (420 x 33280 x 896 32.3
+    // and 35.5 us, 1466 x 10816 x 768 34.1 and 37.0; 77 launches of up to 33 row tiles).  Not with one row tile more than the
+    // groups of eight that walk a column of weights together (1038 x 14976 x 896 43.3 and 40.8, 545 x 28480 x 512 32.1 and 29.3, 2090 x 7808 x 768
+    // 43.4 and 40.2; 1036 x 14848 x 512 is 31.2 and 33.3), nor below K = 512 (384: 0.95 to 0.98 with row scales, 1.02 with blocks)
+    const bool few_blocks = !persistent_256 && K >= 512 && K < 1152 && ((M + 63) / 64 & 7) != 1;
+    const double weight = bm == 64 ? (rounds == 1 ? 1.6 : few_blocks ? 1.78 : 2.0) : bm == 128 ? 1.2 : bm == 192 ? (M <= bm ? 1.0 : slices > 3 ? 1.12 : 1.06) : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
     // a single row of tiles only loads the rows that exist: M = 192 in 256-row tiles costs what 192 rows cost
     // (gate_up at M = 192: 89.6 us in 256-row tiles against 102.5 in 64-row tiles, which need two rounds)
     const double rows = M <= bm ? (double)((M + 63) / 64 * 64) : (double)bm;

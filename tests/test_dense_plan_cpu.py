@@ -112,3 +112,19 @@ def test_scratch_is_asked_for_where_it_is_used():
 def test_tile_heights_at_129_to_192_rows(M, N, K, rows, block):
     form, plan = _plan(M, N, K, block)
     assert form == TILES and plan[0] == rows
+
+
+@pytest.mark.parametrize("M,N,K,rows", [
+    # four rounds of 64-row tiles or three of 128 (us)
+    (420, 33280, 896, 64),     # 32.1, 35.2
+    (448, 33792, 640, 64),     # 28.2, 30.6
+    (1466, 10816, 768, 64),    # 33.8, 36.8
+    (545, 28480, 512, 128),    # 32.1, 29.3
+    (1038, 14976, 896, 128),   # 43.3, 40.8
+    (2090, 7808, 768, 128),    # 43.4, 40.2
+    (315, 25024, 768, 256),    # 21.2, - (256-row tiles 19.8)
+    (420, 33280, 384, 128),    # 24.6, 24.0
+])
+def test_tile_heights_of_a_short_k(M, N, K, rows):
+    form, plan = _plan(M, N, K, block=False)
+    assert form == TILES and plan[0] == rows
