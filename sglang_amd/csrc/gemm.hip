@@ -100,10 +100,10 @@ extern "C" int sglamd_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, c
                    scales_pow2 != 0, bias);
 }
 
-// Linear layers of up to this many rows may quantise them in the GEMM's own workgroups (0: none).
+// Linear layers of up to this many rows may quantise them in the GEMM's own workgroups (0: none).  The kernel holds one tile of 16.
 static int quantising_max_rows() {
   static const int v = getenv("SGLAMD_LINEAR_FUSE_ROWS") ? atoi(getenv("SGLAMD_LINEAR_FUSE_ROWS")) : 16;  // tuning knob
-  return v;
+  return v < 16 ? v : 16;
 }
 // Which of them do.  A launch less saves 1-2 us; every workgroup quantising every row costs it time that grows with M * K
 // and delays its weight stream.  Two launches -> one, us, weights from HBM, queue kept full, block scales (row scales):

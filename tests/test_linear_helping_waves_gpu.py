@@ -36,3 +36,31 @@ def test_equals_quantise_then_multiply(dev, M, N, K, row_scales, dtype, bias):
             ref = ref + b if bias else ref
         assert torch.equal(out.isnan(), ref.isnan())
         assert torch.equal(out.nan_to_num(), ref.nan_to_num())
+
+
+MORE_ROWS = """
+import torch
+from sglang_amd.quantization.fp8_kernel import sglang_per_token_group_quant_fp8, w8a8_block_fp8_matmul
+from sglang_amd.quantization.fp8_utils import dispatch_w8a8_block_fp8_linear
+g = torch.Generator(device="cuda").manual_seed(1)
+for M in (16, 17, 32):
+    x = torch.randn(M, 512, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(1024, 512, generator=g, device="cuda").mul_(100).clamp_(-448, 448).to(torch.float8_e4m3fn)
+    ws = torch.rand(8, 4, generator=g, device="cuda") * 1e-3 + 1e-4
+    print("rows", M, flush=True)
+    out = dispatch_w8a8_block_fp8_linear()(x, w, [128, 128], ws)
+    q, s = sglang_per_token_group_quant_fp8(x, 128, column_major_scales=True)
+    assert torch.equal(out, w8a8_block_fp8_matmul(q, w, s, ws, [128, 128], output_dtype=torch.bfloat16)), M
+"""
+
+
+def test_a_limit_past_the_tile_is_the_tile(dev):
+    """SGLAMD_LINEAR_FUSE_ROWS above the sixteen rows that a workgroup holds (read once per process)."""
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", MORE_ROWS], env=dict(os.environ, SGLAMD_LINEAR_FUSE_ROWS="64"), cwd=root, timeout=100,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
