@@ -797,9 +797,11 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, int pe
   for (int bm = 64; bm <= 256; bm += 64) {
     if (bm > 128 && M <= 128) break;
     if (bm == 192 && !tall) continue;
-    // up to 192 rows one of the two: gate_up at 150 rows 79 us in 192-row tiles, 86 in 256-row tiles, 7168 x 18432 52.7 and 53.4, but 8192 x
-    // 28672 79.4 and 76.5.  A K too short for 192 rows: 256-row tiles unless 128-row tiles fit one round (192 x 65536 x 1024 in 256-, 128-row
-    // tiles 24.7, 32.0 us, 160 x 57344 x 896 21.0, 24.8, 150 x 33792 x 640 15.3, in 64-row tiles 16.0; 140 x 30720 x 640 15.1, 13.2)
+    // Up to 192 rows one of the two: gate_up at 150 rows 79 us in 192-row tiles, 86 in 256-row tiles, 7168 x 18432 52.7 and 53.4, but 8192 x
+    // 28672 79.4 and 76.5.  The line is not a sharp one: of 96 launches at K = 12288 to 28672 192 rows take 0.92 to 1.06 of 256 (block
+    // scales 0.98 in the mean up to K = 24576 and 1.01 at 28672, row scales 1.00).  A K too short for 192 rows: 256-row tiles unless 128-row
+    // tiles fit one round (192 x 65536 x 1024 in 256- and 128-row tiles 24.7 and 32.0 us, 160 x 57344 x 896 21.0 and 24.8, 150 x 33792 x 640
+    // 15.3, in 64-row tiles 16.0; but 140 x 30720 x 640 15.1 and 13.2).
     if (M <= 192 && (tall ? bm == (K < 20480 ? 256 : 192) : bm == 256 && 2 * whole <= cus)) continue;
     const int64_t tiles = ((M + bm - 1) / bm) * ((N + 255) / 256);
     // 192 rows, between the heights that leave many rows or CUs idle: 8192 x 28672 at 560 / 640 rows 198 / 219 -> 159 / 158 us, 7168 x
@@ -814,11 +816,11 @@ static inline BigConfig gemm8_big_config(int64_t M, int64_t N, int64_t K, int pe
     const int slices = gemm8_big_slices(tiles, N, K);
     const int64_t rounds = (tiles * slices + cus - 1) / cus;
     // (64-row tiles in several rounds read each weight byte once per row tile from further away: gate_up at M = 400, four rounds of
-    // them, 176 us, 158 in 128-row tiles, 138 in 256-row tiles).  Less so where a tile has four to eight K blocks, and neither 192-row tiles nor the
-    // persistent kernel are there: four rounds of them against three of 128-row tiles take 0.86 to 0.98 of the time (420 x 33280 x 896 32.3
-    // and 35.5 us, 1466 x 10816 x 768 34.1 and 37.0; 77 launches of up to 33 row tiles).  Not with one row tile more than the
-    // groups of eight that walk a column of weights together (1038 x 14976 x 896 43.3 and 40.8, 545 x 28480 x 512 32.1 and 29.3, 2090 x 7808 x 768
-    // 43.4 and 40.2; 1036 x 14848 x 512 is 31.2 and 33.3), nor below K = 512 (384: 0.95 to 0.98 with row scales, 1.02 with blocks)
+    // them, 176 us, 158 in 128-row tiles, 138 in 256-row tiles.  Less so where a tile has four to eight K blocks and neither 192-row tiles
+    // nor the persistent kernel are there: four rounds of them against three of 128-row tiles take 0.86 to 0.98 of the time, 420 x 33280
+    // x 896 32.3 and 35.5 us, 1466 x 10816 x 768 34.1 and 37.0, in 77 launches of up to 33 row tiles.  Not with one row tile more than the
+    // groups of eight that walk a column of weights together (1038 x 14976 x 896 43.3 and 40.8, 545 x 28480 x 512 32.1 and 29.3, 2090 x 7808
+    // x 768 43.4 and 40.2; 1036 x 14848 x 512 is 31.2 and 33.3), nor below K = 512 (384: 0.95 to 0.98 with row scales, 1.02 with blocks).)
     const bool few_blocks = !persistent_256 && K >= 512 && K < 1152 && ((M + 63) / 64 & 7) != 1;
     const double weight = bm == 64 ? (rounds == 1 ? 1.6 : few_blocks ? 1.78 : 2.0) : bm == 128 ? 1.2 : bm == 192 ? (M <= bm ? 1.0 : slices > 3 ? 1.12 : 1.06) : (persistent_256 && tiles > cus) ? 0.88 : 1.0;
     // a single row of tiles only loads the rows that exist: M = 192 in 256-row tiles costs what 192 rows cost

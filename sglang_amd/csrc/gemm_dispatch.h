@@ -22,8 +22,8 @@ static int tile_min_m() {
   return v;
 }
 
-// 33 to 64 rows: the tile kernel (64-row tile, K split over the chip) or the streaming kernel?  Up to 32 rows the
-// streaming kernel is the faster one on every weight measured (DeepSeek-V3 gate_up / down / q_b / o_proj at 17 rows:
+// 33 to 64 rows: the tile kernel (64-row tile, K split over the chip) or the streaming kernel, where dense_choice below has nothing
+// faster?  Up to 32 rows the streaming kernel is the faster of these two on every weight measured (past 100 MB strips are: dense_choice; DeepSeek-V3 gate_up / down / q_b / o_proj at 17 rows:
 // 54.5 / 26.1 / 12.1 / 22.8 us against 60.0 / 31.7 / 16.9 / 28.8 in 64-row tiles; at 32 rows 63.9 / 30.4 / 13.9 / 25.6
 // against 61.6 / 32.6 / 17.3 / 30.0; Llama-3-70B o / gate_up / down at 24 rows 15.0 / 86.6 / 43.2 against 19.3 / 104.5 /
 // 50.6).  Its four-tile form for 33..64 rows re-reads the activations too often for large weights (gate_up at 48

@@ -1096,8 +1096,8 @@ static int gemm8_skinny_quantising(const GemmArgs& g0, hipStream_t st, bool laun
   return gemm8_skinny_launch_fn<1, 1, MODE, OT, false, 1>(g, st, 1);
 }
 
-// Wide form for 33..64 activation rows on weights with many rows, where the strip kernel (51 -> 44 us on DeepSeek-V3 gate_up at 64
-// rows) would split K and the caller has given no scratch for it: four row tiles times FN = 6, 8 or 9 column tiles
+// Wide form for 33..64 activation rows on weights with many rows, where the strip kernel (kernel alone 51 -> 46 us on DeepSeek-V3 gate_up at
+// 64 rows) does not take the call: block scales with a K that does not fill its last block, or K split and no scratch for it.  Four row tiles times FN = 6, 8 or 9 column tiles
 // (96..144 weight rows) per workgroup, four waves that share K block by block, one ring slot per wave (the four
 // slots and what is in flight to them fill most of LDS).  Per K block a workgroup then fetches 8 KB of activation
 // rows for 12..18 KB of weight rows, where the two-column-tile form fetches 8 KB for 4 KB; the tile count is made a
