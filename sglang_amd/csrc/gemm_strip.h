@@ -11,11 +11,12 @@
 //   * one barrier a K block: by then every fragment of the block is in registers and the next block has landed;
 //   * tiles of any multiple of 16 weight rows, so that the items fill the chip: 36864 weight rows are 256 tiles of 144 where
 //     the tile kernel has 144 tiles of 256 for 256 CUs.
-// Kernel alone under the tracer, us, tile kernel (64 rows: wide streaming form) -> this, cold weights: 36864 x 7168 at 64 / 96 / 128
-// rows 51 / 66 / 69 -> 46 / 49 / 56 (in a graph, weights in turn: 44 / - / 55 to 59 with the clock; with the quantiser in front 47 / 52 / 57); 57344 x 8192 at 128
-// rows 113 -> 100.  At 128 rows the loaders alone, without a product, need 46: the rest is the clock (1.75 to 1.9 GHz under load) and the fragment reads.  Not faster, and not kept: the loads spread over the
-// multiplying waves (61 at 128 rows), two waves to a strip with half of the rows each (69), four stages instead of three, a
-// fragment copy per row tile (spills), weight rows at another pitch (only multiples of 4096 bytes matter, see `rotate`).
+// Kernel alone under the tracer, us, tile kernel (64 rows: wide streaming form) -> this, cold weights: 36864 x 7168 at 64 / 96 / 128 rows
+// 51 / 66 / 69 -> 46 / 49 / 56 (in a graph, weights in turn: 44 / - / 55 to 59 with the clock; with the quantiser in front 47 / 52 / 57);
+// 57344 x 8192 at 128 rows 113 -> 100.  At 128 rows the loaders alone, without a product, need 46: the rest is the clock (1.75 to 1.9 GHz
+// under load) and the fragment reads.  Not faster, and not kept: the loads spread over the multiplying waves (61 at 128 rows), two waves
+// to a strip with half of the rows each (69), four stages instead of three, a fragment copy per row tile (spills), weight rows at another
+// pitch (only multiples of 4096 bytes matter, see `rotate`).
 #pragma once
 #include "gemm_big.h"
 
